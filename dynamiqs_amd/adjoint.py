@@ -270,7 +270,7 @@ class AdjointPlan:
         ]
         t0 = time.perf_counter()
         self.fwd = dense.build_plan('tsit5', fwd_insts, fwd_ts, exp_ops=[Ok for _, Ok in losses], rtol=rtol,
-                                    atol=atol)
+                                    atol=atol, dia_ops=True)
         t1 = time.perf_counter()
 
         # Gauss-Legendre nodes per segment
@@ -292,7 +292,7 @@ class AdjointPlan:
                                    mod=fmods, tsave=node_t[k0 * nodes : k1 * nodes], t0=float(times[k0]), key_H=(),
                                    key_L=(), key_rho=())
                 )
-        self.rec = dense.build_plan('tsit5', rec_insts, rec_insts[0].tsave, rtol=rtol, atol=atol)
+        self.rec = dense.build_plan('tsit5', rec_insts, rec_insts[0].tsave, rtol=rtol, atol=atol, dia_ops=True)
         t2 = time.perf_counter()
 
         # backward adjoint in reversed time s = T - t: Hnh' = iH - 1/2 sum L^dag L,
@@ -315,7 +315,7 @@ class AdjointPlan:
         # lambda starts at O_k: the absolute tolerance scales with |O| so that the
         # backward solve keeps the forward's relative accuracy (|rho| <= 1)
         atol_b = atol * max(1.0, max(float(np.linalg.norm(Ok, 2)) for _, Ok in losses))
-        self.bwd = dense.build_plan('tsit5', bwd_insts, bwd_ts, rtol=rtol, atol=atol_b)
+        self.bwd = dense.build_plan('tsit5', bwd_insts, bwd_ts, rtol=rtol, atol=atol_b, dia_ops=True)
         # node q (in t order) takes the loss terms whose time is after it
         self.loss_mask = np.array([[node_t[q] < tk for q in range(self.Q)] for tk, _ in losses])
         self.node_t = node_t

@@ -1,0 +1,675 @@
+// Adaptive Tsit5 / Dopri5 for small master equations whose operators have few nonzero
+// diagonals (gfx950), n <= 64: one workgroup per instance.
+//
+// The vector field G rho + rho G^dag + sum_k L_k rho L_k^dag of such operators is a
+// stencil, f[i][j] = sum_t C_t(i, j) rho[i + a_t][j + b_t]: one shift (o, 0) and one
+// (0, o) per off-diagonal o of G, one (p, q) per pair of diagonals of a jump operator,
+// equal shifts merged. A driven oscillator has 5 shifts and a driven Kerr oscillator
+// with two-photon loss 6, against (1 + 2K) n multiply-adds per element of the dense
+// products, so the matrix cores have nothing to do here and a step is bound by the
+// latency of its dependent stages (n <= 32) and by FP64 issue and LDS reads (n = 64).
+//
+// A thread owns NE elements of the upper triangle (u = thread + NTH q, row by row, of
+// the n (n + 1) / 2 that exist: no work on padding). Its coefficients C_t, the FP64
+// diagonal generator g = d_i + conj(d_j), the FP64 state, the candidate and the seven
+// FP32 stages stay in registers for the whole solve. The stage input goes to LDS in
+// FP32 (both triangles), the neighbours come back with one 8-byte read per shift, and
+// the FP64 diagonal term takes the thread's own input unrounded. Two LDS copies
+// alternate, so a stage costs one barrier, and the stages are unrolled with the
+// tableau's weights in scalar registers. Measured against the resident dense body:
+// oscillator n = 16, 85 steps and 101 saves 1.20 -> 0.297 ms; 128 driven Kerr oscillators
+// n = 64 (2 jump operators, about 440 steps) 57.4 -> 7.28 ms; the three solves of a
+// gradient at n = 32, 64 control vectors, 6.4 -> 1.7 ms. The controller, step clipping, FSAL, saving and the
+// precision of the operators and stages are those of the dense kernels.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "dqh.h"
+#include "dqh_common.h"
+#include "dqh_mfma.h"
+#include "dqh_tsit5_tableau.h"
+
+namespace dqh {
+namespace diag {
+
+constexpr int kMaxShift = 12;  // shifts of the stencil (register coefficients per element)
+constexpr int kMaxPart = 48;   // contributions to the shifts' coefficients
+
+// A contribution to a coefficient: kind 0 G_x[i] (row diagonal x of the generator),
+// kind 1 conj(G_x[j]), kind 2 L_x[i] conj(L_y[j]) (x, y: rows of the jump-operator table).
+struct Part {
+  uint8_t kind, x, y, pad;
+};
+
+struct Pattern {
+  int32_t nterm, nH, nLrow, nzero;  // shifts, off-diagonals of G, jump-operator rows, parts of shift (0, 0)
+  int32_t guard;                    // largest |a LD + b|
+  int32_t a[kMaxShift], b[kMaxShift];
+  int32_t first[kMaxShift + 1];  // parts of shift t: part[first[t]] .. part[first[t + 1] - 1]
+  Part part[kMaxPart];
+  Part zero[kMaxPart];
+};
+
+// x + (x of the lane that the DPP control names)
+template <int CTRL>
+__device__ __forceinline__ double dpp_sum(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return x + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double lane_of(double x, int lane) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// sum over the wave, the same value in every lane: butterfly over quads, half rows and
+// rows of 16 lanes on the VALU, then the four rows through scalar registers
+__device__ __forceinline__ double wave_sum(double x) {
+  x = dpp_sum<0xB1>(x);   // lane ^ 1
+  x = dpp_sum<0x4E>(x);   // lane ^ 2
+  x = dpp_sum<0x141>(x);  // the other quad of the half row
+  x = dpp_sum<0x140>(x);  // the other half of the row
+  return (lane_of(x, 0) + lane_of(x, 16)) + (lane_of(x, 32) + lane_of(x, 48));
+}
+
+// workgroup sums of N values with one barrier; red alternates between two halves, so a
+// second call need not wait for the readers of the first
+template <int NTH, int N>
+__device__ __forceinline__ void block_sums(double (&x)[N], double *red, int &par) {
+  constexpr int NW = NTH / 64;
+#pragma unroll
+  for (int k = 0; k < N; ++k) x[k] = wave_sum(x[k]);
+  double *r = red + par * (NW * 2);
+  par ^= 1;
+  if constexpr (NW > 1) {
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) r[2 * (threadIdx.x >> 6) + k] = x[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s += r[2 * w + k];
+      x[k] = s;
+    }
+  }
+}
+
+// LDS: two copies of the stage input (rows of LD = n | 1 float2, one slot that elements
+// past the end write, a guard of G zeros before, between and after them so that a shift
+// may leave the matrix: its coefficient is zero there), the generator's off-diagonals and
+// the jump operators' rows (n each), its diagonal (FP64), partial sums.
+__host__ __device__ inline int row_stride(int n) { return n | 1; }
+__host__ __device__ inline int copy_stride(int n, int guard) { return n * row_stride(n) + 1 + guard; }
+template <int NTH>
+__host__ __device__ inline size_t lds_bytes(int n, int nH, int nLrow, int guard) {
+  return (size_t)(2 * copy_stride(n, guard) + guard + (nH + nLrow) * n) * sizeof(float2) +
+         (size_t)n * sizeof(double2) + (size_t)(4 * (NTH / 64)) * sizeof(double);
+}
+
+// the tableau through a scalar pointer that the optimiser cannot see through: its loads
+// stay where they are used (as literals, or hoisted out of the loop, the weights would
+// fill the registers that the stages need)
+typedef const __attribute__((address_space(4))) RKTab CTab;
+template <int TAB>
+__device__ __forceinline__ CTab *weights() {
+  CTab *r = (CTab *)&kRK[TAB];
+  asm volatile("" : "+s"(r));
+  return r;
+}
+
+template <int NTH, int NE, int T, int TAB>
+__global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restrict__ insts, Pattern pat) {
+  extern __shared__ __align__(16) char smem[];
+  const dqh_me_inst &p = insts[blockIdx.x];
+  constexpr RKTab rk = kRKTabs[TAB];
+  const int n = (int)p.n, np = (int)p.np, nE = (int)p.nE, ntsave = (int)p.ntsave, nseg = (int)p.nseg;
+  const int LD = row_stride(n), tid = (int)threadIdx.x;
+  const int npwc = (int)p.npwc;
+  const bool pwc = npwc > 0;
+  double2 *dcur = reinterpret_cast<double2 *>(smem);  // n: diagonal of the current generator
+  double *red = reinterpret_cast<double *>(dcur + n);  // 4 NW
+  const int CS = copy_stride(n, pat.guard);
+  float2 *ysA = reinterpret_cast<float2 *>(red + 4 * (NTH / 64)) + pat.guard;
+  float2 *Gt = ysA + 2 * CS;        // nH x n: G[i][i + o] of the current generator
+  float2 *Lt = Gt + pat.nH * n;     // nLrow x n: L[i][i + p]
+  int64_t *stats = gp<int64_t>(p.stats);
+  if (n > 64 || n * (n + 1) / 2 > NTH * NE || p.nmod != 0 || (pwc && nseg < 2) ||
+      (p.flags & (DQH_FLAG_GLOBAL | DQH_FLAG_LMOD | DQH_FLAG_DOPRI8 | DQH_FLAG_EULER)) ||
+      ((p.flags & DQH_FLAG_DOPRI5) != 0) != (TAB == 1)) {
+    if (tid == 0) stats[3] = DQH_UNSUPPORTED;
+    return;
+  }
+  const double *tsave = gp<const double>(p.tsave);
+  const double *ptimes = gp<const double>(p.pwc_times);
+  const double rtol = p.rtol, atol = p.atol, t_end = p.t1;
+  const double inv_nn = 1.0 / ((double)n * n);
+  const bool save_states = (p.flags & DQH_FLAG_SAVE_STATES) != 0;
+
+  // owned elements; at / am: slots of the element and of its mirror image in a copy (the
+  // spare slot past the end)
+  const int NU = n * (n + 1) / 2;
+  int ei[NE], ej[NE], at[NE], am[NE];
+  double wt[NE];  // weight in a sum over the full matrix
+#pragma unroll
+  for (int q = 0; q < NE; ++q) {
+    int rem = tid + NTH * q, i = 0;
+    ei[q] = -1;
+    ej[q] = 0;
+    at[q] = am[q] = n * LD;
+    wt[q] = 0.0;
+    if (rem < NU) {
+      while (rem >= n - i) {
+        rem -= n - i;
+        ++i;
+      }
+      ei[q] = i;
+      ej[q] = i + rem;
+      at[q] = i * LD + i + rem;
+      am[q] = (i + rem) * LD + i;
+      wt[q] = rem == 0 ? 1.0 : 2.0;
+    }
+  }
+  for (int e = tid; e < 2 * CS + pat.guard; e += NTH) (ysA - pat.guard)[e] = make_float2(0.f, 0.f);
+  for (int e = tid; e < pat.nLrow * n; e += NTH) {
+    const int r = e / n, i = e - r * n;
+    Lt[e] = gp<const float2>(p.Dops)[(size_t)r * np + i];
+  }
+
+  // Gt, dcur <- the constant generator plus the PWC terms of segment seg
+  const float2 *G0 = gp<const float2>(p.Hnh);
+  const double2 *d0g = gp<const double2>(p.hdiag);
+  const float2 *Hp = gp<const float2>(p.Hpwc);
+  const double *vals = gp<const double>(p.pwc_vals);
+  float cr[T][NE], ci[T][NE];
+  double gr[NE], gi[NE];
+  auto build = [&](int seg) {
+    const int nv = nseg - 1;
+    const bool inside = pwc && seg >= 0 && seg < nv;
+    for (int e = tid; e < (pat.nH + 1) * n; e += NTH) {
+      const int r = e / n, i = e - r * n;
+      double re, im;
+      if (r < pat.nH) {
+        const float2 o = G0[(size_t)r * np + i];
+        re = o.x;
+        im = o.y;
+      } else {
+        re = d0g[i].x;
+        im = d0g[i].y;
+      }
+      if (inside) {
+        for (int j = 0; j < npwc; ++j) {
+          const double vr = vals[2 * (j * nv + seg)], vi = vals[2 * (j * nv + seg) + 1];
+          const float2 o = Hp[((size_t)j * (pat.nH + 1) + r) * np + i];
+          re += vr * o.x - vi * o.y;
+          im += vr * o.y + vi * o.x;
+        }
+      }
+      if (r < pat.nH)
+        Gt[e] = make_float2((float)re, (float)im);
+      else
+        dcur[i] = make_double2(re, im);
+    }
+    __syncthreads();
+    int z = 0;  // keeps the pattern's scalar loads here
+    asm volatile("" : "+s"(z));
+    auto coef = [&](const Part &s, int i, int j) -> float2 {
+      if (s.kind == 0) return Gt[s.x * n + i];
+      if (s.kind == 1) {
+        const float2 c = Gt[s.x * n + j];
+        return make_float2(c.x, -c.y);
+      }
+      const float2 a = Lt[s.x * n + i], c = Lt[s.y * n + j];
+      return make_float2(a.x * c.x + a.y * c.y, a.y * c.x - a.x * c.y);
+    };
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const bool on = ei[q] >= 0;
+      const int i = on ? ei[q] : 0, j = ej[q];
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        float ar = 0.f, ai = 0.f;
+        for (int s = pat.first[t + z]; s < pat.first[t + 1 + z]; ++s) {
+          const float2 c = coef(pat.part[s], i, j);
+          ar += c.x;
+          ai += c.y;
+        }
+        cr[t][q] = on ? ar : 0.f;
+        ci[t][q] = on ? ai : 0.f;
+      }
+      const double2 da = dcur[i], db = dcur[j];
+      double r = da.x + db.x, m = da.y - db.y;
+      for (int s = z; s < pat.nzero; ++s) {
+        // products of the jump operators' main diagonals, in FP64
+        const float2 a = Lt[pat.zero[s].x * n + i], c = Lt[pat.zero[s].y * n + j];
+        r += (double)a.x * c.x + (double)a.y * c.y;
+        m += (double)a.y * c.x - (double)a.x * c.y;
+      }
+      gr[q] = on ? r : 0.0;
+      gi[q] = on ? m : 0.0;
+    }
+  };
+
+  // state
+  double2 y[NE], y1[NE];
+  float2 k[7][NE];
+  {
+    const double2 *y0 = gp<const double2>(p.y);
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      y[q] = ei[q] >= 0 ? y0[(size_t)ei[q] * np + ej[q]] : make_double2(0.0, 0.0);
+      if (ei[q] == ej[q]) y[q].y = 0.0;
+      y1[q] = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int s = 0; s < 7; ++s) k[s][q] = make_float2(0.f, 0.f);
+    }
+  }
+  int cur = 0;  // LDS copy of the next stage input
+  int sh[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) sh[t] = t < pat.nterm ? pat.a[t] * LD + pat.b[t] : 0;
+
+  // out = f(v): v (FP64) to LDS in FP32 on both triangles, one barrier, the stencil in
+  // FP32 and the diagonal term in FP64
+  auto field = [&](const double2 (&v)[NE], float2 (&out)[NE]) {
+    float2 *b = ysA + cur * CS;
+    cur ^= 1;
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const float2 x = make_float2((float)v[q].x, (float)v[q].y);
+      b[am[q]] = make_float2(x.x, -x.y);
+      b[at[q]] = x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      int e = at[q];
+      if constexpr (NE > 1) asm volatile("" : "+v"(e));  // the T addresses are formed here, not kept
+      float2 x[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t) x[t] = b[e + sh[t]];
+      float fr = 0.f, fi = 0.f;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        fr = fmaf(cr[t][q], x[t].x, fmaf(-ci[t][q], x[t].y, fr));
+        fi = fmaf(cr[t][q], x[t].y, fmaf(ci[t][q], x[t].x, fi));
+      }
+      const double re = (double)fr + (gr[q] * v[q].x - gi[q] * v[q].y);
+      const double im = (double)fi + (gr[q] * v[q].y + gi[q] * v[q].x);
+      // the diagonal of a Hermitian field is real
+      out[q] = make_float2((float)re, ei[q] == ej[q] ? 0.f : (float)im);
+    }
+  };
+
+  // the FP64 conversions of the stages are made anew in every combination: kept from one
+  // to the next (as common subexpressions) they would not fit the registers
+  auto pin_stages = [&](int m) {
+#pragma unroll
+    for (int j = 0; j < 7; ++j) {
+      if (j < m) {
+#pragma unroll
+        for (int q = 0; q < NE; ++q) asm volatile("" : "+v"(k[j][q].x), "+v"(k[j][q].y));
+      }
+    }
+  };
+
+  int par = 0;
+  // y + h sum_j w_j k_j at save index isave: states on both triangles, Tr(E rho) over the
+  // owned elements and their mirror images
+  auto save = [&](double h, const double (&w)[7], int isave) {
+    float2 *st = gp<float2>(p.states) + (size_t)isave * n * n;
+    double vr[NE], vi[NE];
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      double re = 0.0, im = 0.0;
+#pragma unroll
+      for (int j = 0; j < 7; ++j) {
+        re += w[j] * (double)k[j][q].x;
+        im += w[j] * (double)k[j][q].y;
+      }
+      vr[q] = y[q].x + h * re;
+      vi[q] = y[q].y + h * im;
+      if (save_states && ei[q] >= 0) {
+        st[(size_t)ei[q] * n + ej[q]] = make_float2((float)vr[q], (float)vi[q]);
+        if (ei[q] != ej[q]) st[(size_t)ej[q] * n + ei[q]] = make_float2((float)vr[q], (float)-vi[q]);
+      }
+    }
+    const float2 *ET = gp<const float2>(p.EopsT);
+    for (int e = 0; e < nE; ++e) {
+      const float2 *E = ET + (size_t)e * np * np;
+      double s[2] = {0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < NE; ++q) {
+        if (ei[q] >= 0) {
+          const float2 o = E[(size_t)ei[q] * np + ej[q]];
+          s[0] += o.x * vr[q] - o.y * vi[q];
+          s[1] += o.x * vi[q] + o.y * vr[q];
+          if (ei[q] != ej[q]) {
+            const float2 m = E[(size_t)ej[q] * np + ei[q]];
+            s[0] += m.x * vr[q] + m.y * vi[q];
+            s[1] += m.y * vr[q] - m.x * vi[q];
+          }
+        }
+      }
+      block_sums<NTH>(s, red, par);
+      if (tid == 0) gp<float2>(p.expects)[(size_t)e * ntsave + isave] = make_float2((float)s[0], (float)s[1]);
+    }
+  };
+  const double w0[7] = {0, 0, 0, 0, 0, 0, 0};
+
+  double t = p.t0;
+  int isave = 0, status = 0;
+  int64_t nsteps = 0, nacc = 0, nrej = 0, nrhs = 0;
+  double next_save = ntsave > 0 ? tsave[0] : 0.0;
+  auto advance = [&]() {
+    ++isave;
+    if (isave < ntsave) next_save = tsave[isave];
+  };
+  // segment of t (searchsorted right, -1 before the first breakpoint) and the breakpoint
+  // after it; t only grows, so both move forward
+  int seg = -1;
+  double next_break = pwc ? ptimes[0] : 0.0;
+  auto locate = [&]() {
+    bool moved = false;
+    while (seg + 1 < nseg && next_break <= t) {
+      ++seg;
+      moved = true;
+      if (seg + 1 < nseg) next_break = ptimes[seg + 1];
+    }
+    return moved;
+  };
+  if (pwc) locate();
+  __syncthreads();  // the LDS tables and the zeroed copies
+  build(seg);
+  while (isave < ntsave && next_save <= t) {
+    save(0.0, w0, isave);
+    advance();
+  }
+  field(y, k[0]);
+  ++nrhs;
+
+  // initial step (Hairer-Norsett-Wanner II.4), scale atol + rtol |y0|
+  double dt;
+  {
+    double s[2] = {0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const double ay2 = y[q].x * y[q].x + y[q].y * y[q].y;
+      const double sc = atol + rtol * sqrt(ay2);
+      s[0] += wt[q] * ay2 / (sc * sc);
+      s[1] += wt[q] * ((double)k[0][q].x * k[0][q].x + (double)k[0][q].y * k[0][q].y) / (sc * sc);
+    }
+    block_sums<NTH>(s, red, par);
+    const double d0 = sqrt(s[0] * inv_nn), d1 = sqrt(s[1] * inv_nn);
+    const double h0 = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
+#pragma unroll
+    for (int q = 0; q < NE; ++q) y1[q] = make_double2(y[q].x + h0 * k[0][q].x, y[q].y + h0 * k[0][q].y);
+    field(y1, k[1]);
+    ++nrhs;
+    double s2[1] = {0.0};
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const double sc = atol + rtol * sqrt(y[q].x * y[q].x + y[q].y * y[q].y);
+      const double dr = (double)k[1][q].x - k[0][q].x, di = (double)k[1][q].y - k[0][q].y;
+      s2[0] += wt[q] * (dr * dr + di * di) / (sc * sc);
+    }
+    block_sums<NTH>(s2, red, par);
+    const double d2 = sqrt(s2[0] * inv_nn) / h0;
+    const double md = fmax(d1, d2);
+    const double h1 = md <= 1e-15 ? fmax(1e-6, h0 * 1e-3) : ctrl_pow(0.01 / md, kInitExp);
+    dt = fmin(100.0 * h0, h1);
+  }
+
+  bool need_k0 = false;
+  while (t < t_end) {
+    if (nsteps >= p.max_steps) {
+      status = DQH_MAX_STEPS;
+      break;
+    }
+    if (pwc && locate()) {
+      __syncthreads();  // no wave still reads the previous tables
+      build(seg);
+    }
+    if (need_k0) {
+      field(y, k[0]);
+      ++nrhs;
+      need_k0 = false;
+    }
+    // clip the step to the end time or the next breakpoint strictly after t
+    double h = dt, target = t_end;
+    bool target_jump = false;
+    if (pwc && seg + 1 < nseg && next_break < t_end) {
+      target = next_break;
+      target_jump = true;
+    }
+    bool made_jump = false;
+    double t_new = t + h;
+    if (snaps_to(t, h, target)) {
+      h = target - t;
+      t_new = target;
+      made_jump = target_jump;
+    }
+    if (!(h > 0.0) || !(h > 1e-14 * fmax(1.0, fabs(t)))) {
+      status = DQH_NONFINITE;
+      break;
+    }
+    // stages 1..5 evaluate the field on the increment Delta_s = h sum_j a_sj k_j alone
+    // (the generator is constant over the step): k[1..5] hold g_s = f(Delta_s), k_s =
+    // k_0 + g_s, and every combination folds k_0 into the weight of k[0]. Stage 6 is a
+    // full evaluation at y1 (the next k_0).
+#pragma unroll
+    for (int s = 1; s < 7; ++s) {
+      CTab *w = weights<TAB>();
+      if constexpr (NE > 1) pin_stages(s);
+      const double a0 = w->C[s];  // row sum of A: the weight of k_0 with the increments folded in
+#pragma unroll
+      for (int q = 0; q < NE; ++q) {
+        double re = a0 * (double)k[0][q].x, im = a0 * (double)k[0][q].y;
+#pragma unroll
+        for (int j = 1; j < s; ++j) {
+          if (rk.A[s][j] != 0.0) {  // compile-time
+            re += w->A[s][j] * (double)k[j][q].x;
+            im += w->A[s][j] * (double)k[j][q].y;
+          }
+        }
+        y1[q] = s < 6 ? make_double2(h * re, h * im) : make_double2(y[q].x + h * re, y[q].y + h * im);
+      }
+      field(y1, k[s]);
+    }
+    nrhs += 6;
+    // error norm in FP64; y1 is the candidate of stage 6
+    double ss[1] = {0.0};
+    CTab *we = weights<TAB>();
+    if constexpr (NE > 1) pin_stages(7);
+    double e0 = 0.0;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) e0 += we->E[j];
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      double er = e0 * (double)k[0][q].x, em = e0 * (double)k[0][q].y;
+#pragma unroll
+      for (int j = 1; j < 7; ++j) {
+        if (rk.E[j] != 0.0) {
+          er += we->E[j] * (double)k[j][q].x;
+          em += we->E[j] * (double)k[j][q].y;
+        }
+      }
+      er *= h;
+      em *= h;
+      const double sc = atol + rtol * sqrt(fmax(y[q].x * y[q].x + y[q].y * y[q].y,
+                                                y1[q].x * y1[q].x + y1[q].y * y1[q].y));
+      ss[0] += wt[q] * (er * er + em * em) / (sc * sc);
+    }
+    block_sums<NTH>(ss, red, par);
+    const double norm = sqrt(ss[0] * inv_nn);
+    const bool finite = isfinite(norm);
+    const bool keep = finite && norm < 1.0;
+    double factor;
+    if (!finite)
+      factor = p.factormin;
+    else if (norm == 0.0)
+      factor = p.factormax;
+    else
+      factor = p.safety * ctrl_pow(norm, -0.2);
+    factor = fmin(fmax(factor, keep ? 1.0 : p.factormin), p.factormax);
+    ++nsteps;
+    if (keep) {
+      if (tid == 0 && nacc < p.step_log_cap) gp<double>(p.step_log)[nacc] = t_new;
+      ++nacc;
+      while (isave < ntsave && next_save <= t_new) {
+        const double th = (next_save - t) / h;
+        CTab *wr = weights<TAB>();
+        double w[7];
+#pragma unroll
+        for (int j = 0; j < 7; ++j)
+          w[j] = th * (wr->R[j][0] + th * (wr->R[j][1] + th * (wr->R[j][2] + th * wr->R[j][3])));
+        fold_k0(w);
+        save(h, w, isave);
+        advance();
+      }
+#pragma unroll
+      for (int q = 0; q < NE; ++q) {
+        k[0][q] = k[6][q];
+        y[q] = y1[q];
+      }
+      t = t_new;
+      need_k0 = made_jump;
+    } else {
+      ++nrej;
+    }
+    dt = factor * h;
+  }
+  while (isave < ntsave) {
+    save(0.0, w0, isave);
+    advance();
+  }
+  float2 *fin = gp<float2>(p.final_state);
+  float2 *st = gp<float2>(p.states);
+#pragma unroll
+  for (int q = 0; q < NE; ++q) {
+    if (ei[q] >= 0) {
+      const float2 v = make_float2((float)y[q].x, (float)y[q].y), vc = make_float2(v.x, -v.y);
+      fin[(size_t)ei[q] * n + ej[q]] = v;
+      if (ei[q] != ej[q]) fin[(size_t)ej[q] * n + ei[q]] = vc;
+      if (!save_states) {
+        st[(size_t)ei[q] * n + ej[q]] = v;
+        if (ei[q] != ej[q]) st[(size_t)ej[q] * n + ei[q]] = vc;
+      }
+    }
+  }
+  if (tid == 0) {
+    stats[0] = nsteps;
+    stats[1] = nacc;
+    stats[2] = nrej;
+    stats[3] = status;
+    stats[4] = nrhs;
+  }
+}
+
+// Shifts of the operators' stencil and the parts of their coefficients, sorted by shift
+// (so that an operator set and its zero-extended superset add up in the same order).
+// False when they exceed kMaxShift or kMaxPart.
+bool make_pattern(const dqh_dia_ops &ops, int n, Pattern &pt) {
+  std::memset(&pt, 0, sizeof(pt));
+  std::vector<std::pair<std::pair<int, int>, Part>> parts;
+  pt.nH = ops.noff[0];
+  for (int x = 0; x < ops.noff[0]; ++x) {
+    const int o = ops.off[0][x];
+    if (o == 0) return false;  // the main diagonal goes in hdiag
+    parts.push_back({{o, 0}, Part{0, (uint8_t)x, 0, 0}});
+    parts.push_back({{0, o}, Part{1, (uint8_t)x, 0, 0}});
+  }
+  int row = 0;
+  for (int s = 1; s < ops.nops; ++s) {
+    for (int u = 0; u < ops.noff[s]; ++u)
+      for (int v = 0; v < ops.noff[s]; ++v) {
+        const int a = ops.off[s][u], b = ops.off[s][v];
+        const Part part{2, (uint8_t)(row + u), (uint8_t)(row + v), 0};
+        if (a == 0 && b == 0) {
+          if (pt.nzero >= kMaxPart) return false;
+          pt.zero[pt.nzero++] = part;
+        } else {
+          parts.push_back({{a, b}, part});
+        }
+      }
+    row += ops.noff[s];
+  }
+  pt.nLrow = row;
+  if ((int)parts.size() > kMaxPart) return false;
+  std::stable_sort(parts.begin(), parts.end(), [](const auto &l, const auto &r) { return l.first < r.first; });
+  for (size_t i = 0; i < parts.size(); ++i) {
+    if (i == 0 || parts[i].first != parts[i - 1].first) {
+      if (pt.nterm >= kMaxShift) return false;
+      pt.a[pt.nterm] = parts[i].first.first;
+      pt.b[pt.nterm] = parts[i].first.second;
+      pt.first[pt.nterm++] = (int32_t)i;
+    }
+    pt.part[i] = parts[i].second;
+  }
+  for (int t = pt.nterm; t <= kMaxShift; ++t) pt.first[t] = (int32_t)parts.size();
+  for (int t = 0; t < pt.nterm; ++t) pt.guard = std::max(pt.guard, std::abs(pt.a[t] * row_stride(n) + pt.b[t]));
+  return true;
+}
+
+template <int NTH, int NE, int T, int TAB>
+int launch(const dqh_me_inst *d, int64_t ninst, int n, const Pattern &pt, hipStream_t st) {
+  const size_t lds = lds_bytes<NTH>(n, pt.nH, pt.nLrow, pt.guard);
+  const void *fn = reinterpret_cast<const void *>(&k_tsit5_diag<NTH, NE, T, TAB>);
+  hipError_t err = hipSuccess;
+  if (lds > 65536) err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (err == hipSuccess) {
+    hipLaunchKernelGGL((k_tsit5_diag<NTH, NE, T, TAB>), dim3((unsigned)ninst), dim3(NTH), lds, st, d, pt);
+    err = hipGetLastError();
+  }
+  return err == hipSuccess ? DQH_OK : fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_diag: ") + hipGetErrorString(err));
+}
+
+template <int T, int TAB>
+int launch_size(const dqh_me_inst *d, int64_t ninst, int n, const Pattern &pt, hipStream_t st) {
+  const int nu = n * (n + 1) / 2;
+  if (nu <= 64) return launch<64, 1, T, TAB>(d, ninst, n, pt, st);
+  if (nu <= 192) return launch<192, 1, T, TAB>(d, ninst, n, pt, st);
+  if (nu <= 576) return launch<576, 1, T, TAB>(d, ninst, n, pt, st);
+  if (nu <= 1152) return launch<576, 2, T, TAB>(d, ninst, n, pt, st);
+  return launch<704, 3, T, TAB>(d, ninst, n, pt, st);
+}
+
+}  // namespace diag
+}  // namespace dqh
+
+using namespace dqh;
+
+extern "C" int dqh_mesolve_tsit5_diag(const dqh_me_inst *d_insts, int64_t ninst, int64_t n, const dqh_dia_ops *ops,
+                                      int64_t flags, void *stream) {
+  if (!d_insts || !ops || ninst <= 0 || ninst > (1 << 30))
+    return fail(DQH_BAD_ARG, "dqh_mesolve_tsit5_diag: bad arguments");
+  if (n <= 0 || n > 64) return fail(DQH_BAD_SHAPE, "dqh_mesolve_tsit5_diag: 1 <= n <= 64");
+  if (ops->nops < 1 || ops->nops > DQH_DIA_MAXOPS)
+    return fail(DQH_BAD_ARG, "dqh_mesolve_tsit5_diag: 1 <= nops <= 8 (the generator, then the jump operators)");
+  for (int s = 0; s < ops->nops; ++s) {
+    if (ops->noff[s] < 0 || ops->noff[s] > DQH_DIA_MAXOFF)
+      return fail(DQH_BAD_ARG, "dqh_mesolve_tsit5_diag: bad number of diagonals");
+    for (int u = 0; u < ops->noff[s]; ++u)
+      if (ops->off[s][u] <= -n || ops->off[s][u] >= n)
+        return fail(DQH_BAD_ARG, "dqh_mesolve_tsit5_diag: offset outside (-n, n)");
+  }
+  diag::Pattern pt;
+  if (!diag::make_pattern(*ops, (int)n, pt))
+    return fail(DQH_BAD_SHAPE, "dqh_mesolve_tsit5_diag: at most 12 shifts and no main diagonal in operator 0");
+  hipStream_t st = (hipStream_t)stream;
+  const bool dopri5 = (flags & DQH_FLAG_DOPRI5) != 0;
+  if (pt.nterm <= 6)
+    return dopri5 ? diag::launch_size<6, 1>(d_insts, ninst, (int)n, pt, st)
+                  : diag::launch_size<6, 0>(d_insts, ninst, (int)n, pt, st);
+  return dopri5 ? diag::launch_size<12, 1>(d_insts, ninst, (int)n, pt, st)
+                : diag::launch_size<12, 0>(d_insts, ninst, (int)n, pt, st);
+}

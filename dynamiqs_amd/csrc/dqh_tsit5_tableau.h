@@ -26,7 +26,7 @@ struct RKTab {
 // output is the quartic through y0, y1, f0, f1 and Shampine's midpoint value, in
 // the same b_i(theta) form. Its theta^4 column equals the dense-output constants
 // of the DOPRI5 code.
-static __constant__ RKTab kRK[2] = {
+constexpr RKTab kRKTabs[2] = {
     {{0, 0.161, 0.327, 0.9, 0.9800255409045097, 1, 1},
      {{0, 0, 0, 0, 0, 0, 0},
       {0.161, 0, 0, 0, 0, 0, 0},
@@ -62,6 +62,10 @@ static __constant__ RKTab kRK[2] = {
       {0, -1.3744241142186024, 3.272657752246729, -1.7672812570757455},
       {0, 1.3824689317781436, -3.764937863556287, 2.382468931778144}}},
 };
+
+// the tableaus for kernels that select the pair at run time; kernels compiled for one
+// pair read kRKTabs, whose entries become literals
+static __constant__ RKTab kRK[2] = {kRKTabs[0], kRKTabs[1]};
 
 // Initial step h1 = (0.01 / max(d1, d2))^kInitExp (Hairer-Norsett-Wanner II.4). The
 // exponent is one over the order of the embedded solution (4), while the

@@ -201,6 +201,7 @@ class DensePlan:
         self.uniform_np = 0  # every instance takes the resident Tsit5 body of this np
         self.fp64_diag = False  # ... with the generator's diagonal in FP64 (hdiag)
         self.step_log = None
+        self.stencil = None  # Stencil of the few-diagonal Tsit5 kernel (dqh_mesolve_tsit5_diag)
 
     # ------------------------------------------------------------------ launch
     def reset(self):
@@ -222,6 +223,16 @@ class DensePlan:
                     scratch.numel(), steps, c_p(flags.data_ptr()), sp,
                 ),
                 'dqh_mesolve_tsit5_dense_grid',
+            )
+            return
+        if self.stencil is not None:
+            c_p = _native.ctypes.c_void_p
+            _native.check(
+                lib.dqh_mesolve_tsit5_diag(
+                    c_p(self.d_descs.data_ptr()), self.ninst, self.n, _native.ctypes.byref(self.stencil.ops),
+                    int(self.descs['flags'][0]) & _native.FLAG_DOPRI5, sp,
+                ),
+                'dqh_mesolve_tsit5_diag',
             )
             return
         if self.uniform_np:
@@ -494,6 +505,112 @@ def _hmods(inst: Instance) -> list:
     return out
 
 
+# limits of dqh_mesolve_tsit5_diag (dqh_diag.hip)
+STENCIL_MAX_N = 64
+STENCIL_MAX_SHIFTS = 12
+STENCIL_MAX_PARTS = 48
+STENCIL_MAX_LDS = 150 * 1024
+
+
+@dataclass
+class Stencil:
+    """Operators of a batch by their nonzero diagonals: ``offH`` the off-diagonals of the
+    generators (their union over the batch), ``offL`` those of each jump operator, and
+    ``ops`` the same for the kernel; ``G`` / ``gdiag`` (off-diagonals and main diagonal of
+    every distinct generator) and ``L`` (rows of every distinct set of jump operators) as
+    rows of ``np`` elements, with ``ig`` / ``il`` the instances' indices into them."""
+
+    offH: list
+    offL: list
+    ops: object
+    G: np.ndarray  # (nG, nH, np) complex64
+    gdiag: np.ndarray  # (nG, np) complex128
+    L: np.ndarray  # (nSets, nLrow, np) complex64
+    ig: np.ndarray
+    il: np.ndarray
+
+
+def _rows_on(x: np.ndarray, offs, npad: int) -> np.ndarray:
+    """Diagonals of ``x`` (..., n, n) at ``offs`` as rows (..., len(offs), npad) indexed by
+    the matrix row: element i of offset o is x[i, i + o], zero outside the matrix."""
+    n = x.shape[-1]
+    out = np.zeros((*x.shape[:-2], len(offs), npad), dtype=np.complex128)
+    for k, o in enumerate(offs):
+        lo, hi = max(0, -o), min(n, n - o)
+        out[..., k, lo:hi] = np.diagonal(x, offset=o, axis1=-2, axis2=-1)
+    return out
+
+
+def _offsets(mask: np.ndarray) -> list:
+    i, j = np.nonzero(mask)
+    return [int(o) for o in np.unique(j - i)]
+
+
+def few_diagonals(instances: list, npad: int) -> Stencil | None:
+    """The :class:`Stencil` of a batch, or None where the few-diagonal kernel does not take
+    it: n above STENCIL_MAX_N, time-dependent jump operators or modulated terms, or more
+    shifts, coefficient parts or LDS than the kernel holds. At n = 64 with 12 shifts the
+    stencil needs 13 multiply-adds per element against (1 + 2K) 64 of the dense products,
+    so within these limits it is always the faster form."""
+    n = instances[0].H.shape[-1]
+    K = len(instances[0].Ls)
+    if n > STENCIL_MAX_N or K > 7:
+        return None
+    if any(i.mod or i.Cs is not None or i.expanded or i.Lsum or any(x is not None for x in i.Lmod or [])
+           or any(x is not None for x in i.Lpwc or []) for i in instances):
+        return None
+    ids = {}
+
+    def index(key):  # an instance without keys shares nothing
+        return ids.setdefault(key, len(ids))
+
+    il, Lsets = np.zeros(len(instances), dtype=np.int64), []
+    for b, inst in enumerate(instances):
+        il[b] = index(('L', b if inst.key_L is None else inst.key_L))
+        if il[b] == len(Lsets):
+            Lsets.append(inst.Ls)
+    ids = {}
+    ig, first = np.zeros(len(instances), dtype=np.int64), []
+    for b, inst in enumerate(instances):
+        ig[b] = index(('G', b) if inst.key_H is None or inst.key_L is None else (inst.key_H, inst.key_L))
+        if ig[b] == len(first):
+            first.append(b)
+    Lall = np.stack([np.stack(Ls) if K else np.zeros((0, n, n)) for Ls in Lsets]).astype(np.complex128)
+    LdL = np.swapaxes(Lall.conj(), -1, -2) @ Lall
+    LdL = LdL.sum(axis=1)
+    explicit = [instances[b].Hnh is not None for b in first]
+    G = -1j * np.stack([instances[b].H for b in first]) - 0.5 * LdL[il[first]]
+    for k, b in enumerate(first):
+        if explicit[k]:
+            G[k] = instances[b].Hnh
+    mask = np.any(G != 0, axis=0)
+    for inst in {id(o): o for i in instances for (_, _, o) in i.pwc}.values():
+        mask = mask | (np.asarray(inst) != 0)
+    offH = [o for o in _offsets(mask) if o != 0]
+    offL = [_offsets(m) for m in np.any(Lall != 0, axis=0)] if K else []
+    rowsL = sum(len(o) for o in offL)
+    shifts = {(o, 0) for o in offH} | {(0, o) for o in offH} | {(p, q) for o in offL for p in o for q in o}
+    shifts.discard((0, 0))
+    parts = 2 * len(offH) + sum(len(o) ** 2 for o in offL)
+    guard = max((abs(a * (n | 1) + b) for a, b in shifts), default=0)
+    lds = 8 * (2 * (n * (n | 1) + 1 + guard) + guard + (len(offH) + rowsL) * n) + 16 * n + 1024
+    if (len(shifts) > STENCIL_MAX_SHIFTS or parts > STENCIL_MAX_PARTS or lds > STENCIL_MAX_LDS
+            or len(offH) > 16 or any(len(o) > 16 for o in offL)):
+        return None
+    from .dia import DiaOps
+
+    ops = DiaOps()
+    ops.nops = 1 + K
+    for k, offs in enumerate([offH, *offL]):
+        ops.noff[k] = len(offs)
+        for u, o in enumerate(offs):
+            ops.off[k][u] = o
+    L = [_rows_on(Lall[:, k], offs, npad) for k, offs in enumerate(offL)]
+    return Stencil(offH, offL, ops, _rows_on(G, offH, npad).astype(np.complex64), _rows_on(G, [0], npad)[:, 0],
+                   np.concatenate(L, axis=1).astype(np.complex64) if K else np.zeros((len(Lsets), 0, npad), np.complex64),
+                   ig, il)
+
+
 def build_plan(
     kind: str,
     instances: list,
@@ -517,6 +634,7 @@ def build_plan(
     tableau: str = 'tsit5',
     rouchon_order: int = 1,
     fp64_diag: bool = True,
+    dia_ops: bool = False,
 ) -> DensePlan:
     """Pack ``instances`` (same Hilbert dimension) for ``kind`` in {'tsit5', 'rouchon1', 'rhs'}.
 
@@ -544,7 +662,11 @@ def build_plan(
     FP64 at every vector-field evaluation, the off-diagonal part stays on FP32 MFMA.
     The diagonal holds the largest single terms (energies and decay rates), so this
     removes their FP32 rounding from every stage (about 3x lower error against the
-    FP64 oracle on stiff problems such as the driven Kerr batch)."""
+    FP64 oracle on stiff problems such as the driven Kerr batch).
+
+    ``dia_ops`` (Tsit5 / Dopri5 with every other choice left open): the operators were
+    given by their diagonals, so a batch with few of them runs on the stencil kernel
+    (:func:`few_diagonals`, ``dqh_mesolve_tsit5_diag``) instead of dense products."""
     import torch
 
     if tableau not in ('tsit5', 'dopri5', 'dopri8'):
@@ -593,7 +715,10 @@ def build_plan(
     if form not in ('auto', 'resident', 'global'):
         raise ValueError("form must be 'auto', 'resident' or 'global'")
     use_global = form == 'global'
-    if form == 'auto' and kind in ('tsit5', 'rhs') and not dopri8:
+    stencil = None
+    if dia_ops and kind == 'tsit5' and not dopri8 and form == 'auto' and fp64_diag and grid_tsit5 == 'auto':
+        stencil = few_diagonals(instances, npad)
+    if form == 'auto' and kind in ('tsit5', 'rhs') and not dopri8 and stencil is None:
         from .. import autotune
 
         use_global = autotune.dense_global(npad, K, B)
@@ -643,7 +768,7 @@ def build_plan(
     npwc_all = max((len(inst.pwc) + sum(lp is not None for lp in (inst.Lpwc or [])) for inst in instances), default=0)
     grid_plan = kind == 'tsit5' and not dopri8 and use_grid(grid_tsit5, n, B, npwc_all + nmod_max, nE, save_states)
     hdiag_plan = (fp64_diag and kind == 'tsit5' and npad in (16, 32, 48, 64) and K <= 3 and not use_global
-                  and not lmod_any and not grid_plan)
+                  and not lmod_any and not grid_plan and stencil is None)
     t_stop = float(tsave[-1])
     if instances[0].tsave is not None:
         t_stop = max(float(inst.tsave[-1]) for inst in instances)
@@ -678,6 +803,24 @@ def build_plan(
     descs['max_steps'] = max_steps
     descs['t0'], descs['t1'] = t_start, t_end
     descs['tsave'] = p_tsave
+    if stencil is not None:
+        u = np.uint64
+        descs['EopsT'] = p_E
+        descs['flags'] = ((_native.FLAG_SAVE_STATES if save_states else 0)
+                          | (_native.FLAG_DOPRI5 if tableau == 'dopri5' else 0))
+        descs['nL'] = K
+        for f, block, idx in (('Hnh', stencil.G, stencil.ig), ('hdiag', stencil.gdiag, stencil.ig),
+                              ('Dops', stencil.L, stencil.il)):
+            if block.size:
+                descs[f] = u(arena.put(block)) + idx.astype(u) * u(block[0].nbytes)
+
+    def bpwc(inst):
+        """-i O_j of the PWC terms: matrices, or their rows for the stencil kernel."""
+        if stencil is None:
+            return _pad(np.stack([-1j * o for (_, _, o) in inst.pwc]), npad).astype(np.complex64)
+        O = -1j * np.stack([np.asarray(o, dtype=np.complex128) for (_, _, o) in inst.pwc])
+        return _rows_on(O, [*stencil.offH, 0], npad).astype(np.complex64)
+
     for b, inst in enumerate(instances):
         d = descs[b]
         if per_inst_ts:
@@ -685,6 +828,16 @@ def build_plan(
             d['tsave'] = arena.put(ts_i)
             d['t0'] = float(ts_i[0] if inst.t0 is None else inst.t0)
             d['t1'] = float(ts_i[-1])
+        if stencil is not None:
+            if inst.pwc:
+                grid, samplers = pwc_sampling(inst.pwc)
+                vals = np.stack([np.where(inside, np.asarray(v, dtype=np.complex128)[idx], 0.0)
+                                 for (_, v, _), (idx, inside) in zip(inst.pwc, samplers)])
+                d['npwc'], d['nseg'] = len(inst.pwc), len(grid)
+                d['Hpwc'] = shared(('Hpwc', inst.key_H), lambda inst=inst: bpwc(inst))
+                d['pwc_times'] = shared(('ptimes', inst.key_H), lambda grid=grid: grid)
+                d['pwc_vals'] = arena.put(np.ascontiguousarray(vals).view(np.float64))
+            continue
         d['EopsT'] = p_E
         d['flags'] = _native.FLAG_SAVE_STATES if save_states else 0
         if kind in ('tsit5', 'rhs'):
@@ -769,9 +922,7 @@ def build_plan(
                 d['npwc'] = len(inst.pwc)
                 d['nseg'] = len(grid)
                 npwc_max = max(npwc_max, len(inst.pwc))
-                d['Hpwc'] = shared(
-                    ('Hpwc', inst.key_H), lambda inst=inst: _pad(np.stack([-1j * o for (_, _, o) in inst.pwc]), npad).astype(np.complex64)
-                )
+                d['Hpwc'] = shared(('Hpwc', inst.key_H), lambda inst=inst: bpwc(inst))
                 d['pwc_times'] = shared(('ptimes', inst.key_H), lambda grid=grid: grid)
                 d['pwc_vals'] = arena.put(np.ascontiguousarray(vals).view(np.float64))
             hm = _hmods(inst)
@@ -875,6 +1026,8 @@ def build_plan(
         welems += 2 * nLdev * nn
     if dopri8:  # stages 7..12 after the generator slot: (16 + nL) np^2
         welems = max(welems, (16 + nLdev) * nn)
+    if stencil is not None:  # everything lives in registers and LDS
+        welems = 0
     work = arena.empty(B * welems * 8)
     y = torch.zeros((B, 2, nn, 2), dtype=torch.float64, device=dev)
     y0 = np.zeros((B, npad, npad), dtype=np.complex128)
@@ -897,7 +1050,7 @@ def build_plan(
     for b in range(B):
         d = descs[b]
         d['y'] = y.data_ptr() + b * 2 * nn * 16
-        d['work'] = work.data_ptr() + b * welems * 8
+        d['work'] = work.data_ptr() + b * welems * 8 if welems else 0
         d['states'] = states.data_ptr() + b * ns * n * n * 8
         d['final_state'] = final.data_ptr() + b * n * n * 8
         d['expects'] = expects.data_ptr() + b * max(nE, 1) * len(tsave) * 8
@@ -909,11 +1062,22 @@ def build_plan(
             descs[b]['step_log'] = step_log.data_ptr() + b * int(step_log_cap) * 8
             descs[b]['step_log_cap'] = int(step_log_cap)
     plan.step_log = step_log
-    check_descriptors(descs, [*arena.tensors, work, states, final, expects, stats] + ([step_log] if step_log is not None else []))
+    extents = None
+    if stencil is not None:
+        row, u = npad * 8, np.uint64
+        extents = {'Hnh': np.full(B, len(stencil.offH) * row, dtype=u), 'Dops': np.full(B, stencil.L.shape[1] * row, dtype=u),
+                   'Hpwc': descs['npwc'].astype(u) * u((len(stencil.offH) + 1) * row),
+                   'pwc_times': descs['nseg'].astype(u) * u(8),
+                   'pwc_vals': descs['npwc'].astype(u) * np.maximum(descs['nseg'].astype(np.int64) - 1, 0).astype(u) * u(16)}
+    check_descriptors(descs, [*arena.tensors, work, states, final, expects, stats] + ([step_log] if step_log is not None else []),
+                      extents)
+    plan.stencil = stencil
     plan.descs = descs
     plan.d_descs = torch.from_numpy(descs.view(np.uint8).copy()).to(dev)
     plan.K = K
-    if (
+    if stencil is not None:
+        pass
+    elif (
         kind == 'tsit5'
         and npad in (16, 32, 48, 64)
         and np.all(descs['nL'] <= 3)

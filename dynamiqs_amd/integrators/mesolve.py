@@ -22,8 +22,9 @@ from ..gradient import Gradient, reject_gradient
 from ..method import Dopri5, Dopri8, Euler, Expm, Method, Rouchon1, Rouchon2, Rouchon3, Tsit5, _DEAdaptiveStep
 from ..options import Options, check_options
 from ..qarrays import QArray, asqarray
+from ..qarrays import dia as dia_layout
 from ..result import AdaptiveStepInfos, FixedStepInfos, MESolveResult
-from ..time_qarray import TimeQArray, astimeqarray
+from ..time_qarray import SummedTimeQArray, TimeQArray, astimeqarray
 from . import dense
 from . import dia as dia_path
 from .operators import decompose, resolve_callables
@@ -118,6 +119,12 @@ def dia_route(method, H: TimeQArray, Ls, n: int):
     if n > dense.MAX_NP:
         return 'batched', Ht, Lts
     return None
+
+
+def given_by_diagonals(x: TimeQArray) -> bool:
+    """Whether every term of a time-qarray has the DIA layout."""
+    terms = x.timeqarrays if isinstance(x, SummedTimeQArray) else [x]
+    return all(getattr(getattr(t, 'qarray', None), 'layout', None) is dia_layout for t in terms)
 
 
 def enumerate_instances(H: TimeQArray, Ls, rho0: QArray, cartesian: bool):
@@ -316,6 +323,7 @@ def mesolve(
             max_steps=method.max_steps,
             save_states=save_all,
             tableau=_tableau(method),
+            dia_ops=all(given_by_diagonals(x) for x in (H, *Ls)),
         )
     else:
         plan = dense.build_plan(

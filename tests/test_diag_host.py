@@ -1,0 +1,94 @@
+"""CPU checks of the few-diagonal form of a batch (``dense.few_diagonals``): the stencil
+of the staged rows is the Lindblad vector field of the dense operators, for every kind of
+pattern the rule accepts, and everything else is left to the dense kernels."""
+
+import numpy as np
+import pytest
+
+from dynamiqs_amd.integrators import dense
+from oracle import lindblad
+
+
+def _banded(rng, n, offs):
+    x = np.zeros((n, n), dtype=np.complex128)
+    for o in offs:
+        m = n - abs(o)
+        x += np.diag(rng.normal(size=m) + 1j * rng.normal(size=m), k=o)
+    return x
+
+
+def _field(st, b, rho):
+    """The kernel's evaluation: zero outside the matrix, one coefficient per shift."""
+    n = rho.shape[-1]
+    G, g, L = st.G[st.ig[b]].astype(np.complex128), st.gdiag[st.ig[b]], st.L[st.il[b]].astype(np.complex128)
+    pad = np.zeros((3 * n, 3 * n), dtype=np.complex128)
+    pad[n : 2 * n, n : 2 * n] = rho
+    at = lambda a, c: pad[n + a : 2 * n + a, n + c : 2 * n + c]  # noqa: E731  rho[i + a][j + c]
+    f = (g[:n, None] + g[None, :n].conj()) * rho
+    for k, o in enumerate(st.offH):
+        f = f + G[k, :n, None] * at(o, 0) + G[k, None, :n].conj() * at(0, o)
+    row = 0
+    for offs in st.offL:
+        for u, a in enumerate(offs):
+            for v, c in enumerate(offs):
+                f = f + L[row + u, :n, None] * L[row + v, None, :n].conj() * at(a, c)
+        row += len(offs)
+    return f
+
+
+@pytest.mark.parametrize('n,offH,offL', [
+    (1, [0], [[0]]), (2, [-1, 1], [[1]]), (5, [0], []), (16, [-1, 0, 1], [[1]]), (64, [-2, 0, 2], [[1], [2]]),
+    (33, [-4, 4], [[0], [-3]]), (20, [0], [[-1, 1]]), (9, [-8, 8], [[8], [-8]]), (12, [], [[0, 1]]),
+])
+def test_stencil_rows_give_the_vector_field(n, offH, offL):
+    rng = np.random.default_rng(n)
+    insts, Ls = [], [_banded(rng, n, o) for o in offL]
+    for b in range(3):
+        H = _banded(rng, n, offH)
+        insts.append(dense.Instance(H=H + H.conj().T, Ls=Ls, rho0=np.eye(n) / n, key_H=(b,), key_L=(), key_rho=()))
+    st = dense.few_diagonals(insts, dense.pad16(n))
+    assert st is not None and st.G.shape[0] == 3 and st.L.shape[0] == 1
+    for b, inst in enumerate(insts):
+        r = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
+        r = r + r.conj().T
+        ref = lindblad.rhs_hermitian(inst.H, inst.Ls, r)
+        # the off-diagonal rows are rounded to complex64 (6e-8 each), the rest is FP64
+        assert np.linalg.norm(_field(st, b, r) - ref) <= 1e-6 * max(1.0, np.linalg.norm(ref))
+
+
+def test_explicit_generators_and_instances_without_keys():
+    rng = np.random.default_rng(0)
+    n = 8
+    insts = []
+    for _ in range(2):
+        G = _banded(rng, n, [0, 1])
+        insts.append(dense.Instance(H=np.zeros((n, n)), Ls=[_banded(rng, n, [1])], rho0=np.eye(n) / n, Hnh=G))
+    st = dense.few_diagonals(insts, 16)
+    assert st.offH == [1] and list(st.ig) == [0, 1] and list(st.il) == [0, 1]
+    for b, inst in enumerate(insts):
+        assert np.array_equal(st.gdiag[b, :n], np.diag(inst.Hnh))
+        assert np.array_equal(st.L[b, 0, : n - 1], np.diag(inst.Ls[0], 1).astype(np.complex64))
+
+
+@pytest.mark.parametrize('why,kw', [
+    ('dense', dict(offH=list(range(-9, 10)))), ('shifts', dict(offL=[[0, 1, 2, 3]])), ('size', dict(n=65)),
+    ('jump operators', dict(offL=[[0]] * 8)), ('LDS', dict(n=64, offH=[60], offL=[[60]])),
+])
+def test_everything_else_stays_on_the_dense_kernels(why, kw):
+    rng = np.random.default_rng(1)
+    n = kw.get('n', 20)
+    H = _banded(rng, n, kw.get('offH', [0]))
+    inst = dense.Instance(H=H + H.conj().T, Ls=[_banded(rng, n, o) for o in kw.get('offL', [[1]])], rho0=np.eye(n) / n)
+    assert dense.few_diagonals([inst], dense.pad16(n)) is None, why
+
+
+def test_time_dependent_terms():
+    n, H = 8, np.diag(np.arange(8.0)).astype(np.complex128)
+    X = np.diag(np.ones(7), 1) + np.diag(np.ones(7), -1)
+    kw = dict(H=H, Ls=[np.diag(np.ones(7), 1)], rho0=np.eye(n) / n)
+    st = dense.few_diagonals([dense.Instance(**kw, pwc=[(np.array([0.0, 1.0]), np.ones(1), X)])], 16)
+    assert st.offH == [-1, 1]  # the PWC term's diagonals join the generator's
+    g = lambda t: 1.0  # noqa: E731
+    assert dense.few_diagonals([dense.Instance(**kw, mod=[(g, X, None)])], 16) is None
+    assert dense.few_diagonals([dense.Instance(**kw, Lmod=[(g, None)])], 16) is None
+    assert dense.few_diagonals([dense.Instance(**kw, Lpwc=[(np.array([0.0, 1.0]), np.ones(1))])], 16) is None
