@@ -1,5 +1,5 @@
 // Adaptive Tsit5 / Dopri5 for small master equations whose operators have few nonzero
-// diagonals (gfx950), n <= 64: one workgroup per instance.
+// diagonals (gfx950), n < 128: one workgroup per instance.
 //
 // The vector field G rho + rho G^dag + sum_k L_k rho L_k^dag of such operators is a
 // stencil, f[i][j] = sum_t C_t(i, j) rho[i + a_t][j + b_t]: one shift (o, 0) and one
@@ -9,7 +9,7 @@
 // products, so the matrix cores have nothing to do here and a step is bound by the
 // latency of its dependent stages (n <= 32) and by FP64 issue and LDS reads (n = 64).
 //
-// A thread owns NE elements of the upper triangle (u = thread + NTH q, row by row, of
+// k_tsit5_diag, n <= 64 and at most 12 shifts: a thread owns NE elements of the upper triangle (u = thread + NTH q, row by row, of
 // the n (n + 1) / 2 that exist: no work on padding). Its coefficients C_t, the FP64
 // diagonal generator g = d_i + conj(d_j), the FP64 state, the candidate and the seven
 // FP32 stages stay in registers for the whole solve. The stage input goes to LDS in
@@ -40,6 +40,7 @@ namespace diag {
 
 constexpr int kMaxShift = 12;  // shifts of the stencil (register coefficients per element)
 constexpr int kMaxPart = 48;   // contributions to the shifts' coefficients
+constexpr int kMaxOff = 16;    // off-diagonals of the generator
 
 // A contribution to a coefficient: kind 0 G_x[i] (row diagonal x of the generator),
 // kind 1 conj(G_x[j]), kind 2 L_x[i] conj(L_y[j]) (x, y: rows of the jump-operator table).
@@ -54,6 +55,12 @@ struct Pattern {
   int32_t first[kMaxShift + 1];  // parts of shift t: part[first[t]] .. part[first[t + 1] - 1]
   Part part[kMaxPart];
   Part zero[kMaxPart];
+  // the same for the table form: off-diagonals of G, and the pairs of jump-operator rows
+  // (kind 2 parts) with their shifts, (0, 0) excepted
+  int32_t offH[kMaxOff];
+  int32_t npair;
+  Part pair[kMaxPart];
+  int16_t pa[kMaxPart], pb[kMaxPart];
 };
 
 // x + (x of the lane that the DPP control names)
@@ -575,9 +582,546 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
   }
 }
 
+// The same solve with the coefficients read from LDS tables at every evaluation (one copy
+// of the stage input, two barriers per stage): for 64 < n < 128, for more than kMaxShift
+// shifts, and for modulated terms, whose tables are rebuilt at every stage time. The terms
+// are an outer loop, so that each one keeps NE independent reads in flight. KM: the stages
+// and the state are in global memory (work: 7 NU float2, y: NU double2, in owner order; L2
+// serves them), for n > 90, where they do not fit the registers.
+// Bound by the LDS reads, three 8-byte ones per term and element. 48 two-mode problems of
+// n = 81 (10 parts, about 150 steps): 61.2 -> 3.83 ms against the dense body; 32 problems
+// of n = 127 with one jump diagonal, 8 steps: 12.7 -> 1.28 ms (memory form).
+template <int NTH, int NE, bool KM, int TAB>
+__global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__restrict__ insts, Pattern pat) {
+  extern __shared__ __align__(16) char smem[];
+  const dqh_me_inst &p = insts[blockIdx.x];
+  constexpr RKTab rk = kRKTabs[TAB];
+  constexpr int QC = NE < 2 ? NE : 2;
+  const int n = (int)p.n, np = (int)p.np, nE = (int)p.nE, ntsave = (int)p.ntsave, nseg = (int)p.nseg;
+  const int LD = row_stride(n), NLD = n * LD, tid = (int)threadIdx.x;
+  const int npwc = (int)p.npwc, nmod = (int)p.nmod;
+  const bool pwc = npwc > 0, smooth = nmod > 0;
+  double2 *dcur = reinterpret_cast<double2 *>(smem);
+  double *red = reinterpret_cast<double *>(dcur + n);
+  float2 *ys = reinterpret_cast<float2 *>(red + 4 * (NTH / 64));
+  float2 *Gt = ys + NLD + 1;
+  float2 *Lt = Gt + pat.nH * n;
+  int64_t *stats = gp<int64_t>(p.stats);
+  const int NU = n * (n + 1) / 2;
+  if (n >= 128 || NU > NTH * NE || nmod > DQH_MAX_MOD || (pwc && nseg < 2) || (smooth && p.mod_nint < 1) ||
+      (KM && !p.work) || (p.flags & (DQH_FLAG_GLOBAL | DQH_FLAG_LMOD | DQH_FLAG_DOPRI8 | DQH_FLAG_EULER)) ||
+      ((p.flags & DQH_FLAG_DOPRI5) != 0) != (TAB == 1)) {
+    if (tid == 0) stats[3] = DQH_UNSUPPORTED;
+    return;
+  }
+  const double *tsave = gp<const double>(p.tsave);
+  const double *ptimes = gp<const double>(p.pwc_times);
+  const double rtol = p.rtol, atol = p.atol, t_end = p.t1;
+  const double inv_nn = 1.0 / ((double)n * n);
+  const bool save_states = (p.flags & DQH_FLAG_SAVE_STATES) != 0;
+
+  // owned elements, packed i | j << 8 (i <= j; -1 past the end)
+  int ij[NE];
+#pragma unroll
+  for (int q = 0; q < NE; ++q) {
+    int rem = tid + NTH * q, i = 0;
+    ij[q] = -1;
+    if (rem < NU) {
+      while (rem >= n - i) {
+        rem -= n - i;
+        ++i;
+      }
+      ij[q] = i | ((i + rem) << 8);
+    }
+  }
+  // row and column of element q (0, 0 past the end), formed where they are used
+  auto at = [&](int q, int &i, int &j) {
+    int x = ij[q];
+    asm volatile("" : "+v"(x));
+    x = max(x, 0);
+    i = x & 255;
+    j = x >> 8;
+  };
+  for (int e = tid; e <= NLD; e += NTH) ys[e] = make_float2(0.f, 0.f);
+  for (int e = tid; e < pat.nLrow * n; e += NTH) {
+    const int r = e / n, i = e - r * n;
+    Lt[e] = gp<const float2>(p.Dops)[(size_t)r * np + i];
+  }
+  // Gt, dcur <- the constant generator + the PWC terms of segment seg + f_j(tau) O_j
+  auto tables = [&](int seg, double tau) {
+    const float2 *G0 = gp<const float2>(p.Hnh);
+    const double2 *d0g = gp<const double2>(p.hdiag);
+    const float2 *Hp = gp<const float2>(p.Hpwc), *Hm = gp<const float2>(p.Hmod);
+    const double *vals = gp<const double>(p.pwc_vals);
+    const int nv = nseg - 1, rows = pat.nH + 1;
+    const bool inside = pwc && seg >= 0 && seg < nv;
+    double2 fm[DQH_MAX_MOD];
+#pragma unroll
+    for (int j = 0; j < DQH_MAX_MOD; ++j) fm[j] = make_double2(0.0, 0.0);
+    if (smooth) {
+      const int64_t nint = p.mod_nint;
+      int64_t m = (int64_t)floor((tau - p.mod_t0) / p.mod_dt);
+      m = m < 0 ? 0 : (m >= nint ? nint - 1 : m);
+      const double x = tau - (p.mod_t0 + (double)m * p.mod_dt);
+#pragma unroll
+      for (int j = 0; j < DQH_MAX_MOD; ++j) {
+        if (j < nmod) {
+          const double2 *c = gp<const double2>(p.mod_coef) + ((size_t)j * nint + m) * 4;
+          double re = c[0].x, im = c[0].y;
+#pragma unroll
+          for (int d = 1; d < 4; ++d) {
+            re = re * x + c[d].x;
+            im = im * x + c[d].y;
+          }
+          fm[j] = make_double2(re, im);
+        }
+      }
+    }
+    for (int e = tid; e < rows * n; e += NTH) {
+      const int r = e / n, i = e - r * n;
+      const size_t w = (size_t)r * np + i, stride = (size_t)rows * np;
+      double re, im;
+      if (r < pat.nH) {
+        const float2 o = G0[w];
+        re = o.x;
+        im = o.y;
+      } else {
+        re = d0g[i].x;
+        im = d0g[i].y;
+      }
+      if (inside) {
+        for (int j = 0; j < npwc; ++j) {
+          const double vr = vals[2 * (j * nv + seg)], vi = vals[2 * (j * nv + seg) + 1];
+          const float2 o = Hp[j * stride + w];
+          re += vr * o.x - vi * o.y;
+          im += vr * o.y + vi * o.x;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < DQH_MAX_MOD; ++j) {
+        if (j < nmod) {
+          const float2 o = Hm[j * stride + w];
+          re += fm[j].x * o.x - fm[j].y * o.y;
+          im += fm[j].x * o.y + fm[j].y * o.x;
+        }
+      }
+      if (r < pat.nH)
+        Gt[e] = make_float2((float)re, (float)im);
+      else
+        dcur[i] = make_double2(re, im);
+    }
+  };
+
+  // state and stages: registers, or global memory in owner order (KM)
+  double2 yr[KM ? 1 : NE], v[NE];
+  float2 kr[KM ? 1 : 7][KM ? 1 : NE];
+  double2 *const ym = gp<double2>(p.y) + (size_t)np * np;
+  float2 *const km = gp<float2>(p.work);
+  int k0 = 0, k6 = 6;  // KM: slots of stages 0 and 6, swapped on accepted steps
+  // a uniform base per access and the thread as a 32-bit lane offset (the opaque zero keeps
+  // the bases from being formed ahead and held)
+  auto slot = [&](int j, int q) -> float2 * {
+    int u = (j == 0 ? k0 : (j == 6 ? k6 : j)) * NU + NTH * q;
+    asm volatile("" : "+s"(u));
+    return km + u + (unsigned)tid;
+  };
+  auto own = [&](int q) { return tid + NTH * q < NU; };
+  auto yget = [&](int q) -> double2 {
+    if constexpr (KM)
+      return own(q) ? (ym + NTH * q)[(unsigned)tid] : make_double2(0.0, 0.0);
+    else
+      return yr[q];
+  };
+  auto yset = [&](int q, double2 x) {
+    if constexpr (KM) {
+      if (own(q)) (ym + NTH * q)[(unsigned)tid] = x;
+    } else {
+      yr[q] = x;
+    }
+  };
+  auto kget = [&](int j, int q) -> float2 {
+    if constexpr (KM)
+      return own(q) ? *slot(j, q) : make_float2(0.f, 0.f);
+    else
+      return kr[j][q];
+  };
+  auto kset = [&](int j, int q, float2 x) {
+    if constexpr (KM) {
+      if (own(q)) *slot(j, q) = x;
+    } else {
+      kr[j][q] = x;
+    }
+  };
+  {
+    const double2 *y0 = gp<const double2>(p.y);
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      int i, j;
+      at(q, i, j);
+      double2 x = own(q) ? y0[(size_t)i * np + j] : make_double2(0.0, 0.0);
+      if (i == j) x.y = 0.0;
+      yset(q, x);
+      v[q] = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int s = 0; s < 7; ++s) kset(s, q, make_float2(0.f, 0.f));
+    }
+  }
+
+  // k_s = f(v), with the tables rebuilt at (seg, tau) when asked
+  auto field = [&](int s, bool rebuild, int seg, double tau) {
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      int i, j;
+      at(q, i, j);
+      const float2 x = make_float2((float)v[q].x, (float)v[q].y);
+      const bool on = own(q);
+      ys[on ? j * LD + i : NLD] = make_float2(x.x, -x.y);
+      ys[on ? i * LD + j : NLD] = x;
+    }
+    if (rebuild) tables(seg, tau);
+    __syncthreads();
+    // QC elements at a time: each term keeps their reads in flight
+#pragma unroll
+    for (int c = 0; c < NE; c += QC) {
+      float fr[QC], fi[QC];
+      int i[QC], j[QC];
+#pragma unroll
+      for (int q = 0; q < QC; ++q) {
+        fr[q] = fi[q] = 0.f;
+        at(c + q, i[q], j[q]);
+      }
+#pragma unroll 2
+      for (int x = 0; x < pat.nH; ++x) {
+        const int o = pat.offH[x];
+#pragma unroll
+        for (int q = 0; q < QC; ++q) {
+          const float2 cr = Gt[x * n + i[q]], cc = Gt[x * n + j[q]];
+          const int e = i[q] * LD + j[q];
+          const float2 a = ys[min(max(e + o * LD, 0), NLD)], b = ys[min(max(e + o, 0), NLD)];
+          fr[q] = fmaf(cr.x, a.x, fmaf(-cr.y, a.y, fmaf(cc.x, b.x, fmaf(cc.y, b.y, fr[q]))));
+          fi[q] = fmaf(cr.x, a.y, fmaf(cr.y, a.x, fmaf(cc.x, b.y, fmaf(-cc.y, b.x, fi[q]))));
+        }
+      }
+#pragma unroll 2
+      for (int x = 0; x < pat.npair; ++x) {
+        const Part pr = pat.pair[x];
+        const int sh = pat.pa[x] * LD + pat.pb[x];
+#pragma unroll
+        for (int q = 0; q < QC; ++q) {
+          const float2 l = Lt[pr.x * n + i[q]], m = Lt[pr.y * n + j[q]];
+          const float2 z = ys[min(max(i[q] * LD + j[q] + sh, 0), NLD)];
+          const float cr = l.x * m.x + l.y * m.y, ci = l.y * m.x - l.x * m.y;
+          fr[q] = fmaf(cr, z.x, fmaf(-ci, z.y, fr[q]));
+          fi[q] = fmaf(cr, z.y, fmaf(ci, z.x, fi[q]));
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < QC; ++q) {
+        const double2 da = dcur[i[q]], db = dcur[j[q]];
+        double gr = da.x + db.x, gi = da.y - db.y;
+#pragma unroll 1
+        for (int x = 0; x < pat.nzero; ++x) {  // products of the main diagonals, in FP64
+          const float2 l = Lt[pat.zero[x].x * n + i[q]], m = Lt[pat.zero[x].y * n + j[q]];
+          gr += (double)l.x * m.x + (double)l.y * m.y;
+          gi += (double)l.y * m.x - (double)l.x * m.y;
+        }
+        const double2 u = v[c + q];
+        const double re = (double)fr[q] + (gr * u.x - gi * u.y);
+        const double im = (double)fi[q] + (gr * u.y + gi * u.x);
+        kset(s, c + q, make_float2((float)re, i[q] == j[q] ? 0.f : (float)im));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // the next stage overwrites ys
+  };
+
+  int par = 0;
+  auto save = [&](double h, const double (&w)[7], int isave) {
+    float2 *st = gp<float2>(p.states) + (size_t)isave * n * n;
+    double2 sv[NE];
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const double2 y = yget(q);
+      double re = 0.0, im = 0.0;
+      if (h != 0.0) {
+#pragma unroll
+        for (int j = 0; j < 7; ++j) {
+          const float2 kq = kget(j, q);
+          re += w[j] * (double)kq.x;
+          im += w[j] * (double)kq.y;
+        }
+      }
+      sv[q] = make_double2(y.x + h * re, y.y + h * im);
+      int i, j;
+      at(q, i, j);
+      if (save_states && own(q)) {
+        st[(size_t)i * n + j] = make_float2((float)sv[q].x, (float)sv[q].y);
+        if (i != j) st[(size_t)j * n + i] = make_float2((float)sv[q].x, (float)-sv[q].y);
+      }
+    }
+    const float2 *ET = gp<const float2>(p.EopsT);
+    for (int e = 0; e < nE; ++e) {
+      const float2 *E = ET + (size_t)e * np * np;
+      double s[2] = {0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < NE; ++q) {
+        if (own(q)) {
+          int i, j;
+          at(q, i, j);
+          const float2 o = E[(size_t)i * np + j];
+          s[0] += o.x * sv[q].x - o.y * sv[q].y;
+          s[1] += o.x * sv[q].y + o.y * sv[q].x;
+          if (i != j) {
+            const float2 m = E[(size_t)j * np + i];
+            s[0] += m.x * sv[q].x + m.y * sv[q].y;
+            s[1] += m.y * sv[q].x - m.x * sv[q].y;
+          }
+        }
+      }
+      block_sums<NTH>(s, red, par);
+      if (tid == 0) gp<float2>(p.expects)[(size_t)e * ntsave + isave] = make_float2((float)s[0], (float)s[1]);
+    }
+  };
+  const double w0[7] = {0, 0, 0, 0, 0, 0, 0};
+  auto weight = [&](int q) {
+    int i, j;
+    at(q, i, j);
+    return !own(q) ? 0.0 : (i == j ? 1.0 : 2.0);
+  };
+
+  double t = p.t0;
+  int isave = 0, status = 0;
+  int64_t nsteps = 0, nacc = 0, nrej = 0, nrhs = 0;
+  double next_save = ntsave > 0 ? tsave[0] : 0.0;
+  auto advance = [&]() {
+    ++isave;
+    if (isave < ntsave) next_save = tsave[isave];
+  };
+  int seg = -1;
+  double next_break = pwc ? ptimes[0] : 0.0;
+  auto locate = [&]() {
+    bool moved = false;
+    while (seg + 1 < nseg && next_break <= t) {
+      ++seg;
+      moved = true;
+      if (seg + 1 < nseg) next_break = ptimes[seg + 1];
+    }
+    return moved;
+  };
+  if (pwc) locate();
+  __syncthreads();  // the tables and the zeroed copy
+  while (isave < ntsave && next_save <= t) {
+    save(0.0, w0, isave);
+    advance();
+  }
+#pragma unroll
+  for (int q = 0; q < NE; ++q) v[q] = yget(q);
+  field(0, true, seg, t);
+  ++nrhs;
+
+  double dt;  // initial step, as in k_tsit5_diag
+  {
+    double s[2] = {0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const float2 kq = kget(0, q);
+      const double ay2 = v[q].x * v[q].x + v[q].y * v[q].y;
+      const double sc = atol + rtol * sqrt(ay2);
+      s[0] += weight(q) * ay2 / (sc * sc);
+      s[1] += weight(q) * ((double)kq.x * kq.x + (double)kq.y * kq.y) / (sc * sc);
+    }
+    block_sums<NTH>(s, red, par);
+    const double d0 = sqrt(s[0] * inv_nn), d1 = sqrt(s[1] * inv_nn);
+    const double h0 = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const float2 kq = kget(0, q);
+      v[q] = make_double2(v[q].x + h0 * kq.x, v[q].y + h0 * kq.y);
+    }
+    field(1, smooth, seg, t + h0);
+    ++nrhs;
+    double s2[1] = {0.0};
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const double2 y = yget(q);
+      const float2 ka = kget(0, q), kb = kget(1, q);
+      const double sc = atol + rtol * sqrt(y.x * y.x + y.y * y.y);
+      const double dr = (double)kb.x - ka.x, di = (double)kb.y - ka.y;
+      s2[0] += weight(q) * (dr * dr + di * di) / (sc * sc);
+    }
+    block_sums<NTH>(s2, red, par);
+    const double d2 = sqrt(s2[0] * inv_nn) / h0;
+    const double md = fmax(d1, d2);
+    const double h1 = md <= 1e-15 ? fmax(1e-6, h0 * 1e-3) : ctrl_pow(0.01 / md, kInitExp);
+    dt = fmin(100.0 * h0, h1);
+  }
+
+  bool need_k0 = false;
+  while (t < t_end) {
+    if (nsteps >= p.max_steps) {
+      status = DQH_MAX_STEPS;
+      break;
+    }
+    bool fresh = pwc && locate();  // the tables of the new segment, rebuilt with the next field
+    if (need_k0) {
+#pragma unroll
+      for (int q = 0; q < NE; ++q) v[q] = yget(q);
+      field(0, fresh || smooth, seg, t);
+      fresh = false;
+      ++nrhs;
+      need_k0 = false;
+    }
+    double h = dt, target = t_end;
+    bool target_jump = false;
+    if (pwc && seg + 1 < nseg && next_break < t_end) {
+      target = next_break;
+      target_jump = true;
+    }
+    bool made_jump = false;
+    double t_new = t + h;
+    if (snaps_to(t, h, target)) {
+      h = target - t;
+      t_new = target;
+      made_jump = target_jump;
+    }
+    if (!(h > 0.0) || !(h > 1e-14 * fmax(1.0, fabs(t)))) {
+      status = DQH_NONFINITE;
+      break;
+    }
+    // the increment form of k_tsit5_diag for constant generators (stages 1..5 on the
+    // increment alone); modulated ones evaluate every stage at the full input
+#pragma unroll
+    for (int s = 1; s < 7; ++s) {
+      CTab *w = weights<TAB>();
+      const double a0 = smooth ? w->A[s][0] : w->C[s];
+      if constexpr (!KM && NE > 1) {  // as pin_stages in k_tsit5_diag
+#pragma unroll
+        for (int j = 0; j < s; ++j)
+#pragma unroll
+          for (int q = 0; q < NE; ++q) asm volatile("" : "+v"(kr[j][q].x), "+v"(kr[j][q].y));
+      }
+#pragma unroll
+      for (int q = 0; q < NE; ++q) {
+        if constexpr (KM || NE > 2) __builtin_amdgcn_sched_barrier(0);
+        const float2 ka = kget(0, q);
+        double re = a0 * (double)ka.x, im = a0 * (double)ka.y;
+#pragma unroll
+        for (int j = 1; j < s; ++j) {
+          if (rk.A[s][j] != 0.0) {
+            const float2 kq = kget(j, q);
+            re += w->A[s][j] * (double)kq.x;
+            im += w->A[s][j] * (double)kq.y;
+          }
+        }
+        double2 y = make_double2(0.0, 0.0);
+        if (smooth || s == 6) y = yget(q);
+        v[q] = make_double2(y.x + h * re, y.y + h * im);
+      }
+      field(s, smooth || fresh, seg, t + w->C[s] * h);
+      fresh = false;
+    }
+    nrhs += 6;
+    CTab *we = weights<TAB>();
+    double ss[1] = {0.0};
+    double e0 = we->E[0];
+    if (!smooth) {
+#pragma unroll
+      for (int j = 1; j < 6; ++j) e0 += we->E[j];
+    }
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const float2 ka = kget(0, q);
+      const double2 y = yget(q);
+      double er = e0 * (double)ka.x, em = e0 * (double)ka.y;
+#pragma unroll
+      for (int j = 1; j < 7; ++j) {
+        if (rk.E[j] != 0.0) {
+          const float2 kq = kget(j, q);
+          er += we->E[j] * (double)kq.x;
+          em += we->E[j] * (double)kq.y;
+        }
+      }
+      er *= h;
+      em *= h;
+      const double sc = atol + rtol * sqrt(fmax(y.x * y.x + y.y * y.y, v[q].x * v[q].x + v[q].y * v[q].y));
+      ss[0] += weight(q) * (er * er + em * em) / (sc * sc);
+    }
+    block_sums<NTH>(ss, red, par);
+    const double norm = sqrt(ss[0] * inv_nn);
+    const bool finite = isfinite(norm);
+    const bool keep = finite && norm < 1.0;
+    double factor;
+    if (!finite)
+      factor = p.factormin;
+    else if (norm == 0.0)
+      factor = p.factormax;
+    else
+      factor = p.safety * ctrl_pow(norm, -0.2);
+    factor = fmin(fmax(factor, keep ? 1.0 : p.factormin), p.factormax);
+    ++nsteps;
+    if (keep) {
+      if (tid == 0 && nacc < p.step_log_cap) gp<double>(p.step_log)[nacc] = t_new;
+      ++nacc;
+      while (isave < ntsave && next_save <= t_new) {
+        const double th = (next_save - t) / h;
+        CTab *wr = weights<TAB>();
+        double w[7];
+#pragma unroll
+        for (int j = 0; j < 7; ++j)
+          w[j] = th * (wr->R[j][0] + th * (wr->R[j][1] + th * (wr->R[j][2] + th * wr->R[j][3])));
+        if (!smooth) fold_k0(w);
+        save(h, w, isave);
+        advance();
+      }
+#pragma unroll
+      for (int q = 0; q < NE; ++q) {
+        if constexpr (!KM) kr[0][q] = kr[6][q];
+        yset(q, v[q]);
+      }
+      const int sw = k0;
+      k0 = k6;
+      k6 = sw;
+      t = t_new;
+      need_k0 = made_jump;
+    } else {
+      ++nrej;
+    }
+    dt = factor * h;
+  }
+  while (isave < ntsave) {
+    save(0.0, w0, isave);
+    advance();
+  }
+  float2 *fin = gp<float2>(p.final_state);
+  float2 *st = gp<float2>(p.states);
+#pragma unroll
+  for (int q = 0; q < NE; ++q) {
+    if (own(q)) {
+      int i, j;
+      at(q, i, j);
+      const double2 y = yget(q);
+      const float2 x = make_float2((float)y.x, (float)y.y), xc = make_float2(x.x, -x.y);
+      fin[(size_t)i * n + j] = x;
+      if (i != j) fin[(size_t)j * n + i] = xc;
+      if (!save_states) {
+        st[(size_t)i * n + j] = x;
+        if (i != j) st[(size_t)j * n + i] = xc;
+      }
+    }
+  }
+  if (tid == 0) {
+    stats[0] = nsteps;
+    stats[1] = nacc;
+    stats[2] = nrej;
+    stats[3] = status;
+    stats[4] = nrhs;
+  }
+}
+
 // Shifts of the operators' stencil and the parts of their coefficients, sorted by shift
 // (so that an operator set and its zero-extended superset add up in the same order).
-// False when they exceed kMaxShift or kMaxPart.
+// nterm is kMaxShift + 1 when there are more shifts than the register form holds. False
+// when the parts exceed kMaxPart.
 bool make_pattern(const dqh_dia_ops &ops, int n, Pattern &pt) {
   std::memset(&pt, 0, sizeof(pt));
   std::vector<std::pair<std::pair<int, int>, Part>> parts;
@@ -585,6 +1129,7 @@ bool make_pattern(const dqh_dia_ops &ops, int n, Pattern &pt) {
   for (int x = 0; x < ops.noff[0]; ++x) {
     const int o = ops.off[0][x];
     if (o == 0) return false;  // the main diagonal goes in hdiag
+    pt.offH[x] = o;
     parts.push_back({{o, 0}, Part{0, (uint8_t)x, 0, 0}});
     parts.push_back({{0, o}, Part{1, (uint8_t)x, 0, 0}});
   }
@@ -598,6 +1143,10 @@ bool make_pattern(const dqh_dia_ops &ops, int n, Pattern &pt) {
           if (pt.nzero >= kMaxPart) return false;
           pt.zero[pt.nzero++] = part;
         } else {
+          if (pt.npair >= kMaxPart) return false;
+          pt.pa[pt.npair] = (int16_t)a;
+          pt.pb[pt.npair] = (int16_t)b;
+          pt.pair[pt.npair++] = part;
           parts.push_back({{a, b}, part});
         }
       }
@@ -608,7 +1157,10 @@ bool make_pattern(const dqh_dia_ops &ops, int n, Pattern &pt) {
   std::stable_sort(parts.begin(), parts.end(), [](const auto &l, const auto &r) { return l.first < r.first; });
   for (size_t i = 0; i < parts.size(); ++i) {
     if (i == 0 || parts[i].first != parts[i - 1].first) {
-      if (pt.nterm >= kMaxShift) return false;
+      if (pt.nterm >= kMaxShift) {
+        pt.nterm = kMaxShift + 1;
+        return true;
+      }
       pt.a[pt.nterm] = parts[i].first.first;
       pt.b[pt.nterm] = parts[i].first.second;
       pt.first[pt.nterm++] = (int32_t)i;
@@ -643,16 +1195,40 @@ int launch_size(const dqh_me_inst *d, int64_t ninst, int n, const Pattern &pt, h
   return launch<704, 3, T, TAB>(d, ninst, n, pt, st);
 }
 
+template <int NTH, int NE, bool KM, int TAB>
+int launch_tab(const dqh_me_inst *d, int64_t ninst, int n, const Pattern &pt, hipStream_t st) {
+  const size_t lds = (size_t)(n * row_stride(n) + 1 + (pt.nH + pt.nLrow) * n) * sizeof(float2) +
+                     (size_t)n * sizeof(double2) + (size_t)(4 * (NTH / 64)) * sizeof(double);
+  const void *fn = reinterpret_cast<const void *>(&k_tsit5_diag_tab<NTH, NE, KM, TAB>);
+  hipError_t err = hipSuccess;
+  if (lds > 160 * 1024) return fail(DQH_BAD_SHAPE, "dqh_mesolve_tsit5_diag: the operators' diagonals exceed the LDS");
+  if (lds > 65536) err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (err == hipSuccess) {
+    hipLaunchKernelGGL((k_tsit5_diag_tab<NTH, NE, KM, TAB>), dim3((unsigned)ninst), dim3(NTH), lds, st, d, pt);
+    err = hipGetLastError();
+  }
+  return err == hipSuccess ? DQH_OK : fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_diag: ") + hipGetErrorString(err));
+}
+
+template <int TAB>
+int launch_tab_size(const dqh_me_inst *d, int64_t ninst, int n, const Pattern &pt, hipStream_t st) {
+  const int nu = n * (n + 1) / 2;
+  if (nu <= 576) return launch_tab<576, 1, false, TAB>(d, ninst, n, pt, st);
+  if (nu <= 2048) return launch_tab<1024, 2, false, TAB>(d, ninst, n, pt, st);
+  if (nu <= 4096) return launch_tab<1024, 4, false, TAB>(d, ninst, n, pt, st);
+  return launch_tab<1024, 8, true, TAB>(d, ninst, n, pt, st);
+}
+
 }  // namespace diag
 }  // namespace dqh
 
 using namespace dqh;
 
 extern "C" int dqh_mesolve_tsit5_diag(const dqh_me_inst *d_insts, int64_t ninst, int64_t n, const dqh_dia_ops *ops,
-                                      int64_t flags, void *stream) {
+                                      int64_t flags, int64_t modulated, void *stream) {
   if (!d_insts || !ops || ninst <= 0 || ninst > (1 << 30))
     return fail(DQH_BAD_ARG, "dqh_mesolve_tsit5_diag: bad arguments");
-  if (n <= 0 || n > 64) return fail(DQH_BAD_SHAPE, "dqh_mesolve_tsit5_diag: 1 <= n <= 64");
+  if (n <= 0 || n >= 128) return fail(DQH_BAD_SHAPE, "dqh_mesolve_tsit5_diag: 1 <= n < 128");
   if (ops->nops < 1 || ops->nops > DQH_DIA_MAXOPS)
     return fail(DQH_BAD_ARG, "dqh_mesolve_tsit5_diag: 1 <= nops <= 8 (the generator, then the jump operators)");
   for (int s = 0; s < ops->nops; ++s) {
@@ -664,9 +1240,15 @@ extern "C" int dqh_mesolve_tsit5_diag(const dqh_me_inst *d_insts, int64_t ninst,
   }
   diag::Pattern pt;
   if (!diag::make_pattern(*ops, (int)n, pt))
-    return fail(DQH_BAD_SHAPE, "dqh_mesolve_tsit5_diag: at most 12 shifts and no main diagonal in operator 0");
+    return fail(DQH_BAD_SHAPE, "dqh_mesolve_tsit5_diag: at most 48 parts and no main diagonal in operator 0");
   hipStream_t st = (hipStream_t)stream;
   const bool dopri5 = (flags & DQH_FLAG_DOPRI5) != 0;
+  // the register form for what fits its registers and LDS (the guards of far shifts) and is
+  // constant over a step; the table form for the rest
+  if (n > 64 || pt.nterm > diag::kMaxShift || modulated ||
+      diag::lds_bytes<704>((int)n, pt.nH, pt.nLrow, pt.guard) > 150 * 1024)
+    return dopri5 ? diag::launch_tab_size<1>(d_insts, ninst, (int)n, pt, st)
+                  : diag::launch_tab_size<0>(d_insts, ninst, (int)n, pt, st);
   if (pt.nterm <= 6)
     return dopri5 ? diag::launch_size<6, 1>(d_insts, ninst, (int)n, pt, st)
                   : diag::launch_size<6, 0>(d_insts, ninst, (int)n, pt, st);

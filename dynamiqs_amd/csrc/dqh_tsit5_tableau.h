@@ -63,8 +63,8 @@ constexpr RKTab kRKTabs[2] = {
       {0, 1.3824689317781436, -3.764937863556287, 2.382468931778144}}},
 };
 
-// the tableaus for kernels that select the pair at run time; kernels compiled for one
-// pair read kRKTabs, whose entries become literals
+// the tableaus in device memory; kernels compiled for one pair also read kRKTabs where
+// they drop zero weights at compile time
 static __constant__ RKTab kRK[2] = {kRKTabs[0], kRKTabs[1]};
 
 // Initial step h1 = (0.01 / max(d1, d2))^kInitExp (Hairer-Norsett-Wanner II.4). The

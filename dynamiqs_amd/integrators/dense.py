@@ -230,7 +230,7 @@ class DensePlan:
             _native.check(
                 lib.dqh_mesolve_tsit5_diag(
                     c_p(self.d_descs.data_ptr()), self.ninst, self.n, _native.ctypes.byref(self.stencil.ops),
-                    int(self.descs['flags'][0]) & _native.FLAG_DOPRI5, sp,
+                    int(self.descs['flags'][0]) & _native.FLAG_DOPRI5, int(np.any(self.descs['nmod'] > 0)), sp,
                 ),
                 'dqh_mesolve_tsit5_diag',
             )
@@ -506,10 +506,9 @@ def _hmods(inst: Instance) -> list:
 
 
 # limits of dqh_mesolve_tsit5_diag (dqh_diag.hip)
-STENCIL_MAX_N = 64
-STENCIL_MAX_SHIFTS = 12
+STENCIL_MAX_N = 127
 STENCIL_MAX_PARTS = 48
-STENCIL_MAX_LDS = 150 * 1024
+STENCIL_WORK_N = 90  # above it the stages and the state are in global memory
 
 
 @dataclass
@@ -548,15 +547,18 @@ def _offsets(mask: np.ndarray) -> list:
 
 def few_diagonals(instances: list, npad: int) -> Stencil | None:
     """The :class:`Stencil` of a batch, or None where the few-diagonal kernel does not take
-    it: n above STENCIL_MAX_N, time-dependent jump operators or modulated terms, or more
-    shifts, coefficient parts or LDS than the kernel holds. At n = 64 with 12 shifts the
-    stencil needs 13 multiply-adds per element against (1 + 2K) 64 of the dense products,
-    so within these limits it is always the faster form."""
+    it: n above STENCIL_MAX_N, time-dependent jump operators, or more diagonals than pay.
+    The parts of the stencil are two per off-diagonal and one per pair of diagonals of a
+    jump operator. Up to 12 shifts run from registers, always faster (n = 64, 10 parts, 32
+    instances, 18 steps: 0.50 ms against 2.73 dense); beyond, the parts are read from LDS:
+    n = 16, 16 parts 0.25 against 0.27 ms, n = 32, 28 parts 0.41 against 0.60, n = 64, 41
+    parts 2.6 against 1.9. Above n = 64 the dense form holds nothing in LDS (n = 90, 41
+    parts: 2.4 against 15.4 ms)."""
     n = instances[0].H.shape[-1]
     K = len(instances[0].Ls)
     if n > STENCIL_MAX_N or K > 7:
         return None
-    if any(i.mod or i.Cs is not None or i.expanded or i.Lsum or any(x is not None for x in i.Lmod or [])
+    if any(i.Cs is not None or i.expanded or i.Lsum or any(x is not None for x in i.Lmod or [])
            or any(x is not None for x in i.Lpwc or []) for i in instances):
         return None
     ids = {}
@@ -584,18 +586,12 @@ def few_diagonals(instances: list, npad: int) -> Stencil | None:
         if explicit[k]:
             G[k] = instances[b].Hnh
     mask = np.any(G != 0, axis=0)
-    for inst in {id(o): o for i in instances for (_, _, o) in i.pwc}.values():
-        mask = mask | (np.asarray(inst) != 0)
+    for term in {id(o): o for i in instances for o in [p[2] for p in i.pwc] + [m[1] for m in i.mod]}.values():
+        mask = mask | (np.asarray(term) != 0)
     offH = [o for o in _offsets(mask) if o != 0]
     offL = [_offsets(m) for m in np.any(Lall != 0, axis=0)] if K else []
-    rowsL = sum(len(o) for o in offL)
-    shifts = {(o, 0) for o in offH} | {(0, o) for o in offH} | {(p, q) for o in offL for p in o for q in o}
-    shifts.discard((0, 0))
     parts = 2 * len(offH) + sum(len(o) ** 2 for o in offL)
-    guard = max((abs(a * (n | 1) + b) for a, b in shifts), default=0)
-    lds = 8 * (2 * (n * (n | 1) + 1 + guard) + guard + (len(offH) + rowsL) * n) + 16 * n + 1024
-    if (len(shifts) > STENCIL_MAX_SHIFTS or parts > STENCIL_MAX_PARTS or lds > STENCIL_MAX_LDS
-            or len(offH) > 16 or any(len(o) > 16 for o in offL)):
+    if parts > (max(12, min(n, 24)) if n <= 64 else STENCIL_MAX_PARTS) or len(offH) > 16:
         return None
     from .dia import DiaOps
 
@@ -814,12 +810,34 @@ def build_plan(
             if block.size:
                 descs[f] = u(arena.put(block)) + idx.astype(u) * u(block[0].nbytes)
 
-    def bpwc(inst):
-        """-i O_j of the PWC terms: matrices, or their rows for the stencil kernel."""
-        if stencil is None:
-            return _pad(np.stack([-1j * o for (_, _, o) in inst.pwc]), npad).astype(np.complex64)
-        O = -1j * np.stack([np.asarray(o, dtype=np.complex128) for (_, _, o) in inst.pwc])
-        return _rows_on(O, [*stencil.offH, 0], npad).astype(np.complex64)
+    def bterms(ops):
+        """-i O_j of time-dependent terms: matrices, or their rows for the stencil kernel."""
+        O = -1j * np.stack([np.asarray(o, dtype=np.complex128) for o in ops])
+        return (_pad(O, npad) if stencil is None else _rows_on(O, [*stencil.offH, 0], npad)).astype(np.complex64)
+
+    def pack_pwc(d, inst):
+        if not inst.pwc:
+            return
+        grid, samplers = pwc_sampling(inst.pwc)
+        vals = np.stack([np.where(inside, np.asarray(v, dtype=np.complex128)[idx], 0.0)
+                         for (_, v, _), (idx, inside) in zip(inst.pwc, samplers)])
+        d['npwc'], d['nseg'] = len(inst.pwc), len(grid)
+        d['Hpwc'] = shared(('Hpwc', inst.key_H), lambda: bterms([o for (_, _, o) in inst.pwc]))
+        d['pwc_times'] = shared(('ptimes', inst.key_H), lambda: grid)
+        d['pwc_vals'] = arena.put(np.ascontiguousarray(vals).view(np.float64))
+
+    def pack_mod(d, inst, hm, fns, hkey):
+        """Tables of the functions ``fns`` [(g, key)] on one grid, and the operators of the
+        Hamiltonian-side terms ``hm`` (the first of them)."""
+        tabs = [mod_table(g, key) for (g, key) in fns]
+        nint = max(len(c) for (_, _, c) in tabs)
+        tabs = [spline_table(g, t_tab, t_stop, n0=nint, nmax=nint) if len(c) != nint else (a, dtt, c)
+                for (g, _), (a, dtt, c) in zip(fns, tabs)]
+        d['nmod'] = len(hm)
+        d['mod_t0'], d['mod_dt'], d['mod_nint'] = tabs[0][0], tabs[0][1], nint
+        d['mod_coef'] = arena.put(np.ascontiguousarray(np.stack([c for (_, _, c) in tabs])).view(np.float64))
+        if hm:
+            d['Hmod'] = shared(hkey, lambda: bterms([o for (_, o, _) in hm]))
 
     for b, inst in enumerate(instances):
         d = descs[b]
@@ -829,14 +847,9 @@ def build_plan(
             d['t0'] = float(ts_i[0] if inst.t0 is None else inst.t0)
             d['t1'] = float(ts_i[-1])
         if stencil is not None:
-            if inst.pwc:
-                grid, samplers = pwc_sampling(inst.pwc)
-                vals = np.stack([np.where(inside, np.asarray(v, dtype=np.complex128)[idx], 0.0)
-                                 for (_, v, _), (idx, inside) in zip(inst.pwc, samplers)])
-                d['npwc'], d['nseg'] = len(inst.pwc), len(grid)
-                d['Hpwc'] = shared(('Hpwc', inst.key_H), lambda inst=inst: bpwc(inst))
-                d['pwc_times'] = shared(('ptimes', inst.key_H), lambda grid=grid: grid)
-                d['pwc_vals'] = arena.put(np.ascontiguousarray(vals).view(np.float64))
+            pack_pwc(d, inst)
+            if inst.mod:
+                pack_mod(d, inst, inst.mod, [(g, key) for (g, _, key) in inst.mod], ('Hmod', inst.key_H, None))
             continue
         d['EopsT'] = p_E
         d['flags'] = _native.FLAG_SAVE_STATES if save_states else 0
@@ -915,16 +928,9 @@ def build_plan(
                 )
                 d['pwc_times'] = shared(('ptimes', inst.key_H, inst.key_L, tuple(lpwc)), lambda grid=grid: grid)
                 d['pwc_vals'] = arena.put(np.ascontiguousarray(np.stack(rows)).view(np.float64))
-            elif inst.pwc:
-                grid, samplers = pwc_sampling(inst.pwc)
-                vals = np.stack([np.where(inside, np.asarray(v, dtype=np.complex128)[idx], 0.0)
-                                 for (_, v, _), (idx, inside) in zip(inst.pwc, samplers)])
-                d['npwc'] = len(inst.pwc)
-                d['nseg'] = len(grid)
+            else:
+                pack_pwc(d, inst)
                 npwc_max = max(npwc_max, len(inst.pwc))
-                d['Hpwc'] = shared(('Hpwc', inst.key_H), lambda inst=inst: bpwc(inst))
-                d['pwc_times'] = shared(('ptimes', inst.key_H), lambda grid=grid: grid)
-                d['pwc_vals'] = arena.put(np.ascontiguousarray(vals).view(np.float64))
             hm = _hmods(inst)
             if hm or any(lmod):
                 # tables: the nmod Hamiltonian-side terms, then (DQH_FLAG_LMOD) one per jump
@@ -935,18 +941,7 @@ def build_plan(
                             else (_one, ('one',)) for k in range(K)]
                 if inst.expanded:
                     fns += [inst.Lbmod[k] if inst.Lbmod[k] is not None else (_one, ('one',)) for k in range(K)]
-                tabs = [mod_table(g, key) for (g, key) in fns]
-                nint = max(len(c) for (_, _, c) in tabs)
-                tabs = [spline_table(g, t_tab, t_stop, n0=nint, nmax=nint) if len(c) != nint else (a, dtt, c)
-                        for (g, _), (a, dtt, c) in zip(fns, tabs)]
-                d['nmod'] = len(hm)
-                d['mod_t0'], d['mod_dt'], d['mod_nint'] = tabs[0][0], tabs[0][1], nint
-                d['mod_coef'] = arena.put(np.ascontiguousarray(np.stack([c for (_, _, c) in tabs])).view(np.float64))
-                if hm:
-                    d['Hmod'] = shared(
-                        ('Hmod', inst.key_H, inst.key_L if any(lmod) else None),
-                        lambda hm=hm: _pad(np.stack([-1j * o for (_, o, _) in hm]), npad).astype(np.complex64),
-                    )
+                pack_mod(d, inst, hm, fns, ('Hmod', inst.key_H, inst.key_L if any(lmod) else None))
         else:  # rouchon1: Kraus sets per (PWC segment, step length)
             d['nL'] = nLdev
             grid = None
@@ -1026,8 +1021,8 @@ def build_plan(
         welems += 2 * nLdev * nn
     if dopri8:  # stages 7..12 after the generator slot: (16 + nL) np^2
         welems = max(welems, (16 + nLdev) * nn)
-    if stencil is not None:  # everything lives in registers and LDS
-        welems = 0
+    if stencil is not None:  # everything lives in registers and LDS, or the stages in work
+        welems = 7 * (n * (n + 1) // 2) if n > STENCIL_WORK_N else 0
     work = arena.empty(B * welems * 8)
     y = torch.zeros((B, 2, nn, 2), dtype=torch.float64, device=dev)
     y0 = np.zeros((B, npad, npad), dtype=np.complex128)
@@ -1067,6 +1062,8 @@ def build_plan(
         row, u = npad * 8, np.uint64
         extents = {'Hnh': np.full(B, len(stencil.offH) * row, dtype=u), 'Dops': np.full(B, stencil.L.shape[1] * row, dtype=u),
                    'Hpwc': descs['npwc'].astype(u) * u((len(stencil.offH) + 1) * row),
+                   'Hmod': descs['nmod'].astype(u) * u((len(stencil.offH) + 1) * row),
+                   'work': np.full(B, welems * 8, dtype=u),
                    'pwc_times': descs['nseg'].astype(u) * u(8),
                    'pwc_vals': descs['npwc'].astype(u) * np.maximum(descs['nseg'].astype(np.int64) - 1, 0).astype(u) * u(16)}
     check_descriptors(descs, [*arena.tensors, work, states, final, expects, stats] + ([step_log] if step_log is not None else []),

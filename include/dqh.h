@@ -341,25 +341,27 @@ typedef struct dqh_dia_ops {
   uint64_t diags[DQH_DIA_MAXOPS];
 } dqh_dia_ops;
 
-/* Adaptive Tsit5 / Dopri5 of small instances (n <= 64) whose operators have few nonzero
- * diagonals, one workgroup per instance: the vector field as a stencil of at most 12
- * shifts (two per off-diagonal of the generator, one per pair of diagonals of a jump
- * operator, equal shifts once). ``ops`` names the diagonals, shared by the batch:
- * operator 0 the generator G = -iH - 1/2 sum L^dag L without its main diagonal, operators
- * 1.. the jump operators (``ops->diags`` is not read). The descriptors carry the values,
- * as rows of np elements indexed by the row of the matrix (row of offset o holds
- * A[i][i + o] at i, zero where i + o is outside):
+/* Adaptive Tsit5 / Dopri5 of small instances (n < 128) whose operators have few nonzero
+ * diagonals, one workgroup per instance: the vector field as a stencil with two shifts per
+ * off-diagonal of the generator and one per pair of diagonals of a jump operator (at most
+ * 48 in all). ``ops`` names the diagonals, shared by the batch: operator 0 the generator
+ * G = -iH - 1/2 sum L^dag L without its main diagonal, operators 1.. the jump operators
+ * (``ops->diags`` is not read). The descriptors carry the values, as rows of np elements
+ * indexed by the row of the matrix (row of offset o holds A[i][i + o] at i, zero where
+ * i + o is outside):
  *   Hnh   const c64[noff[0]][np]              off-diagonals of the constant part of G
  *   hdiag const double2[np]                   its main diagonal
  *   Dops  const c64[sum noff[1..]][np]        diagonals of the jump operators, in order
  *   Hpwc  const c64[npwc][noff[0] + 1][np]    -i O_j of each PWC term: its values on the
  *                                             offsets of operator 0, then its main diagonal
- * Cops, work, nL and HAS_HNH are not read; nmod must be 0 and DQH_FLAG_GLOBAL, _LMOD,
- * _DOPRI8 unset. ``flags``: DQH_FLAG_DOPRI5 or 0, as in every descriptor. Everything
- * else is as in dqh_mesolve_tsit5_dense. An instance that does not fit gets the status
- * DQH_UNSUPPORTED. */
+ *   Hmod  const c64[nmod][noff[0] + 1][np]    the same for the modulated terms
+ * work: 7 n (n + 1) / 2 complex64 elements for n > 90, else not read. Cops, nL and HAS_HNH
+ * are not read; DQH_FLAG_GLOBAL, _LMOD and _DOPRI8 must be unset. ``flags``:
+ * DQH_FLAG_DOPRI5 or 0, as in every descriptor; ``modulated``: nonzero if any descriptor has
+ * nmod > 0. Everything else is as in dqh_mesolve_tsit5_dense. An instance that does not
+ * fit gets the status DQH_UNSUPPORTED. */
 int dqh_mesolve_tsit5_diag(const dqh_me_inst *d_insts, int64_t ninst, int64_t n, const dqh_dia_ops *ops,
-                           int64_t flags, void *stream);
+                           int64_t flags, int64_t modulated, void *stream);
 
 /* A batch of Rouchon1 solves sharing their (constant, DIA) operators and differing
  * in rho0. Set 0 is used for every step but the last, set nsets-1 for the last one

@@ -38,7 +38,7 @@ def _field(st, b, rho):
 
 @pytest.mark.parametrize('n,offH,offL', [
     (1, [0], [[0]]), (2, [-1, 1], [[1]]), (5, [0], []), (16, [-1, 0, 1], [[1]]), (64, [-2, 0, 2], [[1], [2]]),
-    (33, [-4, 4], [[0], [-3]]), (20, [0], [[-1, 1]]), (9, [-8, 8], [[8], [-8]]), (12, [], [[0, 1]]),
+    (33, [-4, 4], [[0], [-3]]), (20, [0], [[-1, 1]]), (65, [-8, -1, 1, 8], [[1], [8], [0, 3]]), (127, [0, 1], [[-11, 1]]), (100, [-3, -2, -1, 1, 2, 3], [[0, 1, 2, 3], [-5, 5]]), (9, [-8, 8], [[8], [-8]]), (12, [], [[0, 1]]),
 ])
 def test_stencil_rows_give_the_vector_field(n, offH, offL):
     rng = np.random.default_rng(n)
@@ -71,8 +71,8 @@ def test_explicit_generators_and_instances_without_keys():
 
 
 @pytest.mark.parametrize('why,kw', [
-    ('dense', dict(offH=list(range(-9, 10)))), ('shifts', dict(offL=[[0, 1, 2, 3]])), ('size', dict(n=65)),
-    ('jump operators', dict(offL=[[0]] * 8)), ('LDS', dict(n=64, offH=[60], offL=[[60]])),
+    ('dense', dict(offH=list(range(-9, 10)))), ('pairs', dict(offL=[[0, 1, 2, 3]])), ('parts', dict(n=100, offL=[list(range(7))])), ('size', dict(n=128)),
+    ('jump operators', dict(offL=[[0]] * 8)),
 ])
 def test_everything_else_stays_on_the_dense_kernels(why, kw):
     rng = np.random.default_rng(1)
@@ -89,6 +89,6 @@ def test_time_dependent_terms():
     st = dense.few_diagonals([dense.Instance(**kw, pwc=[(np.array([0.0, 1.0]), np.ones(1), X)])], 16)
     assert st.offH == [-1, 1]  # the PWC term's diagonals join the generator's
     g = lambda t: 1.0  # noqa: E731
-    assert dense.few_diagonals([dense.Instance(**kw, mod=[(g, X, None)])], 16) is None
+    assert dense.few_diagonals([dense.Instance(**kw, mod=[(g, X, None)])], 16).offH == [-1, 1]
     assert dense.few_diagonals([dense.Instance(**kw, Lmod=[(g, None)])], 16) is None
     assert dense.few_diagonals([dense.Instance(**kw, Lpwc=[(np.array([0.0, 1.0]), np.ones(1))])], 16) is None

@@ -1,7 +1,8 @@
 """GPU parity of the few-diagonal Tsit5 / Dopri5 kernel (``dqh_mesolve_tsit5_diag``)
 against the complex128 oracle replaying the GPU's own accepted steps, at the edges of its
-size classes (1, 64, 192 and 576 threads with one element, then two and three elements per
-thread), with no, one and several shifts, and with PWC terms."""
+size classes (64, 192 and 576 threads with one element, then two and three elements per
+thread; with tables up to n = 90 in registers and above in memory), with no, one and many
+shifts, far offsets, and with PWC and modulated terms."""
 
 import numpy as np
 import pytest
@@ -18,7 +19,11 @@ def _banded(rng, n, offs, scale=1.0):
     return x
 
 
-def _insts(n, offH, offL, B, pwc=False):
+def _drive(t):
+    return 0.7 * np.cos(5.0 * t)
+
+
+def _insts(n, offH, offL, B, pwc=False, mod=False):
     from dynamiqs_amd.integrators.dense import Instance
 
     rng = np.random.default_rng(n + len(offH))
@@ -30,7 +35,8 @@ def _insts(n, offH, offL, B, pwc=False):
         psi /= np.linalg.norm(psi)
         X = _banded(rng, n, [1, 0])
         terms = [(np.array([0.1, 0.5, 0.8]), rng.normal(size=2) + 0j, X + X.conj().T)] if pwc else []
-        out.append(Instance(H=H + H.conj().T, Ls=Ls, rho0=psi @ psi.conj().T, pwc=terms, key_H=(b,), key_L=(), key_rho=(b,)))
+        mods = [(_drive, X + X.conj().T, ('drive',))] if mod else []
+        out.append(Instance(H=H + H.conj().T, Ls=Ls, rho0=psi @ psi.conj().T, pwc=terms, mod=mods, key_H=(b,), key_L=(), key_rho=(b,)))
     return out
 
 
@@ -42,6 +48,8 @@ def _replay(inst, tsave, ends, method):
         for times, vals, op in inst.pwc:
             if times[0] <= tseg < times[-1]:
                 H = H + vals[np.searchsorted(times, tseg, side='right') - 1] * op
+        for g, op, _ in inst.mod:
+            H = H + g(t) * op
         return lindblad.rhs_hermitian(H, inst.Ls, y)
 
     kw = dict(tab=tsit5.tableau('dopri5')) if method == 'dopri5' else {}
@@ -55,6 +63,10 @@ CASES = [
     (33, [-1, 0, 1], [[1], [-1], [0]], 'tsit5'), (34, [-5, -1, 0, 1, 5], [[1], [5]], 'tsit5'),
     (47, [0, 1], [[1]], 'tsit5'), (48, [-1, 1], [[2]], 'dopri5'), (64, [-2, 0, 2], [[1], [2]], 'tsit5'),
     (64, [-8, -1, 0, 1, 8], [[1], [8], [0]], 'tsit5'),
+    # the table form: far offsets, many pairs, sizes above 64
+    (64, [-62, 62], [[62], [-60]], 'tsit5'), (20, [0, 1], [[0, 1, 2], [1]], 'dopri5'), (63, [-1, 1], [[-1, 0, 1], [5]], 'tsit5'),
+    (65, [-8, -1, 0, 1, 8], [[1], [8]], 'tsit5'), (90, [-9, 9], [[9], [1], [0]], 'dopri5'),
+    (91, [-10, 10], [[10], [0, 1]], 'tsit5'), (127, [-1, 0, 1], [[1], [126]], 'tsit5'),
 ]
 
 
@@ -63,8 +75,8 @@ def test_matches_fp64_replay(n, offH, offL, method):
     from dynamiqs_amd.integrators import dense
 
     tsave = np.linspace(0.0, 1.0, 6)
-    for pwc in (False, True):
-        insts = _insts(n, offH, offL, 3, pwc)
+    for pwc, mod in ((False, False), (True, False), (True, True)):
+        insts = _insts(n, offH, offL, 3, pwc, mod)
         E = np.diag(np.arange(n)) + 0j
         plan = dense.build_plan('tsit5', insts, tsave, exp_ops=[E], rtol=1e-6, atol=1e-8, step_log_cap=4000,
                                 tableau=method, dia_ops=True)
@@ -75,14 +87,18 @@ def test_matches_fp64_replay(n, offH, offL, method):
         for b, inst in enumerate(insts):
             ref = _replay(inst, tsave, out['step_ends'][b], method)
             # FP32 stages: about nsteps^(1/2) roundings of 6e-8 (the dense kernels' replay bar)
-            assert np.linalg.norm(out['states'][b] - ref, axis=(-2, -1)).max() <= 2e-6, (n, pwc, b)
+            assert np.linalg.norm(out['states'][b] - ref, axis=(-2, -1)).max() <= 2e-6, (n, pwc, mod, b)
             assert np.abs(out['expects'][b, 0] - np.einsum('ij,tji->t', E, out['states'][b])).max() <= 1e-5 * n
             assert np.array_equal(out['states'][b], np.swapaxes(out['states'][b].conj(), -1, -2))
             assert np.array_equal(out['final_state'][b], out['states'][b, -1])
-        # the same step sequence as the dense kernels up to rounding, and bit-identical alone
-        dplan = dense.build_plan('tsit5', insts, tsave, rtol=1e-6, atol=1e-8, tableau=method)
-        dplan.run()
-        assert np.all(np.abs(dplan.results()['nsteps'] - out['nsteps']) <= 2)
+        if not mod:
+            # the step sequence of the dense kernels up to rounding. (With modulated terms the
+            # stages are evaluated at the full state, and their FP32 rounding, 6e-8 |f| each,
+            # is of the size of atol in the error estimate, so the sequences differ.)
+            dplan = dense.build_plan('tsit5', insts, tsave, rtol=1e-6, atol=1e-8, tableau=method)
+            dplan.run()
+            assert np.all(np.abs(dplan.results()['nsteps'] - out['nsteps']) <= 2)
+        # bit-identical alone
         solo = dense.build_plan('tsit5', insts[1:2], tsave, rtol=1e-6, atol=1e-8, tableau=method, dia_ops=True)
         solo.run()
         assert np.array_equal(solo.results()['states'][0], out['states'][1])
