@@ -890,9 +890,8 @@ extern "C" int dqh_mesolve_rouchon1_dia(const dqh_dia_rouchon1 *pb, void *stream
     ++isave;
   }
   if (p.nE > 0)
-    hipLaunchKernelGGL(k_expect_states, dim3((unsigned)p.nsave, (unsigned)p.ninst), dim3(256), 0, st, p.n_true, p.nsave,
-                       p.nE, states, reinterpret_cast<const float2 *>(p.EopsT),
-                       reinterpret_cast<float2 *>(p.expects));
+    launch_expect(p.n_true, p.nsave, p.ninst, p.nE, p.states, p.EopsT, p.expects, reinterpret_cast<void *>(p.work),
+                  2 * (size_t)p.n * p.n * p.ninst * sizeof(float2), st);
   hipError_t err = hipGetLastError();
   if (err == hipSuccess && t_count > 0) {
     err = hipEventSynchronize(ev[3 * t_count - 1]);

@@ -1,54 +1,88 @@
-// Adaptive Tsit5 for sparse-DIA master equations (gfx950).
+// Adaptive Tsit5 / Dopri5 for sparse-DIA master equations (gfx950).
 //
 // The large-n counterpart of the persistent dense kernel: a state of n = 1024
-// does not fit one workgroup, so every Tsit5 stage is one grid-wide launch over
-// all instances (64 x 64 output tiles per workgroup, the DIA Lindblad stencil
-// of dqh_dia_tile.h) and the step controller lives on the device:
-//   stage s = 1..6  k_s = f(ys_s) at the tile, then ys_{s+1} = y + h sum a_{s+1,j} k_j
-//                   at the same elements (only k_j of the element itself is
-//                   needed, so no second sweep); stage 6 also accumulates the
-//                   scaled error of y1 = y + h sum b_j k_j in FP64 per workgroup;
-//   commit          every workgroup reduces its instance's partial sums in the same
-//                   order (identical accept/reject and dt everywhere, no atomics),
-//                   writes dense-output saves, y <- y1 in FP64 on accept, and forms
-//                   ys_1 = y + h' a_10 k_0 of the next attempt; workgroup 0 writes
-//                   the instance's control block for the next step.
-// Control blocks are double-buffered by step parity (every kernel of a step reads
-// block `cur`, the commit writes block `1 - cur`), so a fixed sequence of launches
-// is valid for any step and is captured once as a hipGraph of graph_steps steps
-// and replayed. Instances keep their own t, dt, counters and save cursor; an
-// instance that is done turns every later launch into an early return. The host
-// loop reads a completion count after each replay; max_steps bounds the number of
-// replays. Semantics follow diffrax_integrator.py:59-81, 101-147 (Tsit5 + PID
-// controller + SaveAt dense output) as the dense kernel implements them.
+// does not fit one workgroup, so every stage is one grid-wide launch over all
+// instances and the step controller lives on the device. Every launch is bound by HBM
+// (or, for small batches, by the latency of one launch), so the design counts bytes:
+//   * a Hermitian rho0 stays Hermitian, so only the upper triangle is swept (64-column
+//     strips of 4 NE rows). Stencil reads may cross the diagonal by at most `spread`
+//     elements; the writers keep that band below the diagonal up to date. A rho0 that is
+//     not Hermitian (checked on the device) takes the same kernels over the full matrix;
+//   * stages 1..5 evaluate the field on the increment Delta_s = h sum_j a_sj k_j alone
+//     (constant generators): g_s = f(Delta_s) = k_s - k_0, so neither the FP64 state nor
+//     a rounded copy of it is read; stage 1 is h a_10 f(k_0), without an input of its own;
+//   * stage 5 writes the candidate y1 in FP64 (a second state buffer) and stage 6 reads
+//     its stencil input from it, so accepting a step moves nothing: the buffers swap roles;
+//   * accept / reject, saves and the next dt are formed at the start of the next step's
+//     stage 1, by every workgroup from the same partial sums in the same order (identical
+//     decisions everywhere, no atomics).
+// Bytes per element and step: 24 + 40 + 48 + 56 + 88 + 88 = 344, of half the elements,
+// against 496 of all of them with the full-matrix form on rounded states.
+// Measured (rtol 1e-6, atol 1e-8, two coupled modes with 8 shifts): four solves of n = 1024,
+// 36 steps, 22.6 -> 6.9 ms, stages at 3.8 to 5.3 TB/s (a copy reaches 4.7); one of
+// n = 323, 29 steps, 2.8 -> 1.24 ms, bound by the latency of a launch (about 5 us).
+// Time-dependent Hamiltonians take full stage inputs y + Delta_s instead (the generator
+// changes between the stages), and a separate controller launch before the first stage.
+//
+// Control blocks are double-buffered by step parity (a step reads the other block and
+// writes block `cur`), so a fixed sequence of launches is valid for any step and is
+// captured once as a hipGraph of graph_steps steps and replayed. Instances keep their own
+// t, dt, counters and save cursor; an instance that is done turns every later launch into
+// an early return. The host loop reads a completion count after each replay; max_steps
+// bounds the number of replays. Semantics follow diffrax_integrator.py:59-81, 101-147
+// (Tsit5 + PID controller + SaveAt dense output) as the dense kernel implements them.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 
 #include "dqh.h"
 #include "dqh_common.h"
 #include "dqh_dia_tile.h"
+#include "dqh_dia_tri.h"
 #include "dqh_expect.h"
 #include "dqh_tsit5_tableau.h"
 
 namespace dqh {
 namespace diats {
 
+using namespace tri;
+
 struct Ctrl {
   double t, dt;
-  int64_t nsteps, nacc, nrej, status, isave, rot;  // rot: slot of k_0 in the 7 stage buffers
+  int64_t nsteps, nacc, nrej, status, isave, rot;  // rot: slot of k_0 in the 7 stage buffers, and the flags below
 };
 static_assert(sizeof(Ctrl) == 64, "control block is 64 bytes");
 
+// Ctrl::rot: slot of k_0 (bits 0-2), and
+constexpr int64_t kJump = 8;    // the last accepted step ended on a PWC breakpoint: k_0 is evaluated anew
+constexpr int64_t kFresh = 16;  // no attempt to commit yet
+constexpr int64_t kSel = 32;    // the state is in the second FP64 buffer
+
+// One shift of the stencil: f[i][j] += r[i + p] conj(c[j + q]) X[i + p][j + q]. One-sided
+// products have a vector of ones on the other side. tdr / tdc: the vector belongs to the
+// time-dependent generator (one copy per instance).
+struct Term {
+  const float2 *r, *c;
+  int32_t p, q, tdr, tdc;
+};
+static_assert(sizeof(Term) == 32, "terms are read as 32-byte scalars");
+constexpr int kMaxTerm = 2 * DQH_DIA_MAXOFF + (DQH_DIA_MAXOPS - 1) * DQH_DIA_MAXOFF * DQH_DIA_MAXOFF;
+
 struct V {
   int64_t n, n_true, ninst, nsave, max_steps, npart, flags;
+  int32_t herm, spread, nterm, nb, total;  // nb: 64-element blocks per side; total: tiles per instance
+  int32_t presum;  // the control blocks are formed by k_ctl
   double rtol, atol, safety, fmin_, fmax_, t0, t1, inv_nn;
   float2 *k;      // [7][ninst][n][n]
   float2 *ys;     // [2][ninst][n][n]
+  double2 *y2;    // [ninst][n][n]: second FP64 state
+  Term *terms;
+  float2 *ones;   // [n]
   double *part;   // [ninst][2][npart]
   Ctrl *ctrl;     // [2][ninst]
-  int64_t *flag;  // completion count
+  int64_t *flag;  // completion count; before the first step: rho0 is not Hermitian
   double2 *y;     // [ninst][n][n]
   const double *tsave;
   float2 *states;
@@ -66,11 +100,6 @@ struct V {
 };
 
 __device__ __forceinline__ bool is_done(const Ctrl &c, double t1) { return c.status != 0 || !(c.t < t1); }
-// step of the attempt described by c: the proposed dt, or exactly the rest of the
-// interval when it would end within the snapping tolerance of t1
-// Ctrl::rot holds the slot of k_0 (bits 0-2) and kJump: the last accepted step ended on
-// a PWC breakpoint, so k_0 of the next step is evaluated anew (k_stage with s = 0)
-constexpr int64_t kJump = 8;
 
 // searchsorted(ptimes, t, 'right') - 1: the PWC segment of t (-1 before the first breakpoint)
 __device__ __forceinline__ int seg_of(const V &v, double t) {
@@ -92,6 +121,8 @@ __device__ __forceinline__ double target_of(const V &v, double t) {
   }
   return v.t1;
 }
+// step of the attempt described by c: the proposed dt, or exactly the rest of the
+// interval when it would end within the snapping tolerance of t1
 __device__ __forceinline__ double step_h(const V &v, const Ctrl &c) {
   const double tg = target_of(v, c.t);
   return snaps_to(c.t, c.dt, tg) ? tg - c.t : c.dt;
@@ -108,145 +139,124 @@ __device__ __forceinline__ bool ends_on_jump(const V &v, const Ctrl &c) {
 
 __device__ __forceinline__ float2 *kslot(const V &v, int j, int64_t rot, size_t inst) {
   const size_t nn = (size_t)v.n * v.n;
-  return v.k + ((size_t)((j + (rot & 7)) % 7) * v.ninst + inst) * nn;
+  return v.k + ((size_t)((j + (int)(rot & 7)) % 7) * v.ninst + inst) * nn;
 }
 __device__ __forceinline__ float2 *ysbuf(const V &v, int which, size_t inst) {
   const size_t nn = (size_t)v.n * v.n;
   return v.ys + ((size_t)which * v.ninst + inst) * nn;
 }
+// the FP64 state (other = 0) or the buffer of the candidate (other = 1)
+__device__ __forceinline__ double2 *ybuf(const V &v, int64_t rot, int other, size_t inst) {
+  const size_t nn = (size_t)v.n * v.n;
+  return (((rot & kSel) != 0) != (other != 0) ? v.y2 : v.y) + inst * nn;
+}
 __device__ __forceinline__ double *partial(const V &v, size_t inst, int which) {
   return v.part + (inst * 2 + which) * v.npart;
 }
 
-// FP64 sum over the workgroup; every thread returns the same value.
-template <int NT>
+// FP64 sum over a workgroup of 256; every thread returns the same value.
 __device__ __forceinline__ double block_sum(double x, double *sh) {
   for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
   __syncthreads();
-  double s = 0.0;
-#pragma unroll
-  for (int w = 0; w < NT / 64; ++w) s += sh[w];
-  return s;
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-// Sum of one partial array of an instance, the same order in every workgroup.
-template <int NT>
-__device__ __forceinline__ double reduce_partials(const double *p, int64_t npart, double *sh) {
+// Sum of m partials of an instance, the same order in every workgroup.
+__device__ __forceinline__ double reduce_partials(const double *p, int64_t m, double *sh) {
   double s = 0.0;
-  for (int64_t b = threadIdx.x; b < npart; b += NT) s += p[b];
-  return block_sum<NT>(s, sh);
+  for (int64_t b = threadIdx.x; b < m; b += 256) s += p[b];
+  return block_sum(s, sh);
 }
 
 __device__ __forceinline__ double sq(double2 v) { return v.x * v.x + v.y * v.y; }
-
-// Visit the output elements of this workgroup: the tile (HALO > 0, 512 threads,
-// the stage input staged in LDS with that halo) or one element per thread
-// (HALO == 0, 256 threads, neighbours read through the caches). fn(i, j, f)
-// receives the vector field f at (i, j).
-template <int HALO, class Fn>
-__device__ __forceinline__ void sweep(const V &v, const dqh_dia_ops &ops, const float2 *in, float2 *sx, Fn fn,
-                                      const float2 *D0 = nullptr) {
-  const int64_t n = v.n;
-  if constexpr (HALO > 0) {
-    int i0, j0;
-    diat::tile_of(n, i0, j0);
-    diat::load_halo<HALO>(sx, in, nullptr, n, i0, j0);
-    __syncthreads();
-    const int jj = threadIdx.x & (diat::kTJ - 1);
-#pragma unroll 1
-    for (int m = 0; m < diat::kRowsPerThread; ++m) {
-      const int ii = (threadIdx.x >> 6) + (diat::kThreads / diat::kTJ) * m;
-      const int i = i0 + ii, j = j0 + jj;
-      fn(i, j, diat::stencil(diat::LdsX<HALO>::at(sx, ii, jj), ops, false, n, i, j, D0));
-    }
-  } else {
-    int i, j;
-    if (diat::row_elem(n, i, j)) {
-      const diat::GlobalX X{in, nullptr, n, i, j};
-      fn(i, j, diat::stencil(X, ops, false, n, i, j, D0));
-    }
-  }
+__device__ __forceinline__ double2 add(double2 a, double w, float2 x) {
+  return make_double2(a.x + w * (double)x.x, a.y + w * (double)x.y);
 }
+__device__ __forceinline__ float2 f32(double2 a) { return make_float2((float)a.x, (float)a.y); }
 
-template <int HALO>
-constexpr int nthreads() {
-  return HALO > 0 ? diat::kThreads : 256;
+// stencil inputs: an FP32 matrix, an FP64 one, or y + s k
+struct InF {
+  const float2 *b;
+  __device__ __forceinline__ float2 operator()(size_t e) const { return b[e]; }
+};
+struct InY {
+  const double2 *y;
+  __device__ __forceinline__ float2 operator()(size_t e) const { return f32(y[e]); }
+};
+struct InYK {
+  const double2 *y;
+  const float2 *k;
+  double s;
+  __device__ __forceinline__ float2 operator()(size_t e) const { return f32(add(y[e], s, k[e])); }
+};
+
+typedef const __attribute__((address_space(4))) Term CTerm;
+typedef const __attribute__((address_space(4))) float CFloat;
+typedef const __attribute__((address_space(1))) float GFloat;
+
+// f(X) at rows i0 .. i0 + NE - 1 of column j (columns past the matrix read column
+// n_true - 1 and are dropped by the caller). The row factors are wave-uniform scalars,
+// out-of-range neighbours have a zero factor.
+template <int NE, bool TD, class In>
+__device__ __forceinline__ void stencil(const V &v, size_t inst, const In &X, int i0, int j, float2 (&f)[NE]) {
+  const int nt = v.nterm, n = (int)v.n, lim = (int)v.n_true;
+#pragma unroll
+  for (int m = 0; m < NE; ++m) f[m] = make_float2(0.f, 0.f);
+  CTerm *terms = (CTerm *)v.terms;
+  const size_t hs = TD ? inst * (size_t)v.noff0 * v.n : 0;
+  auto group = [&](auto cnt, int t0) {
+    constexpr int U = decltype(cnt)::value;
+    float2 c[U], x[U][NE];
+    float rx[U][NE], ry[U][NE];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      CTerm &t = terms[t0 + u];
+      const int q = j + t.q, qc = min(max(q, 0), lim - 1);
+      GFloat *cp = (GFloat *)t.c;
+      CFloat *rp = (CFloat *)t.r;
+      if (TD && t.tdc) cp += 2 * hs;
+      if (TD && t.tdr) rp += 2 * hs;
+      c[u] = make_float2(cp[2 * qc], cp[2 * qc + 1]);
+      if (q != qc) c[u] = make_float2(0.f, 0.f);
+#pragma unroll
+      for (int m = 0; m < NE; ++m) {
+        const int a = i0 + m + t.p, ac = min(max(a, 0), lim - 1);
+        const float wx = rp[2 * ac], wy = rp[2 * ac + 1];
+        rx[u][m] = a == ac ? wx : 0.f;
+        ry[u][m] = a == ac ? wy : 0.f;
+        x[u][m] = X((size_t)ac * n + qc);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int m = 0; m < NE; ++m) {
+        const float kr = fmaf(rx[u][m], c[u].x, ry[u][m] * c[u].y);
+        const float ki = fmaf(ry[u][m], c[u].x, -(rx[u][m] * c[u].y));
+        f[m].x = fmaf(kr, x[u][m].x, fmaf(-ki, x[u][m].y, f[m].x));
+        f[m].y = fmaf(kr, x[u][m].y, fmaf(ki, x[u][m].x, f[m].y));
+      }
+    }
+  };
+  constexpr int U = NE > 1 ? 4 : 8;
+  int t = 0;
+  for (; t + U <= nt; t += U) group(std::integral_constant<int, U>{}, t);
+  for (; t < nt; ++t) group(std::integral_constant<int, 1>{}, t);
+  if (v.herm) {
+#pragma unroll
+    for (int m = 0; m < NE; ++m)
+      if (i0 + m == j) f[m].y = 0.f;
+  }
 }
 
 // ------------------------------------------------------------------ one step
-template <int HALO>
-__global__ __launch_bounds__(nthreads<HALO>()) void k_stage(V v, dqh_dia_ops ops, int s, int cur) {
-  const RKTab &rk = rk_tab(v.flags);
-  constexpr int NT = nthreads<HALO>();
-  __shared__ double sh[NT / 64];
-  float2 *sx = nullptr;
-  if constexpr (HALO > 0) {
-    __shared__ float2 lds[diat::Tile<HALO>::NX];
-    sx = lds;
-  }
-  const size_t inst = blockIdx.y;
-  const Ctrl c = v.ctrl[(size_t)cur * v.ninst + inst];
-  if (is_done(c, v.t1)) return;
-  // s = 0: k_0 = f(y) after a step that ended on a breakpoint (input: y in ys buffer 1)
-  if (s == 0 && !(c.rot & kJump)) return;
+// The outcome of the attempt of control block c, whose error partials sum to esum (norm
+// squared times n^2): accept or reject and the next dt, as the next attempt's block.
+__device__ __forceinline__ Ctrl outcome(const V &v, const Ctrl &c, double esum) {
   const double h = step_h(v, c);
-  const int64_t n = v.n;
-  const size_t nn = (size_t)n * n;
-  const double2 *y = v.y + inst * nn;
-  float2 *ks = kslot(v, s, c.rot, inst);
-  float2 *nxt = ysbuf(v, s & 1, inst);
-  double acc = 0.0;
-  sweep<HALO>(v, ops, ysbuf(v, (s + 1) & 1, inst), sx, [&](int i, int j, float2 f) {
-    const size_t e = (size_t)i * n + j;
-    ks[e] = f;
-    const double2 yv = y[e];
-    if (s < 6) {
-      double re = yv.x + h * rk.A[s + 1][s] * f.x, im = yv.y + h * rk.A[s + 1][s] * f.y;
-      for (int q = 0; q < s; ++q) {
-        const float2 kq = kslot(v, q, c.rot, inst)[e];
-        re += h * rk.A[s + 1][q] * kq.x;
-        im += h * rk.A[s + 1][q] * kq.y;
-      }
-      nxt[e] = make_float2((float)re, (float)im);
-    } else if (i < v.n_true && j < v.n_true) {
-      double er = rk.E[6] * f.x, ei = rk.E[6] * f.y, yr = yv.x, yi = yv.y;
-      for (int q = 0; q < 6; ++q) {
-        const float2 kq = kslot(v, q, c.rot, inst)[e];
-        er += rk.E[q] * kq.x;
-        ei += rk.E[q] * kq.y;
-        yr += h * rk.A[6][q] * kq.x;
-        yi += h * rk.A[6][q] * kq.y;
-      }
-      er *= h;
-      ei *= h;
-      const double sc = v.atol + v.rtol * fmax(sqrt(sq(yv)), sqrt(yr * yr + yi * yi));
-      acc += (er * er + ei * ei) / (sc * sc);
-    }
-  }, v.hcur ? v.hcur + inst * (size_t)v.noff0 * n : nullptr);
-  if (s == 6) {
-    const double tot = block_sum<NT>(acc, sh);
-    if (threadIdx.x == 0) partial(v, inst, 0)[blockIdx.x] = tot;
-  }
-}
-
-// accept/reject, saves, y update, next stage input; grid (ceil(n^2/256), ninst)
-__global__ __launch_bounds__(256) void k_commit(V v, int cur) {
-  const RKTab &rk = rk_tab(v.flags);
-  __shared__ double sh[4];
-  const size_t inst = blockIdx.y;
-  const Ctrl c = v.ctrl[(size_t)cur * v.ninst + inst];
-  Ctrl *nx = v.ctrl + (size_t)(1 - cur) * v.ninst + inst;
-  const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
-  if (is_done(c, v.t1)) {
-    if (writer) *nx = c;
-    return;
-  }
-  const double h = step_h(v, c);
-  const double t_new = step_end(v, c);
-  const bool jump = ends_on_jump(v, c);
-  const double norm = sqrt(reduce_partials<256>(partial(v, inst, 0), v.npart, sh) * v.inv_nn);
+  const double norm = sqrt(esum * v.inv_nn);
   const bool finite = isfinite(norm);
   const bool keep = finite && norm < 1.0;
   double factor;
@@ -259,16 +269,15 @@ __global__ __launch_bounds__(256) void k_commit(V v, int cur) {
   factor = fmin(fmax(factor, keep ? 1.0 : v.fmin_), v.fmax_);
   Ctrl o = c;
   o.nsteps += 1;
-  int64_t is_end = c.isave;
   if (keep) {
     o.nacc += 1;
-    o.t = t_new;
-    o.rot = ((c.rot & 7) + 6) % 7 + (jump ? kJump : 0);  // FSAL: k_6 of this step is k_0 of the next
-    while (is_end < v.nsave && v.tsave[is_end] <= t_new) ++is_end;
-    o.isave = is_end;
+    o.t = step_end(v, c);
+    // FSAL: k_6 of this step is k_0 of the next; the candidate becomes the state
+    o.rot = (((c.rot & 7) + 6) % 7) | (ends_on_jump(v, c) ? kJump : 0) | ((c.rot & kSel) ^ kSel);
+    while (o.isave < v.nsave && v.tsave[o.isave] <= o.t) ++o.isave;
   } else {
     o.nrej += 1;
-    o.rot = c.rot & 7;
+    o.rot = c.rot & ~kJump;
   }
   o.dt = factor * h;
   if (o.t < v.t1) {
@@ -279,61 +288,231 @@ __global__ __launch_bounds__(256) void k_commit(V v, int cur) {
       if (!(hn > 0.0) || !(hn > 1e-14 * fmax(1.0, fabs(o.t)))) o.status = DQH_NONFINITE;
     }
   }
-  const int64_t n = v.n;
-  const size_t nn = (size_t)n * n;
-  int i, j;
-  if (diat::row_elem(n, i, j)) {
-    const int64_t e = (int64_t)i * n + j;
-    double2 *yp = v.y + inst * nn + e;
-    const double2 yv = *yp;
-    double2 y1 = yv;
-    float2 k0n = kslot(v, 0, c.rot, inst)[e];
-    if (keep) {
+  return o;
+}
+
+__device__ __forceinline__ Ctrl next_ctrl(const V &v, const Ctrl &c, size_t inst, double *sh) {
+  if (is_done(c, v.t1) || (c.rot & kFresh)) {
+    Ctrl o = c;
+    o.rot &= ~kFresh;
+    return o;
+  }
+  return outcome(v, c, reduce_partials(partial(v, inst, 0), v.total, sh));
+}
+
+// The control block of the next attempt (block cur, from block 1 - cur), formed by every
+// workgroup of the instance alike and stored by workgroup 0, or read where k_ctl has
+// formed it; and the saves of the step that block 1 - cur describes.
+template <int NE, bool TD>
+__device__ __forceinline__ Ctrl commit(const V &v, int cur, size_t inst, int id, int i0, int j, double *sh) {
+  const RKTab &rk = rk_tab(v.flags);
+  const Ctrl c = v.ctrl[(size_t)(1 - cur) * v.ninst + inst];
+  Ctrl *nx = v.ctrl + (size_t)cur * v.ninst + inst;
+  Ctrl o;
+  if (v.presum) {
+    o = *nx;
+  } else {
+    o = next_ctrl(v, c, inst, sh);
+    if (id == 0 && threadIdx.x == 0) *nx = o;
+  }
+  const int64_t is_end = o.isave;
+  const double h = step_h(v, c);
+  if (is_end > c.isave) {
+    const int64_t ntn = v.n_true * v.n_true;
+    const double2 *y = ybuf(v, c.rot, 0, inst);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      const int i = i0 + m;
+      if (!owned(v, i, j)) continue;
+      const size_t e = (size_t)i * v.n + j;
       float2 kk[7];
 #pragma unroll
       for (int q = 0; q < 7; ++q) kk[q] = kslot(v, q, c.rot, inst)[e];
-      const int64_t ntn = v.n_true * v.n_true;
+      const double2 yv = y[e];
       for (int64_t is = c.isave; is < is_end; ++is) {
         const double th = (v.tsave[is] - c.t) / h;
-        double re = yv.x, im = yv.y;
+        double w[7];
 #pragma unroll
-        for (int q = 0; q < 7; ++q) {
-          const double w = th * (rk.R[q][0] + th * (rk.R[q][1] + th * (rk.R[q][2] + th * rk.R[q][3])));
-          re += h * w * kk[q].x;
-          im += h * w * kk[q].y;
+        for (int q = 0; q < 7; ++q)
+          w[q] = th * (rk.R[q][0] + th * (rk.R[q][1] + th * (rk.R[q][2] + th * rk.R[q][3])));
+        if (!TD) fold_k0(w);
+        double2 s = yv;
+#pragma unroll
+        for (int q = 0; q < 7; ++q) s = add(s, h * w[q], kk[q]);
+        float2 *st = v.states + (inst * v.nsave + is) * ntn;
+        float2 x = f32(s);
+        st[(size_t)i * v.n_true + j] = x;
+        if (v.herm && i != j) {
+          x.y = -x.y;
+          st[(size_t)j * v.n_true + i] = x;
         }
-        if (i < v.n_true && j < v.n_true)
-          v.states[(inst * v.nsave + is) * ntn + (size_t)i * v.n_true + j] = make_float2((float)re, (float)im);
       }
-#pragma unroll
-      for (int q = 0; q < 6; ++q) {
-        y1.x += h * rk.A[6][q] * kk[q].x;
-        y1.y += h * rk.A[6][q] * kk[q].y;
-      }
-      *yp = y1;
-      k0n = kk[6];
-      // on a breakpoint, the next step evaluates k_0 = f(y1) with the new segment's H
-      if (jump) ysbuf(v, 1, inst)[e] = make_float2((float)y1.x, (float)y1.y);
-    }
-    if (!is_done(o, v.t1)) {
-      const double hn = step_h(v, o);
-      ysbuf(v, 0, inst)[e] = make_float2((float)(y1.x + hn * rk.A[1][0] * k0n.x), (float)(y1.y + hn * rk.A[1][0] * k0n.y));
     }
   }
-  if (writer) *nx = o;
+  return o;
+}
+
+// Stage S. Constant generators (TD = false): slots 1..5 hold the increments g_S.
+// S = 0 (TD only): k_0 = f(y) after a step that ended on a breakpoint.
+template <int S, int NE, bool TD>
+__global__ __launch_bounds__(256) void k_stage(V v, int cur) {
+  const RKTab &rk = rk_tab(v.flags);
+  __shared__ double sh[4];
+  const size_t inst = blockIdx.y;
+  int id, i0, j;
+  if (!tile<NE>(v, id, i0, j)) return;
+  Ctrl c;
+  if constexpr (S == 1 && !TD)
+    c = commit<NE, TD>(v, cur, inst, id, i0, j, sh);
+  else
+    c = v.ctrl[(size_t)cur * v.ninst + inst];
+  if (is_done(c, v.t1)) return;
+  if (S == 0 && !(c.rot & kJump)) return;
+  const double h = step_h(v, c);
+  double acc = 0.0;
+  // a wave without elements (past the matrix, below the diagonal) only joins the sum
+  const int jw = j - ((int)threadIdx.x & 63);
+  if (i0 >= 0 && i0 < (int)v.n_true && jw < (int)v.n_true && (!v.herm || jw + 63 >= i0)) {
+    const int jc = min(j, (int)v.n_true - 1);
+    // this element's own operands: in flight while the stencil runs, except for the many
+    // of stages 5 and 6 with several rows, whose registers would halve the waves per SIMD
+    constexpr int NK = S == 6 ? 6 : S;
+    constexpr bool kAfter = NE > 1 && S >= 5;
+    float2 kq[NK > 0 ? NK : 1][NE];
+    double2 yv[NE], y1[NE];
+    auto own = [&]() {
+#pragma unroll
+      for (int m = 0; m < NE; ++m) {
+        const size_t e = (size_t)min(i0 + m, (int)v.n_true - 1) * v.n + jc;
+#pragma unroll
+        for (int q = 0; q < NK; ++q) kq[q][m] = kslot(v, q, c.rot, inst)[e];
+        if (S >= 5 || (TD && S >= 1)) yv[m] = ybuf(v, c.rot, 0, inst)[e];
+        if (S == 6) y1[m] = ybuf(v, c.rot, 1, inst)[e];
+      }
+    };
+    if (!kAfter) own();
+    float2 f[NE];
+    if constexpr (S == 0)
+      stencil<NE, TD>(v, inst, InY{ybuf(v, c.rot, 0, inst)}, i0, jc, f);
+    else if constexpr (S == 6)
+      stencil<NE, TD>(v, inst, InY{ybuf(v, c.rot, 1, inst)}, i0, jc, f);
+    else if constexpr (S == 1 && TD)
+      stencil<NE, TD>(v, inst, InYK{ybuf(v, c.rot, 0, inst), kslot(v, 0, c.rot, inst), h * rk.A[1][0]}, i0, jc, f);
+    else if constexpr (S == 1)
+      stencil<NE, TD>(v, inst, InF{kslot(v, 0, c.rot, inst)}, i0, jc, f);
+    else
+      stencil<NE, TD>(v, inst, InF{ysbuf(v, S & 1, inst)}, i0, jc, f);
+    if (kAfter) {
+      // the loads stay behind the stencil
+      asm volatile("" ::: "memory");
+      own();
+    }
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      const int i = i0 + m;
+      if (!owned(v, i, j)) continue;
+      const size_t e = (size_t)i * v.n + j;
+      if constexpr (S == 1 && !TD) {  // f is linear: f(h a_10 k_0) = h a_10 f(k_0)
+        const double s = h * rk.A[1][0];
+        f[m] = make_float2((float)(s * (double)f[m].x), (float)(s * (double)f[m].y));
+      }
+      float2 *ks = kslot(v, S, c.rot, inst);
+      if constexpr (S == 0 || S == 6)
+        put(v, ks, i, j, f[m]);
+      else
+        ks[e] = f[m];
+      if constexpr (S >= 1 && S <= 5) {
+        // increments: the weight of k_0 is the row sum C
+        double2 d = add(make_double2(0.0, 0.0), TD ? rk.A[S + 1][0] : rk.C[S + 1], kq[0][m]);
+#pragma unroll
+        for (int q = 1; q < S; ++q) d = add(d, rk.A[S + 1][q], kq[q][m]);
+        d = add(d, rk.A[S + 1][S], f[m]);
+        d.x *= h;
+        d.y *= h;
+        if (TD || S == 5) {
+          d.x += yv[m].x;
+          d.y += yv[m].y;
+        }
+        if constexpr (S == 5)
+          put(v, ybuf(v, c.rot, 1, inst), i, j, d);
+        else
+          put(v, ysbuf(v, (S + 1) & 1, inst), i, j, f32(d));
+      }
+      if constexpr (S == 6) {
+        double e0 = rk.E[0];
+        if (!TD) {
+#pragma unroll
+          for (int q = 1; q < 6; ++q) e0 += rk.E[q];
+        }
+        double2 er = add(make_double2(0.0, 0.0), e0, kq[0][m]);
+#pragma unroll
+        for (int q = 1; q < 6; ++q) er = add(er, rk.E[q], kq[q][m]);
+        er = add(er, rk.E[6], f[m]);
+        er.x *= h;
+        er.y *= h;
+        const double sc = v.atol + v.rtol * sqrt(fmax(sq(yv[m]), sq(y1[m])));
+        acc += (v.herm && i != j ? 2.0 : 1.0) * sq(er) / (sc * sc);
+      }
+    }
+  }
+  if constexpr (S == 6) {
+    const double tot = block_sum(acc, sh);
+    if (threadIdx.x == 0) partial(v, inst, 0)[id] = tot;
+  }
+}
+
+// the controller alone (time-dependent generators: the diagonals are rebuilt between it
+// and the first stage)
+template <int NE>
+__global__ __launch_bounds__(256) void k_commit(V v, int cur) {
+  __shared__ double sh[4];
+  int id, i0, j;
+  if (!tile<NE>(v, id, i0, j)) return;
+  (void)commit<NE, true>(v, cur, blockIdx.y, id, i0, j, sh);
+}
+
+// the control blocks alone, for grids in which every workgroup forming them costs more
+// than one more launch
+__global__ __launch_bounds__(256) void k_ctl(V v, int cur) {
+  __shared__ double sh[4];
+  const size_t inst = blockIdx.x;
+  const Ctrl o = next_ctrl(v, v.ctrl[(size_t)(1 - cur) * v.ninst + inst], inst, sh);
+  if (threadIdx.x == 0) v.ctrl[(size_t)cur * v.ninst + inst] = o;
 }
 
 // number of instances that are done, after an even number of steps (parity 0)
 __global__ __launch_bounds__(256) void k_count(V v) {
   __shared__ double sh[4];
   double cnt = 0.0;
-  for (int64_t b = threadIdx.x; b < v.ninst; b += 256) cnt += is_done(v.ctrl[b], v.t1) ? 1.0 : 0.0;
-  const double tot = block_sum<256>(cnt, sh);
+  for (int64_t b = threadIdx.x; b < v.ninst; b += 256) cnt += is_done(v.ctrl[v.ninst + b], v.t1) ? 1.0 : 0.0;
+  const double tot = block_sum(cnt, sh);
   if (threadIdx.x == 0) *v.flag = (int64_t)(tot + 0.5);
 }
 
 // ------------------------------------------------------------- initial step
-// Control block, stage input ys_0 = y0 and the saves at tsave <= t0.
+// The list of shifts, the vector of ones, and the flag that k_init sets.
+__global__ __launch_bounds__(256) void k_setup(V v, dqh_dia_ops ops) {
+  for (int64_t e = threadIdx.x; e < v.n; e += 256) v.ones[e] = make_float2(1.f, 0.f);
+  if (threadIdx.x != 0) return;
+  *v.flag = 0;
+  int m = 0;
+  const int td = v.hcur != nullptr;
+  const float2 *D0 = td ? v.hcur : diat::cgp<float2>(ops.diags[0]);
+  for (int u = 0; u < ops.noff[0]; ++u) {
+    const float2 *d = D0 + (size_t)u * v.n;
+    const int p = ops.off[0][u];
+    v.terms[m++] = Term{d, v.ones, p, 0, td, 0};
+    v.terms[m++] = Term{v.ones, d, 0, p, 0, td};
+  }
+  for (int s = 1; s < ops.nops; ++s) {
+    const float2 *A = diat::cgp<float2>(ops.diags[s]);
+    for (int u = 0; u < ops.noff[s]; ++u)
+      for (int w = 0; w < ops.noff[s]; ++w)
+        v.terms[m++] = Term{A + (size_t)u * v.n, A + (size_t)w * v.n, ops.off[s][u], ops.off[s][w], 0, 0};
+  }
+}
+
+// Control block and the saves at tsave <= t0; sets the flag where rho0 is not Hermitian.
 __global__ __launch_bounds__(256) void k_init(V v) {
   const size_t inst = blockIdx.y;
   int64_t is0 = 0;
@@ -341,14 +520,15 @@ __global__ __launch_bounds__(256) void k_init(V v) {
   const int64_t n = v.n;
   const size_t nn = (size_t)n * n;
   int i, j;
-  if (diat::row_elem(n, i, j)) {
-    const int64_t e = (int64_t)i * n + j;
-    const double2 yv = v.y[inst * nn + e];
-    const float2 f = make_float2((float)yv.x, (float)yv.y);
-    ysbuf(v, 0, inst)[e] = f;
+  if (diat::row_elem(n, i, j) && i < v.n_true && j < v.n_true) {
+    const double2 *y = v.y + inst * nn;
+    const double2 yv = y[(int64_t)i * n + j];
+    const float2 f = f32(yv);
     const int64_t ntn = v.n_true * v.n_true;
-    if (i < v.n_true && j < v.n_true)
-      for (int64_t is = 0; is < is0; ++is) v.states[(inst * v.nsave + is) * ntn + (size_t)i * v.n_true + j] = f;
+    for (int64_t is = 0; is < is0; ++is) v.states[(inst * v.nsave + is) * ntn + (size_t)i * v.n_true + j] = f;
+    if (j >= i) {
+      if (!hermitian_at(y, n, i, j)) *v.flag = 1;
+    }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     Ctrl c;
@@ -364,100 +544,91 @@ __global__ __launch_bounds__(256) void k_init(V v) {
 }
 
 // pass 0: k_0 = f(y0), partials |y0|^2 / sc^2 and |k_0|^2 / sc^2;
-// pass 1: f(y0 + h0 k_0), partials |f - k_0|^2 / sc^2 (sc = atol + rtol |y0|).
+// pass 1: partials |f(y0 + h0 k_0) - k_0|^2 / sc^2 (sc = atol + rtol |y0|), for constant
+// generators from f(y0 + h0 k_0) - k_0 = h0 f(k_0); h0 is in control block 1.
 // Hairer-Norsett-Wanner II.4 starting step as the dense kernel computes it.
-template <int HALO>
-__global__ __launch_bounds__(nthreads<HALO>()) void k_init_rhs(V v, dqh_dia_ops ops, int pass) {
-  constexpr int NT = nthreads<HALO>();
-  __shared__ double sh[NT / 64];
-  float2 *sx = nullptr;
-  if constexpr (HALO > 0) {
-    __shared__ float2 lds[diat::Tile<HALO>::NX];
-    sx = lds;
-  }
+template <int NE, bool TD>
+__global__ __launch_bounds__(256) void k_init_rhs(V v, int pass) {
+  __shared__ double sh[4];
   const size_t inst = blockIdx.y;
+  int id, i0, j;
+  if (!tile<NE>(v, id, i0, j)) return;
   if (is_done(v.ctrl[inst], v.t1)) return;
-  const int64_t n = v.n;
-  const size_t nn = (size_t)n * n;
-  const double2 *y = v.y + inst * nn;
+  const double2 *y = ybuf(v, 0, 0, inst);
   float2 *k0 = kslot(v, 0, 0, inst);
   double a0 = 0.0, a1 = 0.0;
-  sweep<HALO>(v, ops, ysbuf(v, pass, inst), sx, [&](int i, int j, float2 f) {
-    const size_t e = (size_t)i * n + j;
-    const double2 yv = y[e];
-    const double sc = v.atol + v.rtol * sqrt(sq(yv));
-    if (pass == 0) {
-      k0[e] = f;
-      if (i < v.n_true && j < v.n_true) {
-        a0 += sq(yv) / (sc * sc);
-        a1 += ((double)f.x * f.x + (double)f.y * f.y) / (sc * sc);
+  if (i0 >= 0 && i0 < (int)v.n_true) {
+    const int jc = min(j, (int)v.n_true - 1);
+    const double h0 = pass == 0 ? 0.0 : v.ctrl[v.ninst + inst].dt;
+    float2 f[NE];
+    if (pass == 0)
+      stencil<NE, TD>(v, inst, InY{y}, i0, jc, f);
+    else if (TD)
+      stencil<NE, TD>(v, inst, InYK{y, k0, h0}, i0, jc, f);
+    else
+      stencil<NE, TD>(v, inst, InF{k0}, i0, jc, f);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      const int i = i0 + m;
+      if (!owned(v, i, j)) continue;
+      const size_t e = (size_t)i * v.n + j;
+      const double2 yv = y[e];
+      const double sc = v.atol + v.rtol * sqrt(sq(yv)), w = v.herm && i != j ? 2.0 : 1.0;
+      if (pass == 0) {
+        put(v, k0, i, j, f[m]);
+        a0 += w * sq(yv) / (sc * sc);
+        a1 += w * sq(make_double2(f[m].x, f[m].y)) / (sc * sc);
+      } else {
+        double2 d = make_double2(h0 * (double)f[m].x, h0 * (double)f[m].y);
+        if (TD) {
+          const float2 kq = k0[e];
+          d = make_double2((double)f[m].x - kq.x, (double)f[m].y - kq.y);
+        }
+        a0 += w * sq(d) / (sc * sc);
       }
-    } else if (i < v.n_true && j < v.n_true) {
-      const float2 kq = k0[e];
-      const double dr = (double)f.x - kq.x, di = (double)f.y - kq.y;
-      a0 += (dr * dr + di * di) / (sc * sc);
     }
-  }, v.hcur ? v.hcur + inst * (size_t)v.noff0 * n : nullptr);
-  const double t0s = block_sum<NT>(a0, sh);
-  const double t1s = block_sum<NT>(a1, sh);
+  }
+  const double t0s = block_sum(a0, sh);
+  const double t1s = block_sum(a1, sh);
   if (threadIdx.x == 0) {
-    partial(v, inst, 0)[blockIdx.x] = t0s;
-    if (pass == 0) partial(v, inst, 1)[blockIdx.x] = t1s;
+    partial(v, inst, 0)[id] = t0s;
+    if (pass == 0) partial(v, inst, 1)[id] = t1s;
   }
 }
 
-// h0 from d0, d1; ys_1 = y0 + h0 k_0; h0 parked in control block 1.
+// h0 from d0, d1, parked in control block 1; d1 moves to slot 0 of its partials
 __global__ __launch_bounds__(256) void k_init_h0(V v) {
   __shared__ double sh[4];
-  const size_t inst = blockIdx.y;
+  const size_t inst = blockIdx.x;
   const Ctrl c = v.ctrl[inst];
   if (is_done(c, v.t1)) return;
-  const double d0 = sqrt(reduce_partials<256>(partial(v, inst, 0), v.npart, sh) * v.inv_nn);
-  const double d1 = sqrt(reduce_partials<256>(partial(v, inst, 1), v.npart, sh) * v.inv_nn);
-  const double h0 = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
-  const int64_t n = v.n;
-  const size_t nn = (size_t)n * n;
-  int i, j;
-  if (diat::row_elem(n, i, j)) {
-    const int64_t e = (int64_t)i * n + j;
-    const double2 yv = v.y[inst * nn + e];
-    const float2 kq = kslot(v, 0, 0, inst)[e];
-    ysbuf(v, 1, inst)[e] = make_float2((float)(yv.x + h0 * kq.x), (float)(yv.y + h0 * kq.y));
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  const double d0 = sqrt(reduce_partials(partial(v, inst, 0), v.total, sh) * v.inv_nn);
+  const double d1 = sqrt(reduce_partials(partial(v, inst, 1), v.total, sh) * v.inv_nn);
+  if (threadIdx.x == 0) {
+    partial(v, inst, 1)[0] = d1;
     Ctrl o = c;
-    o.dt = h0;
+    o.dt = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
     v.ctrl[v.ninst + inst] = o;
   }
 }
 
-// dt0 = min(100 h0, (0.01 / max(d1, d2))^kInitExp); control block 0 and ys_1 of the
-// first attempt.
+// dt0 = min(100 h0, (0.01 / max(d1, d2))^kInitExp): control block 1, which the first step reads
 __global__ __launch_bounds__(256) void k_init_dt(V v) {
-  const RKTab &rk = rk_tab(v.flags);
   __shared__ double sh[4];
-  const size_t inst = blockIdx.y;
+  const size_t inst = blockIdx.x;
   const Ctrl c = v.ctrl[v.ninst + inst];
   if (is_done(c, v.t1)) return;
   const double h0 = c.dt;
-  const double d1 = sqrt(reduce_partials<256>(partial(v, inst, 1), v.npart, sh) * v.inv_nn);
-  const double d2 = sqrt(reduce_partials<256>(partial(v, inst, 0), v.npart, sh) * v.inv_nn) / h0;
+  const double d1 = partial(v, inst, 1)[0];
+  const double d2 = sqrt(reduce_partials(partial(v, inst, 0), v.total, sh) * v.inv_nn) / h0;
   const double md = fmax(d1, d2);
   const double h1 = md <= 1e-15 ? fmax(1e-6, h0 * 1e-3) : pow(0.01 / md, kInitExp);
   Ctrl o = c;
   o.dt = fmin(100.0 * h0, h1);
+  o.rot |= kFresh;
   const double hn = step_h(v, o);
   if (!(hn > 0.0) || !(hn > 1e-14 * fmax(1.0, fabs(o.t)))) o.status = DQH_NONFINITE;
-  const int64_t n = v.n;
-  const size_t nn = (size_t)n * n;
-  int i, j;
-  if (diat::row_elem(n, i, j) && o.status == 0) {
-    const int64_t e = (int64_t)i * n + j;
-    const double2 yv = v.y[inst * nn + e];
-    const float2 kq = kslot(v, 0, 0, inst)[e];
-    ysbuf(v, 0, inst)[e] = make_float2((float)(yv.x + hn * rk.A[1][0] * kq.x), (float)(yv.y + hn * rk.A[1][0] * kq.y));
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) v.ctrl[inst] = o;
+  if (threadIdx.x == 0) v.ctrl[v.ninst + inst] = o;
 }
 
 // f_j(tau) of modulated table j (Horner on the interval that contains tau)
@@ -518,20 +689,26 @@ __global__ __launch_bounds__(256) void k_hupd(V v, int cur, int mode) {
   v.hcur[inst * m + e] = make_float2((float)re, (float)im);
 }
 
-// saves not reached (an instance that stopped early keeps its last state) and stats
+// saves not reached (an instance that stopped early keeps its last state), the final state
+// on both triangles in v.y, and stats
 __global__ __launch_bounds__(256) void k_finish(V v) {
   const size_t inst = blockIdx.y;
-  const Ctrl c = v.ctrl[inst];
+  const Ctrl c = v.ctrl[v.ninst + inst];
   const int64_t n = v.n;
   const size_t nn = (size_t)n * n;
   int i, j;
-  if (diat::row_elem(n, i, j)) {
-    const int64_t e = (int64_t)i * n + j;
+  if (diat::row_elem(n, i, j) && owned(v, i, j)) {
     const int64_t ntn = v.n_true * v.n_true;
-    if (i < v.n_true && j < v.n_true) {
-      const double2 yv = v.y[inst * nn + e];
-      for (int64_t is = c.isave; is < v.nsave; ++is)
-        v.states[(inst * v.nsave + is) * ntn + (size_t)i * v.n_true + j] = make_float2((float)yv.x, (float)yv.y);
+    const size_t e = (size_t)i * n + j, em = (size_t)j * n + i;
+    const bool mirror = v.herm && i != j;
+    double2 *y = v.y + inst * nn;
+    const double2 yv = ybuf(v, c.rot, 0, inst)[e], yc = make_double2(yv.x, -yv.y);
+    if (c.rot & kSel) y[e] = yv;
+    if (mirror) y[em] = yc;
+    for (int64_t is = c.isave; is < v.nsave; ++is) {
+      float2 *st = v.states + (inst * v.nsave + is) * ntn;
+      st[(size_t)i * v.n_true + j] = f32(yv);
+      if (mirror) st[(size_t)j * v.n_true + i] = f32(yc);
     }
   }
   if (blockIdx.x == 0 && threadIdx.x < 8) {
@@ -542,19 +719,24 @@ __global__ __launch_bounds__(256) void k_finish(V v) {
 }
 
 struct Layout {
-  size_t k, ys, part, ctrl, flag, total;
+  size_t k, ys, y2, terms, ones, part, ctrl, flag, total;
+  int64_t npart;
 };
 
 inline size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 inline Layout layout(int64_t n, int64_t ninst) {
   const size_t nn = (size_t)n * n;
-  const size_t npart = (size_t)n * ((n + 255) / 256);  // workgroups of a row-blocked launch
+  const int nb = (int)((n + 63) / 64);
   Layout L;
+  L.npart = std::max(tiles_of(nb, false, 1), tiles_of(nb, true, 1));  // tiles of the smallest kind
   L.k = 0;
   L.ys = L.k + align256(7 * (size_t)ninst * nn * sizeof(float2));
-  L.part = L.ys + align256(2 * (size_t)ninst * nn * sizeof(float2));
-  L.ctrl = L.part + align256((size_t)ninst * 2 * npart * sizeof(double));
+  L.y2 = L.ys + align256(2 * (size_t)ninst * nn * sizeof(float2));
+  L.terms = L.y2 + align256((size_t)ninst * nn * sizeof(double2));
+  L.ones = L.terms + align256(kMaxTerm * sizeof(Term));
+  L.part = L.ones + align256((size_t)n * sizeof(float2));
+  L.ctrl = L.part + align256((size_t)ninst * 2 * L.npart * sizeof(double));
   L.flag = L.ctrl + align256(2 * (size_t)ninst * sizeof(Ctrl));
   L.total = L.flag + 256;
   return L;
@@ -578,84 +760,129 @@ namespace {
 inline dim3 hupd_grid(const diats::V &v) {
   return dim3((unsigned)(((size_t)v.noff0 * v.n + 255) / 256), (unsigned)v.ninst);
 }
+inline dim3 tile_grid(const diats::V &v) { return dim3((unsigned)((v.total + 7) / 8 * 8), (unsigned)v.ninst); }
 
-template <int HALO>
-void launch_step(const diats::V &v, const dqh_dia_ops &ops, dim3 gstage, dim3 gflat, int cur, hipStream_t s) {
-  const bool td = v.hcur != nullptr;
-  if (v.npwc > 0) {  // k_0 anew after a breakpoint (instances that did not land on one return at once)
-    hipLaunchKernelGGL(diats::k_hupd, hupd_grid(v), dim3(256), 0, s, v, cur, 0);
-    hipLaunchKernelGGL(diats::k_stage<HALO>, gstage, dim3(diats::nthreads<HALO>()), 0, s, v, ops, 0, cur);
-  }
-  for (int sg = 1; sg <= 6; ++sg) {
-    if (td) hipLaunchKernelGGL(diats::k_hupd, hupd_grid(v), dim3(256), 0, s, v, cur, sg);
-    hipLaunchKernelGGL(diats::k_stage<HALO>, gstage, dim3(diats::nthreads<HALO>()), 0, s, v, ops, sg, cur);
-  }
-  hipLaunchKernelGGL(diats::k_commit, gflat, dim3(256), 0, s, v, cur);
+template <int S, int NE, bool TD>
+void launch_stages(const diats::V &v, int cur, hipStream_t s) {
+  if (TD) hipLaunchKernelGGL(diats::k_hupd, hupd_grid(v), dim3(256), 0, s, v, cur, S);
+  hipLaunchKernelGGL((diats::k_stage<S, NE, TD>), tile_grid(v), dim3(256), 0, s, v, cur);
+  if constexpr (S > 0 && S < 6) launch_stages<S + 1, NE, TD>(v, cur, s);
 }
 
-template <int HALO>
-int drive(const dqh_dia_tsit5 &p, const diats::V &v, hipStream_t st, dim3 gstage, dim3 gflat) {
-  const dqh_dia_ops &ops = p.ops;
-  const bool td = v.hcur != nullptr;
-  hipLaunchKernelGGL(diats::k_init, gflat, dim3(256), 0, st, v);
-  if (td) hipLaunchKernelGGL(diats::k_hupd, hupd_grid(v), dim3(256), 0, st, v, 0, 7);
-  hipLaunchKernelGGL(diats::k_init_rhs<HALO>, gstage, dim3(diats::nthreads<HALO>()), 0, st, v, ops, 0);
-  hipLaunchKernelGGL(diats::k_init_h0, gflat, dim3(256), 0, st, v);
-  if (td) hipLaunchKernelGGL(diats::k_hupd, hupd_grid(v), dim3(256), 0, st, v, 0, 8);
-  hipLaunchKernelGGL(diats::k_init_rhs<HALO>, gstage, dim3(diats::nthreads<HALO>()), 0, st, v, ops, 1);
-  hipLaunchKernelGGL(diats::k_init_dt, gflat, dim3(256), 0, st, v);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia init: ") + hipGetErrorString(err));
+template <int NE, bool TD>
+void launch_step(const diats::V &v, int cur, hipStream_t s) {
+  if (v.presum) hipLaunchKernelGGL(diats::k_ctl, dim3((unsigned)v.ninst), dim3(256), 0, s, v, cur);
+  if constexpr (TD) {
+    hipLaunchKernelGGL(diats::k_commit<NE>, tile_grid(v), dim3(256), 0, s, v, cur);
+    // k_0 anew after a breakpoint (instances that did not land on one return at once)
+    if (v.npwc > 0) launch_stages<0, NE, TD>(v, cur, s);
+  }
+  launch_stages<1, NE, TD>(v, cur, s);
+}
 
-  const int64_t G = p.graph_steps > 0 ? p.graph_steps : 2;
+struct Steps {  // the captured steps and what captured them
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipStream_t cs = nullptr;
-  auto cleanup = [&]() {
+  ~Steps() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     if (cs) (void)hipStreamDestroy(cs);
-  };
-  if (p.graph_steps > 0) {
-    // capture G steps + the completion count once; replay until every instance is done
-    if ((err = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking)) != hipSuccess ||
-        (err = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal)) != hipSuccess) {
-      cleanup();
-      return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia capture: ") + hipGetErrorString(err));
-    }
-    for (int64_t g = 0; g < G; ++g) launch_step<HALO>(v, ops, gstage, gflat, (int)(g & 1), cs);
+  }
+  // G steps + the completion count
+  template <int NE, bool TD>
+  hipError_t capture(const diats::V &v, int64_t G) {
+    hipError_t err = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking);
+    if (err == hipSuccess) err = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
+    if (err != hipSuccess) return err;
+    for (int64_t g = 0; g < G; ++g) launch_step<NE, TD>(v, (int)(g & 1), cs);
     hipLaunchKernelGGL(diats::k_count, dim3(1), dim3(256), 0, cs, v);
     err = hipStreamEndCapture(cs, &graph);
     if (err == hipSuccess) err = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    if (err != hipSuccess) {
-      cleanup();
-      return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia graph: ") + hipGetErrorString(err));
-    }
+    return err;
   }
+};
+
+struct Events {
   hipEvent_t ev[2] = {nullptr, nullptr};
-  for (int q = 0; q < 2; ++q)
-    if ((err = hipEventCreateWithFlags(&ev[q], hipEventDisableTiming)) != hipSuccess) {
-      cleanup();
-      return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia event: ") + hipGetErrorString(err));
-    }
+  ~Events() {
+    for (int q = 0; q < 2; ++q)
+      if (ev[q]) (void)hipEventDestroy(ev[q]);
+  }
+};
+
+// tiles for a sweep over the upper triangle or the full matrix
+template <int NE>
+void set_tiles(diats::V &v, bool herm) {
+  v.herm = herm;
+  v.nb = (int)((v.n_true + 63) / 64);
+  v.total = diats::tiles_of(v.nb, herm, NE);
+  // Forming the control block delays a workgroup of stage 1 by about 5 us: hidden while
+  // they all run at once, less than the launch of k_ctl; paid per round of workgroups in
+  // larger grids (four solves of n = 1024: 30 us -> 4 + 27 with
+  // the saves).
+  v.presum = (int64_t)v.total * v.ninst > 1024;
+}
+
+template <int NE, bool TD>
+int drive(const dqh_dia_tsit5 &p, diats::V v, hipStream_t st) {
+  const dim3 gflat = diat::row_grid(p.n, p.ninst);
+  // Steps per replay: at most 4, because the replay in flight when the count shows the end
+  // and the rest of the last one are launches without work (n = 323, 29
+  // steps: 1.24 ms a solve with 4, 1.40 with 16; four solves of n = 1024: 6.92 and 7.45)
+  const int64_t G = p.graph_steps > 0 ? std::min<int64_t>(p.graph_steps, 4) : 2;
   volatile int64_t *hf = reinterpret_cast<volatile int64_t *>(p.host_flags);
   hf[0] = hf[1] = -1;
-  // every instance stops within max_steps steps, so this many replays always suffice
-  const int64_t max_iters = p.max_steps / G + 3;
+  Events E;
+  hipError_t err = hipSuccess;
+  for (int q = 0; q < 2 && err == hipSuccess; ++q) err = hipEventCreateWithFlags(&E.ev[q], hipEventDisableTiming);
+  if (err != hipSuccess) return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia event: ") + hipGetErrorString(err));
+  hipLaunchKernelGGL(diats::k_setup, dim3(1), dim3(256), 0, st, v, p.ops);
+  hipLaunchKernelGGL(diats::k_init, gflat, dim3(256), 0, st, v);
+  err = hipGetLastError();
+  if (err == hipSuccess)
+    err = hipMemcpyAsync(const_cast<int64_t *>(hf), v.flag, sizeof(int64_t), hipMemcpyDeviceToHost, st);
+  if (err == hipSuccess) err = hipEventRecord(E.ev[0], st);
+  // the steps are captured while the device looks at rho0: for the upper triangle, and
+  // once more for the full matrix where that proves necessary
+  set_tiles<NE>(v, true);
+  Steps steps, full;
+  Steps *use = &steps;
+  if (err == hipSuccess && p.graph_steps > 0) err = steps.template capture<NE, TD>(v, G);
+  if (err == hipSuccess) err = hipEventSynchronize(E.ev[0]);
+  if (err == hipSuccess && hf[0] != 0) {
+    set_tiles<NE>(v, false);
+    use = &full;
+    if (p.graph_steps > 0) err = full.template capture<NE, TD>(v, G);
+  }
+  if (err != hipSuccess) return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia graph: ") + hipGetErrorString(err));
+  hf[0] = -1;
+  const dim3 gt = tile_grid(v), gi((unsigned)v.ninst);
+  if (TD) hipLaunchKernelGGL(diats::k_hupd, hupd_grid(v), dim3(256), 0, st, v, 0, 7);
+  hipLaunchKernelGGL((diats::k_init_rhs<NE, TD>), gt, dim3(256), 0, st, v, 0);
+  hipLaunchKernelGGL(diats::k_init_h0, gi, dim3(256), 0, st, v);
+  if (TD) hipLaunchKernelGGL(diats::k_hupd, hupd_grid(v), dim3(256), 0, st, v, 0, 8);
+  hipLaunchKernelGGL((diats::k_init_rhs<NE, TD>), gt, dim3(256), 0, st, v, 1);
+  hipLaunchKernelGGL(diats::k_init_dt, gi, dim3(256), 0, st, v);
+  err = hipGetLastError();
+  if (err != hipSuccess) return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia init: ") + hipGetErrorString(err));
+  // every instance stops within max_steps attempts, and the step after the last one
+  // commits it, so this many replays always suffice
+  const int64_t max_iters = p.max_steps / G + 4;
   bool finished = false;
   for (int64_t it = 0; it < max_iters && err == hipSuccess; ++it) {
-    if (exec) {
-      err = hipGraphLaunch(exec, st);
+    if (use->exec) {
+      err = hipGraphLaunch(use->exec, st);
     } else {
-      for (int64_t g = 0; g < G; ++g) launch_step<HALO>(v, ops, gstage, gflat, (int)(g & 1), st);
+      for (int64_t g = 0; g < G; ++g) launch_step<NE, TD>(v, (int)(g & 1), st);
       hipLaunchKernelGGL(diats::k_count, dim3(1), dim3(256), 0, st, v);
       err = hipGetLastError();
     }
     if (err == hipSuccess)
       err = hipMemcpyAsync(const_cast<int64_t *>(hf + (it & 1)), v.flag, sizeof(int64_t), hipMemcpyDeviceToHost, st);
-    if (err == hipSuccess) err = hipEventRecord(ev[it & 1], st);
+    if (err == hipSuccess) err = hipEventRecord(E.ev[it & 1], st);
     if (err == hipSuccess && it > 0) {
-      err = hipEventSynchronize(ev[(it - 1) & 1]);
+      err = hipEventSynchronize(E.ev[(it - 1) & 1]);
       if (err == hipSuccess && hf[(it - 1) & 1] >= v.ninst) {
         finished = true;
         break;
@@ -669,14 +896,11 @@ int drive(const dqh_dia_tsit5 &p, const diats::V &v, hipStream_t st, dim3 gstage
     if (err == hipSuccess) err = hipMemcpy(&last, v.flag, sizeof(int64_t), hipMemcpyDeviceToHost);
     finished = err == hipSuccess && last >= v.ninst;
   }
-  for (int q = 0; q < 2; ++q) (void)hipEventDestroy(ev[q]);
-  cleanup();
   if (err != hipSuccess) return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia: ") + hipGetErrorString(err));
   hipLaunchKernelGGL(diats::k_finish, gflat, dim3(256), 0, st, v);
   if (p.nE > 0)
-    hipLaunchKernelGGL(k_expect_states, dim3((unsigned)p.nsave, (unsigned)p.ninst), dim3(256), 0, st, p.n_true,
-                       p.nsave, p.nE, reinterpret_cast<const float2 *>(p.states),
-                       reinterpret_cast<const float2 *>(p.EopsT), reinterpret_cast<float2 *>(p.expects));
+    launch_expect(p.n_true, p.nsave, p.ninst, p.nE, p.states, p.EopsT, p.expects, v.k,
+                  9 * (size_t)v.n * v.n * v.ninst * sizeof(float2), st);
   err = hipGetLastError();
   if (err != hipSuccess) return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dia: ") + hipGetErrorString(err));
   if (!finished) return fail(DQH_HIP_ERROR, "dqh_mesolve_tsit5_dia: instances still running after max_steps steps");
@@ -720,7 +944,6 @@ extern "C" int dqh_mesolve_tsit5_dia(const dqh_dia_tsit5 *pb, void *stream) {
   const int halo = diat::resolve_halo(p.variant, p.n, diat::max_abs_offset(p.ops));
   if (halo < 0)
     return fail(DQH_BAD_ARG, "dqh_mesolve_tsit5_dia: the tiled sweep needs n % 64 == 0 and every |offset| <= its halo");
-  const size_t nn = (size_t)p.n * p.n;
   const diats::Layout L = diats::layout(p.n, p.ninst);
   char *w = reinterpret_cast<char *>(p.work);
   diats::V v;
@@ -740,6 +963,10 @@ extern "C" int dqh_mesolve_tsit5_dia(const dqh_dia_tsit5 *pb, void *stream) {
   v.inv_nn = 1.0 / ((double)p.n_true * (double)p.n_true);
   v.k = reinterpret_cast<float2 *>(w + L.k);
   v.ys = reinterpret_cast<float2 *>(w + L.ys);
+  v.y2 = reinterpret_cast<double2 *>(w + L.y2);
+  v.terms = reinterpret_cast<diats::Term *>(w + L.terms);
+  v.ones = reinterpret_cast<float2 *>(w + L.ones);
+  v.npart = L.npart;
   v.part = reinterpret_cast<double *>(w + L.part);
   v.ctrl = reinterpret_cast<diats::Ctrl *>(w + L.ctrl);
   v.flag = reinterpret_cast<int64_t *>(w + L.flag);
@@ -761,12 +988,20 @@ extern "C" int dqh_mesolve_tsit5_dia(const dqh_dia_tsit5 *pb, void *stream) {
   v.H0 = reinterpret_cast<const float2 *>(p.ops.diags[0]);
   v.Hterms = td ? reinterpret_cast<const float2 *>(p.Hterms) : nullptr;
   v.hcur = td ? reinterpret_cast<float2 *>(p.hcur) : nullptr;
-  const dim3 gflat = diat::row_grid(p.n, p.ninst);
+  v.nterm = 2 * p.ops.noff[0];
+  v.spread = 0;  // largest p - q of a shift (p, q)
+  for (int u = 0; u < p.ops.noff[0]; ++u) v.spread = std::max(v.spread, std::abs(p.ops.off[0][u]));
+  for (int k = 1; k < p.ops.nops; ++k) {
+    v.nterm += p.ops.noff[k] * p.ops.noff[k];
+    for (int u = 0; u < p.ops.noff[k]; ++u)
+      for (int w = 0; w < p.ops.noff[k]; ++w) v.spread = std::max(v.spread, p.ops.off[k][u] - p.ops.off[k][w]);
+  }
+  v.herm = v.nb = v.total = v.presum = 0;
   hipStream_t st = (hipStream_t)stream;
-  const dim3 gtile((unsigned)((p.n / diat::kTI) * (p.n / diat::kTJ)), (unsigned)p.ninst);
-  v.npart = halo > 0 ? gtile.x : gflat.x;
-  if (halo == 8) return drive<8>(p, v, st, gtile, gflat);
-  if (halo == 16) return drive<16>(p, v, st, gtile, gflat);
-  if (halo == 32) return drive<32>(p, v, st, gtile, gflat);
-  return drive<0>(p, v, st, gflat, gflat);
+  // four rows per thread share the column factors and keep more loads in flight; they
+  // leave at least four waves per SIMD from 2^20 elements on. Below, one row per thread
+  // spreads the work over more CUs.
+  const bool large = (double)p.n_true * (double)p.n_true * (double)p.ninst >= (double)(1 << 21);
+  if (td) return large ? drive<4, true>(p, v, st) : drive<1, true>(p, v, st);
+  return large ? drive<4, false>(p, v, st) : drive<1, false>(p, v, st);
 }

@@ -555,13 +555,6 @@ def tsit5_plan(
     n_pad = NB * ((n + NB - 1) // NB)
     LdL = sum((L.conj().T @ L for L in Ls), np.zeros_like(H))
     Hnh = -1j * H - 0.5 * LdL
-    if variant == SWEEP_AUTO:
-        from .. import autotune
-
-        # the sweep form must admit every offset of the time-dependent terms too
-        Hpat = H + sum((np.abs(np.asarray(O)) for O in [o for (_, _, o) in (pwc or [])] + [o for (_, o) in (mod or [])]),
-                       np.zeros(H.shape))
-        variant = autotune.dia_sweep(Hpat, Ls, B)
     arena = _Arena(dev)
     prob = DiaTsit5()
     prob.n, prob.n_true, prob.ninst, prob.nsave = n_pad, n, B, len(tsave)

@@ -452,8 +452,8 @@ typedef struct dqh_dia_tsit5 {
   int64_t nsave;
   int64_t max_steps;
   int64_t nE;
-  int64_t variant;      /* DQH_SWEEP_* */
-  int64_t graph_steps;  /* steps per captured hipGraph (even); 0: plain launches */
+  int64_t variant;      /* DQH_SWEEP_*: checked against the problem; every form runs the same sweep */
+  int64_t graph_steps;  /* most steps per captured hipGraph (even); 0: plain launches */
   double rtol, atol, safety, factormin, factormax, t0, t1;
   int64_t flags;        /* DQH_FLAG_DOPRI5 selects the Dopri5 pair */
   dqh_dia_ops ops;      /* diags[0] = Hnh = -iH - 1/2 sum L^dag L, diags[k] = L_k */

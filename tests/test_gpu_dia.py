@@ -233,6 +233,39 @@ def test_dia_tsit5_matches_oracle(variant):
         assert abs(np.trace(out['final_state'][b]) - 1) < 1e-6
 
 
+@pytest.mark.parametrize('n, hermitian', [(65, True), (130, True), (191, True), (65, False), (191, False)])
+def test_dia_tsit5_any_offsets_and_states(n, hermitian):
+    """Operators with diagonals far apart on both sides (stencil reads up to 2 x 17 elements
+    across the diagonal), n just past and just short of a block of 64, complex elements, a
+    Hermitian rho0 (upper triangle) and one that is not (full matrix). Against the FP64
+    oracle at the same tolerances: 1e-5, the bound of the other solves here."""
+    from dynamiqs_amd.integrators import dia
+    from oracle import tsit5
+
+    rng = np.random.default_rng(n)
+
+    def banded(offs):
+        return sum(np.diag(rng.normal(size=n - abs(o)) + 1j * rng.normal(size=n - abs(o)), o) for o in offs)
+
+    A = banded([0, 3, 17])
+    H, Ls = 0.3 * (A + A.conj().T), [0.2 * banded([-17, 2]), 0.2 * banded([1])]
+    X = rng.normal(size=(2, n, n)) + 1j * rng.normal(size=(2, n, n))
+    rho0 = X @ np.swapaxes(X.conj(), -1, -2) if hermitian else X
+    rho0 /= np.linalg.norm(rho0, axis=(-2, -1), keepdims=True)
+    tsave = np.linspace(0.0, 0.3, 4)
+    plan = dia.tsit5_plan(H, Ls, rho0, tsave, exp_ops=[A])
+    plan.run()
+    out = plan.results()
+    f = _sparse_lindblad(H, Ls)
+    for b in range(2):
+        saved, _, st = tsit5.integrate(f, rho0[b], tsave, rtol=1e-6, atol=1e-6)
+        assert np.linalg.norm(out['states'][b] - np.stack(saved), axis=(-2, -1)).max() <= TOL
+        assert np.linalg.norm(out['final_state'][b] - saved[-1]) <= TOL
+        ex = np.einsum('ij,tji->t', A, np.stack(saved))
+        assert np.abs(out['expects'][b, 0] - ex).max() <= TOL * np.linalg.norm(A)
+        assert abs(int(out['nsteps'][b]) - st.nsteps) <= 2
+
+
 def test_dia_tsit5_graph_replays_equal_plain_launches():
     """The captured hipGraph (replayed many times, 4 steps each) and plain launches
     of the same kernels give bit-identical states and counters."""
