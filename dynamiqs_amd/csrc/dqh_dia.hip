@@ -33,6 +33,7 @@
 #include "dqh.h"
 #include "dqh_common.h"
 #include "dqh_dia_tile.h"
+#include "dqh_dia_tri.h"
 #include "dqh_expect.h"
 
 namespace dqh {
@@ -655,6 +656,203 @@ __global__ __launch_bounds__(256) void k_kraus(int64_t n, int64_t n_true, int64_
   }
 }
 
+// ------------------------------------------------------------- diagonal form
+// When D = T^-dag - I also has few diagonals above FP32 resolution, both halves of a step
+// are stencils, and a Hermitian state needs the upper triangle alone (dqh_dia_tri.h; a
+// state that is not Hermitian takes the same kernels over the full matrix):
+//   k_dnorm   E = D hi + hi D^dag + D hi D^dag, X = hi + E      24 bytes per element
+//   k_dkraus  the Kraus increment of X, the FP64 update          48 bytes per element
+// Bound by those bytes. 16 states of n = 1024 (D with 4 diagonals, 17
+// products of the Kraus map), 40 steps: 24.2 -> 10.4 ms (k_blk_norm 233 us and k_kraus 266 us
+// a step before, 98 and 149 now; a copy of their bytes would take 43 and 86, the rest are the
+// L1 accesses of the 16 and 17 neighbours and the stores below the diagonal). One, two and
+// four rows per thread: 111, 103, 98 us for k_dnorm.
+struct DView {
+  int64_t n, n_true;
+  int32_t herm, spread, nb, total;
+};
+constexpr int kMaxNorm = 6;  // diagonals of D
+constexpr int kMaxKraus = 4;  // diagonals of a Kraus operator
+struct Diags {
+  const float2 *d;
+  int32_t n;
+  int32_t off[kMaxNorm], row[kMaxNorm];  // row: of d
+};
+struct KOps {
+  int32_t nops, pad;
+  const float2 *d[DQH_DIA_MAXOPS];
+  int32_t noff[DQH_DIA_MAXOPS], off[DQH_DIA_MAXOPS][kMaxKraus], row[DQH_DIA_MAXOPS][kMaxKraus];
+};
+
+typedef const __attribute__((address_space(4))) float CFloat;
+typedef const __attribute__((address_space(1))) float GFloat;
+
+// (ONE) A X + X A^dag + A X A^dag, with diagonal 0 of A at offset 0, or A X A^dag, added to
+// f at rows i0 .. i0 + NE - 1 of column j. The row factors are wave-uniform scalars; a
+// neighbour outside the matrix has a zero factor and a clamped address.
+template <int Q, int NE, bool ONE>
+__device__ __forceinline__ void sandwich(const float2 *X, const float2 *d, const int32_t *off, const int32_t *row, int n,
+                                         int lim, int i0, int j, float2 (&f)[NE]) {
+  float2 c[Q];
+  int jc[Q];
+#pragma unroll
+  for (int v = 0; v < Q; ++v) {
+    const int q = j + off[v];
+    jc[v] = min(max(q, 0), lim - 1);
+    GFloat *p = (GFloat *)(d + (size_t)row[v] * n + jc[v]);
+    c[v] = q == jc[v] ? make_float2(p[0], p[1]) : make_float2(0.f, 0.f);
+  }
+#pragma unroll
+  for (int u = 0; u < Q; ++u) {
+    float2 x[Q][NE];
+    float ax[NE], ay[NE];
+    CFloat *dr = (CFloat *)(d + (size_t)row[u] * n);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      const int a = i0 + m + off[u], ac = min(max(a, 0), lim - 1);
+      const float wx = dr[2 * ac], wy = dr[2 * ac + 1];
+      ax[m] = a == ac ? wx : 0.f;
+      ay[m] = a == ac ? wy : 0.f;
+#pragma unroll
+      for (int v = 0; v < Q; ++v) x[v][m] = X[(size_t)ac * n + jc[v]];
+    }
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      float zr = 0.f, zi = 0.f;
+#pragma unroll
+      for (int v = 0; v < Q; ++v) {  // X A^dag
+        zr = fmaf(x[v][m].x, c[v].x, fmaf(x[v][m].y, c[v].y, zr));
+        zi = fmaf(x[v][m].y, c[v].x, fmaf(-x[v][m].x, c[v].y, zi));
+      }
+      if (ONE && u == 0) {
+        f[m].x += zr;
+        f[m].y += zi;
+      }
+      if (ONE) {
+        zr += x[0][m].x;
+        zi += x[0][m].y;
+      }
+      f[m].x = fmaf(ax[m], zr, fmaf(-ay[m], zi, f[m].x));
+      f[m].y = fmaf(ax[m], zi, fmaf(ay[m], zr, f[m].y));
+    }
+  }
+}
+
+template <int NE, bool ONE, int QM, int Q = 1>
+__device__ __forceinline__ void sandwich_of(int q, const float2 *X, const float2 *d, const int32_t *off,
+                                            const int32_t *row, int n, int lim, int i0, int j, float2 (&f)[NE]) {
+  if constexpr (Q <= QM) {
+    if (q == Q)
+      sandwich<Q, NE, ONE>(X, d, off, row, n, lim, i0, j, f);
+    else
+      sandwich_of<NE, ONE, QM, Q + 1>(q, X, d, off, row, n, lim, i0, j, f);
+  }
+}
+
+// the view for the state at hand: *flag != 0 where rho0 is not Hermitian
+template <int NE>
+__device__ __forceinline__ void resolve(DView &v, const int64_t *flag) {
+  v.herm = *flag == 0;
+  v.total = tri::tiles_of(v.nb, v.herm != 0, NE);
+}
+
+template <int NE, int Q>
+__global__ __launch_bounds__(256) void k_dnorm(DView v, const int64_t *__restrict__ flag, Diags D,
+                                               const float2 *__restrict__ hi, float2 *__restrict__ X,
+                                               float2 *__restrict__ E) {
+  resolve<NE>(v, flag);
+  const int lim = (int)v.n_true;
+  const size_t base = (size_t)blockIdx.y * v.n * v.n;
+  int id, i0, j;
+  for (int round = 0; tri::tile<NE>(v, id, i0, j, round); ++round) {
+    if (i0 < 0 || i0 >= lim || (v.herm && (j | 63) < i0)) continue;
+    const int jc = min(j, lim - 1);
+    float2 f[NE];
+#pragma unroll
+    for (int m = 0; m < NE; ++m) f[m] = make_float2(0.f, 0.f);
+    sandwich<Q, NE, true>(hi + base, D.d, D.off, D.row, (int)v.n, lim, i0, jc, f);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      const int i = i0 + m;
+      if (!tri::owned(v, i, j)) continue;
+      const size_t e = base + (size_t)i * v.n + j;
+      if (v.herm && i == j) f[m].y = 0.f;
+      const float2 h = hi[e];
+      E[e] = f[m];
+      tri::put(v, X + base, i, j, make_float2(h.x + f[m].x, h.y + f[m].y));
+    }
+  }
+}
+
+template <int NE>
+__global__ __launch_bounds__(256) void k_dkraus(DView v, const int64_t *__restrict__ flag, KOps ops, int64_t nsave,
+                                                Saves sv, const float2 *__restrict__ X, const float2 *__restrict__ E,
+                                                float2 *__restrict__ hi, float2 *__restrict__ lo,
+                                                float2 *__restrict__ states) {
+  resolve<NE>(v, flag);
+  const int lim = (int)v.n_true, n = (int)v.n;
+  const size_t base = (size_t)blockIdx.y * v.n * v.n;
+  float2 *st_inst = states + (size_t)blockIdx.y * nsave * v.n_true * v.n_true;
+  int id, i0, j;
+  for (int round = 0; tri::tile<NE>(v, id, i0, j, round); ++round) {
+    if (i0 < 0 || i0 >= lim || (v.herm && (j | 63) < i0)) continue;
+    const int jc = min(j, lim - 1);
+    float2 f[NE];
+#pragma unroll
+    for (int m = 0; m < NE; ++m) f[m] = make_float2(0.f, 0.f);
+    sandwich_of<NE, true, kMaxKraus>(ops.noff[0], X + base, ops.d[0], ops.off[0], ops.row[0], n, lim, i0, jc, f);
+    for (int s = 1; s < ops.nops; ++s)
+      sandwich_of<NE, false, kMaxKraus>(ops.noff[s], X + base, ops.d[s], ops.off[s], ops.row[s], n, lim, i0, jc, f);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      const int i = i0 + m;
+      if (!tri::owned(v, i, j)) continue;
+      const size_t e = base + (size_t)i * v.n + j;
+      const float2 x = E[e], h = hi[e], l = lo[e];
+      const double dr = (double)x.x + f[m].x, di = v.herm && i == j ? 0.0 : (double)x.y + f[m].y;
+      const double orr = (double)h.x + (double)l.x, oi = (double)h.y + (double)l.y;
+      for (int k = 0; k < sv.count; ++k) {
+        const double th = sv.theta[k];
+        float2 *st = st_inst + sv.idx[k] * v.n_true * v.n_true;
+        float2 r = make_float2((float)(orr + th * dr), (float)(oi + th * di));
+        st[(size_t)i * v.n_true + j] = r;
+        if (v.herm && i != j) {
+          r.y = -r.y;
+          st[(size_t)j * v.n_true + i] = r;
+        }
+      }
+      if (sv.update) {
+        const double nr = orr + dr, ni = oi + di;
+        const float2 hn = make_float2((float)nr, (float)ni);
+        tri::put(v, hi + base, i, j, hn);
+        lo[e] = make_float2((float)(nr - (double)hn.x), (float)(ni - (double)hn.y));
+      }
+    }
+  }
+}
+
+// sets the flag where rho0 is not Hermitian
+__global__ __launch_bounds__(256) void k_herm(int64_t n, int64_t n_true, const double2 *__restrict__ r64, int64_t *flag) {
+  int i, j;
+  if (!diat::row_elem(n, i, j) || i >= n_true || j >= n_true || j < i) return;
+  if (!tri::hermitian_at(r64 + (size_t)blockIdx.y * n * n, n, i, j)) *flag = 1;
+}
+__global__ void k_zero(int64_t *flag) { *flag = 0; }
+
+// rho = hi + lo in FP64 (end of the solve), the lower triangle from the upper one
+__global__ __launch_bounds__(256) void k_dcombine(int64_t n, const int64_t *__restrict__ flag,
+                                                  const float2 *__restrict__ hi, const float2 *__restrict__ lo,
+                                                  double2 *__restrict__ r64) {
+  int i, j;
+  if (!diat::row_elem(n, i, j)) return;
+  const size_t base = (size_t)blockIdx.y * n * n;
+  const bool mirror = *flag == 0 && j < i;
+  const size_t e = base + (mirror ? (size_t)j * n + i : (size_t)i * n + j);
+  const float2 h = hi[e], l = lo[e];
+  const double im = (double)h.y + (double)l.y;
+  r64[base + (size_t)i * n + j] = make_double2((double)h.x + (double)l.x, mirror ? -im : im);
+}
+
 // LDS-tiled form of k_kraus (all offsets within the halo, n % 64 == 0): one
 // workgroup per 64 x 64 tile of one instance, X staged with its halo.
 template <int HALO>
@@ -774,6 +972,59 @@ extern "C" int dqh_mesolve_rouchon1_dia(const dqh_dia_rouchon1 *pb, void *stream
   const dim3 gtile((unsigned)((n / diat::kTI) * (n / diat::kTJ)), (unsigned)p.ninst);
   int maxoff = 0;
   for (int s = 0; s < p.nsets; ++s) maxoff = std::max(maxoff, diat::max_abs_offset(p.ops[s]));
+  const bool dnorm = p.nd > 0;
+  // dx, dv: how far below the diagonal X and hi are kept
+  dia::DView dv{n, p.n_true, 1, 0, (int32_t)((p.n_true + 63) / 64), 0}, dx;
+  dia::Diags dd[2] = {};
+  dia::KOps dk[2] = {};
+  int64_t *flag = reinterpret_cast<int64_t *>(p.flag);
+  if (dnorm) {
+    if (p.nd > dia::kMaxNorm || p.nd_off[0] != 0 || !flag)
+      return fail(DQH_BAD_ARG, "dqh_mesolve_rouchon1_dia: the diagonal normalisation takes 1 to 6 diagonals, the first at offset 0, and a flag");
+    int dmin = 0, dmax = 0;
+    for (int u = 0; u < p.nd; ++u) {
+      if (p.nd_off[u] <= -n || p.nd_off[u] >= n)
+        return fail(DQH_BAD_ARG, "dqh_mesolve_rouchon1_dia: normalisation offset outside (-n, n)");
+      dmin = std::min(dmin, p.nd_off[u]);
+      dmax = std::max(dmax, p.nd_off[u]);
+    }
+    dv.spread = dmax - dmin;
+    dx = dv;
+    dx.spread = 0;
+    for (int s = 0; s < p.nsets; ++s) {
+      if (!p.Nd[s]) return fail(DQH_BAD_ARG, "dqh_mesolve_rouchon1_dia: null diagonals of the normalisation");
+      dd[s].d = reinterpret_cast<const float2 *>(p.Nd[s]);
+      dd[s].n = (int32_t)p.nd;
+      for (int u = 0; u < p.nd; ++u) {
+        dd[s].off[u] = p.nd_off[u];
+        dd[s].row[u] = u;
+      }
+      const dqh_dia_ops &o = p.ops[s];
+      dk[s].nops = o.nops;
+      for (int k = 0; k < o.nops; ++k) {
+        if (o.noff[k] > dia::kMaxKraus)
+          return fail(DQH_BAD_ARG, "dqh_mesolve_rouchon1_dia: the diagonal form takes at most 4 diagonals per Kraus operator");
+        dk[s].d[k] = reinterpret_cast<const float2 *>(o.diags[k]);
+        dk[s].noff[k] = o.noff[k];
+        int omin = k ? n : 0, omax = k ? -n : 0;
+        for (int u = 0; u < o.noff[k]; ++u) {
+          dk[s].off[k][u] = o.off[k][u];
+          dk[s].row[k][u] = u;
+          omin = std::min(omin, o.off[k][u]);
+          omax = std::max(omax, o.off[k][u]);
+          if (k == 0 && o.off[k][u] == 0 && u > 0) {  // offset 0 first
+            std::swap(dk[s].off[k][0], dk[s].off[k][u]);
+            std::swap(dk[s].row[k][0], dk[s].row[k][u]);
+          }
+        }
+        if (k == 0 && dk[s].off[0][0] != 0)
+          return fail(DQH_BAD_ARG, "dqh_mesolve_rouchon1_dia: the diagonal form needs the main diagonal of operator 0");
+        dx.spread = std::max(dx.spread, omax - omin);
+      }
+    }
+    dv.total = dx.total = tri::tiles_of(dv.nb, true, 4);
+  }
+  const dim3 gtri((unsigned)((dv.total + 7) / 8 * 8), (unsigned)p.ninst);
   // the fused sweep has a global form (GLOBAL, and SPLIT, which names the former
   // two-pass form) and LDS-tiled forms
   const int halo = p.variant == DQH_SWEEP_SPLIT ? 0 : diat::resolve_halo(p.variant, n, maxoff);
@@ -782,6 +1033,10 @@ extern "C" int dqh_mesolve_rouchon1_dia(const dqh_dia_rouchon1 *pb, void *stream
   const int64_t total = p.ninst * nn;
   const unsigned gflat = (unsigned)((total + 255) / 256);
   hipLaunchKernelGGL(dia::k_split, dim3(gflat), dim3(256), 0, st, total, r64, hi, lo);
+  if (dnorm) {
+    hipLaunchKernelGGL(dia::k_zero, dim3(1), dim3(1), 0, st, flag);
+    hipLaunchKernelGGL(dia::k_herm, gel, dim3(256), 0, st, n, p.n_true, r64, flag);
+  }
   const int64_t *hs_step = reinterpret_cast<const int64_t *>(p.save_step);
   const double *hs_theta = reinterpret_cast<const double *>(p.save_theta);
   int64_t isave = 0;
@@ -798,8 +1053,11 @@ extern "C" int dqh_mesolve_rouchon1_dia(const dqh_dia_rouchon1 *pb, void *stream
   // global sweep: IB instances per thread (up to dia::kKrausIB)
   const int kib = p.ninst >= dia::kKrausIB ? dia::kKrausIB : (p.ninst >= 4 ? 4 : (p.ninst >= 2 ? 2 : 1));
   const dim3 gkr(gel.x, (unsigned)((p.ninst + kib - 1) / kib));
-  auto sweep = [&](const dqh_dia_ops &ops, const dia::Saves &sv) {
-    if (halo == 8)
+  auto sweep = [&](int set, const dia::Saves &sv) {
+    const dqh_dia_ops &ops = p.ops[set];
+    if (dnorm)
+      hipLaunchKernelGGL(dia::k_dkraus<4>, gtri, dim3(256), 0, st, dv, flag, dk[set], p.nsave, sv, X, E, hi, lo, states);
+    else if (halo == 8)
       hipLaunchKernelGGL(dia::k_kraus_tiled<8>, gtile, dim3(diat::kThreads), 0, st, n, p.n_true, ops, X, E, hi, lo,
                          states, p.nsave, sv);
     else if (halo == 16)
@@ -829,7 +1087,20 @@ extern "C" int dqh_mesolve_rouchon1_dia(const dqh_dia_rouchon1 *pb, void *stream
     const bool timed = tk >= 0 && tk < t_count;
     if (timed) hipEventRecord(ev[3 * tk], st);
     // D1 = T^-dag hi - hi into the X buffer, then E and X = hi + E (over D1)
-    if (blocks) {
+    if (dnorm) {
+      if (p.nd == 1)
+        hipLaunchKernelGGL((dia::k_dnorm<4, 1>), gtri, dim3(256), 0, st, dx, flag, dd[set], hi, X, E);
+      else if (p.nd == 2)
+        hipLaunchKernelGGL((dia::k_dnorm<4, 2>), gtri, dim3(256), 0, st, dx, flag, dd[set], hi, X, E);
+      else if (p.nd == 3)
+        hipLaunchKernelGGL((dia::k_dnorm<4, 3>), gtri, dim3(256), 0, st, dx, flag, dd[set], hi, X, E);
+      else if (p.nd == 4)
+        hipLaunchKernelGGL((dia::k_dnorm<4, 4>), gtri, dim3(256), 0, st, dx, flag, dd[set], hi, X, E);
+      else if (p.nd == 5)
+        hipLaunchKernelGGL((dia::k_dnorm<4, 5>), gtri, dim3(256), 0, st, dx, flag, dd[set], hi, X, E);
+      else
+        hipLaunchKernelGGL((dia::k_dnorm<4, 6>), gtri, dim3(256), 0, st, dx, flag, dd[set], hi, X, E);
+    } else if (blocks) {
       const float2 *Lm = reinterpret_cast<const float2 *>(p.Lm[set]);
       const float2 *Rm = reinterpret_cast<const float2 *>(p.Rm[set]);
       if (fused) {
@@ -880,11 +1151,14 @@ extern "C" int dqh_mesolve_rouchon1_dia(const dqh_dia_rouchon1 *pb, void *stream
       isave += sv.count;
       nin -= sv.count;
       sv.update = nin == 0;
-      sweep(p.ops[set], sv);
+      sweep(set, sv);
     } while (nin > 0);
     if (timed) hipEventRecord(ev[3 * tk + 2], st);
   }
-  hipLaunchKernelGGL(dia::k_combine, dim3(gflat), dim3(256), 0, st, total, hi, lo, r64);
+  if (dnorm)
+    hipLaunchKernelGGL(dia::k_dcombine, gel, dim3(256), 0, st, n, flag, hi, lo, r64);
+  else
+    hipLaunchKernelGGL(dia::k_combine, dim3(gflat), dim3(256), 0, st, total, hi, lo, r64);
   while (isave < p.nsave) {
     hipLaunchKernelGGL(dia::k_save, gel, dim3(256), 0, st, n, p.n_true, r64, states, p.nsave, isave);
     ++isave;

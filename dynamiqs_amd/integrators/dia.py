@@ -68,6 +68,10 @@ class DiaRouchon1(ctypes.Structure):
         ('blk_mat', ctypes.c_uint64),
         ('Lm', ctypes.c_uint64 * 2),
         ('Rm', ctypes.c_uint64 * 2),
+        ('nd', ctypes.c_int64),
+        ('nd_off', ctypes.c_int32 * 6),
+        ('Nd', ctypes.c_uint64 * 2),
+        ('flag', ctypes.c_uint64),
     ]
 
 
@@ -158,6 +162,35 @@ def block_normalisation(S: np.ndarray, sets):
         Rs.append((Ti - np.eye(d)).T.reshape(-1))
     idx_all = np.concatenate(sets).astype(np.int32)
     return of, loc, start, idx_all, mat, np.concatenate(Ls).astype(np.complex64), np.concatenate(Rs).astype(np.complex64)
+
+
+MAXNORM, MAXKRAUS = 6, 4  # diagonals of T^-dag - I and of a Kraus operator in the diagonal form
+
+
+def diagonal_normalisation(of, loc, idx, start, mat, Lm, n: int):
+    """T^-dag - I by its diagonals, from its sets' blocks (``block_normalisation``):
+    (offsets, diags) with offset 0 first, or None above MAXNORM diagonals. Diagonals are
+    dropped, smallest first, while their largest elements add up to less than 2^-30 of the
+    largest element: 1/64 of the FP32 rounding of the kept ones."""
+    offs, rows, vals = [], [], []
+    for b in range(len(start) - 1):
+        s = idx[start[b] : start[b + 1]].astype(np.int64)
+        offs.append((s[None, :] - s[:, None]).reshape(-1))
+        rows.append(np.broadcast_to(s[None, :], (len(s), len(s))).reshape(-1))
+        vals.append(Lm[mat[b] : mat[b + 1]])
+    offs, rows, vals = np.concatenate(offs), np.concatenate(rows), np.concatenate(vals)
+    top = np.zeros(2 * n - 1)
+    np.maximum.at(top, offs + n - 1, np.abs(vals))
+    order = np.argsort(top)
+    keep = np.sort(order[np.cumsum(top[order]) >= 2.0**-30 * top.max()]) - (n - 1)
+    keep = [0] + [int(o) for o in keep if o != 0 and top[o + n - 1] > 0]
+    if len(keep) > MAXNORM:
+        return None
+    d = np.zeros((len(keep), n), dtype=np.complex64)
+    for u, o in enumerate(keep):
+        m = offs == o
+        d[u, rows[m]] = vals[m]
+    return keep, d
 
 
 def block_solve_operators(H: np.ndarray, Ls, dt: float, n_pad: int, banded: bool = True):
@@ -296,11 +329,7 @@ def build_plan(
     arena = _Arena(dev)
     prob = DiaRouchon1()
     prob.n, prob.n_true, prob.nb, prob.ninst = n_pad, n, NB, B
-    if variant == SWEEP_AUTO:
-        from .. import autotune
-
-        variant = autotune.dia_sweep(H, Ls, B, kind='kraus', dt=float(dt))
-    prob.nsteps, prob.nsets, prob.variant, prob.solve_panel = nsteps, len(sets), variant, int(solve_panel)
+    prob.nsteps, prob.nsets, prob.solve_panel = nsteps, len(sets), int(solve_panel)
     # normalisation: block form when S decouples into small index sets (the same
     # sets for every step length: they follow the sparsity of Hnh and L^dag L)
     if normalisation not in ('auto', 'banded', 'blocks'):
@@ -311,13 +340,36 @@ def build_plan(
     if normalisation == 'blocks' and isets is None:
         raise ValueError('the normalisation matrix S does not decouple into sets of at most '
                          f'{MAXBLK} indices (or n > {MAXN_BLOCKS})')
+    # the diagonal form where every choice is open: its sweeps need no halo, and half the
+    # elements of a Hermitian state
+    diagonal = (isets is not None and normalisation == 'auto' and variant == SWEEP_AUTO and solve_panel == 0)
+    packs = [block_solve_operators(H, Ls, h, n_pad, banded=isets is None) for h in sets]
+    blks = [block_normalisation(normalisation_S(H, Ls, h, n_pad), isets) for h in sets] if isets is not None else []
+    if diagonal:
+        nds = [diagonal_normalisation(of, loc, idx, start, mat, Lm, n_pad)
+               for (of, loc, start, idx, mat, Lm, _) in blks]
+        diagonal = (all(x is not None for x in nds) and all(x[0] == nds[0][0] for x in nds)
+                    and all(len(o) <= MAXKRAUS for _, _, ops in packs for o, _ in ops)
+                    and all(0 in ops[0][0] for _, _, ops in packs))
+    if variant == SWEEP_AUTO and not diagonal:
+        from .. import autotune
+
+        variant = autotune.dia_sweep(H, Ls, B, kind='kraus', dt=float(dt))
+    prob.variant = variant
+    flag = torch.zeros(1, dtype=torch.int64, device=dev)
+    if diagonal:
+        prob.nd, prob.flag = len(nds[0][0]), flag.data_ptr()
+        for u, o in enumerate(nds[0][0]):
+            prob.nd_off[u] = o
+        for si, (_, d) in enumerate(nds):
+            prob.Nd[si] = arena.put_now(d)
     for si, h in enumerate(sets):
-        Vp, Wn, ops = block_solve_operators(H, Ls, h, n_pad, banded=isets is None)
+        Vp, Wn, ops = packs[si]
         if isets is None:
             prob.Vp[si] = arena.put_now(Vp.astype(np.complex64))
             prob.Wn[si] = arena.put_now(Wn.astype(np.complex64))
-        else:
-            of, loc, start, idx, mat, Lm, Rm = block_normalisation(normalisation_S(H, Ls, h, n_pad), isets)
+        elif not diagonal:
+            of, loc, start, idx, mat, Lm, Rm = blks[si]
             if si == 0:
                 prob.nblk, prob.blk_maxd = len(isets), max(len(x) for x in isets)
                 prob.blk_of, prob.blk_loc = arena.put_now(of), arena.put_now(loc)
@@ -346,14 +398,16 @@ def build_plan(
         prob.expects = expects.data_ptr()
     plan = DiaPlan()
     plan.problem, plan.arena = prob, arena
-    plan.keep = [steps_h, thetas_h, rho32, work]
+    plan.keep = [steps_h, thetas_h, rho32, work, flag]
     plan.rho64, plan.rho64_0, plan.states, plan.expects = rho64, rho64_0, states, expects
     plan.ninst, plan.n, plan.n_true, plan.nsave, plan.nsteps, plan.nE = B, n_pad, n, len(tsave), nsteps, nE
     # roofline units: the Kraus sweep reads rho and writes rho' (2 n^2 complex64) per step and instance
     plan.sweep_bytes_per_step = 2.0 * n * n * 8 * B
     plan.solve_flops_per_step = 2 * 2 * 8.0 * NB * NB * n_pad * (n_pad // NB) * B
-    plan.normalisation = 'banded' if isets is None else 'blocks'
-    if isets is not None:  # two one-sided products of d x d triangular blocks per row / column
+    plan.normalisation = 'banded' if isets is None else 'diagonals' if diagonal else 'blocks'
+    if diagonal:  # (nd + 1) nd products per element
+        plan.solve_flops_per_step = 8.0 * prob.nd * (prob.nd + 1) * n * n * B
+    elif isets is not None:  # two one-sided products of d x d triangular blocks per row / column
         d2 = float(sum(len(x) * (len(x) + 1) / 2 for x in isets))
         plan.solve_flops_per_step = 2 * 8.0 * d2 * n_pad * B
     return plan

@@ -409,6 +409,13 @@ typedef struct dqh_dia_rouchon1 {
   uint64_t Lm[2];      /* device c64[sum d^2] per step set: T_b^-dag - I, row-major (upper) */
   uint64_t Rm[2];      /* device c64[sum d^2] per step set: (T_b^-1 - I)^T, row-major, so that
                           column l of T_b^-1 - I (nonzero from row l on) is contiguous */
+  /* Diagonal form (nd = 0: one of the forms above): T^-dag - I by its diagonals, in the
+   * layout of dqh_dia_ops, for operators of at most 4 diagonals (operator 0 with its main
+   * one). Sweeps the upper triangle alone when rho0 is Hermitian. */
+  int64_t nd;          /* diagonals (at most 6) */
+  int32_t nd_off[6];   /* their offsets, nd_off[0] = 0 */
+  uint64_t Nd[2];      /* device c64[nd][n] per step set */
+  uint64_t flag;       /* device int64 scratch */
 } dqh_dia_rouchon1;
 
 #define DQH_DIA_MAXBLK 64

@@ -206,6 +206,40 @@ def _sparse_lindblad(H, Ls):
     return f
 
 
+@pytest.mark.parametrize('na, nb_, dt, hermitian', [(5, 13, 1e-3, True), (12, 16, 2e-2, True), (10, 13, 1e-3, False)])
+def test_dia_rouchon1_diagonal_form(na, nb_, dt, hermitian):
+    """The diagonal form of the normalisation (the default for these operators) at n = 65,
+    192 and 130 with 3 to 6 diagonals of T^-dag - I, a last step of another length, an
+    initial state that is Hermitian and one that is not: against the FP64 Kraus map, within
+    the FP32 rounding of the increments (40 steps of at most 1e-7 of the state)."""
+    from dynamiqs_amd.integrators import dia
+
+    H, Ls, _ = _two_mode(na, nb_)
+    n = na * nb_
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(2, n, 3)) + 1j * rng.normal(size=(2, n, 3))
+    rho0 = X @ np.swapaxes(X.conj(), -1, -2)
+    if not hermitian:
+        rho0 = rho0 + 0.3 * (rng.normal(size=rho0.shape) + 1j * rng.normal(size=rho0.shape))
+    rho0 /= np.linalg.norm(rho0, axis=(-2, -1), keepdims=True)
+    tsave = np.array([0.0, 10 * dt, 39.5 * dt])
+    plan = dia.build_plan(H, Ls, rho0, tsave, dt)
+    assert plan.normalisation == 'diagonals'
+    plan.run()
+    out = plan.results()
+    steps = [dt] * 39 + [0.5 * dt]
+    for b in range(2):
+        rho = rho0[b]
+        for m, h in enumerate(steps):
+            M = [np.eye(n) - 1j * h * (H - 0.5j * sum(L.conj().T @ L for L in Ls)), *[np.sqrt(h) * L for L in Ls]]
+            Tdi = np.linalg.inv(np.linalg.cholesky(sum(A.conj().T @ A for A in M))).conj().T
+            rho = sum((A @ Tdi) @ rho @ (A @ Tdi).conj().T for A in M)
+            if m == 9:
+                assert np.linalg.norm(out['states'][b, 1] - rho) <= 1e-6
+        assert np.linalg.norm(out['states'][b, 2] - rho) <= 4e-6
+        assert np.linalg.norm(out['final_state'][b] - rho) <= 4e-6
+
+
 @pytest.mark.parametrize('variant', ['tiled', 'global'])
 def test_dia_tsit5_matches_oracle(variant):
     """Adaptive Tsit5 on the DIA sweeps (n = 144, padded to 192) against the oracle's
