@@ -103,6 +103,7 @@ SYMBOLS = {
     'dqh_dia_tsit5_work_bytes': (_I64, [_I64, _I64]),
     'dqh_mesolve_tsit5_dia': (ctypes.c_int, [_P, _P]),
     'dqh_sesolve_tsit5': (ctypes.c_int, [_P, _I64, _I64, _P]),
+    'dqh_sesolve_tsit5_const': (ctypes.c_int, [_P, _I64, _I64, _I64, _P]),
     'dqh_expm_work_bytes': (_I64, [_I64, _I64, _I64]),
     'dqh_expm_propagators': (ctypes.c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P]),
     'dqh_expm_propagators_noalloc': (ctypes.c_int, [_P, _P, _I64, _I64, _I64, _I64, _I64, _P]),

@@ -34,6 +34,7 @@
 #include "dqh_common.h"
 #include "dqh_mfma.h"
 #include "dqh_tsit5_tableau.h"
+#include "dqh_wave.h"
 
 namespace dqh {
 namespace diag {
@@ -63,54 +64,6 @@ struct Pattern {
   int16_t pa[kMaxPart], pb[kMaxPart];
 };
 
-// x + (x of the lane that the DPP control names)
-template <int CTRL>
-__device__ __forceinline__ double dpp_sum(double x) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
-  return x + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double lane_of(double x, int lane) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-// sum over the wave, the same value in every lane: butterfly over quads, half rows and
-// rows of 16 lanes on the VALU, then the four rows through scalar registers
-__device__ __forceinline__ double wave_sum(double x) {
-  x = dpp_sum<0xB1>(x);   // lane ^ 1
-  x = dpp_sum<0x4E>(x);   // lane ^ 2
-  x = dpp_sum<0x141>(x);  // the other quad of the half row
-  x = dpp_sum<0x140>(x);  // the other half of the row
-  return (lane_of(x, 0) + lane_of(x, 16)) + (lane_of(x, 32) + lane_of(x, 48));
-}
-
-// workgroup sums of N values with one barrier; red alternates between two halves, so a
-// second call need not wait for the readers of the first
-template <int NTH, int N>
-__device__ __forceinline__ void block_sums(double (&x)[N], double *red, int &par) {
-  constexpr int NW = NTH / 64;
-#pragma unroll
-  for (int k = 0; k < N; ++k) x[k] = wave_sum(x[k]);
-  double *r = red + par * (NW * 2);
-  par ^= 1;
-  if constexpr (NW > 1) {
-    if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-      for (int k = 0; k < N; ++k) r[2 * (threadIdx.x >> 6) + k] = x[k];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-      double s = 0.0;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) s += r[2 * w + k];
-      x[k] = s;
-    }
-  }
-}
-
 // LDS: two copies of the stage input (rows of LD = n | 1 float2, one slot that elements
 // past the end write, a guard of G zeros before, between and after them so that a shift
 // may leave the matrix: its coefficient is zero there), the generator's off-diagonals and
@@ -121,17 +74,6 @@ template <int NTH>
 __host__ __device__ inline size_t lds_bytes(int n, int nH, int nLrow, int guard) {
   return (size_t)(2 * copy_stride(n, guard) + guard + (nH + nLrow) * n) * sizeof(float2) +
          (size_t)n * sizeof(double2) + (size_t)(4 * (NTH / 64)) * sizeof(double);
-}
-
-// the tableau through a scalar pointer that the optimiser cannot see through: its loads
-// stay where they are used (as literals, or hoisted out of the loop, the weights would
-// fill the registers that the stages need)
-typedef const __attribute__((address_space(4))) RKTab CTab;
-template <int TAB>
-__device__ __forceinline__ CTab *weights() {
-  CTab *r = (CTab *)&kRK[TAB];
-  asm volatile("" : "+s"(r));
-  return r;
 }
 
 template <int NTH, int NE, int T, int TAB>

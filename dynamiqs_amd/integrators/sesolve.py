@@ -28,6 +28,7 @@ from .operators import decompose, resample_pwc, resolve_callables, spline_table,
 
 SUPPORTED_METHODS = (Tsit5, Dopri5, Euler, Expm)
 MAX_PWC = 8
+MAX_N_CONST = 128  # largest dimension of the kernel with G in registers
 MAX_NP = 1024  # padded dimension of the largest sesolve kernel variant
 SE_FIELDS = ('tsave', 'Hnh', 'EopsT', 'Hpwc', 'pwc_times', 'pwc_vals', 'Hmod', 'mod_coef', 'step_t')
 
@@ -53,6 +54,7 @@ class SEPlan:
         self.descs = self.d_descs = None
         self.states = self.final = self.expects = self.stats = self.step_log = None
         self.y = self.y0 = None
+        self.constant = False  # the kernel with G in registers (dqh_sesolve_tsit5_const)
 
     def reset(self):
         self.y.copy_(self.y0)
@@ -62,6 +64,14 @@ class SEPlan:
 
         lib = _native.lib()
         s = stream if stream is not None else torch.cuda.current_stream()
+        if self.constant:
+            _native.check(
+                lib.dqh_sesolve_tsit5_const(_native.ctypes.c_void_p(self.d_descs.data_ptr()), self.ninst, self.n,
+                                            int(self.descs['flags'][0]) & _native.FLAG_DOPRI5,
+                                            _native.ctypes.c_void_p(s.cuda_stream)),
+                'dqh_sesolve_tsit5_const',
+            )
+            return
         _native.check(
             lib.dqh_sesolve_tsit5(_native.ctypes.c_void_p(self.d_descs.data_ptr()), self.ninst, self.np,
                                   _native.ctypes.c_void_p(s.cuda_stream)),
@@ -161,6 +171,8 @@ def _finish(plan: SEPlan, descs, arena, y0: np.ndarray, dev, step_log_cap: int) 
         tensors.append(plan.step_log)
     check_descriptors(descs, tensors, extents)
     plan.tensors = tensors
+    plan.constant = (n <= MAX_N_CONST and not np.any(descs['npwc']) and not np.any(descs['nmod'])
+                     and not np.any(descs['flags'] & _native.FLAG_EULER))
     plan.descs = descs
     plan.d_descs = torch.from_numpy(descs.view(np.uint8).copy()).to(dev)
     return plan

@@ -517,6 +517,11 @@ int dqh_mesolve_tsit5_dia(const dqh_dia_tsit5 *problem, void *stream);
  * expects[e][i] = <psi(tsave[i])| E_e |psi(tsave[i])>. */
 int dqh_sesolve_tsit5(const dqh_me_inst *d_insts, int64_t ninst, int64_t np_max, void *stream);
 
+/* The same for constant Hamiltonians of dimension n <= 128 (npwc = nmod = 0, no Euler steps;
+ * an instance that has them gets status DQH_UNSUPPORTED): every instance of the batch has
+ * dimension n, and the pair that ``flags`` (DQH_FLAG_DOPRI5) and its descriptor name. */
+int dqh_sesolve_tsit5_const(const dqh_me_inst *d_insts, int64_t ninst, int64_t n, int64_t flags, void *stream);
+
 /* ------------------------------------------------------------------ Expm */
 /* Propagators of piecewise-constant generators by explicit exponentiation
  * (replaces ExpmIntegrator.run, expm_integrator.py:60-90: expm of dt_k A_k on every

@@ -182,6 +182,29 @@ def test_batching_shapes_and_instance_independence():
     np.testing.assert_array_equal(fin.final_state.to_numpy(), res.states.to_numpy()[:, :, -1])
 
 
+@pytest.mark.parametrize('method', ['tsit5', 'dopri5'])
+@pytest.mark.parametrize('n', [1, 2, 16, 17, 33, 64, 65, 128])
+def test_constant_kernel_sizes(n, method):
+    """The kernel with the generator in registers at the edges of its sizes (16, 32, 64, 128
+    rows): replay error within the bound of n <= 64 (2e-6; FP32 sums of up to 128 terms), and
+    both expectation values (the first from registers) of the saved kets."""
+    from oracle import mesolve as om
+
+    from dynamiqs_amd.integrators.sesolve import SEInstance
+
+    rng = np.random.default_rng(n)
+    Hs = [_herm(rng, n, 2.0) for _ in range(3)]
+    psis = [_ket(rng, n) for _ in Hs]
+    Es = [_herm(rng, n), rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))]
+    tsave = np.linspace(0.0, 1.5, 7)
+    insts = [SEInstance(H=H, psi0=p, key_H=(b,)) for b, (H, p) in enumerate(zip(Hs, psis))]
+    res, errs = _run_plan(insts, tsave, [om.TimeOp(H) for H in Hs], psis, method, exp_ops=Es)
+    assert np.all(errs <= REPLAY_TOL), errs
+    x = res['states'].astype(np.complex128)
+    ex = np.einsum('bti,eij,btj->bet', x.conj(), np.stack(Es), x)
+    assert np.abs(res['expects'] - ex).max() <= 1e-6 * max(np.linalg.norm(E, 2) for E in Es)
+
+
 def test_large_dimension_replay():
     """n = 200 (padded to 208, one row per thread): replay within 1e-5 (FP32
     products over 200-term rows) and the norm conserved to the same level."""
