@@ -3,14 +3,21 @@
 // The persistent kernel gives one workgroup (one CU) to each instance, which is
 // the right shape for batches of small problems but leaves a single n = 256
 // solve on one of 256 CUs. Here every stage of every instance is spread over the
-// whole grid, in three launches:
-//   k_xprod  X_k = L_k ys                          16 x 16 MFMA tiles, one per wave
-//   k_tmp    tmp = Hnh ys + sum_k X_k (L_k^dag / 2) 16 x 16 MFMA tiles, one per wave
-//   k_body   f = tmp + tmp^dag; k_s = f; ys <- the next stage input, in place (the
-//            GEMMs that read ys are done): the increment h sum a_{s+1,j} k_j for
-//            stages 1..5 (the generator is constant, so f(y + Delta) = k_0 + f(Delta)
-//            and k_1..k_5 hold f(Delta_s) only), y + that increment for stage 6;
-//            or on the last stage the FP64 partial sums of the scaled error
+// whole grid, in two launches:
+//   k_xprod  X_k = L_k ys          32 x 32 tiles, the k range split over four waves
+//   k_stage  f = Hnh ys + (Hnh ys)^dag + sum_k X_k L_k^dag on the 16 x 16 tiles of the
+//            upper triangle (f is Hermitian), the products' k ranges split over eight
+//            waves; then k_s = f and the next stage input, on the tile and its mirror
+//            image: the increment h sum a_{s+1,j} k_j for stages 1..5 (the generator is
+//            constant, so f(y + Delta) = k_0 + f(Delta) and k_1..k_5 hold f(Delta_s)
+//            only), y + that increment for stage 6; or on the last stage the FP64
+//            partial sums of the scaled error. The stage inputs alternate between two
+//            buffers.
+// Bound by the FP32 matrix cores and the L2 reads of their operands; the splits are there
+// because a few hundred tiles of one or two instances would otherwise leave most of the
+// 1024 SIMDs idle. Two instances of n = 233 with 3 jump operators: a stage 46 -> 27 us
+// (before: tmp = Hnh ys + sum_k X_k L_k^dag / 2 on all tiles, one wave each, and a third
+// launch for tmp + tmp^dag). An XCD-aware order of the tiles made no difference.
 // and one commit launch per step (accept/reject, dense-output saves, y <- y1 in
 // FP64, the next stage input), as in the DIA grid integrator: every workgroup
 // reduces its instance's partial sums in the same order, control blocks alternate
@@ -50,13 +57,14 @@ __device__ __forceinline__ bool is_done(const Ctrl &c, double t1) { return c.sta
 __device__ __forceinline__ double step_h(const Ctrl &c, double t1) { return snaps_to(c.t, c.dt, t1) ? t1 - c.t : c.dt; }
 __device__ __forceinline__ double step_end(const Ctrl &c, double t1) { return snaps_to(c.t, c.dt, t1) ? t1 : c.t + c.dt; }
 
-// per-instance scratch (the descriptor's work buffer): k_0..k_6, ys, tmp, X_k
+// per-instance scratch (the descriptor's work buffer): k_0..k_6, the two stage inputs, X_k
 __device__ __forceinline__ float2 *kslot(const dqh_me_inst &p, int j, int64_t rot) {
   const size_t nn = (size_t)p.np * p.np;
   return gp<float2>(p.work) + (size_t)((j + rot) % 7) * nn;
 }
-__device__ __forceinline__ float2 *ysb(const dqh_me_inst &p) { return gp<float2>(p.work) + 7 * (size_t)p.np * p.np; }
-__device__ __forceinline__ float2 *tmpb(const dqh_me_inst &p) { return gp<float2>(p.work) + 8 * (size_t)p.np * p.np; }
+__device__ __forceinline__ float2 *ysb(const dqh_me_inst &p, int which) {
+  return gp<float2>(p.work) + (size_t)(7 + which) * p.np * p.np;
+}
 __device__ __forceinline__ float2 *xb(const dqh_me_inst &p) { return gp<float2>(p.work) + 9 * (size_t)p.np * p.np; }
 __device__ __forceinline__ double *partial(const G &g, size_t inst, int which) {
   return g.part + (inst * 2 + which) * g.npart;
@@ -89,103 +97,223 @@ __device__ __forceinline__ Ctrl ctrl_of(const G &g, int cur) {
 }
 
 // ----------------------------------------------------------- vector field
-// X_k = L_k ys for every jump operator; grid (ceil(maxL * T^2 / 4), ninst), 4 waves
-__global__ __launch_bounds__(256) void k_xprod(const dqh_me_inst *__restrict__ insts, G g, int cur) {
-  const dqh_me_inst &p = insts[blockIdx.y];
-  if (cur >= 0 && is_done(ctrl_of(g, cur), p.t1)) return;
-  const int np = (int)p.np, T = np >> 4;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= (int)p.nL * T * T) return;  // wave-uniform: no barrier follows
-  const int lane = threadIdx.x & 63;
-  const size_t nn = (size_t)np * np;
-  const int kk = t / (T * T), ti = (t / T) % T, tj = t % T;
-  Acc acc;
-  acc_zero(acc);
-  tile_mac(acc, gp<const float2>(p.Dops) + kk * nn, np, ysb(p), np, ti * 16, tj * 16, np, lane);
-  tile_store(acc, xb(p) + kk * nn, np, ti * 16, tj * 16, lane);
+// operands of one k-block of 16 (tile_mac's lane layout) and their products
+struct Ops {
+  float4 a01, a23;
+  float2 b[4];
+};
+__device__ __forceinline__ void load_a(Ops &o, const float2 *A, int ld, int row0, int k0, int lane) {
+  const float2 *p = A + (size_t)(row0 + (lane & 15)) * ld + 4 * (lane >> 4) + k0;
+  o.a01 = *reinterpret_cast<const float4 *>(p);
+  o.a23 = *reinterpret_cast<const float4 *>(p + 2);
+}
+__device__ __forceinline__ void load_b(Ops &o, const float2 *B, int ld, int col0, int k0, int lane) {
+  const float2 *p = B + (size_t)(4 * (lane >> 4) + k0) * ld + col0 + (lane & 15);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o.b[i] = p[(size_t)i * ld];
+}
+__device__ __forceinline__ void mac(Acc &acc, const Ops &a, const Ops &b) {
+  cmfma(acc, a.a01.x, a.a01.y, b.b[0]);
+  cmfma(acc, a.a01.z, a.a01.w, b.b[1]);
+  cmfma(acc, a.a23.x, a.a23.y, b.b[2]);
+  cmfma(acc, a.a23.z, a.a23.w, b.b[3]);
+}
+// accumulator tile of a wave to LDS, row-major
+__device__ __forceinline__ void to_lds(const Acc &acc, float2 *t, int lane) {
+  const int r = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) t[(4 * g + v) * 16 + r] = make_float2(acc.re[v], acc.im[v]);
 }
 
-// tmp = Hnh ys + sum_k X_k C_k; grid (ceil(T^2 / 4), ninst), 4 waves
-__global__ __launch_bounds__(256) void k_tmp(const dqh_me_inst *__restrict__ insts, G g, int cur) {
+// X_k = L_k ys (input buffer `which`) for every jump operator; grid (maxL * ceil(T/2)^2,
+// ninst), 4 waves: wave w sums the k-blocks w, w + 4, .. of the four 16 x 16 tiles
+__global__ __launch_bounds__(256) void k_xprod(const dqh_me_inst *__restrict__ insts, G g, int which, int cur) {
+  __shared__ float2 part[4][4][256];
   const dqh_me_inst &p = insts[blockIdx.y];
   if (cur >= 0 && is_done(ctrl_of(g, cur), p.t1)) return;
-  const int np = (int)p.np, T = np >> 4;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= T * T) return;
-  const int lane = threadIdx.x & 63;
+  const int np = (int)p.np, T = np >> 4, H = (T + 1) >> 1;
+  const int kk = blockIdx.x / (H * H), t = blockIdx.x - kk * H * H;
+  if (kk >= (int)p.nL) return;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const size_t nn = (size_t)np * np;
-  const int ti = t / T, tj = t % T;
-  Acc acc;
-  acc_zero(acc);
-  if (p.flags & DQH_FLAG_HAS_HNH) tile_mac(acc, gp<const float2>(p.Hnh), np, ysb(p), np, ti * 16, tj * 16, np, lane);
-  const float2 *X = xb(p), *C = gp<const float2>(p.Cops);
-  for (int kk = 0; kk < (int)p.nL; ++kk) tile_mac(acc, X + kk * nn, np, C + kk * nn, np, ti * 16, tj * 16, np, lane);
-  tile_store(acc, tmpb(p), np, ti * 16, tj * 16, lane);
+  const int ti = 2 * (t / H), tj = 2 * (t % H);
+  // an odd T: the tiles past the end repeat the last ones and are not stored
+  const int ri[2] = {ti, min(ti + 1, T - 1)}, cj[2] = {tj, min(tj + 1, T - 1)};
+  const float2 *A = gp<const float2>(p.Dops) + kk * nn, *Y = ysb(p, which);
+  Acc acc[2][2];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) acc_zero(acc[x >> 1][x & 1]);
+  Ops o[2], nx[2];
+  auto fetch = [&](Ops (&q)[2], int kb) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      load_a(q[x], A, np, 16 * ri[x], 16 * kb, lane);
+      load_b(q[x], Y, np, 16 * cj[x], 16 * kb, lane);
+    }
+  };
+  if (w < T) fetch(o, w);
+  for (int kb = w; kb < T; kb += 4) {
+    if (kb + 4 < T) fetch(nx, kb + 4);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) mac(acc[x][y], o[x], o[y]);
+    o[0] = nx[0];
+    o[1] = nx[1];
+  }
+#pragma unroll
+  for (int x = 0; x < 4; ++x) to_lds(acc[x >> 1][x & 1], part[w][x], lane);
+  __syncthreads();
+  float2 *X = xb(p) + kk * nn;
+  const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    if (ti + (x >> 1) >= T || tj + (x & 1) >= T) continue;
+    float2 v = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v.x += part[q][x][threadIdx.x].x;
+      v.y += part[q][x][threadIdx.x].y;
+    }
+    X[(size_t)(16 * (ti + (x >> 1)) + r) * np + 16 * (tj + (x & 1)) + c] = v;
+  }
 }
 
-__device__ __forceinline__ float2 field_at(const float2 *tmp, int np, int i, int j) {
-  const float2 a = tmp[(size_t)i * np + j], b = tmp[(size_t)j * np + i];
-  return make_float2(a.x + b.x, a.y - b.y);
+// tile (ti <= tj) of the upper triangle by its number
+__device__ __forceinline__ void upper_tile(int t, int T, int &ti, int &tj) {
+  // rows of T, T - 1, .. tiles: ti is the largest row whose first tile is <= t
+  const float b = 2.f * T + 1.f;
+  ti = (int)((b - sqrtf(b * b - 8.f * t)) * 0.5f);
+  auto first = [&](int r) { return r * T - r * (r - 1) / 2; };
+  while (ti > 0 && first(ti) > t) --ti;
+  while (first(ti + 1) <= t) ++ti;
+  tj = ti + t - first(ti);
 }
 
 // ------------------------------------------------------------------ one step
-// stage s = 1..6 after k_xprod / k_tmp on ys; grid (ceil(np^2 / 256), ninst)
-__global__ __launch_bounds__(256) void k_body(const dqh_me_inst *__restrict__ insts, G g, int s, int cur) {
-  __shared__ double sh[4];
+// f at an upper tile and its mirror image, then by mode s:
+//   1..6  the stage: k_s = f, the next stage input or the error partials
+//   0     (initial step) f -> k_0
+//   7     (initial step) f -> stage input buffer 1
+// Input: buffer (s + 1) & 1 for stages, buffer 0 for the initial step.
+// grid (T (T + 1) / 2, ninst), 8 waves
+__global__ __launch_bounds__(512) void k_stage(const dqh_me_inst *__restrict__ insts, G g, int s, int cur) {
+  __shared__ float2 part[8][2][256];
+  __shared__ double sh[8];
   const dqh_me_inst &p = insts[blockIdx.y];
   const RKTab &rk = rk_tab(p.flags);
   const Ctrl c = ctrl_of(g, cur);
-  if (is_done(c, p.t1)) return;
-  const double h = step_h(c, p.t1);
-  const int np = (int)p.np, n = (int)p.n;
+  if (cur >= 0 && is_done(c, p.t1)) return;
+  const int np = (int)p.np, n = (int)p.n, T = np >> 4;
   const size_t nn = (size_t)np * np;
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  int ti, tj;
+  upper_tile((int)blockIdx.x, T, ti, tj);
+  const bool stage = s >= 1 && s <= 6;
+  const float2 *Y = ysb(p, stage ? (s + 1) & 1 : 0);
+  const float2 *Hn = gp<const float2>(p.Hnh), *X = xb(p), *C = gp<const float2>(p.Cops);
+  // product 0: (Hnh ys)[ti][tj], 1: (Hnh ys)[tj][ti], 2 + k: 2 X_k C_k = X_k L_k^dag at [ti][tj]
+  Acc up, lo;
+  acc_zero(up);
+  acc_zero(lo);
+  const int first = (p.flags & DQH_FLAG_HAS_HNH) ? 0 : 2 * T, last = (2 + (int)p.nL) * T;
+  auto fetch = [&](Ops &o, int b) {
+    const int m = b / T, kb = b - m * T;
+    if (m < 2) {
+      load_a(o, Hn, np, 16 * (m ? tj : ti), 16 * kb, lane);
+      load_b(o, Y, np, 16 * (m ? ti : tj), 16 * kb, lane);
+    } else {
+      load_a(o, X + (m - 2) * nn, np, 16 * ti, 16 * kb, lane);
+      load_b(o, C + (m - 2) * nn, np, 16 * tj, 16 * kb, lane);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        o.b[i].x *= 2.f;
+        o.b[i].y *= 2.f;
+      }
+    }
+  };
+  Ops o, nx;
+  if (first + w < last) fetch(o, first + w);
+  for (int b = first + w; b < last; b += 8) {
+    if (b + 8 < last) fetch(nx, b + 8);
+    if (b >= T && b < 2 * T)
+      mac(lo, o, o);
+    else
+      mac(up, o, o);
+    o = nx;
+  }
+  to_lds(up, part[w][0], lane);
+  to_lds(lo, part[w][1], lane);
+  __syncthreads();
+  // threads 0..255: the tile; 256..511: its mirror image (not for a tile on the diagonal)
+  const int half = threadIdx.x >> 8, a = (threadIdx.x >> 4) & 15, b = threadIdx.x & 15;
   double acc = 0.0;
-  if (e < (int64_t)nn) {
-    const int i = (int)e / np, j = (int)e - ((int)e / np) * np;  // e < np^2 < 2^31
-    const float2 f = field_at(tmpb(p), np, i, j);
-    kslot(p, s, c.rot)[e] = f;
-    // increment form (constant generators): stages 1..5 hold g_s = f(Delta_s),
-    // k_s = k_0 + g_s, folded into the weight of k_0 (stage 6 is f(y1))
-    const float2 k0 = kslot(p, 0, c.rot)[e];
-    if (s < 6) {
-      double a0 = 0.0;
-      for (int q = 0; q <= s; ++q) a0 += rk.A[s + 1][q];
-      double re = h * a0 * k0.x + h * rk.A[s + 1][s] * f.x, im = h * a0 * k0.y + h * rk.A[s + 1][s] * f.y;
-      if (s + 1 == 6) {
+  if (half == 0 || ti != tj) {
+    // position in the upper tile: (a, b), or (b, a) for the mirror image
+    int pr = half ? b : a, pc = half ? a : b;
+    bool conj = half != 0;
+    if (ti == tj && pr > pc) {  // below the diagonal of a diagonal tile
+      const int x = pr;
+      pr = pc;
+      pc = x;
+      conj = true;
+    }
+    float2 f = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float2 u = part[q][0][pr * 16 + pc], l = part[q][1][pc * 16 + pr];
+      f.x += u.x + l.x;
+      f.y += u.y - l.y;
+    }
+    if (conj) f.y = -f.y;
+    const int i = 16 * (half ? tj : ti) + a, j = 16 * (half ? ti : tj) + b;
+    if (i == j) f.y = 0.f;
+    const size_t e = (size_t)i * np + j;
+    if (!stage) {
+      (s == 0 ? kslot(p, 0, 0) : ysb(p, 1))[e] = f;
+    } else {
+      const double h = step_h(c, p.t1);
+      kslot(p, s, c.rot)[e] = f;
+      const float2 k0 = kslot(p, 0, c.rot)[e];
+      if (s < 6) {
+        double a0 = 0.0;
+        for (int q = 0; q <= s; ++q) a0 += rk.A[s + 1][q];
+        double re = h * a0 * k0.x + h * rk.A[s + 1][s] * f.x, im = h * a0 * k0.y + h * rk.A[s + 1][s] * f.y;
+        if (s + 1 == 6) {
+          const double2 yv = gp<const double2>(p.y)[e];
+          re += yv.x;
+          im += yv.y;
+        }
+        for (int q = 1; q < s; ++q) {
+          const float2 kq = kslot(p, q, c.rot)[e];
+          re += h * rk.A[s + 1][q] * kq.x;
+          im += h * rk.A[s + 1][q] * kq.y;
+        }
+        ysb(p, s & 1)[e] = make_float2((float)re, (float)im);
+      } else if (i < n && j < n) {
         const double2 yv = gp<const double2>(p.y)[e];
-        re += yv.x;
-        im += yv.y;
+        double ew[7], bw[7];
+        for (int q = 0; q < 7; ++q) ew[q] = rk.E[q], bw[q] = rk.A[6][q];
+        fold_k0(ew);
+        fold_k0(bw);
+        double er = ew[6] * f.x + ew[0] * k0.x, ei = ew[6] * f.y + ew[0] * k0.y;
+        double yr = yv.x + h * bw[0] * k0.x, yi = yv.y + h * bw[0] * k0.y;
+        for (int q = 1; q < 6; ++q) {
+          const float2 kq = kslot(p, q, c.rot)[e];
+          er += ew[q] * kq.x;
+          ei += ew[q] * kq.y;
+          yr += h * bw[q] * kq.x;
+          yi += h * bw[q] * kq.y;
+        }
+        er *= h;
+        ei *= h;
+        const double sc = p.atol + p.rtol * fmax(sqrt(sq(yv)), sqrt(yr * yr + yi * yi));
+        acc += (er * er + ei * ei) / (sc * sc);
       }
-      for (int q = 1; q < s; ++q) {
-        const float2 kq = kslot(p, q, c.rot)[e];
-        re += h * rk.A[s + 1][q] * kq.x;
-        im += h * rk.A[s + 1][q] * kq.y;
-      }
-      ysb(p)[e] = make_float2((float)re, (float)im);
-    } else if (i < n && j < n) {
-      const double2 yv = gp<const double2>(p.y)[e];
-      double ew[7], bw[7];
-      for (int q = 0; q < 7; ++q) ew[q] = rk.E[q], bw[q] = rk.A[6][q];
-      fold_k0(ew);
-      fold_k0(bw);
-      double er = ew[6] * f.x + ew[0] * k0.x, ei = ew[6] * f.y + ew[0] * k0.y;
-      double yr = yv.x + h * bw[0] * k0.x, yi = yv.y + h * bw[0] * k0.y;
-      for (int q = 1; q < 6; ++q) {
-        const float2 kq = kslot(p, q, c.rot)[e];
-        er += ew[q] * kq.x;
-        ei += ew[q] * kq.y;
-        yr += h * bw[q] * kq.x;
-        yi += h * bw[q] * kq.y;
-      }
-      er *= h;
-      ei *= h;
-      const double sc = p.atol + p.rtol * fmax(sqrt(sq(yv)), sqrt(yr * yr + yi * yi));
-      acc += (er * er + ei * ei) / (sc * sc);
     }
   }
   if (s == 6) {
-    const double tot = block_sum<256>(acc, sh);
+    const double tot = block_sum<512>(acc, sh);
     if (threadIdx.x == 0) partial(g, blockIdx.y, 0)[blockIdx.x] = tot;
   }
 }
@@ -206,7 +334,8 @@ __global__ __launch_bounds__(256) void k_commit(const dqh_me_inst *__restrict__ 
   const double h = step_h(c, p.t1);
   const double t_new = step_end(c, p.t1);
   const double inv_nn = 1.0 / ((double)p.n * (double)p.n);
-  const double norm = sqrt(reduce_partials<256>(partial(g, inst, 0), g.npart, sh) * inv_nn);
+  const int T = (int)p.np >> 4;
+  const double norm = sqrt(reduce_partials<256>(partial(g, inst, 0), T * (T + 1) / 2, sh) * inv_nn);
   const bool finite = isfinite(norm);
   const bool keep = finite && norm < 1.0;
   double factor;
@@ -285,7 +414,7 @@ __global__ __launch_bounds__(256) void k_commit(const dqh_me_inst *__restrict__ 
     // stage 1 input of the next attempt: the increment hn a_10 k_0
     if (!is_done(o, p.t1)) {
       const double hn = step_h(o, p.t1);
-      ysb(p)[e] = make_float2((float)(hn * rk.A[1][0] * k0n.x), (float)(hn * rk.A[1][0] * k0n.y));
+      ysb(p, 0)[e] = make_float2((float)(hn * rk.A[1][0] * k0n.x), (float)(hn * rk.A[1][0] * k0n.y));
     }
   }
   if (writer) *nx = o;
@@ -313,7 +442,7 @@ __global__ __launch_bounds__(256) void k_init(const dqh_me_inst *__restrict__ in
   if (e < (int64_t)nn) {
     const double2 yv = gp<const double2>(p.y)[e];
     const float2 f = make_float2((float)yv.x, (float)yv.y);
-    ysb(p)[e] = f;
+    ysb(p, 0)[e] = f;
     const int i = (int)e / np, j = (int)e - ((int)e / np) * np;  // e < np^2 < 2^31
     if ((p.flags & DQH_FLAG_SAVE_STATES) && i < n && j < n) {
       float2 *st = gp<float2>(p.states);
@@ -333,8 +462,8 @@ __global__ __launch_bounds__(256) void k_init(const dqh_me_inst *__restrict__ in
   }
 }
 
-// pass 0: k_0 = f(y0) and the partials of d0, d1; pass 1: partials of d2 for
-// f(y0 + h0 k_0) (Hairer-Norsett-Wanner II.4, as the persistent kernel)
+// pass 0: the partials of d0, d1 from k_0 = f(y0); pass 1: partials of d2 from
+// f(y0 + h0 k_0) in stage input buffer 1 (Hairer-Norsett-Wanner II.4, as the persistent kernel)
 __global__ __launch_bounds__(256) void k_init_body(const dqh_me_inst *__restrict__ insts, G g, int pass) {
   __shared__ double sh[4];
   const size_t inst = blockIdx.y;
@@ -346,12 +475,11 @@ __global__ __launch_bounds__(256) void k_init_body(const dqh_me_inst *__restrict
   double a0 = 0.0, a1 = 0.0;
   if (e < (int64_t)nn) {
     const int i = (int)e / np, j = (int)e - ((int)e / np) * np;  // e < np^2 < 2^31
-    const float2 f = field_at(tmpb(p), np, i, j);
+    const float2 *k0 = kslot(p, 0, 0);
+    const float2 f = (pass == 0 ? k0 : ysb(p, 1))[e];
     const double2 yv = gp<const double2>(p.y)[e];
     const double sc = p.atol + p.rtol * sqrt(sq(yv));
-    float2 *k0 = kslot(p, 0, 0);
     if (pass == 0) {
-      k0[e] = f;
       if (i < n && j < n) {
         a0 = sq(yv) / (sc * sc);
         a1 = ((double)f.x * f.x + (double)f.y * f.y) / (sc * sc);
@@ -385,7 +513,7 @@ __global__ __launch_bounds__(256) void k_init_h0(const dqh_me_inst *__restrict__
   if (e < (int64_t)nn) {
     const double2 yv = gp<const double2>(p.y)[e];
     const float2 kq = kslot(p, 0, 0)[e];
-    ysb(p)[e] = make_float2((float)(yv.x + h0 * kq.x), (float)(yv.y + h0 * kq.y));
+    ysb(p, 0)[e] = make_float2((float)(yv.x + h0 * kq.x), (float)(yv.y + h0 * kq.y));
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     Ctrl o = c;
@@ -415,7 +543,7 @@ __global__ __launch_bounds__(256) void k_init_dt(const dqh_me_inst *__restrict__
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e < (int64_t)nn && o.status == 0) {  // stage 1 input (increment form)
     const float2 kq = kslot(p, 0, 0)[e];
-    ysb(p)[e] = make_float2((float)(hn * rk.A[1][0] * kq.x), (float)(hn * rk.A[1][0] * kq.y));
+    ysb(p, 0)[e] = make_float2((float)(hn * rk.A[1][0] * kq.x), (float)(hn * rk.A[1][0] * kq.y));
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) g.ctrl[inst] = o;
 }
@@ -505,16 +633,14 @@ struct Launch {
   dim3 gx, gt, gflat;
 };
 
-void launch_field(const dqh_me_inst *d, const dgrid::G &g, const Launch &L, int cur, hipStream_t s) {
-  hipLaunchKernelGGL(dgrid::k_xprod, L.gx, dim3(256), 0, s, d, g, cur);
-  hipLaunchKernelGGL(dgrid::k_tmp, L.gt, dim3(256), 0, s, d, g, cur);
+// mode s of k_stage on its input
+void launch_stage(const dqh_me_inst *d, const dgrid::G &g, const Launch &L, int s, int cur, hipStream_t st) {
+  hipLaunchKernelGGL(dgrid::k_xprod, L.gx, dim3(256), 0, st, d, g, s >= 1 && s <= 6 ? (s + 1) & 1 : 0, cur);
+  hipLaunchKernelGGL(dgrid::k_stage, L.gt, dim3(512), 0, st, d, g, s, cur);
 }
 
 void launch_step(const dqh_me_inst *d, const dgrid::G &g, const Launch &L, int cur, hipStream_t s) {
-  for (int sg = 1; sg <= 6; ++sg) {
-    launch_field(d, g, L, cur, s);
-    hipLaunchKernelGGL(dgrid::k_body, L.gflat, dim3(256), 0, s, d, g, sg, cur);
-  }
+  for (int sg = 1; sg <= 6; ++sg) launch_stage(d, g, L, sg, cur, s);
   hipLaunchKernelGGL(dgrid::k_commit, L.gflat, dim3(256), 0, s, d, g, cur);
 }
 
@@ -560,24 +686,26 @@ extern "C" int dqh_mesolve_tsit5_dense_grid(const dqh_me_inst *d_insts, const dq
   g.flag = reinterpret_cast<int64_t *>(w + Ly.flag);
   const int64_t T = np / 16;
   Launch L;
-  L.gx = dim3((unsigned)std::max<int64_t>(1, (maxL * T * T + 3) / 4), (unsigned)ninst);
-  L.gt = dim3((unsigned)((T * T + 3) / 4), (unsigned)ninst);
+  const int64_t H = (T + 1) / 2;
+  L.gx = dim3((unsigned)std::max<int64_t>(1, maxL * H * H), (unsigned)ninst);
+  L.gt = dim3((unsigned)(T * (T + 1) / 2), (unsigned)ninst);
   L.gflat = dim3((unsigned)((np * np + 255) / 256), (unsigned)ninst);
   g.npart = L.gflat.x;
   hipStream_t st = (hipStream_t)stream;
 
   hipLaunchKernelGGL(dgrid::k_init, L.gflat, dim3(256), 0, st, d_insts, g);
-  launch_field(d_insts, g, L, -1, st);
+  launch_stage(d_insts, g, L, 0, -1, st);
   hipLaunchKernelGGL(dgrid::k_init_body, L.gflat, dim3(256), 0, st, d_insts, g, 0);
   hipLaunchKernelGGL(dgrid::k_init_h0, L.gflat, dim3(256), 0, st, d_insts, g);
-  launch_field(d_insts, g, L, -1, st);
+  launch_stage(d_insts, g, L, 7, -1, st);
   hipLaunchKernelGGL(dgrid::k_init_body, L.gflat, dim3(256), 0, st, d_insts, g, 1);
   hipLaunchKernelGGL(dgrid::k_init_dt, L.gflat, dim3(256), 0, st, d_insts, g);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess)
     return fail(DQH_HIP_ERROR, std::string("dqh_mesolve_tsit5_dense_grid init: ") + hipGetErrorString(err));
 
-  const int64_t G = graph_steps > 0 ? graph_steps : 2;
+  // at most 4 steps per replay: what is launched past the last step is lost
+  const int64_t G = graph_steps > 0 ? std::min<int64_t>(graph_steps, 4) : 2;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipStream_t cs = nullptr;
