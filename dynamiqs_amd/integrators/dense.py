@@ -168,6 +168,18 @@ def check_descriptors(descs: np.ndarray, tensors, extents: dict | None = None) -
         raise RuntimeError(f'descriptor field {POINTER_FIELDS[j // B]} = {int(v[j]):#x} is outside the plan allocations')
 
 
+def to_host(t) -> np.ndarray:
+    """The device tensor ``t`` as a new host array. numpy asks for huge pages for its large
+    arrays and torch does not: 53 MB take 5.4 ms here and 13.4 ms with ``t.cpu()``, which
+    spends them on page faults."""
+    import torch
+
+    if t.numel() == 0:
+        return t.cpu().numpy()
+    out = torch.from_numpy(np.empty(tuple(t.shape), dtype=t.new_empty(0, device='cpu').numpy().dtype))
+    return out.copy_(t).numpy()
+
+
 def _device():
     import torch
 
@@ -247,17 +259,19 @@ class DensePlan:
         }[self.kind]
         _native.check(fn(_native.ctypes.c_void_p(self.d_descs.data_ptr()), self.ninst, sp), f'dqh {self.kind}')
 
-    def results(self) -> dict:
+    def results(self, final: bool = True) -> dict:
+        """The results on the host; without the final states unless ``final``."""
         import torch
 
         torch.cuda.synchronize()
         n = self.n
         out = {}
-        c64 = lambda t: t.cpu().numpy().view(np.complex64)  # noqa: E731
+        c64 = lambda t: to_host(t).view(np.complex64)  # noqa: E731
         if self.states is not None:
             shp = (self.ninst, self.ntsave, n, n) if self.save_states else (self.ninst, 1, n, n)
             out['states'] = c64(self.states).reshape(shp)
-        out['final_state'] = c64(self.final).reshape(self.ninst, n, n)
+        if final:
+            out['final_state'] = c64(self.final).reshape(self.ninst, n, n)
         if self.nE:
             out['expects'] = c64(self.expects).reshape(self.ninst, self.nE, self.ntsave)
         st = self.stats.cpu().numpy()
@@ -580,12 +594,21 @@ def few_diagonals(instances: list, npad: int) -> Stencil | None:
     Lall = np.stack([np.stack(Ls) if K else np.zeros((0, n, n)) for Ls in Lsets]).astype(np.complex128)
     LdL = np.swapaxes(Lall.conj(), -1, -2) @ Lall
     LdL = LdL.sum(axis=1)
-    explicit = [instances[b].Hnh is not None for b in first]
-    G = -1j * np.stack([instances[b].H for b in first]) - 0.5 * LdL[il[first]]
-    for k, b in enumerate(first):
-        if explicit[k]:
-            G[k] = instances[b].Hnh
-    mask = np.any(G != 0, axis=0)
+    # generators -i H - 1/2 sum L^dag L, or the explicit ones; formed on their diagonals only
+    explicit = np.array([instances[b].Hnh is not None for b in first])
+    Hs = np.stack([instances[b].Hnh if e else instances[b].H for b, e in zip(first, explicit)])
+    mask = np.zeros((n, n), dtype=bool)
+    for x in Hs:
+        mask |= x != 0
+    if not explicit.all():
+        mask |= np.any(LdL != 0, axis=0)
+
+    def generators(offs):
+        rows = _rows_on(Hs, offs, npad)
+        plain = ~explicit
+        rows[plain] = -1j * rows[plain] - 0.5 * _rows_on(LdL, offs, npad)[il[first]][plain]
+        return rows
+
     for term in {id(o): o for i in instances for o in [p[2] for p in i.pwc] + [m[1] for m in i.mod]}.values():
         mask = mask | (np.asarray(term) != 0)
     offH = [o for o in _offsets(mask) if o != 0]
@@ -602,7 +625,7 @@ def few_diagonals(instances: list, npad: int) -> Stencil | None:
         for u, o in enumerate(offs):
             ops.off[k][u] = o
     L = [_rows_on(Lall[:, k], offs, npad) for k, offs in enumerate(offL)]
-    return Stencil(offH, offL, ops, _rows_on(G, offH, npad).astype(np.complex64), _rows_on(G, [0], npad)[:, 0],
+    return Stencil(offH, offL, ops, generators(offH).astype(np.complex64), generators([0])[:, 0],
                    np.concatenate(L, axis=1).astype(np.complex64) if K else np.zeros((len(Lsets), 0, npad), np.complex64),
                    ig, il)
 
@@ -756,6 +779,7 @@ def build_plan(
         return cache[key]
 
     npwc_max = 0
+    decay = {}  # sum L^dag L of the constant jump operators, by their arrays
     kraus_index = {}  # ('kraus', key_H, key_L) -> step key -> set index, for sets already built
     kraus_bytes = [0]  # device bytes of the Kraus sets built for this batch
     nmod_max = max((len(_hmods(inst)) for inst in instances), default=0)
@@ -878,19 +902,26 @@ def build_plan(
                 if inst.Hnh is not None:
                     return _pad(np.asarray(inst.Hnh, dtype=np.complex128), npad)
                 # the time-dependent jump operators' L^dag L terms are in Hmod / Hpwc
-                LdL = sum((_dag(L) @ L for k, L in enumerate(inst.Ls) if not lmod[k]), np.zeros_like(inst.H))
-                return _pad(-1j * inst.H - 0.5 * LdL, npad)
+                lkey = (tuple(id(L) for L in inst.Ls), tuple(lmod))  # the arrays live as long as the instances
+                if lkey not in decay:
+                    decay[lkey] = sum((_dag(L) @ L for k, L in enumerate(inst.Ls) if not lmod[k]),
+                                      np.zeros((n, n), dtype=np.complex128))
+                return _pad(-1j * inst.H - 0.5 * decay[lkey], npad)
 
             hkey = ('Hnh', inst.key_H, inst.key_L, tuple(lmod))
             if hdiag_plan:
                 # the resident body adds the diagonal in FP64 (hdiag); Hnh keeps the rest
-                def bHoff(bH128=bH128):
-                    a = np.array(bH128(), dtype=np.complex128)  # a copy: bH128 may return the caller's Hnh
+                diag = []
+
+                def bHoff(bH128=bH128, diag=diag):
+                    a = bH128()
+                    diag.append(np.diag(a).astype(np.complex128))
+                    a = a.astype(np.complex64)  # a copy: bH128 may return the caller's Hnh
                     np.fill_diagonal(a, 0.0)
-                    return a.astype(np.complex64)
+                    return a
 
                 d['Hnh'] = shared(hkey + ('off',), bHoff)
-                d['hdiag'] = shared(hkey + ('diag',), lambda bH128=bH128: np.ascontiguousarray(np.diag(bH128())))
+                d['hdiag'] = shared(hkey + ('diag',), lambda diag=diag: diag[0])
             else:
                 d['Hnh'] = shared(hkey, lambda bH128=bH128: bH128().astype(np.complex64))
             if K and inst.Cs is not None:  # D/C pairs of expanded jump-operator sums
@@ -1012,8 +1043,10 @@ def build_plan(
 
     # ---- one host-to-device transfer for every staged operator, then real addresses
     arena.upload()
+    u = np.uint64
     for f in ARENA_FIELDS:
-        descs[f] = [arena.patch(int(v)) for v in descs[f]]
+        v = descs[f]
+        descs[f] = np.where(v != 0, v + u(arena.base) - u(1), u(0))
 
     # ---- state, scratch, outputs
     welems = _native.work_elems(npad, nLdev, npwc_max + nmod_max)
@@ -1025,14 +1058,18 @@ def build_plan(
         welems = 7 * (n * (n + 1) // 2) if n > STENCIL_WORK_N else 0
     work = arena.empty(B * welems * 8)
     y = torch.zeros((B, 2, nn, 2), dtype=torch.float64, device=dev)
-    y0 = np.zeros((B, npad, npad), dtype=np.complex128)
-    rho_cache = {}
-    for b, inst in enumerate(instances):
-        key = inst.key_rho
-        y0[b, :n, :n] = inst.rho0
-        if key is not None:
-            rho_cache[key] = b
-    y0_t = torch.from_numpy(y0.reshape(B, nn).view(np.float64).reshape(B, nn, 2)).to(dev)
+    # one copy per distinct state array goes to the device
+    slot, distinct = {}, []
+    for inst in instances:
+        if id(inst.rho0) not in slot:
+            slot[id(inst.rho0)] = len(distinct)
+            distinct.append(inst.rho0)
+    y0 = np.zeros((len(distinct), npad, npad), dtype=np.complex128)
+    for k, rho in enumerate(distinct):
+        y0[k, :n, :n] = rho
+    y0_t = torch.from_numpy(y0.reshape(-1, nn).view(np.float64).reshape(-1, nn, 2)).to(dev)
+    if len(distinct) < B:
+        y0_t = y0_t[torch.tensor([slot[id(inst.rho0)] for inst in instances], device=dev)]
     y[:, 0].copy_(y0_t)
     plan.y, plan.y0 = y, y0_t
     arena.tensors.append(y)
@@ -1042,14 +1079,17 @@ def build_plan(
     expects = torch.zeros((B, max(nE, 1) * len(tsave) * 2), dtype=torch.float32, device=dev)
     stats = torch.zeros((B, 8), dtype=torch.int64, device=dev)
     plan.states, plan.final, plan.expects, plan.stats = states, final, expects, stats
-    for b in range(B):
-        d = descs[b]
-        d['y'] = y.data_ptr() + b * 2 * nn * 16
-        d['work'] = work.data_ptr() + b * welems * 8 if welems else 0
-        d['states'] = states.data_ptr() + b * ns * n * n * 8
-        d['final_state'] = final.data_ptr() + b * n * n * 8
-        d['expects'] = expects.data_ptr() + b * max(nE, 1) * len(tsave) * 8
-        d['stats'] = stats.data_ptr() + b * 64
+    at = np.arange(B, dtype=u)
+
+    def column(t, stride):
+        return u(t.data_ptr()) + at * u(stride)
+
+    descs['y'] = column(y, 2 * nn * 16)
+    descs['work'] = column(work, welems * 8) if welems else 0
+    descs['states'] = column(states, ns * n * n * 8)
+    descs['final_state'] = column(final, n * n * 8)
+    descs['expects'] = column(expects, max(nE, 1) * len(tsave) * 8)
+    descs['stats'] = column(stats, 64)
     step_log = None
     if step_log_cap > 0 and kind == 'tsit5':
         step_log = torch.zeros((B, int(step_log_cap)), dtype=torch.float64, device=dev)

@@ -148,6 +148,19 @@ def enumerate_instances(H: TimeQArray, Ls, rho0: QArray, cartesian: bool):
     else:
         out_shape = tuple(np.broadcast_shapes(*shapes))
     insts = []
+    # a batch element's operators and state are formed once, however many instances use them
+    rhos, Hs, Lcs = {}, {}, {}
+    has_const = [Lt.const is not None and bool(np.any(Lt.const)) for Lt in Lts]
+
+    def once(memo, key, make):
+        if key not in memo:
+            memo[key] = make()
+        return memo[key]
+
+    def state(ir):
+        rho = r[ir]
+        return rho @ rho.conj().T if rho.shape[-1] == 1 else rho
+
     for idx in np.ndindex(*out_shape) if out_shape else [()]:
         if cartesian:
             parts, o = [], 0
@@ -157,15 +170,13 @@ def enumerate_instances(H: TimeQArray, Ls, rho0: QArray, cartesian: bool):
         else:
             parts = [_broadcast_index(idx, s) for s in shapes]
         iH, iLs, ir = parts[0], parts[1:-1], parts[-1]
-        rho = r[ir]
-        if rho.shape[-1] == 1:
-            rho = rho @ rho.conj().T
+        rho = once(rhos, ir, lambda: state(ir))
         Lmods, Lpwcs, Lsums, Lops = [], [], [], []
-        for Lt, i in zip(Lts, iLs):
-            nterms = len(Lt.mod) + len(Lt.pwc) + (Lt.const is not None and bool(np.any(Lt.const)))
+        for q, (Lt, i) in enumerate(zip(Lts, iLs)):
+            nterms = len(Lt.mod) + len(Lt.pwc) + has_const[q]
             if (Lt.mod or Lt.pwc) and nterms > 1:
                 terms = []
-                if Lt.const is not None and np.any(Lt.const):
+                if has_const[q]:
                     terms.append((('const', 1.0), Lt.const_at(i)))
                 for g, o, f in Lt.mod_at(i):
                     terms.append((('mod', g, (id(f), i if np.ndim(f(0.0)) else None)), o))
@@ -190,10 +201,10 @@ def enumerate_instances(H: TimeQArray, Ls, rho0: QArray, cartesian: bool):
             else:
                 Lmods.append(None)
                 Lpwcs.append(None)
-                Lops.append(Lt.const_at(i))
+                Lops.append(once(Lcs, (q, i), lambda: Lt.const_at(i)))
         insts.append(
             dense.Instance(
-                H=Ht.const_at(iH),
+                H=once(Hs, iH, lambda: Ht.const_at(iH)),
                 Ls=Lops,
                 Lmod=Lmods if any(m is not None for m in Lmods) else [],
                 Lpwc=Lpwcs if any(m is not None for m in Lpwcs) else [],
@@ -273,8 +284,8 @@ def mesolve(
 
     out_shape, insts = enumerate_instances(H, Ls, rho0, options.cartesian_batching)
     if options.assume_hermitian and isinstance(method, ADAPTIVE):
-        for inst in insts:
-            check_hermitian(inst.rho0, 'y0')
+        for rho in {id(inst.rho0): inst.rho0 for inst in insts}.values():
+            check_hermitian(rho, 'y0')
     parts, pindex = hermitian_parts([inst.rho0 for inst in insts], options.assume_hermitian and isinstance(method, ADAPTIVE))
     if len(parts) > len(insts):
         solve = []
@@ -284,7 +295,8 @@ def mesolve(
                 solve.append(replace(inst, rho0=parts[ib], key_rho=None))
         insts = solve
     else:
-        insts = [replace(inst, rho0=a) for inst, a in zip(insts, parts)]
+        for inst, a in zip(insts, parts):
+            inst.rho0 = a
     Es = [E.to_numpy() for E in exp_ops] if exp_ops is not None else None
     t0 = None if options.t0 is None else float(options.t0)
     # save_extra sees the state at every save time, whatever save_states is
@@ -338,7 +350,7 @@ def mesolve(
             rouchon_order=_fixed_step_order(method),
         )
     plan.run()
-    res = plan.results()
+    res = plan.results() if adaptive_rouchon else plan.results(final=False)
     if adaptive_rouchon:  # FP64 on the device; results in the dtype of the other paths
         res['states'] = res['states'].astype(np.complex64)
         if 'expects' in res:
@@ -507,24 +519,33 @@ def hermitian_parts(rhos, assume_hermitian: bool):
     parts are solved as separate instances. Returns the list of states to solve and, per input, the index of A
     and of B (-1 when there is no B part)."""
     parts, index = [], []
-    for r in rhos:
+    split = {}  # by array: instances that share a state share its parts
+
+    def parts_of(r):
         r = np.asarray(r)
-        a = 0.5 * (r + r.conj().T)
-        ia = len(parts)
-        parts.append(a)
-        ib = -1
-        asym = np.max(np.abs(r - r.conj().T), initial=0.0)
-        if not assume_hermitian and asym > 1e-14 * max(1.0, np.max(np.abs(r), initial=0.0)):
-            ib = len(parts)
-            parts.append(-0.5j * (r - r.conj().T))
-        index.append((ia, ib))
+        a, b = 0.5 * (r + r.conj().T), None
+        if not assume_hermitian:
+            asym = np.max(np.abs(r - r.conj().T), initial=0.0)
+            if asym > 1e-14 * max(1.0, np.max(np.abs(r), initial=0.0)):
+                b = -0.5j * (r - r.conj().T)
+        return a, b
+
+    for r in rhos:
+        if id(r) not in split:
+            split[id(r)] = parts_of(r)
+        a, b = split[id(r)]
+        index.append((len(parts), -1 if b is None else len(parts) + 1))
+        parts.extend([a] if b is None else [a, b])
     return parts, np.asarray(index, dtype=np.int64).reshape(-1, 2)
 
 
 def combine_parts(x: np.ndarray, index: np.ndarray) -> np.ndarray:
     """x[A] + i x[B] over the first axis (the inverse of ``hermitian_parts``)."""
-    out = x[index[:, 0]].astype(np.result_type(x.dtype, np.complex64))
     has_b = index[:, 1] >= 0
+    dtype = np.result_type(x.dtype, np.complex64)
+    if not np.any(has_b) and x.dtype == dtype and np.array_equal(index[:, 0], np.arange(len(x))):
+        return x  # nothing to recombine
+    out = x[index[:, 0]].astype(dtype)
     if np.any(has_b):
         out[has_b] = out[has_b] + 1j * x[index[has_b, 1]]
     return out

@@ -101,22 +101,29 @@ def check_expm_size(nchain: int, nint: int, N: int) -> None:
         )
 
 
-def expm_chain(X: np.ndarray, Y0: np.ndarray | None = None) -> np.ndarray:
-    """Chained exponentials on the GPU: ``X`` (nchain, nint, N, N) complex holds
-    dt_k A_k; returns U (nchain, nint, N, N) complex64 with
-    U[b, k] = expm(X[b, k]) ... expm(X[b, 0]) (``dqh_expm_propagators``), or, with
-    ``Y0`` (nchain, N, M) a block of initial states per chain as columns, the states
-    U[b, k] Y0[b] (nchain, nint, N, M) (``dqh_cgemm_batched`` on the resident U)."""
+def _norm1(A: np.ndarray) -> float:
+    return float(np.max(np.sum(np.abs(A), axis=-2), initial=0.0))
+
+
+def expm_chain(gens, dts, Y0: np.ndarray | None = None) -> np.ndarray:
+    """Chained exponentials on the GPU: ``gens[b][k]`` is the generator A_k (N, N) of
+    interval k of chain b with its 1-norm and ``dts[k]`` the interval's length; returns U
+    (nchain, nint, N, N) complex64 with U[b, k] = expm(dt_k A_k) ... expm(dt_0 A_0)
+    (``dqh_expm_propagators``), or, with ``Y0`` (nchain, N, M) a block of initial states
+    per chain as columns, the states U[b, k] Y0[b] (nchain, nint, N, M)
+    (``dqh_cgemm_batched`` on the resident U)."""
     import torch
 
-    from .dense import _device
+    from .dense import _device, to_host
 
-    nchain, nint, N = X.shape[0], X.shape[1], X.shape[-1]
+    nchain, nint, N = len(gens), len(dts), gens[0][0][0].shape[-1]
     Np = pad16(N)
-    norm = float(np.max(np.sum(np.abs(X), axis=-2), initial=0.0))  # largest 1-norm
+    norm = max(abs(float(dt)) * size for g in gens for (_, size), dt in zip(g, dts))
     s = int(max(0, np.ceil(np.log2(norm / THETA)))) if norm > THETA else 0
-    Xs = np.zeros((nchain, nint, Np, Np), dtype=np.complex64)
-    Xs[..., :N, :N] = X / 2.0**s
+    Xs = (np.empty if Np == N else np.zeros)((nchain, nint, Np, Np), dtype=np.complex64)
+    for b, g in enumerate(gens):
+        for k, (A, _) in enumerate(g):
+            Xs[b, k, :N, :N] = (dts[k] / 2.0**s) * A
     dev = _device()
     lib = _native.lib()
     x = torch.from_numpy(Xs.view(np.float32)).to(dev)
@@ -144,10 +151,10 @@ def expm_chain(X: np.ndarray, Y0: np.ndarray | None = None) -> np.ndarray:
                 'dqh_cgemm_batched',
             )
             torch.cuda.synchronize()
-            blocks.append(Y.cpu().numpy().view(np.complex64).reshape(nchain, nint, Np, Np)[..., :N, : c1 - c0])
+            blocks.append(to_host(Y).view(np.complex64).reshape(nchain, nint, Np, Np)[..., :N, : c1 - c0])
         return np.concatenate(blocks, axis=-1)
     torch.cuda.synchronize()
-    out = U.cpu().numpy().view(np.complex64).reshape(nchain, nint, Np, Np)
+    out = to_host(U).view(np.complex64).reshape(nchain, nint, Np, Np)
     return out[..., :N, :N]
 
 
@@ -171,16 +178,18 @@ def _expm_result(ops_at, build, chains, N, dims, out_shape, tsave, t0, disc, met
     if nint > 0:
         check_expm_size(len(chains), nint, N)
         dts = np.diff(times)
-        X = np.empty((len(chains), nint, N, N), dtype=np.complex128)
-        for b, c in enumerate(chains):
+        gens = []
+        for c in chains:
             cache = {}  # one generator per distinct set of operators (a constant one: once)
+            gens.append([])
             for k in range(nint):
                 ops = ops_at(c, times[k])
                 key = b''.join(o.tobytes() for o in ops)
                 if key not in cache:
-                    cache[key] = build(ops)
-                X[b, k] = dts[k] * cache[key]
-        Uc = expm_chain(X)
+                    A = build(ops)
+                    cache[key] = (A, _norm1(A))
+                gens[-1].append(cache[key])
+        Uc = expm_chain(gens, dts)
     eye = np.eye(N, dtype=np.complex64)
     for i, nb in enumerate(nbefore):
         U[:, i] = eye if nb == 0 else Uc[:, nb - 1]
@@ -501,16 +510,18 @@ def expm_solve(H, Ls, y0: QArray, tsave, Es, method, gradient, options, me: bool
     if nint > 0:
         check_expm_size(len(chain_keys), nint, N)
         dts = np.diff(times)
-        X = np.empty((len(chain_keys), nint, N, N), dtype=np.complex128)
-        for ci, key in enumerate(chain_keys):
+        gens = []
+        for key in chain_keys:
             cache = {}
+            gens.append([])
             for k in range(nint):
                 ops = (_op_at(Ht, key[0], times[k]), *[_op_at(Lt, p, times[k]) for Lt, p in zip(Lts, key[1:])])
                 kb = b''.join(o.tobytes() for o in ops)
                 if kb not in cache:
-                    cache[kb] = slindbladian(ops[0], ops[1:]) if me else -1j * ops[0]
-                X[ci, k] = dts[k] * cache[kb]
-        Y = expm_chain(X, Y0)
+                    A = slindbladian(ops[0], ops[1:]) if me else -1j * ops[0]
+                    cache[kb] = (A, _norm1(A))
+                gens[-1].append(cache[kb])
+        Y = expm_chain(gens, dts, Y0)
     for ci, mem in enumerate(members):
         for j, (b, _) in enumerate(mem):
             for i, nb in enumerate(nbefore):

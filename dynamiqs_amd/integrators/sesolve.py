@@ -22,7 +22,7 @@ from ..options import Options, check_options
 from ..qarrays import QArray, asqarray
 from ..result import AdaptiveStepInfos, FixedStepInfos, SESolveResult
 from ..time_qarray import TimeQArray, astimeqarray
-from .dense import _Arena, _device, _pad, check_descriptors, pad16, rouchon_step_times
+from .dense import _Arena, _device, _pad, check_descriptors, pad16, rouchon_step_times, to_host
 from .mesolve import assert_method_supported, max_steps_error, save_extra_outputs
 from .operators import decompose, resample_pwc, resolve_callables, spline_table, union_breakpoints
 
@@ -83,7 +83,7 @@ class SEPlan:
 
         torch.cuda.synchronize()
         n, ns = self.n, (self.ntsave if self.save_states else 1)
-        c64 = lambda t: t.cpu().numpy().view(np.complex64)  # noqa: E731
+        c64 = lambda t: to_host(t).view(np.complex64)  # noqa: E731
         out = {
             'states': c64(self.states).reshape(self.ninst, ns, n),
             'final_state': c64(self.final).reshape(self.ninst, n),
