@@ -109,6 +109,7 @@ SYMBOLS = {
     'dqh_expm_propagators_noalloc': (ctypes.c_int, [_P, _P, _I64, _I64, _I64, _I64, _I64, _P]),
     'dqh_cgemm_batched': (ctypes.c_int, [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _I64, _P]),
     'dqh_adjoint_pwc_quadrature': (ctypes.c_int, [_I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _P]),
+    'dqh_adjoint_lambda_nodes': (ctypes.c_int, [_I64, _I64, _I64, _I64, _P, _P, _P, _P, _P]),
     'dqh_adjoint_pwc_quadrature_dia': (ctypes.c_int, [_I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _P]),
     'dqh_adjoint_rate_quadrature': (ctypes.c_int, [_I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P]),
     'dqh_host_device_pointer': (ctypes.c_int, [_P, ctypes.POINTER(_P)]),

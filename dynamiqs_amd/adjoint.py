@@ -429,14 +429,18 @@ class AdjointPlan:
         ex = fwd.expects.view(B, K, fwd.ntsave, 2).to(torch.float64).cpu().numpy()
         J = sum(ex[:, k, int(self.loss_pos[k]), 0] for k in range(K))
         rho_nodes_dev = rec.states  # (B * nck, Qc n n 2) float32 == (B, Q, n, n) complex64
-        bst = bwd.states.view(B, K, 2 + Q, n * n * 2)
-        lam_k = torch.flip(bst[:, :, 1 : 1 + Q], dims=[2])  # (B, K, Q, .) in t order
-        lam_dev = (lam_k * self.mask_t[None, :, :, None]).sum(dim=1).contiguous()
-        lambda0 = bst[:, :, 1 + Q].sum(dim=1).cpu().numpy().view(np.complex64).reshape(B, n, n)
+        lam_dev = torch.empty((B, Q, n * n * 2), dtype=torch.float32, device=self.dev)
+        lam0 = torch.empty((B, n * n * 2), dtype=torch.float32, device=self.dev)
 
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         lib = _native.lib()
         P = ctypes.c_void_p
+        _native.check(
+            lib.dqh_adjoint_lambda_nodes(B, K, Q, n, P(bwd.states.data_ptr()), P(self.mask_t.data_ptr()),
+                                         P(lam_dev.data_ptr()), P(lam0.data_ptr()), stream),
+            'dqh_adjoint_lambda_nodes',
+        )
+        lambda0 = lam0.cpu().numpy().view(np.complex64).reshape(B, n, n)
         t5 = time.perf_counter()
         grad = np.zeros((B, nterms, nseg))
         if nterms:

@@ -101,69 +101,96 @@ __global__ __launch_bounds__(kThreads) void k_quad(int n, int nnodes, int nterms
 // diags[u][a + p]): with the integrand Im(Tr(lam O rho) - Tr(lam rho O)),
 //   Tr(lam O rho) = sum_u sum_{a,c} lam[c][a] O[a][a+p] rho[a+p][c],
 //   Tr(lam rho O) = sum_u sum_{a,b} lam[b+p][a] rho[a][b] O[b][b+p],
-// 2 d n^2 complex products per node instead of 2 n^3 (d diagonals). lam is
-// staged in LDS (n <= 64), rho is read from global memory along its rows.
+// 2 d n^2 complex products per node instead of 2 n^3 (d diagonals). lam and the diagonals
+// are in LDS (n <= 64), rho is read along its rows into registers, at most M elements per
+// thread. Bound by reading rho and lam once, and by latency: every node is one round trip to
+// memory and one barrier (64 x 200 nodes of n = 32: 319 -> 126 us against one
+// dependent load per diagonal and element).
+template <int M>
 __global__ __launch_bounds__(kThreads) void k_quad_dia(int n, int nnodes, int nseg, dqh_dia_ops ops,
                                                        const float2 *__restrict__ rho, const float2 *__restrict__ lam,
                                                        const double *__restrict__ weights,
                                                        const int *__restrict__ seg_first, double *__restrict__ grad) {
-  __shared__ float2 sL[kMaxLds * (kMaxLds + 1)];
+  extern __shared__ float2 smem[];
   __shared__ double red[kThreads / 64];
   const int seg = blockIdx.x;
   const size_t inst = blockIdx.y;
-  const size_t nn = (size_t)n * n;
-  const int ld = kMaxLds + 1;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nn = n * n, ld = n + 1, tid = (int)threadIdx.x;
+  float2 *sL = smem, *sD = smem + n * ld;  // lam [n][ld]; the diagonals of every operator [n]
+  const int lane = tid & 63, wave = tid >> 6;
   const int nterms = ops.nops;
+  for (int j = 0, row = 0; j < nterms; row += ops.noff[j], ++j) {
+    const float2 *D = reinterpret_cast<const float2 *>(ops.diags[j]);
+    for (int e = tid; e < ops.noff[j] * n; e += kThreads) sD[row * n + e] = D[e];
+  }
+  // row and column of this thread's elements
+  int ra[M], rc[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const int e = tid + kThreads * m;
+    ra[m] = e / n;
+    rc[m] = e - ra[m] * n;
+  }
   double acc[DQH_DIA_MAXOPS];
+#pragma unroll
   for (int j = 0; j < DQH_DIA_MAXOPS; ++j) acc[j] = 0.0;
   for (int q = seg_first[seg]; q < seg_first[seg + 1]; ++q) {
     const float2 *R = rho + (inst * nnodes + q) * nn;
     const float2 *Lm = lam + (inst * nnodes + q) * nn;
+    float2 r[M], l0[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const int e = tid + kThreads * m;
+      r[m] = e < nn ? R[e] : make_float2(0.f, 0.f);  // rho[a][c]
+      l0[m] = e < nn ? Lm[e] : make_float2(0.f, 0.f);
+    }
     __syncthreads();
-    for (size_t e = threadIdx.x; e < nn; e += kThreads) sL[(e / n) * ld + e % n] = Lm[e];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+      if (tid + kThreads * m < nn) sL[ra[m] * ld + rc[m]] = l0[m];
     __syncthreads();
     const double wq = weights[q];
-    for (int j = 0; j < nterms; ++j) {
-      const float2 *D = reinterpret_cast<const float2 *>(ops.diags[j]);
-      double im = 0.0;
-      for (size_t e = threadIdx.x; e < nn; e += kThreads) {
-        const int a = (int)(e / n), c = (int)(e % n);  // rho[a][c] is contiguous in e
-        const float2 r = R[e];
-        float sr = 0.f, si = 0.f;
-        for (int u = 0; u < ops.noff[j]; ++u) {
-          const int p = ops.off[j][u];
-          // Tr(lam O rho): rho[a][c] pairs with lam[c][a - p] O[a - p][a]
-          const int a2 = a - p;
-          if (a2 >= 0 && a2 < n) {
-            const float2 o = D[(size_t)u * n + a];
-            const float2 l = sL[c * ld + a2];
-            const float lr = l.x * o.x - l.y * o.y, li = l.x * o.y + l.y * o.x;
-            sr += lr * r.x - li * r.y;
-            si += lr * r.y + li * r.x;
-          }
-          // Tr(lam rho O): rho[a][c] pairs with lam[c + p][a] O[c][c + p]
-          const int c2 = c + p;
-          if (c2 >= 0 && c2 < n) {
-            const float2 o = D[(size_t)u * n + c2];
-            const float2 l = sL[c2 * ld + a];
-            const float lr = l.x * o.x - l.y * o.y, li = l.x * o.y + l.y * o.x;
-            sr -= lr * r.x - li * r.y;
-            si -= lr * r.y + li * r.x;
-          }
+    int row = 0;
+#pragma unroll
+    for (int j = 0; j < DQH_DIA_MAXOPS; ++j) {
+      if (j >= nterms) break;
+      float si[M];
+#pragma unroll
+      for (int m = 0; m < M; ++m) si[m] = 0.f;
+      for (int u = 0; u < ops.noff[j]; ++u, ++row) {
+        const int p = ops.off[j][u];
+        const float2 *D = sD + row * n;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          if (kThreads * m >= nn) break;
+          const int a = ra[m], c = rc[m];
+          // Tr(lam O rho): rho[a][c] pairs with lam[c][a - p] O[a - p][a]; Tr(lam rho O):
+          // with lam[c + p][a] O[c][c + p]. Elements past the matrix and neighbours outside
+          // it read element 0 and drop out.
+          const bool in = a < n, in1 = in && (unsigned)(a - p) < (unsigned)n, in2 = in && (unsigned)(c + p) < (unsigned)n;
+          const float2 o1 = D[in1 ? a : 0], l1 = sL[in1 ? c * ld + a - p : 0];
+          const float2 o2 = D[in2 ? c + p : 0], l2 = sL[in2 ? (c + p) * ld + a : 0];
+          const float x1 = l1.x * o1.x - l1.y * o1.y, y1 = l1.x * o1.y + l1.y * o1.x;
+          const float x2 = l2.x * o2.x - l2.y * o2.y, y2 = l2.x * o2.y + l2.y * o2.x;
+          if (in1) si[m] += x1 * r[m].y + y1 * r[m].x;
+          if (in2) si[m] -= x2 * r[m].y + y2 * r[m].x;
         }
-        im += (double)si;
       }
+      double im = 0.0;
+#pragma unroll
+      for (int m = 0; m < M; ++m) im += (double)si[m];
       acc[j] += wq * im;
     }
   }
-  for (int j = 0; j < nterms; ++j) {
+#pragma unroll
+  for (int j = 0; j < DQH_DIA_MAXOPS; ++j) {
+    if (j >= nterms) break;
     double v = acc[j];
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     __syncthreads();
     if (lane == 0) red[wave] = v;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
       double s = 0;
       for (int w = 0; w < kThreads / 64; ++w) s += red[w];
       grad[(inst * nterms + j) * nseg + seg] = s;
@@ -247,6 +274,38 @@ __global__ __launch_bounds__(kThreads) void k_rate_quad(int n, int nnodes, int n
   }
 }
 
+// The adjoint states at the quadrature nodes from the backward solves: lam[b][q] =
+// sum_k mask[k][q] bst[b][k][Q - q], and lambda0[b] = sum_k bst[b][k][Q + 1] (the backward
+// solve k saves its start, the nodes in reversed order and its end). One pass over the
+// saved states, bound by reading them and writing lam (64 x 200 nodes of n = 32: 0.36 ms as
+// a flip, a product and sums before; below 0.1 ms here). grid
+// ((Q + 1) ceil(nn / 1024), B)
+__global__ __launch_bounds__(kThreads) void k_lambda_nodes(int K, int Q, int64_t nn, const float2 *__restrict__ bst,
+                                                           const float *__restrict__ mask, float2 *__restrict__ lam,
+                                                           float2 *__restrict__ lambda0) {
+  const unsigned chunks = (unsigned)((nn + 4 * kThreads - 1) / (4 * kThreads));
+  const int q = (int)(blockIdx.x / chunks);
+  const int64_t e0 = (int64_t)(blockIdx.x - q * chunks) * 4 * kThreads + threadIdx.x;
+  const size_t b = blockIdx.y;
+  float2 s[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) s[m] = make_float2(0.f, 0.f);
+  for (int k = 0; k < K; ++k) {
+    const float2 *x = bst + ((b * K + k) * (Q + 2) + (q < Q ? Q - q : Q + 1)) * nn;
+    const float w = q < Q ? mask[(size_t)k * Q + q] : 1.f;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const float2 v = x[min(e0 + m * kThreads, nn - 1)];
+      s[m].x += w * v.x;
+      s[m].y += w * v.y;
+    }
+  }
+  float2 *o = q < Q ? lam + (b * Q + q) * nn : lambda0 + b * nn;
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+    if (e0 + m * kThreads < nn) o[e0 + m * kThreads] = s[m];
+}
+
 }  // namespace adj
 }  // namespace dqh
 
@@ -264,6 +323,23 @@ extern "C" int dqh_adjoint_pwc_quadrature(int64_t ninst, int64_t n, int64_t nnod
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess)
     return dqh::fail(DQH_HIP_ERROR, std::string("dqh_adjoint_pwc_quadrature: ") + hipGetErrorString(err));
+  return DQH_OK;
+}
+
+extern "C" int dqh_adjoint_lambda_nodes(int64_t ninst, int64_t nloss, int64_t nnodes, int64_t n, const void *bstates,
+                                        const float *mask, void *lam, void *lambda0, void *stream) {
+  if (ninst <= 0 || ninst > 65535 || nloss <= 0 || nnodes <= 0 || n <= 0 || n > 1024 ||
+      (nnodes + 1) * ((n * n + 4 * dqh::adj::kThreads - 1) / (4 * dqh::adj::kThreads)) > 0x7fffffff || !bstates || !mask || !lam || !lambda0)
+    return dqh::fail(DQH_BAD_ARG, "dqh_adjoint_lambda_nodes: bad arguments");
+  const int64_t nn = n * n;
+  hipLaunchKernelGGL(dqh::adj::k_lambda_nodes,
+                     dim3((unsigned)((nnodes + 1) * ((nn + 4 * dqh::adj::kThreads - 1) / (4 * dqh::adj::kThreads))), (unsigned)ninst),
+                     dim3(dqh::adj::kThreads), 0, (hipStream_t)stream, (int)nloss, (int)nnodes, nn,
+                     reinterpret_cast<const float2 *>(bstates), mask, reinterpret_cast<float2 *>(lam),
+                     reinterpret_cast<float2 *>(lambda0));
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess)
+    return dqh::fail(DQH_HIP_ERROR, std::string("dqh_adjoint_lambda_nodes: ") + hipGetErrorString(err));
   return DQH_OK;
 }
 
@@ -301,11 +377,23 @@ extern "C" int dqh_adjoint_pwc_quadrature_dia(int64_t ninst, int64_t n, int64_t 
       if (ops->off[k][u] <= -n || ops->off[k][u] >= n)
         return dqh::fail(DQH_BAD_ARG, "dqh_adjoint_pwc_quadrature_dia: offset outside (-n, n)");
   }
-  hipLaunchKernelGGL(dqh::adj::k_quad_dia, dim3((unsigned)nseg, (unsigned)ninst), dim3(dqh::adj::kThreads), 0,
-                     (hipStream_t)stream, (int)n, (int)nnodes, (int)nseg, *ops,
-                     reinterpret_cast<const float2 *>(rho_nodes), reinterpret_cast<const float2 *>(lam_nodes), weights,
-                     reinterpret_cast<const int *>(seg_first), grad);
-  const hipError_t err = hipGetLastError();
+  int rows = 0;
+  for (int k = 0; k < ops->nops; ++k) rows += ops->noff[k];
+  const size_t lds = (size_t)(n * (n + 1) + rows * n) * sizeof(float2);
+  hipError_t err = hipSuccess;
+  auto launch = [&](auto kernel) {
+    if (lds > 65536)
+      err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (err != hipSuccess) return;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nseg, (unsigned)ninst), dim3(dqh::adj::kThreads), lds, (hipStream_t)stream,
+                       (int)n, (int)nnodes, (int)nseg, *ops, reinterpret_cast<const float2 *>(rho_nodes),
+                       reinterpret_cast<const float2 *>(lam_nodes), weights, reinterpret_cast<const int *>(seg_first), grad);
+  };
+  if (n <= 32)
+    launch(dqh::adj::k_quad_dia<4>);
+  else
+    launch(dqh::adj::k_quad_dia<16>);
+  if (err == hipSuccess) err = hipGetLastError();
   if (err != hipSuccess)
     return dqh::fail(DQH_HIP_ERROR, std::string("dqh_adjoint_pwc_quadrature_dia: ") + hipGetErrorString(err));
   return DQH_OK;
