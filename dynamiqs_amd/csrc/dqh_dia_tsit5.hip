@@ -8,21 +8,23 @@
 //     strips of 4 NE rows). Stencil reads may cross the diagonal by at most `spread`
 //     elements; the writers keep that band below the diagonal up to date. A rho0 that is
 //     not Hermitian (checked on the device) takes the same kernels over the full matrix;
-//   * stages 1..5 evaluate the field on the increment Delta_s = h sum_j a_sj k_j alone
-//     (constant generators): g_s = f(Delta_s) = k_s - k_0, so neither the FP64 state nor
-//     a rounded copy of it is read; stage 1 is h a_10 f(k_0), without an input of its own;
+//   * stage 1 forms its input y + h a_10 k_0 where the stencil reads it, so that no pass
+//     over the matrix has to follow the choice of h;
 //   * stage 5 writes the candidate y1 in FP64 (a second state buffer) and stage 6 reads
 //     its stencil input from it, so accepting a step moves nothing: the buffers swap roles;
 //   * accept / reject, saves and the next dt are formed at the start of the next step's
 //     stage 1, by every workgroup from the same partial sums in the same order (identical
 //     decisions everywhere, no atomics).
-// Bytes per element and step: 24 + 40 + 48 + 56 + 88 + 88 = 344, of half the elements,
-// against 496 of all of them with the full-matrix form on rounded states.
+// Bytes per element and step: 40 + 56 + 64 + 72 + 88 + 88 = 408, of half the elements,
+// against 496 of all of them with full-matrix sweeps and a commit pass. The stages are
+// evaluated on the rounded states y + Delta_s as before: on the increments alone (344 bytes,
+// 6.7 ms below) the error estimate loses the FP32 noise that holds the steps down in the
+// full-matrix form, and the solutions moved by up to 8e-3 of the largest elements' scale.
 // Measured (rtol 1e-6, atol 1e-8, two coupled modes with 8 shifts): four solves of n = 1024,
 // 36 steps, 22.6 -> 6.9 ms, stages at 3.8 to 5.3 TB/s (a copy reaches 4.7); one of
 // n = 323, 29 steps, 2.8 -> 1.24 ms, bound by the latency of a launch (about 5 us).
-// Time-dependent Hamiltonians take full stage inputs y + Delta_s instead (the generator
-// changes between the stages), and a separate controller launch before the first stage.
+// Time-dependent Hamiltonians take a separate controller launch before the first stage,
+// because their diagonals are rebuilt in between.
 //
 // Control blocks are double-buffered by step parity (a step reads the other block and
 // writes block `cur`), so a fixed sequence of launches is valid for any step and is
@@ -335,7 +337,6 @@ __device__ __forceinline__ Ctrl commit(const V &v, int cur, size_t inst, int id,
 #pragma unroll
         for (int q = 0; q < 7; ++q)
           w[q] = th * (rk.R[q][0] + th * (rk.R[q][1] + th * (rk.R[q][2] + th * rk.R[q][3])));
-        if (!TD) fold_k0(w);
         double2 s = yv;
 #pragma unroll
         for (int q = 0; q < 7; ++q) s = add(s, h * w[q], kk[q]);
@@ -352,8 +353,8 @@ __device__ __forceinline__ Ctrl commit(const V &v, int cur, size_t inst, int id,
   return o;
 }
 
-// Stage S. Constant generators (TD = false): slots 1..5 hold the increments g_S.
-// S = 0 (TD only): k_0 = f(y) after a step that ended on a breakpoint.
+// Stage S: k_S and the input of stage S + 1, or the error partials (S = 6). S = 0 (TD only):
+// k_0 = f(y) after a step that ended on a breakpoint.
 template <int S, int NE, bool TD>
 __global__ __launch_bounds__(256) void k_stage(V v, int cur) {
   const RKTab &rk = rk_tab(v.flags);
@@ -386,7 +387,7 @@ __global__ __launch_bounds__(256) void k_stage(V v, int cur) {
         const size_t e = (size_t)min(i0 + m, (int)v.n_true - 1) * v.n + jc;
 #pragma unroll
         for (int q = 0; q < NK; ++q) kq[q][m] = kslot(v, q, c.rot, inst)[e];
-        if (S >= 5 || (TD && S >= 1)) yv[m] = ybuf(v, c.rot, 0, inst)[e];
+        if (S >= 1) yv[m] = ybuf(v, c.rot, 0, inst)[e];
         if (S == 6) y1[m] = ybuf(v, c.rot, 1, inst)[e];
       }
     };
@@ -396,10 +397,8 @@ __global__ __launch_bounds__(256) void k_stage(V v, int cur) {
       stencil<NE, TD>(v, inst, InY{ybuf(v, c.rot, 0, inst)}, i0, jc, f);
     else if constexpr (S == 6)
       stencil<NE, TD>(v, inst, InY{ybuf(v, c.rot, 1, inst)}, i0, jc, f);
-    else if constexpr (S == 1 && TD)
-      stencil<NE, TD>(v, inst, InYK{ybuf(v, c.rot, 0, inst), kslot(v, 0, c.rot, inst), h * rk.A[1][0]}, i0, jc, f);
     else if constexpr (S == 1)
-      stencil<NE, TD>(v, inst, InF{kslot(v, 0, c.rot, inst)}, i0, jc, f);
+      stencil<NE, TD>(v, inst, InYK{ybuf(v, c.rot, 0, inst), kslot(v, 0, c.rot, inst), h * rk.A[1][0]}, i0, jc, f);
     else
       stencil<NE, TD>(v, inst, InF{ysbuf(v, S & 1, inst)}, i0, jc, f);
     if (kAfter) {
@@ -412,41 +411,25 @@ __global__ __launch_bounds__(256) void k_stage(V v, int cur) {
       const int i = i0 + m;
       if (!owned(v, i, j)) continue;
       const size_t e = (size_t)i * v.n + j;
-      if constexpr (S == 1 && !TD) {  // f is linear: f(h a_10 k_0) = h a_10 f(k_0)
-        const double s = h * rk.A[1][0];
-        f[m] = make_float2((float)(s * (double)f[m].x), (float)(s * (double)f[m].y));
-      }
       float2 *ks = kslot(v, S, c.rot, inst);
       if constexpr (S == 0 || S == 6)
         put(v, ks, i, j, f[m]);
       else
         ks[e] = f[m];
       if constexpr (S >= 1 && S <= 5) {
-        // increments: the weight of k_0 is the row sum C
-        double2 d = add(make_double2(0.0, 0.0), TD ? rk.A[S + 1][0] : rk.C[S + 1], kq[0][m]);
+        double2 d = yv[m];
 #pragma unroll
-        for (int q = 1; q < S; ++q) d = add(d, rk.A[S + 1][q], kq[q][m]);
-        d = add(d, rk.A[S + 1][S], f[m]);
-        d.x *= h;
-        d.y *= h;
-        if (TD || S == 5) {
-          d.x += yv[m].x;
-          d.y += yv[m].y;
-        }
+        for (int q = 0; q < S; ++q) d = add(d, h * rk.A[S + 1][q], kq[q][m]);
+        d = add(d, h * rk.A[S + 1][S], f[m]);
         if constexpr (S == 5)
           put(v, ybuf(v, c.rot, 1, inst), i, j, d);
         else
           put(v, ysbuf(v, (S + 1) & 1, inst), i, j, f32(d));
       }
       if constexpr (S == 6) {
-        double e0 = rk.E[0];
-        if (!TD) {
+        double2 er = make_double2(0.0, 0.0);
 #pragma unroll
-          for (int q = 1; q < 6; ++q) e0 += rk.E[q];
-        }
-        double2 er = add(make_double2(0.0, 0.0), e0, kq[0][m]);
-#pragma unroll
-        for (int q = 1; q < 6; ++q) er = add(er, rk.E[q], kq[q][m]);
+        for (int q = 0; q < 6; ++q) er = add(er, rk.E[q], kq[q][m]);
         er = add(er, rk.E[6], f[m]);
         er.x *= h;
         er.y *= h;
@@ -544,8 +527,8 @@ __global__ __launch_bounds__(256) void k_init(V v) {
 }
 
 // pass 0: k_0 = f(y0), partials |y0|^2 / sc^2 and |k_0|^2 / sc^2;
-// pass 1: partials |f(y0 + h0 k_0) - k_0|^2 / sc^2 (sc = atol + rtol |y0|), for constant
-// generators from f(y0 + h0 k_0) - k_0 = h0 f(k_0); h0 is in control block 1.
+// pass 1: partials |f(y0 + h0 k_0) - k_0|^2 / sc^2 (sc = atol + rtol |y0|), h0 in control
+// block 1.
 // Hairer-Norsett-Wanner II.4 starting step as the dense kernel computes it.
 template <int NE, bool TD>
 __global__ __launch_bounds__(256) void k_init_rhs(V v, int pass) {
@@ -563,10 +546,8 @@ __global__ __launch_bounds__(256) void k_init_rhs(V v, int pass) {
     float2 f[NE];
     if (pass == 0)
       stencil<NE, TD>(v, inst, InY{y}, i0, jc, f);
-    else if (TD)
-      stencil<NE, TD>(v, inst, InYK{y, k0, h0}, i0, jc, f);
     else
-      stencil<NE, TD>(v, inst, InF{k0}, i0, jc, f);
+      stencil<NE, TD>(v, inst, InYK{y, k0, h0}, i0, jc, f);
 #pragma unroll
     for (int m = 0; m < NE; ++m) {
       const int i = i0 + m;
@@ -579,12 +560,8 @@ __global__ __launch_bounds__(256) void k_init_rhs(V v, int pass) {
         a0 += w * sq(yv) / (sc * sc);
         a1 += w * sq(make_double2(f[m].x, f[m].y)) / (sc * sc);
       } else {
-        double2 d = make_double2(h0 * (double)f[m].x, h0 * (double)f[m].y);
-        if (TD) {
-          const float2 kq = k0[e];
-          d = make_double2((double)f[m].x - kq.x, (double)f[m].y - kq.y);
-        }
-        a0 += w * sq(d) / (sc * sc);
+        const float2 kq = k0[e];
+        a0 += w * sq(make_double2((double)f[m].x - kq.x, (double)f[m].y - kq.y)) / (sc * sc);
       }
     }
   }

@@ -406,9 +406,8 @@ __global__ __launch_bounds__(T) void k_sesolve(const dqh_me_inst *__restrict__ i
 // Constant Hamiltonians up to n = 128: four lanes per row, each with a quarter of the row's
 // columns of G = -i H in registers, and the state and stages of the row in registers too
 // (alike in its four lanes). The stage input goes through LDS (two copies alternate, one
-// barrier per stage), the four partial sums are added within the quad. Stages 1..5 evaluate
-// the field on the increment alone (fold_k0). Up to n = 64 the first expectation operator is in
-// registers as well. Bound by the latency of a stage. A call,
+// barrier per stage), the four partial sums are added within the quad. Up to n = 64 the first
+// expectation operator is in registers as well. Bound by the latency of a stage. A call,
 // against reading G from the caches at every stage: 48 solves of n = 64 (50 saves, Dopri5)
 // 2.44 -> 1.01 ms, 3000 two-level solves 2.00 -> 1.88 ms (the host's share), up to 7 times
 // less at 64 < n <= 128.
@@ -559,26 +558,22 @@ __global__ __launch_bounds__(4 * NR) void k_sesolve_const(const dqh_me_inst *__r
 #pragma unroll
     for (int s = 1; s < 7; ++s) {
       CTab *w = weights<TAB>();
-      const double a0 = w->C[s];  // row sum of A: the weight of k_0 with the increments folded in
-      double re = a0 * (double)k[0].x, im = a0 * (double)k[0].y;
+      double re = 0.0, im = 0.0;
 #pragma unroll
-      for (int j = 1; j < s; ++j) {
+      for (int j = 0; j < s; ++j) {
         if (rk.A[s][j] != 0.0) {  // compile-time
           re += w->A[s][j] * (double)k[j].x;
           im += w->A[s][j] * (double)k[j].y;
         }
       }
-      y1 = s < 6 ? make_double2(h * re, h * im) : make_double2(y.x + h * re, y.y + h * im);
+      y1 = make_double2(y.x + h * re, y.y + h * im);
       k[s] = field(y1);
     }
     nrhs += 6;
     CTab *we = weights<TAB>();
-    double e0 = 0.0;
+    double er = 0.0, em = 0.0;
 #pragma unroll
-    for (int j = 0; j < 6; ++j) e0 += we->E[j];
-    double er = e0 * (double)k[0].x, em = e0 * (double)k[0].y;
-#pragma unroll
-    for (int j = 1; j < 7; ++j) {
+    for (int j = 0; j < 7; ++j) {
       if (rk.E[j] != 0.0) {
         er += we->E[j] * (double)k[j].x;
         em += we->E[j] * (double)k[j].y;
@@ -604,7 +599,6 @@ __global__ __launch_bounds__(4 * NR) void k_sesolve_const(const dqh_me_inst *__r
 #pragma unroll
         for (int j = 0; j < 7; ++j)
           w[j] = th * (wr->R[j][0] + th * (wr->R[j][1] + th * (wr->R[j][2] + th * wr->R[j][3])));
-        fold_k0(w);
         save(h, w, isave);
         advance();
       }
