@@ -9,18 +9,22 @@
 // products, so the matrix cores have nothing to do here and a step is bound by the
 // latency of its dependent stages (n <= 32) and by FP64 issue and LDS reads (n = 64).
 //
-// k_tsit5_diag, n <= 64 and at most 12 shifts: a thread owns NE elements of the upper triangle (u = thread + NTH q, row by row, of
-// the n (n + 1) / 2 that exist: no work on padding). Its coefficients C_t, the FP64
-// diagonal generator g = d_i + conj(d_j), the FP64 state, the candidate and the seven
-// FP32 stages stay in registers for the whole solve. The stage input goes to LDS in
-// FP32 (both triangles), the neighbours come back with one 8-byte read per shift, and
-// the FP64 diagonal term takes the thread's own input unrounded. Two LDS copies
-// alternate, so a stage costs one barrier, and the stages are unrolled with the
-// tableau's weights in scalar registers. Measured against the resident dense body:
-// oscillator n = 16, 85 steps and 101 saves 1.20 -> 0.297 ms; 128 driven Kerr oscillators
-// n = 64 (2 jump operators, about 440 steps) 57.4 -> 7.28 ms; the three solves of a
-// gradient at n = 32, 64 control vectors, 6.4 -> 1.7 ms. The controller, step clipping, FSAL, saving and the
-// precision of the operators and stages are those of the dense kernels.
+// k_tsit5_diag, n <= 64 and at most 12 shifts: a thread owns NE elements of the upper
+// triangle (u = thread + NTH q, row by row, of the n (n + 1) / 2 that exist: no work on
+// padding). Its coefficients C_t, the FP64 diagonal generator g = d_i + conj(d_j), the FP64
+// state, the candidate and the seven FP32 stages stay in registers for the whole solve. The
+// stage input goes to LDS in FP32 (both triangles), the neighbours come back with one
+// 8-byte read per shift, and the FP64 diagonal term takes the thread's own input unrounded.
+// Two LDS copies alternate, so a stage costs one barrier, and the stages are unrolled with
+// the tableau's weights in scalar registers. With several elements per thread the saves
+// form one element at a time, slots are recomputed and uniform doubles are scalar: without
+// that the three elements of n = 64 spilled 340 registers in every step.
+// Measured against the resident dense body: oscillator n = 16, 85 steps and 101 saves 1.20
+// -> 0.31 ms; 128 driven Kerr oscillators n = 64 (2 jump operators, about 440 steps) 57.4 ->
+// 4.5 ms (7.3 with the spills); the solves of a gradient at n = 32, 64 control vectors, 6.4
+// -> 1.3 ms (500 saves of the backward solve: 1.19 -> 1.00 ms with the weights of all saves
+// of a step formed at once, one per lane). The controller, step clipping, FSAL, saving and
+// the precision of the operators and stages are those of the dense kernels.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -76,6 +80,16 @@ __host__ __device__ inline size_t lds_bytes(int n, int nH, int nLrow, int guard)
          (size_t)n * sizeof(double2) + (size_t)(4 * (NTH / 64)) * sizeof(double);
 }
 
+// a double that is the same in all lanes, in scalar registers where several elements per
+// thread need the vector ones (ON); a single element is bound by latency instead
+template <bool ON>
+__device__ __forceinline__ double uniform(double x) {
+  if constexpr (!ON) return x;
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
 template <int NTH, int NE, int T, int TAB>
 __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restrict__ insts, Pattern pat) {
   extern __shared__ __align__(16) char smem[];
@@ -101,33 +115,34 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
   const double *tsave = gp<const double>(p.tsave);
   const double *ptimes = gp<const double>(p.pwc_times);
   const double rtol = p.rtol, atol = p.atol, t_end = p.t1;
-  const double inv_nn = 1.0 / ((double)n * n);
+  const double inv_nn = uniform<(NE > 1)>(1.0 / ((double)n * n));
   const bool save_states = (p.flags & DQH_FLAG_SAVE_STATES) != 0;
 
-  // owned elements; at / am: slots of the element and of its mirror image in a copy (the
-  // spare slot past the end)
+  // owned elements, packed i | j << 8 (i <= j; -1 past the end): their slots in a copy are
+  // formed where they are used, or the registers would not hold the stages
   const int NU = n * (n + 1) / 2;
-  int ei[NE], ej[NE], at[NE], am[NE];
-  double wt[NE];  // weight in a sum over the full matrix
+  int ij[NE];
 #pragma unroll
   for (int q = 0; q < NE; ++q) {
     int rem = tid + NTH * q, i = 0;
-    ei[q] = -1;
-    ej[q] = 0;
-    at[q] = am[q] = n * LD;
-    wt[q] = 0.0;
+    ij[q] = -1;
     if (rem < NU) {
       while (rem >= n - i) {
         rem -= n - i;
         ++i;
       }
-      ei[q] = i;
-      ej[q] = i + rem;
-      at[q] = i * LD + i + rem;
-      am[q] = (i + rem) * LD + i;
-      wt[q] = rem == 0 ? 1.0 : 2.0;
+      ij[q] = i | ((i + rem) << 8);
     }
   }
+  // row and column of element q; past the end 0, 0
+  auto at = [&](int q, int &i, int &j) {
+    int x = ij[q];
+    if constexpr (NE > 1) asm volatile("" : "+v"(x));
+    const int z = x < 0 ? 0 : x;
+    i = z & 255;
+    j = z >> 8;
+    return x >= 0;
+  };
   for (int e = tid; e < 2 * CS + pat.guard; e += NTH) (ysA - pat.guard)[e] = make_float2(0.f, 0.f);
   for (int e = tid; e < pat.nLrow * n; e += NTH) {
     const int r = e / n, i = e - r * n;
@@ -182,8 +197,8 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
     };
 #pragma unroll
     for (int q = 0; q < NE; ++q) {
-      const bool on = ei[q] >= 0;
-      const int i = on ? ei[q] : 0, j = ej[q];
+      int i, j;
+      const bool on = at(q, i, j);
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         float ar = 0.f, ai = 0.f;
@@ -215,8 +230,9 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
     const double2 *y0 = gp<const double2>(p.y);
 #pragma unroll
     for (int q = 0; q < NE; ++q) {
-      y[q] = ei[q] >= 0 ? y0[(size_t)ei[q] * np + ej[q]] : make_double2(0.0, 0.0);
-      if (ei[q] == ej[q]) y[q].y = 0.0;
+      int i, j;
+      y[q] = at(q, i, j) ? y0[(size_t)i * np + j] : make_double2(0.0, 0.0);
+      if (i == j) y[q].y = 0.0;
       y1[q] = make_double2(0.0, 0.0);
 #pragma unroll
       for (int s = 0; s < 7; ++s) k[s][q] = make_float2(0.f, 0.f);
@@ -235,14 +251,17 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
 #pragma unroll
     for (int q = 0; q < NE; ++q) {
       const float2 x = make_float2((float)v[q].x, (float)v[q].y);
-      b[am[q]] = make_float2(x.x, -x.y);
-      b[at[q]] = x;
+      int i, j;
+      const bool on = at(q, i, j);
+      b[on ? j * LD + i : n * LD] = make_float2(x.x, -x.y);
+      b[on ? i * LD + j : n * LD] = x;
     }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < NE; ++q) {
-      int e = at[q];
-      if constexpr (NE > 1) asm volatile("" : "+v"(e));  // the T addresses are formed here, not kept
+      int i, j;
+      const bool on = at(q, i, j);
+      const int e = on ? i * LD + j : n * LD;
       float2 x[T];
 #pragma unroll
       for (int t = 0; t < T; ++t) x[t] = b[e + sh[t]];
@@ -255,7 +274,8 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
       const double re = (double)fr + (gr[q] * v[q].x - gi[q] * v[q].y);
       const double im = (double)fi + (gr[q] * v[q].y + gi[q] * v[q].x);
       // the diagonal of a Hermitian field is real
-      out[q] = make_float2((float)re, ei[q] == ej[q] ? 0.f : (float)im);
+      out[q] = make_float2((float)re, i == j ? 0.f : (float)im);
+      if constexpr (NE > 2) __builtin_amdgcn_sched_barrier(0);  // one element's neighbours in registers at a time
     }
   };
 
@@ -273,23 +293,33 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
 
   int par = 0;
   // y + h sum_j w_j k_j at save index isave: states on both triangles, Tr(E rho) over the
-  // owned elements and their mirror images
+  // owned elements and their mirror images. One element at a time and formed anew for every
+  // operator: kept, the values would not fit beside the stages.
   auto save = [&](double h, const double (&w)[7], int isave) {
     float2 *st = gp<float2>(p.states) + (size_t)isave * n * n;
-    double vr[NE], vi[NE];
-#pragma unroll
-    for (int q = 0; q < NE; ++q) {
+    auto value = [&](int q) {
       double re = 0.0, im = 0.0;
 #pragma unroll
       for (int j = 0; j < 7; ++j) {
-        re += w[j] * (double)k[j][q].x;
-        im += w[j] * (double)k[j][q].y;
+        float2 x = k[j][q];
+        if constexpr (NE > 1) asm volatile("" : "+v"(x.x), "+v"(x.y));
+        re += w[j] * (double)x.x;
+        im += w[j] * (double)x.y;
       }
-      vr[q] = y[q].x + h * re;
-      vi[q] = y[q].y + h * im;
-      if (save_states && ei[q] >= 0) {
-        st[(size_t)ei[q] * n + ej[q]] = make_float2((float)vr[q], (float)vi[q]);
-        if (ei[q] != ej[q]) st[(size_t)ej[q] * n + ei[q]] = make_float2((float)vr[q], (float)-vi[q]);
+      return make_double2(y[q].x + h * re, y[q].y + h * im);
+    };
+    double2 single = make_double2(0.0, 0.0);
+    if constexpr (NE == 1) single = value(0);
+    if (save_states) {
+#pragma unroll
+      for (int q = 0; q < NE; ++q) {
+        const double2 v = NE == 1 ? single : value(q);
+        int i, j;
+        if (at(q, i, j)) {
+          st[(size_t)i * n + j] = make_float2((float)v.x, (float)v.y);
+          if (i != j) st[(size_t)j * n + i] = make_float2((float)v.x, (float)-v.y);
+        }
+        if constexpr (NE > 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
     const float2 *ET = gp<const float2>(p.EopsT);
@@ -298,30 +328,46 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
       double s[2] = {0.0, 0.0};
 #pragma unroll
       for (int q = 0; q < NE; ++q) {
-        if (ei[q] >= 0) {
-          const float2 o = E[(size_t)ei[q] * np + ej[q]];
-          s[0] += o.x * vr[q] - o.y * vi[q];
-          s[1] += o.x * vi[q] + o.y * vr[q];
-          if (ei[q] != ej[q]) {
-            const float2 m = E[(size_t)ej[q] * np + ei[q]];
-            s[0] += m.x * vr[q] + m.y * vi[q];
-            s[1] += m.y * vr[q] - m.x * vi[q];
+        const double2 v = NE == 1 ? single : value(q);
+        int i, j;
+        if (at(q, i, j)) {
+          const float2 o = E[(size_t)i * np + j];
+          s[0] += o.x * v.x - o.y * v.y;
+          s[1] += o.x * v.y + o.y * v.x;
+          if (i != j) {
+            const float2 m = E[(size_t)j * np + i];
+            s[0] += m.x * v.x + m.y * v.y;
+            s[1] += m.y * v.x - m.x * v.y;
           }
         }
+        if constexpr (NE > 1) __builtin_amdgcn_sched_barrier(0);
       }
       block_sums<NTH>(s, red, par);
       if (tid == 0) gp<float2>(p.expects)[(size_t)e * ntsave + isave] = make_float2((float)s[0], (float)s[1]);
     }
+  };
+  // weight of element q in a sum over the full matrix
+  auto weight = [&](int q) {
+    int i, j;
+    return at(q, i, j) ? (i == j ? 1.0 : 2.0) : 0.0;
   };
   const double w0[7] = {0, 0, 0, 0, 0, 0, 0};
 
   double t = p.t0;
   int isave = 0, status = 0;
   int64_t nsteps = 0, nacc = 0, nrej = 0, nrhs = 0;
+  // NE = 1: the save times sbase .. sbase + 63, one per lane, and how many are due by x
+  const int lane = tid & 63;
+  int sbase = 0;
+  double ts = NE == 1 && lane < ntsave ? tsave[lane] : 0.0;
+  auto due = [&](double x) {
+    const int i = sbase + lane;
+    return (int)__popcll(__ballot(i >= isave && i < ntsave && ts <= x));
+  };
   double next_save = ntsave > 0 ? tsave[0] : 0.0;
   auto advance = [&]() {
     ++isave;
-    if (isave < ntsave) next_save = tsave[isave];
+    if (isave < ntsave) next_save = uniform<(NE > 1)>(tsave[isave]);
   };
   // segment of t (searchsorted right, -1 before the first breakpoint) and the breakpoint
   // after it; t only grows, so both move forward
@@ -343,6 +389,10 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
     save(0.0, w0, isave);
     advance();
   }
+  if (NE == 1 && isave >= 64) {
+    sbase = isave;
+    ts = sbase + lane < ntsave ? tsave[sbase + lane] : 0.0;
+  }
   field(y, k[0]);
   ++nrhs;
 
@@ -354,8 +404,8 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
     for (int q = 0; q < NE; ++q) {
       const double ay2 = y[q].x * y[q].x + y[q].y * y[q].y;
       const double sc = atol + rtol * sqrt(ay2);
-      s[0] += wt[q] * ay2 / (sc * sc);
-      s[1] += wt[q] * ((double)k[0][q].x * k[0][q].x + (double)k[0][q].y * k[0][q].y) / (sc * sc);
+      s[0] += weight(q) * ay2 / (sc * sc);
+      s[1] += weight(q) * ((double)k[0][q].x * k[0][q].x + (double)k[0][q].y * k[0][q].y) / (sc * sc);
     }
     block_sums<NTH>(s, red, par);
     const double d0 = sqrt(s[0] * inv_nn), d1 = sqrt(s[1] * inv_nn);
@@ -369,7 +419,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
     for (int q = 0; q < NE; ++q) {
       const double sc = atol + rtol * sqrt(y[q].x * y[q].x + y[q].y * y[q].y);
       const double dr = (double)k[1][q].x - k[0][q].x, di = (double)k[1][q].y - k[0][q].y;
-      s2[0] += wt[q] * (dr * dr + di * di) / (sc * sc);
+      s2[0] += weight(q) * (dr * dr + di * di) / (sc * sc);
     }
     block_sums<NTH>(s2, red, par);
     const double d2 = sqrt(s2[0] * inv_nn) / h0;
@@ -407,6 +457,8 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
       t_new = target;
       made_jump = target_jump;
     }
+    h = uniform<(NE > 1)>(h);
+    t_new = uniform<(NE > 1)>(t_new);
     if (!(h > 0.0) || !(h > 1e-14 * fmax(1.0, fabs(t)))) {
       status = DQH_NONFINITE;
       break;
@@ -431,6 +483,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
           }
         }
         y1[q] = s < 6 ? make_double2(h * re, h * im) : make_double2(y[q].x + h * re, y[q].y + h * im);
+        if constexpr (NE > 2) __builtin_amdgcn_sched_barrier(0);
       }
       field(y1, k[s]);
     }
@@ -456,7 +509,8 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
       em *= h;
       const double sc = atol + rtol * sqrt(fmax(y[q].x * y[q].x + y[q].y * y[q].y,
                                                 y1[q].x * y1[q].x + y1[q].y * y1[q].y));
-      ss[0] += wt[q] * (er * er + em * em) / (sc * sc);
+      ss[0] += weight(q) * (er * er + em * em) / (sc * sc);
+      if constexpr (NE > 2) __builtin_amdgcn_sched_barrier(0);
     }
     block_sums<NTH>(ss, red, par);
     const double norm = sqrt(ss[0] * inv_nn);
@@ -474,44 +528,68 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
     if (keep) {
       if (tid == 0 && nacc < p.step_log_cap) gp<double>(p.step_log)[nacc] = t_new;
       ++nacc;
-      while (isave < ntsave && next_save <= t_new) {
-        const double th = (next_save - t) / h;
-        CTab *wr = weights<TAB>();
-        double w[7];
+      if constexpr (NE == 1) {
+        // the dense-output weights of all saves that are due at once, one save per lane
+        // (several elements per thread have no registers for them)
+        for (int m = due(t_new); m > 0; m = due(t_new)) {
+          CTab *wr = weights<TAB>();
+          const double th = (ts - t) / h;
+          double wl[7];
 #pragma unroll
-        for (int j = 0; j < 7; ++j)
-          w[j] = th * (wr->R[j][0] + th * (wr->R[j][1] + th * (wr->R[j][2] + th * wr->R[j][3])));
-        fold_k0(w);
-        save(h, w, isave);
-        advance();
+          for (int j = 0; j < 7; ++j)
+            wl[j] = th * (wr->R[j][0] + th * (wr->R[j][1] + th * (wr->R[j][2] + th * wr->R[j][3])));
+          fold_k0(wl);
+          for (; m > 0; --m, ++isave) {
+            double w[7];
+#pragma unroll
+            for (int j = 0; j < 7; ++j) w[j] = lane_of(wl[j], isave - sbase);
+            save(h, w, isave);
+          }
+          if (isave == sbase + 64) {
+            sbase = isave;
+            ts = sbase + lane < ntsave ? tsave[sbase + lane] : 0.0;
+          }
+        }
+      } else {
+        while (isave < ntsave && next_save <= t_new) {
+          const double th = (next_save - t) / h;
+          CTab *wr = weights<TAB>();
+          double w[7];
+#pragma unroll
+          for (int j = 0; j < 7; ++j)
+            w[j] = th * (wr->R[j][0] + th * (wr->R[j][1] + th * (wr->R[j][2] + th * wr->R[j][3])));
+          fold_k0(w);
+#pragma unroll
+          for (int j = 0; j < 7; ++j) w[j] = uniform<(NE > 1)>(w[j]);
+          save(h, w, isave);
+          advance();
+        }
       }
 #pragma unroll
       for (int q = 0; q < NE; ++q) {
         k[0][q] = k[6][q];
         y[q] = y1[q];
       }
-      t = t_new;
+      t = uniform<(NE > 1)>(t_new);
       need_k0 = made_jump;
     } else {
       ++nrej;
     }
-    dt = factor * h;
+    dt = uniform<(NE > 1)>(factor * h);
   }
-  while (isave < ntsave) {
-    save(0.0, w0, isave);
-    advance();
-  }
+  for (; isave < ntsave; ++isave) save(0.0, w0, isave);
   float2 *fin = gp<float2>(p.final_state);
   float2 *st = gp<float2>(p.states);
 #pragma unroll
   for (int q = 0; q < NE; ++q) {
-    if (ei[q] >= 0) {
+    int i, j;
+    if (at(q, i, j)) {
       const float2 v = make_float2((float)y[q].x, (float)y[q].y), vc = make_float2(v.x, -v.y);
-      fin[(size_t)ei[q] * n + ej[q]] = v;
-      if (ei[q] != ej[q]) fin[(size_t)ej[q] * n + ei[q]] = vc;
+      fin[(size_t)i * n + j] = v;
+      if (i != j) fin[(size_t)j * n + i] = vc;
       if (!save_states) {
-        st[(size_t)ei[q] * n + ej[q]] = v;
-        if (ei[q] != ej[q]) st[(size_t)ej[q] * n + ei[q]] = vc;
+        st[(size_t)i * n + j] = v;
+        if (i != j) st[(size_t)j * n + i] = vc;
       }
     }
   }
@@ -531,7 +609,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
 // and the state are in global memory (work: 7 NU float2, y: NU double2, in owner order; L2
 // serves them), for n > 90, where they do not fit the registers.
 // Bound by the LDS reads, three 8-byte ones per term and element. 48 two-mode problems of
-// n = 81 (10 parts, about 150 steps): 61.2 -> 3.83 ms against the dense body; 32 problems
+// n = 81 (10 parts, about 150 steps): 61.2 -> 2.94 ms against the dense body; 32 problems
 // of n = 127 with one jump diagonal, 8 steps: 12.7 -> 1.28 ms (memory form).
 template <int NTH, int NE, bool KM, int TAB>
 __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__restrict__ insts, Pattern pat) {
@@ -559,7 +637,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
   const double *tsave = gp<const double>(p.tsave);
   const double *ptimes = gp<const double>(p.pwc_times);
   const double rtol = p.rtol, atol = p.atol, t_end = p.t1;
-  const double inv_nn = 1.0 / ((double)n * n);
+  const double inv_nn = uniform<(NE > 1)>(1.0 / ((double)n * n));
   const bool save_states = (p.flags & DQH_FLAG_SAVE_STATES) != 0;
 
   // owned elements, packed i | j << 8 (i <= j; -1 past the end)
@@ -778,27 +856,34 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
   };
 
   int par = 0;
+  // as in k_tsit5_diag: one element at a time, formed anew for every operator
   auto save = [&](double h, const double (&w)[7], int isave) {
     float2 *st = gp<float2>(p.states) + (size_t)isave * n * n;
-    double2 sv[NE];
-#pragma unroll
-    for (int q = 0; q < NE; ++q) {
+    auto value = [&](int q) {
       const double2 y = yget(q);
       double re = 0.0, im = 0.0;
       if (h != 0.0) {
 #pragma unroll
         for (int j = 0; j < 7; ++j) {
-          const float2 kq = kget(j, q);
-          re += w[j] * (double)kq.x;
-          im += w[j] * (double)kq.y;
+          float2 x = kget(j, q);
+          asm volatile("" : "+v"(x.x), "+v"(x.y));
+          re += w[j] * (double)x.x;
+          im += w[j] * (double)x.y;
         }
       }
-      sv[q] = make_double2(y.x + h * re, y.y + h * im);
-      int i, j;
-      at(q, i, j);
-      if (save_states && own(q)) {
-        st[(size_t)i * n + j] = make_float2((float)sv[q].x, (float)sv[q].y);
-        if (i != j) st[(size_t)j * n + i] = make_float2((float)sv[q].x, (float)-sv[q].y);
+      return make_double2(y.x + h * re, y.y + h * im);
+    };
+    if (save_states) {
+#pragma unroll
+      for (int q = 0; q < NE; ++q) {
+        const double2 v = value(q);
+        int i, j;
+        at(q, i, j);
+        if (own(q)) {
+          st[(size_t)i * n + j] = make_float2((float)v.x, (float)v.y);
+          if (i != j) st[(size_t)j * n + i] = make_float2((float)v.x, (float)-v.y);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
     const float2 *ET = gp<const float2>(p.EopsT);
@@ -807,18 +892,20 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
       double s[2] = {0.0, 0.0};
 #pragma unroll
       for (int q = 0; q < NE; ++q) {
+        const double2 v = value(q);
         if (own(q)) {
           int i, j;
           at(q, i, j);
           const float2 o = E[(size_t)i * np + j];
-          s[0] += o.x * sv[q].x - o.y * sv[q].y;
-          s[1] += o.x * sv[q].y + o.y * sv[q].x;
+          s[0] += o.x * v.x - o.y * v.y;
+          s[1] += o.x * v.y + o.y * v.x;
           if (i != j) {
             const float2 m = E[(size_t)j * np + i];
-            s[0] += m.x * sv[q].x + m.y * sv[q].y;
-            s[1] += m.y * sv[q].x - m.x * sv[q].y;
+            s[0] += m.x * v.x + m.y * v.y;
+            s[1] += m.y * v.x - m.x * v.y;
           }
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
       block_sums<NTH>(s, red, par);
       if (tid == 0) gp<float2>(p.expects)[(size_t)e * ntsave + isave] = make_float2((float)s[0], (float)s[1]);
@@ -837,7 +924,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
   double next_save = ntsave > 0 ? tsave[0] : 0.0;
   auto advance = [&]() {
     ++isave;
-    if (isave < ntsave) next_save = tsave[isave];
+    if (isave < ntsave) next_save = uniform<(NE > 1)>(tsave[isave]);
   };
   int seg = -1;
   double next_break = pwc ? ptimes[0] : 0.0;
@@ -926,6 +1013,8 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
       t_new = target;
       made_jump = target_jump;
     }
+    h = uniform<(NE > 1)>(h);
+    t_new = uniform<(NE > 1)>(t_new);
     if (!(h > 0.0) || !(h > 1e-14 * fmax(1.0, fabs(t)))) {
       status = DQH_NONFINITE;
       break;
@@ -987,6 +1076,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
       em *= h;
       const double sc = atol + rtol * sqrt(fmax(y.x * y.x + y.y * y.y, v[q].x * v[q].x + v[q].y * v[q].y));
       ss[0] += weight(q) * (er * er + em * em) / (sc * sc);
+      if constexpr (KM || NE > 2) __builtin_amdgcn_sched_barrier(0);
     }
     block_sums<NTH>(ss, red, par);
     const double norm = sqrt(ss[0] * inv_nn);
@@ -1012,6 +1102,8 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
         for (int j = 0; j < 7; ++j)
           w[j] = th * (wr->R[j][0] + th * (wr->R[j][1] + th * (wr->R[j][2] + th * wr->R[j][3])));
         if (!smooth) fold_k0(w);
+#pragma unroll
+        for (int j = 0; j < 7; ++j) w[j] = uniform<(NE > 1)>(w[j]);
         save(h, w, isave);
         advance();
       }
@@ -1028,7 +1120,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
     } else {
       ++nrej;
     }
-    dt = factor * h;
+    dt = uniform<(NE > 1)>(factor * h);
   }
   while (isave < ntsave) {
     save(0.0, w0, isave);
