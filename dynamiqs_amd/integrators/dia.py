@@ -335,8 +335,10 @@ def build_plan(
     if normalisation not in ('auto', 'banded', 'blocks'):
         raise ValueError("normalisation must be 'auto', 'banded' or 'blocks'")
     isets = None
+    Ss = []
     if normalisation != 'banded' and n_pad <= MAXN_BLOCKS:
-        isets = coupled_sets(normalisation_S(H, Ls, sets[0], n_pad))
+        Ss = [normalisation_S(H, Ls, h, n_pad) for h in sets]
+        isets = coupled_sets(Ss[0])
     if normalisation == 'blocks' and isets is None:
         raise ValueError('the normalisation matrix S does not decouple into sets of at most '
                          f'{MAXBLK} indices (or n > {MAXN_BLOCKS})')
@@ -344,7 +346,7 @@ def build_plan(
     # elements of a Hermitian state
     diagonal = (isets is not None and normalisation == 'auto' and variant == SWEEP_AUTO and solve_panel == 0)
     packs = [block_solve_operators(H, Ls, h, n_pad, banded=isets is None) for h in sets]
-    blks = [block_normalisation(normalisation_S(H, Ls, h, n_pad), isets) for h in sets] if isets is not None else []
+    blks = [block_normalisation(S, isets) for S in Ss] if isets is not None else []
     if diagonal:
         nds = [diagonal_normalisation(of, loc, idx, start, mat, Lm, n_pad)
                for (of, loc, start, idx, mat, Lm, _) in blks]
