@@ -609,7 +609,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
 // and the state are in global memory (work: 7 NU float2, y: NU double2, in owner order; L2
 // serves them), for n > 90, where they do not fit the registers.
 // Bound by the LDS reads, three 8-byte ones per term and element. 48 two-mode problems of
-// n = 81 (10 parts, about 150 steps): 61.2 -> 2.94 ms against the dense body; 32 problems
+// n = 81 (10 parts, about 150 steps): 61.2 -> 2.12 ms against the dense body; 32 problems
 // of n = 127 with one jump diagonal, 8 steps: 12.7 -> 1.28 ms (memory form).
 template <int NTH, int NE, bool KM, int TAB>
 __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__restrict__ insts, Pattern pat) {
@@ -803,10 +803,11 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
     // QC elements at a time: each term keeps their reads in flight
 #pragma unroll
     for (int c = 0; c < NE; c += QC) {
+      const int nq = NE - c < QC ? NE - c : QC;  // constant once unrolled
       float fr[QC], fi[QC];
       int i[QC], j[QC];
 #pragma unroll
-      for (int q = 0; q < QC; ++q) {
+      for (int q = 0; q < nq; ++q) {
         fr[q] = fi[q] = 0.f;
         at(c + q, i[q], j[q]);
       }
@@ -814,7 +815,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
       for (int x = 0; x < pat.nH; ++x) {
         const int o = pat.offH[x];
 #pragma unroll
-        for (int q = 0; q < QC; ++q) {
+        for (int q = 0; q < nq; ++q) {
           const float2 cr = Gt[x * n + i[q]], cc = Gt[x * n + j[q]];
           const int e = i[q] * LD + j[q];
           const float2 a = ys[min(max(e + o * LD, 0), NLD)], b = ys[min(max(e + o, 0), NLD)];
@@ -827,7 +828,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
         const Part pr = pat.pair[x];
         const int sh = pat.pa[x] * LD + pat.pb[x];
 #pragma unroll
-        for (int q = 0; q < QC; ++q) {
+        for (int q = 0; q < nq; ++q) {
           const float2 l = Lt[pr.x * n + i[q]], m = Lt[pr.y * n + j[q]];
           const float2 z = ys[min(max(i[q] * LD + j[q] + sh, 0), NLD)];
           const float cr = l.x * m.x + l.y * m.y, ci = l.y * m.x - l.x * m.y;
@@ -836,7 +837,7 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag_tab(const dqh_me_inst *__res
         }
       }
 #pragma unroll
-      for (int q = 0; q < QC; ++q) {
+      for (int q = 0; q < nq; ++q) {
         const double2 da = dcur[i[q]], db = dcur[j[q]];
         double gr = da.x + db.x, gi = da.y - db.y;
 #pragma unroll 1
@@ -1249,7 +1250,15 @@ int launch_tab_size(const dqh_me_inst *d, int64_t ninst, int n, const Pattern &p
   const int nu = n * (n + 1) / 2;
   if (nu <= 576) return launch_tab<576, 1, false, TAB>(d, ninst, n, pt, st);
   if (nu <= 2048) return launch_tab<1024, 2, false, TAB>(d, ninst, n, pt, st);
+  // 704 threads (11 waves) have 168 registers each, which hold the stages of 4 elements and
+  // nearly those of 5; 1024 have 128 (48 two-mode solves: n = 72 2.98 ms with 1024 threads,
+  // 1.61 with 704; n = 81 2.93 and 2.12). In memory, the fewest elements per thread that cover
+  // the triangle (n = 100: 8.1 ms with 8, 4.5 with 5).
+  if (nu <= 2816) return launch_tab<704, 4, false, TAB>(d, ninst, n, pt, st);
+  if (nu <= 3520) return launch_tab<704, 5, false, TAB>(d, ninst, n, pt, st);
   if (nu <= 4096) return launch_tab<1024, 4, false, TAB>(d, ninst, n, pt, st);
+  if (nu <= 5120) return launch_tab<1024, 5, true, TAB>(d, ninst, n, pt, st);
+  if (nu <= 6144) return launch_tab<1024, 6, true, TAB>(d, ninst, n, pt, st);
   return launch_tab<1024, 8, true, TAB>(d, ninst, n, pt, st);
 }
 

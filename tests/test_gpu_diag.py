@@ -67,6 +67,10 @@ CASES = [
     (64, [-62, 62], [[62], [-60]], 'tsit5'), (20, [0, 1], [[0, 1, 2], [1]], 'dopri5'), (63, [-1, 1], [[-1, 0, 1], [5]], 'tsit5'),
     (65, [-8, -1, 0, 1, 8], [[1], [8]], 'tsit5'), (90, [-9, 9], [[9], [1], [0]], 'dopri5'),
     (91, [-10, 10], [[10], [0, 1]], 'tsit5'), (127, [-1, 0, 1], [[1], [126]], 'tsit5'),
+    # the last of one and the first of the next number of elements per thread
+    (74, [-1, 1], [[1]], 'tsit5'), (75, [-1, 1], [[1]], 'dopri5'), (83, [-9, 9], [[9], [0, 1]], 'tsit5'),
+    (84, [-1, 1], [[1], [83]], 'tsit5'), (100, [-10, 10], [[10], [1]], 'dopri5'), (101, [-1, 0, 1], [[1]], 'tsit5'),
+    (110, [-1, 1], [[1]], 'tsit5'), (111, [-1, 1], [[2]], 'dopri5'),
 ]
 
 
