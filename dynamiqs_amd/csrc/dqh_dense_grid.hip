@@ -13,11 +13,6 @@
 //            only), y + that increment for stage 6; or on the last stage the FP64
 //            partial sums of the scaled error. The stage inputs alternate between two
 //            buffers.
-// Bound by the FP32 matrix cores and the L2 reads of their operands; the splits are there
-// because a few hundred tiles of one or two instances would otherwise leave most of the
-// 1024 SIMDs idle. Two instances of n = 233 with 3 jump operators: a stage 46 -> 27 us
-// (before: tmp = Hnh ys + sum_k X_k L_k^dag / 2 on all tiles, one wave each, and a third
-// launch for tmp + tmp^dag). An XCD-aware order of the tiles made no difference.
 // and one commit launch per step (accept/reject, dense-output saves, y <- y1 in
 // FP64, the next stage input), as in the DIA grid integrator: every workgroup
 // reduces its instance's partial sums in the same order, control blocks alternate
@@ -26,6 +21,12 @@
 // dqh_mesolve_tsit5_dense (same operators, scratch, outputs and controller,
 // diffrax_integrator.py:59-81, 101-147), so the two entry points are
 // interchangeable for constant generators.
+//
+// Bound by the FP32 matrix cores and the L2 reads of their operands; the splits are there
+// because a few hundred tiles of one or two instances would otherwise leave most of the
+// 1024 SIMDs idle. Two instances of n = 233 with 3 jump operators: a stage 46 -> 27 us
+// (before: tmp = Hnh ys + sum_k X_k L_k^dag / 2 on all tiles, one wave each, and a third
+// launch for tmp + tmp^dag). An XCD-aware order of the tiles made no difference.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -663,10 +663,11 @@ __global__ __launch_bounds__(256) void k_kraus(int64_t n, int64_t n_true, int64_
 //   k_dnorm   E = D hi + hi D^dag + D hi D^dag, X = hi + E      24 bytes per element
 //   k_dkraus  the Kraus increment of X, the FP64 update          48 bytes per element
 // Bound by those bytes. 16 states of n = 1024 (D with 4 diagonals, 17
-// products of the Kraus map), 40 steps: 24.2 -> 10.4 ms (k_blk_norm 233 us and k_kraus 266 us
-// a step before, 98 and 149 now; a copy of their bytes would take 43 and 86, the rest are the
-// L1 accesses of the 16 and 17 neighbours and the stores below the diagonal). One, two and
-// four rows per thread: 111, 103, 98 us for k_dnorm.
+// products of the Kraus map), 40 steps: 24.3 -> 8.7 ms (k_blk_norm 233 us and k_kraus 266 us
+// a step before; now 98 and 149 for all 16 states at once, 47 and 55 for each of two groups
+// that fit the Infinity Cache; a copy of the bytes of all from HBM would take 43 and 86, the
+// rest are the L1 accesses of the 16 and 17 neighbours and the stores below the diagonal).
+// One, two and four rows per thread: 111, 103, 98 us for k_dnorm.
 struct DView {
   int64_t n, n_true;
   int32_t herm, spread, nb, total;

@@ -18,11 +18,11 @@
 // Bytes per element and step: 40 + 56 + 64 + 72 + 88 + 88 = 408, of half the elements,
 // against 496 of all of them with full-matrix sweeps and a commit pass. The stages are
 // evaluated on the rounded states y + Delta_s as before: on the increments alone (344 bytes,
-// 6.7 ms below) the error estimate loses the FP32 noise that holds the steps down in the
+// about 1 ms less below) the error estimate loses the FP32 noise that holds the steps down in the
 // full-matrix form, and the solutions moved by up to 8e-3 of the largest elements' scale.
 // Measured (rtol 1e-6, atol 1e-8, two coupled modes with 8 shifts): four solves of n = 1024,
-// 36 steps, 22.6 -> 6.9 ms, stages at 3.8 to 5.3 TB/s (a copy reaches 4.7); one of
-// n = 323, 29 steps, 2.8 -> 1.24 ms, bound by the latency of a launch (about 5 us).
+// 36 steps, 21.7 -> 7.3 ms, stages at 3.8 to 5.3 TB/s (a copy reaches 4.7); one of
+// n = 323, 29 steps, 2.4 -> 1.08 ms, bound by the latency of a launch (about 5 us).
 // Time-dependent Hamiltonians take a separate controller launch before the first stage,
 // because their diagonals are rebuilt in between.
 //
@@ -856,7 +856,7 @@ int drive(const dqh_dia_tsit5 &p, diats::V v, hipStream_t st) {
   const dim3 gflat = diat::row_grid(p.n, p.ninst);
   // Steps per replay: at most 4, because the replay in flight when the count shows the end
   // and the rest of the last one are launches without work (n = 323, 29
-  // steps: 1.24 ms a solve with 4, 1.40 with 16; four solves of n = 1024: 6.92 and 7.45)
+  // steps: 1.30 ms a solve with 4, 1.40 with 16; four solves of n = 1024: 7.66 and 8.15)
   const int64_t G = p.graph_steps > 0 ? std::min<int64_t>(p.graph_steps, 4) : 2;
   volatile int64_t *hf = reinterpret_cast<volatile int64_t *>(p.host_flags);
   hf[0] = hf[1] = -1;

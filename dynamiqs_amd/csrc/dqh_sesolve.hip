@@ -409,7 +409,7 @@ __global__ __launch_bounds__(T) void k_sesolve(const dqh_me_inst *__restrict__ i
 // barrier per stage), the four partial sums are added within the quad. Up to n = 64 the first
 // expectation operator is in registers as well. Bound by the latency of a stage. A call,
 // against reading G from the caches at every stage: 48 solves of n = 64 (50 saves, Dopri5)
-// 2.44 -> 1.01 ms, 3000 two-level solves 2.00 -> 1.88 ms (the host's share), up to 7 times
+// 2.45 -> 1.1 ms, 3000 two-level solves 2.0 -> 1.9 ms (the host's share), up to 7 times
 // less at 64 < n <= 128.
 template <int NR, int TAB>
 __global__ __launch_bounds__(4 * NR) void k_sesolve_const(const dqh_me_inst *__restrict__ insts) {
