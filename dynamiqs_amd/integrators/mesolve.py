@@ -519,7 +519,10 @@ def hermitian_parts(rhos, assume_hermitian: bool):
     parts are solved as separate instances. Returns the list of states to solve and, per input, the index of A
     and of B (-1 when there is no B part)."""
     parts, index = [], []
-    split = {}  # by array: instances that share a state share its parts
+    # by array: instances that share a state share its parts. The list keeps the arrays alive
+    # while their ids are keys (iterating over one array makes views that are freed at once)
+    rhos = list(rhos)
+    split = {}
 
     def parts_of(r):
         r = np.asarray(r)

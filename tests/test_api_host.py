@@ -167,6 +167,63 @@ def test_hermitian_parts_split_and_recombine():
     np.testing.assert_allclose(parts[0], 0.5 * (x + x.conj().T))
 
 
+@pytest.mark.parametrize('assume', [True, False])
+@pytest.mark.parametrize('hermitian', [True, False])
+@pytest.mark.parametrize('n', [5, 144])
+def test_hermitian_parts_of_one_array(n, hermitian, assume):
+    """Distinct states given as one array, whose rows are views made on the fly: A + iB of
+    every state is that state (its Hermitian part when the states are assumed Hermitian),
+    and a state that appears twice in a list is split once."""
+    from dynamiqs_amd.integrators.mesolve import combine_parts, hermitian_parts
+
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(8, n, n)) + 1j * rng.normal(size=(8, n, n))
+    h = 0.5 * (x + np.swapaxes(x.conj(), -1, -2))
+    r = h if hermitian else x
+    parts, index = hermitian_parts(r, assume)
+    assert len(parts) == (8 if hermitian or assume else 16)
+    np.testing.assert_allclose(combine_parts(np.stack(parts), index), h if assume else r, atol=1e-14)
+    parts, index = hermitian_parts([r[0], r[1], h[0]], assume)
+    np.testing.assert_allclose(combine_parts(np.stack(parts), index), [h[0], h[1], h[0]] if assume else [r[0], r[1], h[0]], atol=1e-14)
+    same = [h[0]] * 2
+    parts, _ = hermitian_parts(same, assume)
+    assert parts[0] is parts[1]
+
+
+@pytest.mark.parametrize('method', [dq.method.Tsit5(), dq.method.Dopri5(), dq.method.Rouchon1(dt=0.1)])
+@pytest.mark.parametrize('assume', [True, False])
+@pytest.mark.parametrize('kets', [True, False])
+@pytest.mark.parametrize('m', [1, 3, 5, 8])
+def test_dia_route_packs_every_initial_state(monkeypatch, m, kets, assume, method):
+    """dq.mesolve on DIA operators with n >= 128: the states handed to the plan are those of
+    the call, in order."""
+    from dynamiqs_amd.integrators import dia
+
+    na, nb = 12, 12
+    n = na * nb
+    a, b = dq.tensor(dq.destroy(na), dq.eye(nb)), dq.tensor(dq.eye(na), dq.destroy(nb))
+    rng = np.random.default_rng(m)
+    psi = rng.normal(size=(m, n, 1)) + 1j * rng.normal(size=(m, n, 1))
+    psi /= np.linalg.norm(psi, axis=-2, keepdims=True)
+    rho = psi @ np.swapaxes(psi.conj(), -1, -2)
+    seen = []
+
+    class Packed(Exception):
+        pass
+
+    def take(H, Ls, rho0, *args, **kwargs):
+        seen.append(np.array(rho0))
+        raise Packed
+
+    monkeypatch.setattr(dia, 'tsit5_plan', take)
+    monkeypatch.setattr(dia, 'build_plan', take)
+    with pytest.raises(Packed):
+        dq.mesolve(a.dag() @ b + a @ b.dag(), [a, b], psi if kets else rho, np.linspace(0.0, 1.0, 3), method=method,
+                   options=dq.Options(assume_hermitian=assume))
+    assert seen[0].shape == (m, n, n)
+    np.testing.assert_allclose(seen[0], rho, atol=1e-15)
+
+
 def test_save_extra_outputs_stacking():
     """save_extra outputs are stacked leaf by leaf with shape (*batch, ntsave, *leaf)
     (dicts, named tuples, lists, QArray leaves), as the reference's vmapped scan

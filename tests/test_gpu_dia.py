@@ -360,6 +360,26 @@ def test_mesolve_routes_dia_tsit5():
     assert int(res.infos.nsteps) > 0
 
 
+@pytest.mark.parametrize('method', ['tsit5', 'dopri5', 'rouchon1'])
+def test_mesolve_dia_batch_of_states_equals_single_solves(method):
+    """Five different kets in one call at n = 144 against five calls: an instance depends on
+    its own state only, up to the order of FP64 sums (1e-7, one rounding of the results)."""
+    import dynamiqs_amd as dq
+
+    a, b = dq.destroy(12, 12)
+    H = 5 * a.dag() @ a + 6 * b.dag() @ b + 0.1 * (a.dag() @ b + a @ b.dag())
+    Ls = [np.sqrt(0.02) * a, np.sqrt(0.05) * b]
+    m = {'tsit5': dq.method.Tsit5(), 'dopri5': dq.method.Dopri5(), 'rouchon1': dq.method.Rouchon1(dt=1e-2)}[method]
+    kets = np.stack([dq.coherent((12, 12), (al, 0.2)).to_numpy() for al in (0.3, 0.6, 0.9, 1.2, 1.5)])
+    tsave = np.linspace(0.0, 0.2, 3)
+    kw = dict(exp_ops=[a.dag() @ a], method=m)
+    res = dq.mesolve(H, Ls, kets, tsave, **kw)
+    for i, ket in enumerate(kets):
+        one = dq.mesolve(H, Ls, ket, tsave, **kw)
+        assert np.abs(res.states.to_numpy()[i] - one.states.to_numpy()).max() <= 1e-7
+        assert np.abs(res.expects[i] - one.expects).max() <= 1e-6
+
+
 def test_autotuner_times_and_caches_dia_and_dense_forms(tmp_path, monkeypatch):
     """The autotuner times every admissible form on the GPU, keeps the fastest and
     answers the next request for the same key from its cache."""
