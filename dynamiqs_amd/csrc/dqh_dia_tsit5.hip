@@ -20,9 +20,10 @@
 // evaluated on the rounded states y + Delta_s as before: on the increments alone (344 bytes,
 // about 1 ms less below) the error estimate loses the FP32 noise that holds the steps down in the
 // full-matrix form, and the solutions moved by up to 8e-3 of the largest elements' scale.
+// The order of rounding within a field is that of the full-matrix form too (stencil below).
 // Measured (rtol 1e-6, atol 1e-8, two coupled modes with 8 shifts): four solves of n = 1024,
-// 36 steps, 21.7 -> 7.3 ms, stages at 3.8 to 5.3 TB/s (a copy reaches 4.7); one of
-// n = 323, 29 steps, 2.4 -> 1.08 ms, bound by the latency of a launch (about 5 us).
+// 36 steps, 21.7 -> 7.4 ms, stages at 3.8 to 5.3 TB/s (a copy reaches 4.7); one of
+// n = 323, 29 steps, 2.4 -> 1.2 ms, bound by the latency of a launch (about 5 us).
 // Time-dependent Hamiltonians take a separate controller launch before the first stage,
 // because their diagonals are rebuilt in between.
 //
@@ -62,26 +63,31 @@ constexpr int64_t kJump = 8;    // the last accepted step ended on a PWC breakpo
 constexpr int64_t kFresh = 16;  // no attempt to commit yet
 constexpr int64_t kSel = 32;    // the state is in the second FP64 buffer
 
-// One shift of the stencil: f[i][j] += r[i + p] conj(c[j + q]) X[i + p][j + q]. One-sided
-// products have a vector of ones on the other side. tdr / tdc: the vector belongs to the
-// time-dependent generator (one copy per instance).
+// A shift of a jump operator: f[i][j] += r[i + p] z, z = go z_before + X[i + p][j + q] conj(c[j + q]).
+// The column offsets of a row offset share its factor: go = 1 from the second on, and r is a
+// vector of zeros but for the last.
 struct Term {
   const float2 *r, *c;
-  int32_t p, q, tdr, tdc;
+  int32_t p, q;
+  float go;
+  int32_t pad;
 };
 static_assert(sizeof(Term) == 32, "terms are read as 32-byte scalars");
-constexpr int kMaxTerm = 2 * DQH_DIA_MAXOFF + (DQH_DIA_MAXOPS - 1) * DQH_DIA_MAXOFF * DQH_DIA_MAXOFF;
+constexpr int kMaxTerm = (DQH_DIA_MAXOPS - 1) * DQH_DIA_MAXOFF * DQH_DIA_MAXOFF;
+constexpr int kHead = 4;  // terms in the kernel arguments: one round trip less than from the list
 
 struct V {
   int64_t n, n_true, ninst, nsave, max_steps, npart, flags;
-  int32_t herm, spread, nterm, nb, total;  // nb: 64-element blocks per side; total: tiles per instance
+  int32_t herm, spread, npair, nterm, nb, total;  // nb: 64-element blocks per side; total: tiles per instance
   int32_t presum;  // the control blocks are formed by k_ctl
+  int32_t off[DQH_DIA_MAXOFF];  // offsets of the generator (operator 0): npair of them
+  Term head[kHead];             // the first of the nterm terms
   double rtol, atol, safety, fmin_, fmax_, t0, t1, inv_nn;
   float2 *k;      // [7][ninst][n][n]
   float2 *ys;     // [2][ninst][n][n]
   double2 *y2;    // [ninst][n][n]: second FP64 state
-  Term *terms;
-  float2 *ones;   // [n]
+  Term *terms;    // [nterm]
+  float2 *zeros;  // [n]
   double *part;   // [ninst][2][npart]
   Ctrl *ctrl;     // [2][ninst]
   int64_t *flag;  // completion count; before the first step: rho0 is not Hermitian
@@ -196,7 +202,6 @@ struct InYK {
 
 typedef const __attribute__((address_space(4))) Term CTerm;
 typedef int Int8 __attribute__((ext_vector_type(8)));
-typedef const __attribute__((address_space(4))) Int8 CInt8;
 
 // A control block that no workgroup of the launch writes, through the scalar cache
 __device__ __forceinline__ Ctrl read_ctrl(const Ctrl *p) {
@@ -204,96 +209,158 @@ __device__ __forceinline__ Ctrl read_ctrl(const Ctrl *p) {
   return Ctrl{c->t, c->dt, c->nsteps, c->nacc, c->nrej, c->status, c->isave, c->rot};
 }
 
-// The first shifts of the list, requested ahead of the loads that decide whether they are
-// needed: one round trip less in a launch that is bound by its latency (n = 323: a stage 4.7 -> 4.35 us)
-constexpr int kAhead = 8;
-struct Ahead {
-  Int8 t[kAhead];
-};
-template <int NE>
-__device__ __forceinline__ Ahead look_ahead(const V &v) {
-  Ahead a;
-  if constexpr (NE == 1) {
-    CInt8 *p = (CInt8 *)v.terms;
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) a.t[u] = p[u];  // the list has room for more
-  }
-  return a;
-}
-template <int NE>
-__device__ __forceinline__ void arrived(Ahead &a) {
-  if constexpr (NE == 1) {
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) asm volatile("" : "+s"(a.t[u]));
-  }
-}
-__device__ __forceinline__ Term as_term(Int8 x) {
-  Term t;
-  __builtin_memcpy(&t, &x, sizeof(t));
-  return t;
-}
 typedef const __attribute__((address_space(4))) float CFloat;
 typedef const __attribute__((address_space(1))) float GFloat;
 
 // f(X) at rows i0 .. i0 + NE - 1 of column j (columns past the matrix read column
-// n_true - 1 and are dropped by the caller). The row factors are wave-uniform scalars,
+// n_true - 1 and are dropped by the caller). The row factors are alike in a wave,
 // out-of-range neighbours have a zero factor.
+// Order of rounding: every product of complex numbers is rounded before it is added, and
+// X conj(c) is summed over a jump operator's column offsets before the row factor. The error
+// estimate of the first steps lies in the FP32 noise of f, so the step sequence follows the
+// rounding, and the components at the stability limit follow the steps: with the products
+// chained into the sum by fused multiply-adds the states of n = 1024 differed from those of
+// the full-matrix form by up to 2.5e-2 of their rms (12 batches of four), now by up to 3.7e-3
+// (40 batches; the full-matrix form sums the lower triangle in another order).
+// The loads of a chunk are in flight together: with one row per thread those of up to 4
+// offsets of the generator and 4 terms (n = 323: a solve 1.2 ms, 1.4 with terms of one kind
+// in chunks of 8 that share code), with four rows about 16 of the matrix. One row per thread
+// reads its row factors like the column's, because a scalar load is waited for in its block.
 template <int NE, bool TD, class In>
-__device__ __forceinline__ void stencil(const V &v, size_t inst, const In &X, int i0, int j, float2 (&f)[NE],
-                                        const Ahead *ahead = nullptr) {
-  const int nt = v.nterm, n = (int)v.n, lim = (int)v.n_true;
+__device__ __forceinline__ void stencil(const V &v, size_t inst, const In &X, int i0, int j, float2 (&f)[NE]) {
+  const int n = (int)v.n, lim = (int)v.n_true, np = v.npair, nt = v.nterm;
+  const float2 *D = TD ? v.hcur + inst * (size_t)v.noff0 * v.n : v.H0;
+  float2 z[NE];
 #pragma unroll
-  for (int m = 0; m < NE; ++m) f[m] = make_float2(0.f, 0.f);
-  CTerm *terms = (CTerm *)v.terms;
-  const size_t hs = TD ? inst * (size_t)v.noff0 * v.n : 0;
-  auto group = [&](auto cnt, auto first, int t0) {
-    constexpr int U = decltype(cnt)::value;
-    float2 c[U], x[U][NE];
-    float rx[U][NE], ry[U][NE];
+  for (int m = 0; m < NE; ++m) f[m] = z[m] = make_float2(0.f, 0.f);
+  auto clamp = [&](int a) { return min(max(a, 0), lim - 1); };
+  auto outside = [&](int a) { return (unsigned)a >= (unsigned)lim; };
+  auto column = [&](const float2 *d, int qc) {
+    GFloat *cp = (GFloat *)d;
+    return make_float2(cp[2 * qc], cp[2 * qc + 1]);
+  };
+  auto rows = [&](const float2 *d, int p, float2 (&r)[NE]) {
+    CFloat *rp = (CFloat *)d;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      Term t;
-      if constexpr (decltype(first)::value)
-        t = as_term(ahead->t[u]);
-      else
-        t = Term{terms[t0 + u].r, terms[t0 + u].c, terms[t0 + u].p, terms[t0 + u].q, terms[t0 + u].tdr, terms[t0 + u].tdc};
-      const int q = j + t.q, qc = min(max(q, 0), lim - 1);
-      GFloat *cp = (GFloat *)t.c;
-      CFloat *rp = (CFloat *)t.r;
-      if (TD && t.tdc) cp += 2 * hs;
-      if (TD && t.tdr) rp += 2 * hs;
-      c[u] = make_float2(cp[2 * qc], cp[2 * qc + 1]);
-      if (q != qc) c[u] = make_float2(0.f, 0.f);
-#pragma unroll
-      for (int m = 0; m < NE; ++m) {
-        const int a = i0 + m + t.p, ac = min(max(a, 0), lim - 1);
-        const float wx = rp[2 * ac], wy = rp[2 * ac + 1];
-        rx[u][m] = a == ac ? wx : 0.f;
-        ry[u][m] = a == ac ? wy : 0.f;
-        x[u][m] = X((size_t)ac * n + qc);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int m = 0; m < NE; ++m) {
-        const float kr = fmaf(rx[u][m], c[u].x, ry[u][m] * c[u].y);
-        const float ki = fmaf(ry[u][m], c[u].x, -(rx[u][m] * c[u].y));
-        f[m].x = fmaf(kr, x[u][m].x, fmaf(-ki, x[u][m].y, f[m].x));
-        f[m].y = fmaf(kr, x[u][m].y, fmaf(ki, x[u][m].x, f[m].y));
+    for (int m = 0; m < NE; ++m) {
+      int a = clamp(i0 + m + p);
+      if constexpr (NE == 1) {
+        asm volatile("" : "+v"(a));
+        r[m] = column(d, a);
+      } else {
+        r[m] = make_float2(rp[2 * a], rp[2 * a + 1]);
       }
     }
   };
-  constexpr int U = NE > 1 ? 4 : 8;
-  int t = 0;
-  if constexpr (NE == 1) {
-    if (ahead && nt >= kAhead) {
-      group(std::integral_constant<int, kAhead>{}, std::true_type{}, 0);
-      t = kAhead;
+  // an offset p of the generator: G[i][i + p] X[i + p][j], then X[i][j + p] conj(G[j][j + p])
+  struct Pair {
+    int p;
+    float2 c, r[NE], x[NE], w[NE];
+  };
+  auto load_pair = [&](Pair &o, int u, int p) {
+    const float2 *d = D + (size_t)u * n;
+    o.p = p;
+    const int qc = clamp(j + o.p);
+    o.c = column(d, qc);
+    rows(d, o.p, o.r);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      o.x[m] = X((size_t)clamp(i0 + m + o.p) * n + j);
+      o.w[m] = X((size_t)min(i0 + m, lim - 1) * n + qc);
     }
+  };
+  auto add_pair = [&](Pair &o) {
+    if (outside(j + o.p)) o.c = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      if (outside(i0 + m + o.p)) o.r[m] = make_float2(0.f, 0.f);
+      f[m].x += fmaf(o.r[m].x, o.x[m].x, -(o.r[m].y * o.x[m].y));
+      f[m].y += fmaf(o.r[m].x, o.x[m].y, o.r[m].y * o.x[m].x);
+      f[m].x += fmaf(o.w[m].x, o.c.x, o.w[m].y * o.c.y);
+      f[m].y += fmaf(o.w[m].y, o.c.x, -(o.w[m].x * o.c.y));
+    }
+  };
+  struct Jump {
+    int p, q;
+    float go;
+    float2 c, r[NE], x[NE];
+  };
+  auto load_jump = [&](Jump &o, const auto &t) {
+    o.p = t.p;
+    o.q = t.q;
+    o.go = t.go;
+    const int qc = clamp(j + o.q);
+    o.c = column(t.c, qc);
+    rows(t.r, o.p, o.r);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) o.x[m] = X((size_t)clamp(i0 + m + o.p) * n + qc);
+  };
+  auto add_jump = [&](Jump &o) {
+    if (outside(j + o.q)) o.c = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int m = 0; m < NE; ++m) {
+      if (outside(i0 + m + o.p)) o.r[m] = make_float2(0.f, 0.f);
+      z[m].x = fmaf(z[m].x, o.go, fmaf(o.x[m].x, o.c.x, o.x[m].y * o.c.y));
+      z[m].y = fmaf(z[m].y, o.go, fmaf(o.x[m].y, o.c.x, -(o.x[m].x * o.c.y)));
+      f[m].x += fmaf(o.r[m].x, z[m].x, -(o.r[m].y * z[m].y));
+      f[m].y += fmaf(o.r[m].y, z[m].x, o.r[m].x * z[m].y);
+    }
+  };
+  // offsets in chunks of PF, the last PL or fewer together with the first SL terms, the
+  // other terms in chunks of SF
+  constexpr int PF = NE > 1 ? 2 : 4, PL = NE > 1 ? 1 : 4, SL = NE > 1 ? 2 : kHead, SF = 4;
+  int u = 0;
+  for (; np - u > PL; u += PF) {
+    Pair o[PF];
+#pragma unroll
+    for (int x = 0; x < PF; ++x) load_pair(o[x], u + x, v.off[u + x]);
+#pragma unroll
+    for (int x = 0; x < PF; ++x) add_pair(o[x]);
   }
-  for (; t + U <= nt; t += U) group(std::integral_constant<int, U>{}, std::false_type{}, t);
-  for (; t < nt; ++t) group(std::integral_constant<int, 1>{}, std::false_type{}, t);
+  {
+    Pair o[PL];
+    Jump s[SL];
+    int off[PL];
+    Int8 head[SL];
+#pragma unroll
+    for (int x = 0; x < PL; ++x) off[x] = v.off[min(u + x, DQH_DIA_MAXOFF - 1)];
+#pragma unroll
+    for (int x = 0; x < SL; ++x) __builtin_memcpy(&head[x], &v.head[x], sizeof(Term));
+    // these arrive together: in the blocks below each would be waited for by itself
+#pragma unroll
+    for (int x = 0; x < PL; ++x) asm volatile("" : "+s"(off[x]));
+#pragma unroll
+    for (int x = 0; x < SL; ++x) asm volatile("" : "+s"(head[x]));
+#pragma unroll
+    for (int x = 0; x < PL; ++x)
+      if (u + x < np) load_pair(o[x], u + x, off[x]);
+#pragma unroll
+    for (int x = 0; x < SL; ++x) {
+      Term t;
+      __builtin_memcpy(&t, &head[x], sizeof(Term));
+      if (x < nt) load_jump(s[x], t);
+    }
+#pragma unroll
+    for (int x = 0; x < PL; ++x)
+      if (u + x < np) add_pair(o[x]);
+#pragma unroll
+    for (int x = 0; x < SL; ++x)
+      if (x < nt) add_jump(s[x]);
+  }
+  CTerm *terms = (CTerm *)v.terms;
+  int t = SL;
+  for (; t + SF <= nt; t += SF) {
+    Jump s[SF];
+#pragma unroll
+    for (int x = 0; x < SF; ++x) load_jump(s[x], terms[t + x]);
+#pragma unroll
+    for (int x = 0; x < SF; ++x) add_jump(s[x]);
+  }
+  for (; t < nt; ++t) {
+    Jump s;
+    load_jump(s, terms[t]);
+    add_jump(s);
+  }
   if (v.herm) {
 #pragma unroll
     for (int m = 0; m < NE; ++m)
@@ -410,13 +477,11 @@ __global__ __launch_bounds__(256) void k_stage(V v, int cur) {
   const size_t inst = blockIdx.y;
   int id, i0, j;
   if (!tile<NE>(v, id, i0, j)) return;
-  Ahead ahead = look_ahead<NE>(v);
   Ctrl c;
   if constexpr (S == 1 && !TD)
     c = commit<NE, TD>(v, cur, inst, id, i0, j, sh);
   else
     c = read_ctrl(v.ctrl + (size_t)cur * v.ninst + inst);
-  arrived<NE>(ahead);
   if (is_done(c, v.t1)) return;
   if (S == 0 && !(c.rot & kJump)) return;
   const double h = step_h(v, c);
@@ -444,13 +509,13 @@ __global__ __launch_bounds__(256) void k_stage(V v, int cur) {
     if (!kAfter) own();
     float2 f[NE];
     if constexpr (S == 0)
-      stencil<NE, TD>(v, inst, InY{ybuf(v, c.rot, 0, inst)}, i0, jc, f, &ahead);
+      stencil<NE, TD>(v, inst, InY{ybuf(v, c.rot, 0, inst)}, i0, jc, f);
     else if constexpr (S == 6)
-      stencil<NE, TD>(v, inst, InY{ybuf(v, c.rot, 1, inst)}, i0, jc, f, &ahead);
+      stencil<NE, TD>(v, inst, InY{ybuf(v, c.rot, 1, inst)}, i0, jc, f);
     else if constexpr (S == 1)
-      stencil<NE, TD>(v, inst, InYK{ybuf(v, c.rot, 0, inst), kslot(v, 0, c.rot, inst), h * rk.A[1][0]}, i0, jc, f, &ahead);
+      stencil<NE, TD>(v, inst, InYK{ybuf(v, c.rot, 0, inst), kslot(v, 0, c.rot, inst), h * rk.A[1][0]}, i0, jc, f);
     else
-      stencil<NE, TD>(v, inst, InF{ysbuf(v, S & 1, inst)}, i0, jc, f, &ahead);
+      stencil<NE, TD>(v, inst, InF{ysbuf(v, S & 1, inst)}, i0, jc, f);
     if (kAfter) {
       // the loads stay behind the stencil
       asm volatile("" ::: "memory");
@@ -468,9 +533,10 @@ __global__ __launch_bounds__(256) void k_stage(V v, int cur) {
         ks[e] = f[m];
       if constexpr (S >= 1 && S <= 5) {
         double2 d = yv[m];
+        if (S < 5) d = add(d, h * rk.A[S + 1][S], f[m]);
 #pragma unroll
         for (int q = 0; q < S; ++q) d = add(d, h * rk.A[S + 1][q], kq[q][m]);
-        d = add(d, h * rk.A[S + 1][S], f[m]);
+        if (S == 5) d = add(d, h * rk.A[S + 1][S], f[m]);  // the candidate
         if constexpr (S == 5)
           put(v, ybuf(v, c.rot, 1, inst), i, j, d);
         else
@@ -523,26 +589,26 @@ __global__ __launch_bounds__(256) void k_count(V v) {
 }
 
 // ------------------------------------------------------------- initial step
-// The list of shifts, the vector of ones, and the flag that k_init sets.
+// The jump operators' terms, the first `most` of them written to list; returns how many there are.
+__host__ __device__ inline int list_terms(const dqh_dia_ops &ops, int64_t n, const float2 *zeros, Term *list, int most) {
+  int m = 0;
+  for (int s = 1; s < ops.nops; ++s) {
+    const float2 *A = (const float2 *)ops.diags[s];
+    for (int u = 0; u < ops.noff[s]; ++u)
+      for (int w = 0; w < ops.noff[s]; ++w, ++m)
+        if (m < most)
+          list[m] = Term{w + 1 < ops.noff[s] ? zeros : A + (size_t)u * n, A + (size_t)w * n, ops.off[s][u], ops.off[s][w],
+                         w > 0 ? 1.f : 0.f, 0};
+  }
+  return m;
+}
+
+// The list of terms, the vector of zeros, and the flag that k_init sets.
 __global__ __launch_bounds__(256) void k_setup(V v, dqh_dia_ops ops) {
-  for (int64_t e = threadIdx.x; e < v.n; e += 256) v.ones[e] = make_float2(1.f, 0.f);
+  for (int64_t e = threadIdx.x; e < v.n; e += 256) v.zeros[e] = make_float2(0.f, 0.f);
   if (threadIdx.x != 0) return;
   *v.flag = 0;
-  int m = 0;
-  const int td = v.hcur != nullptr;
-  const float2 *D0 = td ? v.hcur : diat::cgp<float2>(ops.diags[0]);
-  for (int u = 0; u < ops.noff[0]; ++u) {
-    const float2 *d = D0 + (size_t)u * v.n;
-    const int p = ops.off[0][u];
-    v.terms[m++] = Term{d, v.ones, p, 0, td, 0};
-    v.terms[m++] = Term{v.ones, d, 0, p, 0, td};
-  }
-  for (int s = 1; s < ops.nops; ++s) {
-    const float2 *A = diat::cgp<float2>(ops.diags[s]);
-    for (int u = 0; u < ops.noff[s]; ++u)
-      for (int w = 0; w < ops.noff[s]; ++w)
-        v.terms[m++] = Term{A + (size_t)u * v.n, A + (size_t)w * v.n, ops.off[s][u], ops.off[s][w], 0, 0};
-  }
+  list_terms(ops, v.n, v.zeros, v.terms, kMaxTerm);
 }
 
 // Control block and the saves at tsave <= t0; sets the flag where rho0 is not Hermitian.
@@ -746,7 +812,7 @@ __global__ __launch_bounds__(256) void k_finish(V v) {
 }
 
 struct Layout {
-  size_t k, ys, y2, terms, ones, part, ctrl, flag, total;
+  size_t k, ys, y2, terms, zeros, part, ctrl, flag, total;
   int64_t npart;
 };
 
@@ -761,8 +827,8 @@ inline Layout layout(int64_t n, int64_t ninst) {
   L.ys = L.k + align256(7 * (size_t)ninst * nn * sizeof(float2));
   L.y2 = L.ys + align256(2 * (size_t)ninst * nn * sizeof(float2));
   L.terms = L.y2 + align256((size_t)ninst * nn * sizeof(double2));
-  L.ones = L.terms + align256(kMaxTerm * sizeof(Term));
-  L.part = L.ones + align256((size_t)n * sizeof(float2));
+  L.zeros = L.terms + align256(kMaxTerm * sizeof(Term));
+  L.part = L.zeros + align256((size_t)n * sizeof(float2));
   L.ctrl = L.part + align256((size_t)ninst * 2 * L.npart * sizeof(double));
   L.flag = L.ctrl + align256(2 * (size_t)ninst * sizeof(Ctrl));
   L.total = L.flag + 256;
@@ -992,7 +1058,7 @@ extern "C" int dqh_mesolve_tsit5_dia(const dqh_dia_tsit5 *pb, void *stream) {
   v.ys = reinterpret_cast<float2 *>(w + L.ys);
   v.y2 = reinterpret_cast<double2 *>(w + L.y2);
   v.terms = reinterpret_cast<diats::Term *>(w + L.terms);
-  v.ones = reinterpret_cast<float2 *>(w + L.ones);
+  v.zeros = reinterpret_cast<float2 *>(w + L.zeros);
   v.npart = L.npart;
   v.part = reinterpret_cast<double *>(w + L.part);
   v.ctrl = reinterpret_cast<diats::Ctrl *>(w + L.ctrl);
@@ -1015,14 +1081,15 @@ extern "C" int dqh_mesolve_tsit5_dia(const dqh_dia_tsit5 *pb, void *stream) {
   v.H0 = reinterpret_cast<const float2 *>(p.ops.diags[0]);
   v.Hterms = td ? reinterpret_cast<const float2 *>(p.Hterms) : nullptr;
   v.hcur = td ? reinterpret_cast<float2 *>(p.hcur) : nullptr;
-  v.nterm = 2 * p.ops.noff[0];
+  v.npair = p.ops.noff[0];
+  for (int u = 0; u < DQH_DIA_MAXOFF; ++u) v.off[u] = u < v.npair ? p.ops.off[0][u] : 0;
+  for (int x = 0; x < diats::kHead; ++x) v.head[x] = diats::Term{};
+  v.nterm = diats::list_terms(p.ops, p.n, v.zeros, v.head, diats::kHead);
   v.spread = 0;  // largest p - q of a shift (p, q)
   for (int u = 0; u < p.ops.noff[0]; ++u) v.spread = std::max(v.spread, std::abs(p.ops.off[0][u]));
-  for (int k = 1; k < p.ops.nops; ++k) {
-    v.nterm += p.ops.noff[k] * p.ops.noff[k];
+  for (int k = 1; k < p.ops.nops; ++k)
     for (int u = 0; u < p.ops.noff[k]; ++u)
       for (int w = 0; w < p.ops.noff[k]; ++w) v.spread = std::max(v.spread, p.ops.off[k][u] - p.ops.off[k][w]);
-  }
   v.herm = v.nb = v.total = v.presum = 0;
   hipStream_t st = (hipStream_t)stream;
   // four rows per thread share the column factors and keep more loads in flight; they

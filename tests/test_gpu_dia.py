@@ -300,6 +300,95 @@ def test_dia_tsit5_any_offsets_and_states(n, hermitian):
         assert abs(int(out['nsteps'][b]) - st.nsteps) <= 2
 
 
+def _fma32(a, b, c):
+    """fmaf: the product of two FP32 numbers is exact in FP64."""
+    return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(np.float32)
+
+
+def _rounded_field(ops, X):
+    """The vector field of a Hermitian X in FP32 (re, im), with every product of complex numbers
+    rounded before it is added: r x per row factor, x conj(c) per column factor, the sum of
+    x conj(c) over a jump operator's column offsets before its row factor. ``ops``:
+    [(offsets, diagonals)], the generator first. The lower triangle mirrors the upper one."""
+    n = X.shape[-1]
+    pad = np.zeros((3 * n, 3 * n), dtype=np.complex64)
+    pad[n : 2 * n, n : 2 * n] = X
+    fr, fi = np.zeros((n, n), np.float32), np.zeros((n, n), np.float32)
+
+    def shifted(p, q):
+        x = pad[n + p : 2 * n + p, n + q : 2 * n + q]
+        return x.real.copy(), x.imag.copy()
+
+    def factor(d, p):  # the diagonal's element of each row: d[i + p], zero outside
+        out = np.zeros(n, dtype=np.complex64)
+        lo, hi = max(0, -p), min(n, n - p)
+        out[lo:hi] = d[lo + p : hi + p]
+        return out.real.copy(), out.imag.copy()
+
+    def times_row(r, zr, zi, jump=False):
+        rx, ry = r[0][:, None], r[1][:, None]
+        return _fma32(rx, zr, -(ry * zi)), _fma32(ry, zr, rx * zi) if jump else _fma32(rx, zi, ry * zr)
+
+    def times_col(c, xr, xi):
+        cx, cy = c[0][None, :], c[1][None, :]
+        return _fma32(xr, cx, xi * cy), _fma32(xi, cx, -(xr * cy))
+
+    offs, D = ops[0]
+    for p, d in zip(offs, D.astype(np.complex64)):
+        for t in (times_row(factor(d, p), *shifted(p, 0)), times_col(factor(d, p), *shifted(0, p))):
+            fr, fi = fr + t[0], fi + t[1]
+    for offs, D in ops[1:]:
+        D = D.astype(np.complex64)
+        for p, dp in zip(offs, D):
+            zr, zi = np.zeros((n, n), np.float32), np.zeros((n, n), np.float32)
+            for q, dq_ in zip(offs, D):
+                t = times_col(factor(dq_, q), *shifted(p, q))
+                zr, zi = zr + t[0], zi + t[1]
+            t = times_row(factor(dp, p), zr, zi, jump=True)
+            fr, fi = fr + t[0], fi + t[1]
+    f = np.triu(fr + 1j * fi, 1)
+    return f + f.conj().T + np.diag(np.diag(fr)).astype(np.complex64)
+
+
+@pytest.mark.parametrize('n, B', [(65, 2), (130, 2), (130, 125)])
+def test_dia_tsit5_rounding_of_one_step(n, B):
+    """One Tsit5 step over the whole interval, with one and four rows per thread, against the
+    same step on the host with the FP32 stages in the stated order of rounding. The saved
+    states are equal except where an FP64 sum in another order (1e-16 relative) crosses an
+    FP32 boundary: fewer than 1e-4 of the elements. (Products chained into the sum by fused
+    multiply-adds change about every second element.)"""
+    from dynamiqs_amd.integrators import dia
+    from oracle import tsit5
+
+    rng = np.random.default_rng(n)
+
+    def banded(offs):
+        return sum(np.diag(rng.normal(size=n - abs(o)) + 1j * rng.normal(size=n - abs(o)), o) for o in offs)
+
+    A = banded([0, 3, 17])
+    H, Ls = 0.3 * (A + A.conj().T), [0.3 * banded([-17, 2]), 0.3 * banded([1])]
+    X = rng.normal(size=(B, n, 3)) + 1j * rng.normal(size=(B, n, 3))
+    rho0 = X @ np.swapaxes(X.conj(), -1, -2)
+    rho0 = 0.5 * (rho0 + np.swapaxes(rho0.conj(), -1, -2))
+    rho0 /= np.linalg.norm(rho0, axis=(-2, -1), keepdims=True)
+    T = 0.25
+    plan = dia.tsit5_plan(H, Ls, rho0, np.array([0.0, T]), rtol=0.5, atol=0.5)
+    plan.run()
+    out = plan.results()
+    assert np.all(out['nsteps'] == 1)
+    Hnh = -1j * H - 0.5 * sum(L.conj().T @ L for L in Ls)
+    ops = [dia._dia_of(x) for x in (Hnh, *Ls)]
+    for b in (0, B - 1):
+        y, ks = rho0[b], []
+        for s in range(7):
+            v = y + sum((T * tsit5.A[s, q] * ks[q].astype(np.complex128) for q in range(s)), np.zeros_like(y))
+            ks.append(_rounded_field(ops, v.astype(np.complex64)))
+        assert np.linalg.norm(T * ks[0]) > 0.1  # the field's rounding shows in the state
+        y1 = y + sum(T * tsit5.B[q] * ks[q].astype(np.complex128) for q in range(7))
+        differ = np.mean(out['states'][b, 1] != y1.astype(np.complex64))
+        assert differ <= 1e-4, differ
+
+
 def test_dia_tsit5_graph_replays_equal_plain_launches():
     """The captured hipGraph (replayed many times, 4 steps each) and plain launches
     of the same kernels give bit-identical states and counters."""
