@@ -292,12 +292,14 @@ __global__ __launch_bounds__(NTH) void k_tsit5_diag(const dqh_me_inst *__restric
   };
 
   int par = 0;
-  // y + h sum_j w_j k_j at save index isave: states on both triangles, Tr(E rho) over the
-  // owned elements and their mirror images. One element at a time and formed anew for every
+  // y + h sum_j w_j k_j at save index isave (h = 0: the state itself, whatever the stages of
+  // a rejected step hold): states on both triangles, Tr(E rho) over the owned elements and
+  // their mirror images. One element at a time and formed anew for every
   // operator: kept, the values would not fit beside the stages.
   auto save = [&](double h, const double (&w)[7], int isave) {
     float2 *st = gp<float2>(p.states) + (size_t)isave * n * n;
     auto value = [&](int q) {
+      if (h == 0.0) return y[q];
       double re = 0.0, im = 0.0;
 #pragma unroll
       for (int j = 0; j < 7; ++j) {

@@ -469,13 +469,16 @@ __global__ __launch_bounds__(4 * NR) void k_sesolve_const(const dqh_me_inst *__r
     return make_float2(quad_sum(ar + br), quad_sum(ai + bi));
   };
   int vcur = 0;
-  // y + h sum_j w_j k_j (state and <psi|E|psi>) at save index isave
+  // y + h sum_j w_j k_j (state and <psi|E|psi>) at save index isave (h = 0: the state itself,
+  // whatever the stages of a rejected step hold)
   auto save = [&](double h, const double (&w)[7], int isave) {
     double re = 0.0, im = 0.0;
+    if (h != 0.0) {
 #pragma unroll
-    for (int j = 0; j < 7; ++j) {
-      re += w[j] * (double)k[j].x;
-      im += w[j] * (double)k[j].y;
+      for (int j = 0; j < 7; ++j) {
+        re += w[j] * (double)k[j].x;
+        im += w[j] * (double)k[j].y;
+      }
     }
     const double2 v = make_double2(y.x + h * re, y.y + h * im);
     if (save_states && one) gp<float2>(p.states)[(size_t)isave * n + i] = make_float2((float)v.x, (float)v.y);

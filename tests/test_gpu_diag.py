@@ -131,3 +131,28 @@ def test_mesolve_takes_dia_operators_there_and_stops_as_before():
     assert seen == [True, False, True, True]
     assert np.abs(r.expects - rd.expects).max() <= 1e-6 and r.states.shape == rd.states.shape
     assert np.linalg.norm(r.states.to_numpy() - rd.states.to_numpy()) <= 1e-6
+
+
+@pytest.mark.parametrize('n', [3, 40, 64, 70, 100])
+def test_saves_after_an_early_stop_are_the_state(n):
+    """A first attempt whose stages overflow FP32 (a coupling of 1e28 that the initial state
+    does not touch) is rejected and max_steps = 1 ends the solve there: the saves not reached
+    are the initial state, as final_state is, in every form of the kernel."""
+    from dynamiqs_amd import _native
+    from dynamiqs_amd.integrators import dense
+
+    H = np.zeros((n, n), dtype=np.complex128)
+    H[0, 1] = H[1, 0] = 1.0
+    H[1, 2] = H[2, 1] = 1e28
+    rho0 = np.zeros((n, n), dtype=np.complex128)
+    rho0[0, 0] = 1.0
+    E = np.diag(np.arange(1.0, n + 1)) + 0j
+    plan = dense.build_plan('tsit5', [dense.Instance(H=H, Ls=[np.diag(np.ones(n - 1), 1) + 0j], rho0=rho0)],
+                            np.linspace(0.0, 1.0, 4), exp_ops=[E], max_steps=1, dia_ops=True)
+    assert plan.stencil is not None
+    plan.run()
+    out = plan.results()
+    assert out['status'][0] == _native.STATUS_MAX_STEPS and out['nrejected'][0] == 1
+    assert np.array_equal(out['final_state'][0], rho0.astype(np.complex64))
+    assert np.array_equal(out['states'][0], np.broadcast_to(rho0.astype(np.complex64), (4, n, n)))
+    assert np.array_equal(out['expects'][0, 0], np.ones(4))

@@ -205,6 +205,30 @@ def test_constant_kernel_sizes(n, method):
     assert np.abs(res['expects'] - ex).max() <= 1e-6 * max(np.linalg.norm(E, 2) for E in Es)
 
 
+@pytest.mark.parametrize('n', [3, 40, 100])
+def test_constant_kernel_saves_after_an_early_stop_are_the_state(n):
+    """A first attempt whose stages overflow FP32 (a coupling of 1e28 that the initial state
+    does not touch) is rejected and max_steps = 1 ends the solve there: the saves not reached
+    are the initial state, as final_state is."""
+    from dynamiqs_amd import _native
+    from dynamiqs_amd.integrators.sesolve import SEInstance, build_plan
+
+    H = np.zeros((n, n), dtype=np.complex128)
+    H[0, 1] = H[1, 0] = 1.0
+    H[1, 2] = H[2, 1] = 1e28
+    psi = np.zeros(n, dtype=np.complex128)
+    psi[0] = 1.0
+    plan = build_plan([SEInstance(H=H, psi0=psi, key_H=(0,))], np.linspace(0.0, 1.0, 4),
+                      exp_ops=[np.diag(np.arange(1.0, n + 1)) + 0j], max_steps=1)
+    assert plan.constant
+    plan.run()
+    out = plan.results()
+    assert out['status'][0] == _native.STATUS_MAX_STEPS and out['nrejected'][0] == 1
+    assert np.array_equal(out['final_state'][0], psi.astype(np.complex64))
+    assert np.array_equal(out['states'][0], np.broadcast_to(psi.astype(np.complex64), (4, n)))
+    assert np.array_equal(out['expects'][0, 0], np.ones(4))
+
+
 def test_large_dimension_replay():
     """n = 200 (padded to 208, one row per thread): replay within 1e-5 (FP32
     products over 200-term rows) and the norm conserved to the same level."""
