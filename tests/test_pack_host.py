@@ -170,3 +170,26 @@ def test_grid_plan_carries_no_fp64_diagonal(host_device, monkeypatch):
     plan = dense.build_plan('tsit5', insts, np.array([0.0, 0.5, 1.0]), form='resident', grid_tsit5=True)
     assert plan.grid is not None and not plan.fp64_diag
     assert np.all(plan.descs['hdiag'] == 0)
+
+
+@pytest.mark.parametrize('N', [1, 2, 8, 9, 16, 17])
+def test_expm_generators_are_staged_alike_at_every_size(N):
+    """Small generators are staged by one array expression, larger ones in a loop: the same
+    bits as the product of every interval, for shared generators, unequal steps and a padded
+    size, and the scaling brings the largest 1-norm below THETA."""
+    from dynamiqs_amd.integrators import propagators as pr
+
+    rng = np.random.default_rng(N)
+    gens = [s * (rng.normal(size=(N, N)) + 1j * rng.normal(size=(N, N))) for s in (1.0, 30.0, 0.1)]
+    index = np.array([[0, 0, 1, 0], [2, 1, 2, 2]])
+    dts = np.array([0.1, 0.3, 0.2, 1.7])
+    X, s = pr.stage_generators(gens, index, dts)
+    norm = max(float(np.max(np.sum(np.abs(dts[k] * gens[index[b, k]]), axis=0))) for b in range(2) for k in range(4))
+    assert norm / 2.0**s <= pr.THETA and (s == 0 or norm / 2.0 ** (s - 1) > pr.THETA * (1 - 1e-12))
+    assert X.shape == (2, 4, pr.pad16(N), pr.pad16(N)) and X.dtype == np.complex64
+    assert not X[..., N:, :].any() and not X[..., :, N:].any()
+    for b in range(2):
+        for k in range(4):
+            assert np.array_equal(X[b, k, :N, :N], ((dts[k] * gens[index[b, k]]) / 2.0**s).astype(np.complex64))
+    with np.errstate(invalid='ignore'):
+        assert pr.stage_generators([np.full((N, N), np.nan)], np.zeros((1, 2), dtype=int), dts[:2])[1] == 0
