@@ -193,3 +193,11 @@ def test_expm_generators_are_staged_alike_at_every_size(N):
             assert np.array_equal(X[b, k, :N, :N], ((dts[k] * gens[index[b, k]]) / 2.0**s).astype(np.complex64))
     with np.errstate(invalid='ignore'):
         assert pr.stage_generators([np.full((N, N), np.nan)], np.zeros((1, 2), dtype=int), dts[:2])[1] == 0
+
+
+@pytest.mark.parametrize('count', [0, 7, (1 << 22) - 1, (1 << 22) + 3])
+def test_to_host_on_both_sides_of_its_line(count):
+    """float32 tensors up to and above 16 MB, and an empty one."""
+    t = torch.arange(count, dtype=torch.float32).reshape(1, -1)
+    out = dense.to_host(t)
+    assert out.dtype == np.float32 and out.shape == (1, count) and np.array_equal(out, t.numpy())
