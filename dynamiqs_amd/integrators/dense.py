@@ -557,18 +557,29 @@ def _rows_on(x: np.ndarray, offs, npad: int) -> np.ndarray:
 
 def _offsets(mask: np.ndarray) -> list:
     i, j = np.nonzero(mask)
-    return [int(o) for o in np.unique(j - i)]
+    n = mask.shape[-1]
+    return (np.flatnonzero(np.bincount(j - i + (n - 1))) - (n - 1)).tolist()
+
+
+def most_parts(n: int) -> int:
+    """Parts of the stencil (two per off-diagonal of the generator, one per pair of diagonals
+    of a jump operator) up to which the few-diagonal kernel takes a batch. Kernel times of the
+    stencil and of the dense form, one and 64 instances:
+    * constant operators, at most 12 shifts, from registers: n = 16, 10 parts, 26 steps 0.09
+      against 0.43 ms; n = 64, 10 parts, 18 steps, 32 instances 0.50 against 2.73;
+    * from LDS tables: n = 4, 12 parts with a modulated term, 41 steps 0.62 against 0.73;
+      n = 16, 14 parts, 40 steps 0.42 against 0.65 (modulated, 42 steps, 0.58 against 0.85);
+      n = 16, 25 parts, 44 steps 0.73 against 0.59; n = 20, 17 parts, 31 steps 0.41 against
+      1.21 (modulated 0.65 against 1.85); n = 32, 28 parts 0.41 against 0.60; n = 64, 41
+      parts 2.6 against 1.9;
+    * above n = 64 the dense form holds nothing in LDS: n = 90, 41 parts 2.4 against 15.4."""
+    return max(12, min(n, 24)) if n <= 64 else STENCIL_MAX_PARTS
 
 
 def few_diagonals(instances: list, npad: int) -> Stencil | None:
     """The :class:`Stencil` of a batch, or None where the few-diagonal kernel does not take
-    it: n above STENCIL_MAX_N, time-dependent jump operators, or more diagonals than pay.
-    The parts of the stencil are two per off-diagonal and one per pair of diagonals of a
-    jump operator. Up to 12 shifts run from registers, always faster (n = 64, 10 parts, 32
-    instances, 18 steps: 0.50 ms against 2.73 dense); beyond, the parts are read from LDS:
-    n = 16, 16 parts 0.25 against 0.27 ms, n = 32, 28 parts 0.41 against 0.60, n = 64, 41
-    parts 2.6 against 1.9. Above n = 64 the dense form holds nothing in LDS (n = 90, 41
-    parts: 2.4 against 15.4 ms)."""
+    it: n above STENCIL_MAX_N, time-dependent jump operators, or more diagonals than pay
+    (:func:`most_parts`)."""
     n = instances[0].H.shape[-1]
     K = len(instances[0].Ls)
     if n > STENCIL_MAX_N or K > 7:
@@ -604,18 +615,12 @@ def few_diagonals(instances: list, npad: int) -> Stencil | None:
     if not explicit.all():
         mask |= np.any(LdL != 0, axis=0)
 
-    def generators(offs):
-        rows = _rows_on(Hs, offs, npad)
-        plain = ~explicit
-        rows[plain] = -1j * rows[plain] - 0.5 * _rows_on(LdL, offs, npad)[il[first]][plain]
-        return rows
-
     for term in {id(o): o for i in instances for o in [p[2] for p in i.pwc] + [m[1] for m in i.mod]}.values():
         mask = mask | (np.asarray(term) != 0)
     offH = [o for o in _offsets(mask) if o != 0]
     offL = [_offsets(m) for m in np.any(Lall != 0, axis=0)] if K else []
     parts = 2 * len(offH) + sum(len(o) ** 2 for o in offL)
-    if parts > (max(12, min(n, 24)) if n <= 64 else STENCIL_MAX_PARTS) or len(offH) > 16:
+    if parts > most_parts(n) or len(offH) > 16:
         return None
     from .dia import DiaOps
 
@@ -625,8 +630,12 @@ def few_diagonals(instances: list, npad: int) -> Stencil | None:
         ops.noff[k] = len(offs)
         for u, o in enumerate(offs):
             ops.off[k][u] = o
+    G = _rows_on(Hs, [*offH, 0], npad)
+    plain = ~explicit
+    if plain.any():
+        G[plain] = -1j * G[plain] - 0.5 * _rows_on(LdL, [*offH, 0], npad)[il[first]][plain]
     L = [_rows_on(Lall[:, k], offs, npad) for k, offs in enumerate(offL)]
-    return Stencil(offH, offL, ops, generators(offH).astype(np.complex64), generators([0])[:, 0],
+    return Stencil(offH, offL, ops, G[:, :-1].astype(np.complex64), np.ascontiguousarray(G[:, -1]),
                    np.concatenate(L, axis=1).astype(np.complex64) if K else np.zeros((len(Lsets), 0, npad), np.complex64),
                    ig, il)
 
