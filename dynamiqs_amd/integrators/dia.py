@@ -656,9 +656,19 @@ def tsit5_plan(
     r64[:, :n, :n] = rho0
     y0 = torch.from_numpy(r64.view(np.float64)).to(dev)
     y = y0.clone()
-    work = torch.empty((int(lib.dqh_dia_tsit5_work_bytes(n_pad, B)),), dtype=torch.uint8, device=dev)
+
+    def large():
+        return (torch.empty((int(lib.dqh_dia_tsit5_work_bytes(n_pad, B)),), dtype=torch.uint8, device=dev),
+                torch.zeros((B * len(tsave) * n * n * 2,), dtype=torch.float32, device=dev))
+
+    try:
+        work, states = large()
+    except torch.OutOfMemoryError:
+        # the copy of rho0 for reset() stays on the host: 16 bytes per element, those of the
+        # second FP64 state in the workspace
+        y0 = torch.from_numpy(r64.view(np.float64))
+        work, states = large()
     ts_d = torch.from_numpy(tsave.copy()).to(dev)
-    states = torch.zeros((B * len(tsave) * n * n * 2,), dtype=torch.float32, device=dev)
     stats = torch.zeros((B, 8), dtype=torch.int64, device=dev)
     flags = torch.zeros((2,), dtype=torch.int64, pin_memory=True)
     nE = 0 if exp_ops is None else len(exp_ops)

@@ -389,6 +389,38 @@ def test_dia_tsit5_rounding_of_one_step(n, B):
         assert differ <= 1e-4, differ
 
 
+def test_dia_tsit5_plan_where_memory_is_short(monkeypatch):
+    """Where the workspace does not fit beside the device copy of rho0, that copy stays on the
+    host: the same solves, the first and after a reset."""
+    import torch
+
+    from dynamiqs_amd.integrators import dia
+    from oracle import operators as op
+
+    H, Ls, _ = _two_mode(8, 9)
+    rho0 = np.stack([op.coherent_dm((8, 9), (al, 0.0)) for al in (0.5, 1.2)])
+    tsave = np.linspace(0.0, 0.2, 3)
+    ref = dia.tsit5_plan(H, Ls, rho0, tsave)
+    ref.run()
+    empty, calls = torch.empty, []
+
+    def short(*args, **kw):
+        calls.append(args)
+        if len(calls) == 1:
+            raise torch.OutOfMemoryError('as if the device were full')
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, 'empty', short)
+    plan = dia.tsit5_plan(H, Ls, rho0, tsave)
+    monkeypatch.undo()
+    assert len(calls) == 2 and ref.y0.device.type == 'cuda' and plan.y0.device.type == 'cpu'
+    for _ in range(2):
+        plan.reset()
+        plan.run()
+        for k, v in plan.results().items():
+            assert np.array_equal(v, ref.results()[k]), k
+
+
 def test_dia_tsit5_graph_replays_equal_plain_launches():
     """The captured hipGraph (replayed many times, 4 steps each) and plain launches
     of the same kernels give bit-identical states and counters."""
