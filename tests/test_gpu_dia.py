@@ -240,18 +240,21 @@ def test_dia_rouchon1_diagonal_form(na, nb_, dt, hermitian):
         assert np.linalg.norm(out['final_state'][b] - rho) <= 4e-6
 
 
-@pytest.mark.parametrize('variant', ['tiled', 'global'])
-def test_dia_tsit5_matches_oracle(variant):
+@pytest.mark.parametrize('variant, batch', [('tiled', 2), ('global', 102)])
+def test_dia_tsit5_matches_oracle(variant, batch):
     """Adaptive Tsit5 on the DIA sweeps (n = 144, padded to 192) against the oracle's
     FP64 Tsit5 on the same problem and tolerances: states within 1e-5, identical
-    step counts up to a few steps (FP32 stages vs FP64 error estimate)."""
+    step counts up to a few steps (FP32 stages vs FP64 error estimate). 2 instances take one
+    row per thread, 102 (more than 2^21 elements) four; ``variant`` is checked, and every
+    form runs the same sweep."""
     from dynamiqs_amd.integrators import dia
     from oracle import mesolve as om
     from oracle import operators as op
 
     H, Ls, _ = _two_mode(12, 12)
     alphas = (0.5, 1.5)
-    rho0 = np.stack([op.coherent_dm((12, 12), (al, 0.0)) for al in alphas])
+    rho0 = np.stack([op.coherent_dm((12, 12), (al, 0.0)) for al in alphas])[np.arange(batch) % 2]
+    assert (rho0.size >= 1 << 21) == (batch > 2)
     tsave = np.linspace(0.0, 0.3, 7)
     v = {'tiled': dia.SWEEP_TILED, 'global': dia.SWEEP_GLOBAL}[variant]
     plan = dia.tsit5_plan(H, Ls, rho0, tsave, variant=v)
@@ -265,6 +268,7 @@ def test_dia_tsit5_matches_oracle(variant):
         nref = int(ref['infos']['nsteps'])
         assert abs(int(out['nsteps'][b]) - nref) <= max(2, nref // 20), (out['nsteps'][b], nref)
         assert abs(np.trace(out['final_state'][b]) - 1) < 1e-6
+        assert np.all(out['states'][b::2] == out['states'][b])  # instances of one rho0
 
 
 @pytest.mark.parametrize('n, hermitian', [(65, True), (130, True), (191, True), (65, False), (191, False)])
@@ -540,7 +544,7 @@ def test_dia_block_solve_panel_widths_agree():
     assert np.array_equal(outs[0]['states'], outs[1]['states'])
 
 
-@pytest.mark.parametrize('normalisation', ['banded', 'blocks'])
+@pytest.mark.parametrize('normalisation', ['banded', 'blocks', 'auto'])
 def test_dia_rouchon1_long_run_is_stable_and_matches_dense(normalisation):
     """5000 steps (T = 5, dt = 1e-3) of the 16 x 16 two-mode problem (n = 256): the
     state stays trace-preserving and Hermitian and agrees with the dense Rouchon1
