@@ -198,8 +198,9 @@ def bench_dia(args):
 
 
 def bench_dia_tsit5(args, H, Ls, rho0, tsave, variant):
-    """The same two-mode batch with adaptive Tsit5 on the DIA sweeps (rtol = atol =
-    1e-6): solves/s and the algorithmic bandwidth of its vector fields."""
+    """The same two-mode batch with adaptive Tsit5 on the DIA sweep (rtol = atol =
+    1e-6; ``variant`` is only checked there): solves/s and the algorithmic bandwidth of its
+    vector fields."""
     import torch
 
     from dynamiqs_amd.integrators import dia
@@ -1024,7 +1025,8 @@ def main(argv=None):
     ap.add_argument('--rates', type=float, nargs='+', default=[100.0, 400.0, 0.0])
     ap.add_argument('--budget-gb', type=float, default=32.0)
     ap.add_argument('--dia-T', type=float, default=5.0)
-    ap.add_argument('--dia-variant', default='auto', choices=['auto', 'global', 'tiled', 'split'])
+    ap.add_argument('--dia-variant', default='auto', choices=['auto', 'global', 'tiled', 'split'],
+                    help='sweep form of Rouchon1 (Tsit5 checks it and has one sweep)')
     ap.add_argument('--dia-method', default='rouchon1', choices=['rouchon1', 'tsit5'])
     ap.add_argument('--gpus', type=int, default=1)
     ap.add_argument('--steps', type=int, default=3)

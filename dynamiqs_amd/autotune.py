@@ -126,8 +126,8 @@ def dia_candidates(n_pad: int, maxoff: int) -> list[int]:
 
 def dia_sweep(H: np.ndarray, Ls, batch: int, kind: str = 'rhs', dt: float = 1e-3) -> int:
     """Fastest sweep form (a ``SWEEP_*`` value) for the DIA operators of (H, Ls):
-    ``kind`` 'rhs' times the Lindblad vector field (DIA Tsit5), 'kraus' times three
-    Rouchon1 steps of length ``dt``."""
+    ``kind`` 'rhs' times the Lindblad vector field (for ``dia.rhs_plan``; DIA Tsit5 has one
+    sweep and nothing to choose), 'kraus' times three Rouchon1 steps of length ``dt``."""
     from .integrators import dia
 
     if not enabled():

@@ -1092,9 +1092,9 @@ extern "C" int dqh_mesolve_tsit5_dia(const dqh_dia_tsit5 *pb, void *stream) {
       for (int w = 0; w < p.ops.noff[k]; ++w) v.spread = std::max(v.spread, p.ops.off[k][u] - p.ops.off[k][w]);
   v.herm = v.nb = v.total = v.presum = 0;
   hipStream_t st = (hipStream_t)stream;
-  // four rows per thread share the column factors and keep more loads in flight; they
-  // leave at least four waves per SIMD from 2^20 elements on. Below, one row per thread
-  // spreads the work over more CUs.
+  // four rows per thread share the column factors and keep more loads in flight; the upper
+  // triangle of 2^21 elements, 2^20, leaves them four waves per SIMD. Below, one row per
+  // thread spreads the work over more CUs.
   const bool large = (double)p.n_true * (double)p.n_true * (double)p.ninst >= (double)(1 << 21);
   if (td) return large ? drive<4, true>(p, v, st) : drive<1, true>(p, v, st);
   return large ? drive<4, false>(p, v, st) : drive<1, false>(p, v, st);

@@ -598,7 +598,9 @@ def tsit5_plan(
     nonzeros lie on few diagonals) and differ in rho0 (B, n, n). ``tableau='dopri5'``
     integrates with the Dopri5 pair instead. Time-dependent Hamiltonian terms, shared
     by the batch: ``pwc`` [(times, values (nv,), O)] (``dq.pwc``) and ``mod`` [(f, O)]
-    (``dq.modulated``, f(t) scalar), with O on few diagonals: H(t) = H + sum c_j(t) O_j."""
+    (``dq.modulated``, f(t) scalar), with O on few diagonals: H(t) = H + sum c_j(t) O_j.
+    ``variant`` is checked against the problem (SWEEP_SPLIT, and a tiled form that does not
+    admit its offsets, are refused); every form runs the same sweep."""
     import torch
 
     dev = _device()
