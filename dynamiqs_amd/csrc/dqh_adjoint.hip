@@ -10,6 +10,7 @@
 // workgroup per (instance, segment) accumulates its nodes in FP64; no atomics.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 
 #include "dqh.h"
@@ -328,15 +329,18 @@ extern "C" int dqh_adjoint_pwc_quadrature(int64_t ninst, int64_t n, int64_t nnod
 
 extern "C" int dqh_adjoint_lambda_nodes(int64_t ninst, int64_t nloss, int64_t nnodes, int64_t n, const void *bstates,
                                         const float *mask, void *lam, void *lambda0, void *stream) {
-  if (ninst <= 0 || ninst > 65535 || nloss <= 0 || nnodes <= 0 || n <= 0 || n > 1024 ||
+  if (ninst <= 0 || nloss <= 0 || nnodes <= 0 || n <= 0 || n > 1024 ||
       (nnodes + 1) * ((n * n + 4 * dqh::adj::kThreads - 1) / (4 * dqh::adj::kThreads)) > 0x7fffffff || !bstates || !mask || !lam || !lambda0)
     return dqh::fail(DQH_BAD_ARG, "dqh_adjoint_lambda_nodes: bad arguments");
   const int64_t nn = n * n;
-  hipLaunchKernelGGL(dqh::adj::k_lambda_nodes,
-                     dim3((unsigned)((nnodes + 1) * ((nn + 4 * dqh::adj::kThreads - 1) / (4 * dqh::adj::kThreads))), (unsigned)ninst),
-                     dim3(dqh::adj::kThreads), 0, (hipStream_t)stream, (int)nloss, (int)nnodes, nn,
-                     reinterpret_cast<const float2 *>(bstates), mask, reinterpret_cast<float2 *>(lam),
-                     reinterpret_cast<float2 *>(lambda0));
+  const float2 *b = reinterpret_cast<const float2 *>(bstates);
+  float2 *l = reinterpret_cast<float2 *>(lam), *l0 = reinterpret_cast<float2 *>(lambda0);
+  for (int64_t i = 0; i < ninst; i += 65535)  // instances of a grid
+    hipLaunchKernelGGL(dqh::adj::k_lambda_nodes,
+                       dim3((unsigned)((nnodes + 1) * ((nn + 4 * dqh::adj::kThreads - 1) / (4 * dqh::adj::kThreads))),
+                            (unsigned)std::min<int64_t>(ninst - i, 65535)),
+                       dim3(dqh::adj::kThreads), 0, (hipStream_t)stream, (int)nloss, (int)nnodes, nn,
+                       b + i * nloss * (nnodes + 2) * nn, mask, l + i * nnodes * nn, l0 + i * nn);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess)
     return dqh::fail(DQH_HIP_ERROR, std::string("dqh_adjoint_lambda_nodes: ") + hipGetErrorString(err));

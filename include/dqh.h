@@ -573,7 +573,7 @@ int dqh_adjoint_pwc_quadrature(int64_t ninst, int64_t n, int64_t nnodes, int64_t
  * (bstates: device c64[ninst][nloss][nnodes + 2][n][n], the start, the nodes in reversed
  * order and the end): lam[b][q] = sum_k mask[k][q] bstates[b][k][nnodes - q] (device
  * c64[ninst][nnodes][n][n]; mask: device float[nloss][nnodes]) and lambda0[b] = sum_k
- * bstates[b][k][nnodes + 1] (device c64[ninst][n][n]). ninst <= 65535, n <= 1024. */
+ * bstates[b][k][nnodes + 1] (device c64[ninst][n][n]). n <= 1024. */
 int dqh_adjoint_lambda_nodes(int64_t ninst, int64_t nloss, int64_t nnodes, int64_t n, const void *bstates,
                              const float *mask, void *lam, void *lambda0, void *stream);
 

@@ -253,3 +253,32 @@ def test_loss_over_several_times_and_modulated_parameter_vs_fd():
         fd_phi = (loss(u[b], ph=phi + hh) - loss(u[b], ph=phi - hh)) / (2 * hh)
         assert abs(res.grad_params[b, 0] - fd_theta) <= 1e-4 * max(1.0, abs(fd_theta)), (res.grad_params[b], fd_theta)
         assert abs(res.grad_params[b, 1] - fd_phi) <= 1e-4 * max(1.0, abs(fd_phi)), (res.grad_params[b], fd_phi)
+
+
+@pytest.mark.parametrize('B, K, Q, n', [(1, 1, 1, 1), (3, 2, 5, 32), (2, 3, 4, 33), (65536, 2, 3, 2), (131071, 1, 1, 1)])
+def test_lambda_nodes_equal_the_sum_over_the_losses(B, K, Q, n):
+    """The adjoint states at the nodes (in time order, masked per loss) and lambda0, at one
+    and several workgroups per state (n^2 = 1024 and 1089) and above 65535 instances, the
+    most of one grid. The same FP32 sums in the same order: equal."""
+    import ctypes
+
+    import torch
+
+    from dynamiqs_amd import _native
+
+    g = torch.Generator(device='cuda').manual_seed(n)
+    b = torch.randn((B, K, Q + 2, 2 * n * n), generator=g, device='cuda')
+    mask = (torch.rand((K, Q), generator=g, device='cuda') < 0.6).to(torch.float32)
+    lam = torch.full((B, Q, 2 * n * n), float('nan'), device='cuda')
+    lam0 = torch.full((B, 2 * n * n), float('nan'), device='cuda')
+    P = ctypes.c_void_p
+    _native.check(
+        _native.lib().dqh_adjoint_lambda_nodes(B, K, Q, n, P(b.data_ptr()), P(mask.data_ptr()), P(lam.data_ptr()),
+                                               P(lam0.data_ptr()), P(torch.cuda.current_stream().cuda_stream)),
+        'dqh_adjoint_lambda_nodes',
+    )
+    ref, ref0 = torch.zeros_like(lam), torch.zeros_like(lam0)
+    for k in range(K):
+        ref += torch.flip(b[:, k, 1 : 1 + Q], dims=[1]) * mask[k][None, :, None]
+        ref0 += b[:, k, 1 + Q]
+    assert torch.equal(lam, ref) and torch.equal(lam0, ref0)
