@@ -928,8 +928,8 @@ extern "C" int dqh_mesolve_rouchon1_dia(const dqh_dia_rouchon1 *pb, void *stream
   const dqh_dia_rouchon1 &p = *pb;
   if (p.nb != dia::kNB || p.n <= 0 || p.n % dia::kNB != 0 || p.ninst <= 0 || p.n_true > p.n)
     return fail(DQH_BAD_SHAPE, "dqh_mesolve_rouchon1_dia: n must be a positive multiple of 64 and nb == 64");
-  if (p.nE < 0 || (p.nE > 0 && (!p.EopsT || !p.expects)))
-    return fail(DQH_BAD_ARG, "dqh_mesolve_rouchon1_dia: nE > 0 needs EopsT and expects");
+  if (p.nE < 0 || (p.nE > 0 && (!p.EopsT || !p.expects || p.nsave < 1)))
+    return fail(DQH_BAD_ARG, "dqh_mesolve_rouchon1_dia: nE > 0 needs EopsT, expects and nsave >= 1");
   if (p.ops[0].nops < 1 || p.ops[0].nops > DQH_DIA_MAXOPS || p.nsets < 1 || p.nsets > 2)
     return fail(DQH_BAD_ARG, "dqh_mesolve_rouchon1_dia: bad operator description");
   for (int s = 0; s < p.nsets; ++s)

@@ -71,7 +71,7 @@ static __global__ __launch_bounds__(256) void k_expect_sum(int64_t nsave, int64_
   expects[(inst * nE + k) * nsave + s] = make_float2((float)sr, (float)si);
 }
 
-// scratch: device memory that is free by then
+// nsave, ninst, nE >= 1; scratch: device memory that is free by then
 static inline void launch_expect(int64_t n_true, int64_t nsave, int64_t ninst, int64_t nE, uint64_t states,
                                  uint64_t EopsT, uint64_t expects, void *scratch, size_t bytes, hipStream_t st) {
   const int64_t count = ninst * nsave * nE, fit = (int64_t)(bytes / sizeof(double2)) / count;

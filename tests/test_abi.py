@@ -37,6 +37,22 @@ def test_descriptor_layout_matches_mirror():
     assert names == list(_native.ME_INST_DTYPE.names)
 
 
+def test_rouchon1_expectations_without_saves_are_refused():
+    """Before any work, and without a division by the number of saves."""
+    from dynamiqs_amd import _native
+    from dynamiqs_amd.integrators.dia import DiaRouchon1
+
+    p = DiaRouchon1()
+    p.nb = p.n = p.n_true = 64
+    p.ninst = p.nsets = p.nE = 1
+    p.EopsT = p.expects = 16
+    p.ops[0].nops = p.ops[0].noff[0] = 1
+    for nsave in (0, -1):
+        p.nsave = nsave
+        assert _native.lib().dqh_mesolve_rouchon1_dia(ctypes.byref(p), None) == -1
+        assert b'nsave >= 1' in _native.lib().dqh_last_error()
+
+
 def test_no_fallback_when_library_missing(monkeypatch, tmp_path):
     import pytest
 
